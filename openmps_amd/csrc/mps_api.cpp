@@ -258,35 +258,25 @@ const std::vector<uint32_t>& storage_order(Context& c) {
 }
 
 void download_caller_order(Context& c, const void* dev, void* host, size_t elem) {
-  const size_t n = c.n;
-  if (n == 0) return;
-  if (c.order_serial == 0) {
-    MPS_HIP(hipMemcpyAsync(host, dev, n * elem, hipMemcpyDeviceToHost, c.stream));
-    MPS_HIP(hipStreamSynchronize(c.stream));
-    return;
+  double* d[kCallerFields] = {};
+  void* h[kCallerFields] = {};
+  void* src = const_cast<void*>(dev);
+  if (elem == 8) {
+    d[0] = static_cast<double*>(src);
+    h[0] = host;
   }
-  const std::vector<uint32_t>& o = storage_order(c);
-  std::vector<unsigned char> tmp(n * elem);
-  MPS_HIP(hipMemcpyAsync(tmp.data(), dev, n * elem, hipMemcpyDeviceToHost, c.stream));
-  MPS_HIP(hipStreamSynchronize(c.stream));
-  unsigned char* h = static_cast<unsigned char*>(host);
-  for (size_t k = 0; k < n; k++) std::memcpy(h + o[k] * elem, tmp.data() + k * elem, elem);
+  caller_order(c, true, d, h, elem == 8 ? nullptr : src, elem == 8 ? nullptr : host, static_cast<int>(elem));
 }
 
 void upload_caller_order(Context& c, const void* host, void* dev, size_t elem) {
-  const size_t n = c.n;
-  if (n == 0) return;
-  if (c.order_serial == 0) {
-    MPS_HIP(hipMemcpyAsync(dev, host, n * elem, hipMemcpyHostToDevice, c.stream));
-    MPS_HIP(hipStreamSynchronize(c.stream));
-    return;
+  double* d[kCallerFields] = {};
+  void* h[kCallerFields] = {};
+  void* src = const_cast<void*>(host);
+  if (elem == 8) {
+    d[0] = static_cast<double*>(dev);
+    h[0] = src;
   }
-  const std::vector<uint32_t>& o = storage_order(c);
-  std::vector<unsigned char> tmp(n * elem);
-  const unsigned char* h = static_cast<const unsigned char*>(host);
-  for (size_t k = 0; k < n; k++) std::memcpy(tmp.data() + k * elem, h + o[k] * elem, elem);
-  MPS_HIP(hipMemcpyAsync(dev, tmp.data(), n * elem, hipMemcpyHostToDevice, c.stream));
-  MPS_HIP(hipStreamSynchronize(c.stream));
+  caller_order(c, false, d, h, elem == 8 ? nullptr : dev, elem == 8 ? nullptr : src, static_cast<int>(elem));
 }
 
 void ensure_ppe_vectors(Context& c, size_t n) {
@@ -537,13 +527,9 @@ int mps_get_particles(mps_ctx* ctx, double* x, double* z, double* u, double* w, 
                       uint8_t* type) {
   return mps::guard(ctx, [&](Context& c) {
     if (c.n == 0) return;
-    if (x) mps::download_caller_order(c, c.x, x, 8);
-    if (z) mps::download_caller_order(c, c.z, z, 8);
-    if (u) mps::download_caller_order(c, c.u, u, 8);
-    if (w) mps::download_caller_order(c, c.w, w, 8);
-    if (p) mps::download_caller_order(c, c.p, p, 8);
-    if (n) mps::download_caller_order(c, c.nd, n, 8);
-    if (type) mps::download_caller_order(c, c.type, type, 1);
+    double* const dev[mps::kCallerFields] = {c.x, c.z, c.u, c.w, c.p, c.nd};
+    void* const host[mps::kCallerFields] = {x, z, u, w, p, n};
+    mps::caller_order(c, true, dev, host, c.type, type, 1);
   });
 }
 
@@ -555,13 +541,10 @@ int mps_set_particles(mps_ctx* ctx, const double* x, const double* z, const doub
     if (type)
       for (size_t k = 0; k < N; k++)
         if (type[k] > MPS_DISABLED) throw Failure{MPS_ERR_BAD_ARG, "particle type out of range"};
-    if (x) mps::upload_caller_order(c, x, c.x, 8);
-    if (z) mps::upload_caller_order(c, z, c.z, 8);
-    if (u) mps::upload_caller_order(c, u, c.u, 8);
-    if (w) mps::upload_caller_order(c, w, c.w, 8);
-    if (p) mps::upload_caller_order(c, p, c.p, 8);
-    if (n) mps::upload_caller_order(c, n, c.nd, 8);
-    if (type) mps::upload_caller_order(c, type, c.type, 1);
+    double* const dev[mps::kCallerFields] = {c.x, c.z, c.u, c.w, c.p, c.nd};
+    void* const host[mps::kCallerFields] = {const_cast<double*>(x), const_cast<double*>(z), const_cast<double*>(u),
+                                            const_cast<double*>(w), const_cast<double*>(p), const_cast<double*>(n)};
+    mps::caller_order(c, false, dev, host, c.type, const_cast<uint8_t*>(type), 1);
     c.ppe_from_particles = false;  // positions no longer those the system was assembled from
   });
 }

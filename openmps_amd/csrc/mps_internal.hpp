@@ -465,10 +465,17 @@ inline unsigned grid_for(size_t n, int block = kBlock) {
 // The caller's index of every stored particle (host copy of orig, refreshed
 // after a permutation; the stream is synchronised when it is refreshed).
 const std::vector<uint32_t>& storage_order(Context& c);
-// host[orig[k]] = dev[k] for the c.n particles (synchronous)
+// host[orig[k]] = dev[k] for the c.n particles (synchronous; elem 1, 4 or 8)
 void download_caller_order(Context& c, const void* dev, void* host, size_t elem);
-// dev[k] = host[orig[k]] for the c.n particles (synchronous)
+// dev[k] = host[orig[k]] for the c.n particles (synchronous; elem 1, 4 or 8)
 void upload_caller_order(Context& c, const void* host, void* dev, size_t elem);
+// Both for several arrays at once (mps_particles.hip; synchronous): out, host[m][orig[k]] =
+// dev[m][k] for every FP64 array m with host[m] and the small one of elem-byte
+// entries (1 or 4) if small_host; else dev[m][k] = host[m][orig[k]].  Uses the
+// permutation's spare arrays.
+constexpr int kCallerFields = 6;
+void caller_order(Context& c, bool out, double* const* dev, void* const* host, void* small_dev, void* small_host,
+                  int elem);
 
 // ---- stage entry points (defined in the .hip units) ------------------------------
 void search(Context& c);                 // mps_search.hip

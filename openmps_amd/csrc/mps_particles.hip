@@ -446,6 +446,49 @@ __global__ void __launch_bounds__(kBlock) k_apply_du(size_t n, double* __restric
   z[i] = z[i] + az * dt;
 }
 
+// The API's per-particle arrays between the caller's order and storage order:
+// caller[orig[k]] = store[k] (OUT) or store[k] = caller[orig[k]], up to
+// kCallerFields FP64 arrays and one of elem-byte entries (1 or 4) in one
+// launch; null pointers are skipped.  The host copies then move whole arrays.
+// (Permuted entry by entry on the host, the six arrays of 1.05M particles took
+// 12-13 ms in and 14-17 ms out; with this kernel 1.9 and 3-6.5 ms, nearly all
+// of it the pageable copies.)  The kernel is bound by the scattered side's
+// 8-byte accesses, which stay near each other because the cell order follows
+// the caller's order inside a cell.
+struct CallerMove {
+  size_t n;
+  const uint32_t* orig;
+  double* store[kCallerFields];
+  double* caller[kCallerFields];
+  void* small_store;
+  void* small_caller;
+  int elem;  // of the small array
+};
+template <bool OUT>
+__global__ void __launch_bounds__(kBlock) k_caller_order(CallerMove a) {
+  const size_t k = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
+  if (k >= a.n) return;
+  const uint32_t o = a.orig[k];
+#pragma unroll
+  for (int m = 0; m < kCallerFields; m++)
+    if (a.store[m]) {
+      if (OUT) a.caller[m][o] = a.store[m][k];
+      else a.store[m][k] = a.caller[m][o];
+    }
+  if (!a.small_store) return;
+  if (a.elem == 1) {
+    uint8_t* st = static_cast<uint8_t*>(a.small_store);
+    uint8_t* ca = static_cast<uint8_t*>(a.small_caller);
+    if (OUT) ca[o] = st[k];
+    else st[k] = ca[o];
+  } else {
+    uint32_t* st = static_cast<uint32_t*>(a.small_store);
+    uint32_t* ca = static_cast<uint32_t*>(a.small_caller);
+    if (OUT) ca[o] = st[k];
+    else st[k] = ca[o];
+  }
+}
+
 // max over particles of u.u ignoring NaN (DetermineDt, Computer.hpp:764-771).
 __global__ void __launch_bounds__(256) k_max_speed2(size_t n, const double* __restrict__ u,
                                                     const double* __restrict__ w,
@@ -613,6 +656,56 @@ void wall_targets_from_callback(Context& c) {
   }
   MPS_HIP(hipMemcpyAsync(c.wall_x, wx.data(), n * 8, hipMemcpyHostToDevice, c.stream));
   MPS_HIP(hipMemcpyAsync(c.wall_z, wz.data(), n * 8, hipMemcpyHostToDevice, c.stream));
+  MPS_HIP(hipStreamSynchronize(c.stream));
+}
+
+void caller_order(Context& c, bool out, double* const* dev, void* const* host, void* small_dev, void* small_host,
+                  int elem) {
+  const size_t n = c.n;
+  if (n == 0) return;
+  // the copies alone would run from a thread on any device; the launch needs this one
+  struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int dev) {
+      int now = dev;
+      if (hipGetDevice(&now) == hipSuccess && now != dev && hipSetDevice(dev) == hipSuccess) prev = now;
+    }
+    ~OnDevice() {
+      if (prev >= 0) (void)hipSetDevice(prev);
+    }
+  } on(c.device);
+  // the spares are free between permutations: the caller-ordered copies
+  const bool moved = c.order_serial != 0;
+  CallerMove a{};
+  a.n = n;
+  a.orig = c.orig;
+  a.elem = elem;
+  for (int m = 0; m < kCallerFields; m++)
+    if (host[m]) {
+      a.store[m] = dev[m];
+      a.caller[m] = moved ? c.spare_d[m] : dev[m];
+    }
+  if (small_host) {
+    a.small_store = small_dev;
+    a.small_caller = !moved ? small_dev : (elem == 1 ? static_cast<void*>(c.spare_type) : static_cast<void*>(c.spare_key));
+  }
+  auto copies = [&] {
+    for (int m = 0; m < kCallerFields; m++)
+      if (host[m])
+        MPS_HIP(hipMemcpyAsync(out ? host[m] : a.caller[m], out ? a.caller[m] : host[m], n * 8,
+                               out ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, c.stream));
+    if (small_host)
+      MPS_HIP(hipMemcpyAsync(out ? small_host : a.small_caller, out ? a.small_caller : small_host,
+                             n * static_cast<size_t>(elem), out ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice,
+                             c.stream));
+  };
+  if (!out) copies();
+  if (moved) {
+    if (out) hipLaunchKernelGGL(k_caller_order<true>, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, a);
+    else hipLaunchKernelGGL(k_caller_order<false>, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, a);
+    check_launch();
+  }
+  if (out) copies();
   MPS_HIP(hipStreamSynchronize(c.stream));
 }
 
