@@ -357,8 +357,8 @@ int mps_device_copy_probe(size_t bytes, double* ms_out);
  * work runs on `stream` (a hipStream_t; NULL: the default stream) of `device`,
  * and the call returns once it has finished.  Allocates nothing: r, p, q, the
  * partial sums and the status live in a fixed array of the library that each
- * device keeps until the process ends (3 MPS_NOALLOC_MAX_ROWS + 3072 doubles,
- * 24 MiB), so n <= MPS_NOALLOC_MAX_ROWS (MPS_ERR_BAD_ARG above, with the
+ * device keeps until the process ends (3 MPS_NOALLOC_MAX_ROWS + 20 k doubles,
+ * 24.2 MiB), so n <= MPS_NOALLOC_MAX_ROWS (MPS_ERR_BAD_ARG above, with the
  * message in err).  Every call on a device shares that array: calls that
  * overlap on one device race.  `err` (may be NULL) receives the message of a
  * failed call; `iterations` (may be NULL) the CG iterations.  Returns

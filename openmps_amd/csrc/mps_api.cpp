@@ -140,6 +140,7 @@ void free_all(Context& c) {
   dfree(c.ml_flag); dfree(c.ml_off); dfree(c.ml_list); dfree(c.ml_active); dfree(c.st_replay);
   dfree(c.ml_pid); dfree(c.ml_dv); dfree(c.ml_sc); dfree(c.zrec);
   dfree(c.amg_S64); dfree(c.amg_S); dfree(c.amg_dinv); dfree(c.amg_r); dfree(c.amg_x); dfree(c.amg_e);
+  dfree(c.res_ctl);
   dfree(c.amg_inv); dfree(c.amg_rows); dfree(c.box_part); dfree(c.amg_q9); dfree(c.amg_tq);
   if (c.flags_host) (void)hipHostFree(c.flags_host);
   if (c.nbr_total_host) (void)hipHostFree(c.nbr_total_host);
@@ -149,6 +150,7 @@ void free_all(Context& c) {
   if (c.st_host) (void)hipHostFree(c.st_host);
   if (c.st32_host) (void)hipHostFree(c.st32_host);
   if (c.ir_host) (void)hipHostFree(c.ir_host);
+  if (c.res_host) (void)hipHostFree(c.res_host);
   for (auto& e : c.events) {
     (void)hipEventDestroy(e.a);
     (void)hipEventDestroy(e.b);
@@ -412,6 +414,7 @@ int mps_create(const mps_env* env, double allowable_residual, int device, mps_ct
     mps::pinned(c.st_host, 1);
     mps::pinned(c.st32_host, 1);
     mps::pinned(c.ir_host, 1);
+    mps::pinned(c.res_host, 2);
     MPS_HIP(hipEventCreate(&c.solve_a));
     MPS_HIP(hipEventCreate(&c.solve_b));
   } catch (Failure& f) {

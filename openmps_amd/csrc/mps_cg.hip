@@ -21,6 +21,7 @@
 // lane.  These kernels use explicit FMA: the CG is checked against the
 // tolerance, not bit for bit.
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdio>
@@ -31,6 +32,7 @@
 
 #include "mps_device.hpp"
 #include "mps_internal.hpp"
+#include "mps_resident.hpp"
 
 namespace mps {
 namespace {
@@ -571,6 +573,316 @@ __global__ void __launch_bounds__(NT) k_cg_check(const double* __restrict__ part
       st->converged = 1;
       st->iterations = it - 1;
     }
+  }
+}
+
+// ---- the FP64 CG with resident workgroups ----
+//
+// The iterations of k_cg_spmv / k_cg_update in one launch, for systems whose
+// rows fit one per thread of the workgroups that the chip holds at once: each
+// thread keeps x, r, p, q and its row's first REG matrix entries in registers,
+// the next entries (10 bytes each) in LDS as far as it goes, and streams the
+// rest.  A workgroup gathers r from an LDS copy of exactly the rows its columns
+// name, reloaded every iteration (cell-ordered rows couple to three short
+// ranges of rows, far apart: copying the whole span took 2 us more per
+// iteration at 131k rows).  Two exchanges per iteration (p.q, then r with
+// r.r).  Every value and every sum is computed in the order of the launched
+// kernels, so the two agree bit for bit.  REG = 32 (170 VGPRs) with one
+// workgroup per compute unit, 20 (128 VGPRs) with two.
+//
+// It is bound by the two exchanges (1.8 us each for 5 workgroups, 2.8 for 256)
+// and the round trip of the gather; launched, by the two launches and, from
+// 100k rows on, by the matrix streams.  Per iteration (dam breaks, 28 entries a
+// row; launched -> resident): 1.5k rows 12.0 -> 4.7 us, 12k 13.0 -> 5.9, 50k
+// 13.7 -> 6.9, 131k 17.9 -> 9.8, 191k 24.0 -> 13.6, 257k 26.5 -> 16.0.
+__global__ void __launch_bounds__(NT) k_resident_clear(ResidentCtl* ctl, CgStatus* st) {
+  resident_clear(ctl);
+  if (threadIdx.x == 0) *st = CgStatus{};
+}
+
+// The entries of row i in stored order: count, column and value of entry k,
+// and the sum's starting value.
+template <class T>
+struct SellRow {
+  const Sell<T>& A;
+  size_t i, base;
+  uint32_t m;
+  __device__ __forceinline__ SellRow(const Sell<T>& a, size_t row, bool in)
+      : A(a), i(row), base(in ? a.off[row >> 6] + (row & 63) : 0), m(in ? a.width[row >> 6] : 0u) {}
+  __device__ __forceinline__ uint32_t col(uint32_t k) const { return sell_col(A, i, base + 64ull * k); }
+  __device__ __forceinline__ T val(uint32_t k) const { return A.val[base + 64ull * k]; }
+  __device__ __forceinline__ T diag() const { return A.diag[i]; }
+};
+struct CsrRow {
+  const Csr& A;
+  uint64_t lo;
+  uint32_t m;
+  __device__ __forceinline__ CsrRow(const Csr& a, size_t row, bool in)
+      : A(a), lo(in ? a.rowptr[row] : 0), m(in ? static_cast<uint32_t>(a.rowptr[row + 1] - lo) : 0u) {}
+  __device__ __forceinline__ uint32_t col(uint32_t k) const { return A.col[lo + k]; }
+  __device__ __forceinline__ double val(uint32_t k) const { return A.val[lo + k]; }
+  __device__ __forceinline__ double diag() const { return 0.0; }
+};
+__device__ __forceinline__ SellRow<double> row_of(const Sell<double>& A, size_t i, bool in) { return {A, i, in}; }
+__device__ __forceinline__ CsrRow row_of(const Csr& A, size_t i, bool in) { return {A, i, in}; }
+
+// Smallest and largest value over the block (every thread contributes).
+__device__ __forceinline__ void block_range(uint32_t& lo, uint32_t& hi) {
+  __shared__ uint32_t s[2 * (NT / 64)];
+  lo = wave_min_u32(lo);
+  hi = wave_max_u32(hi);
+  if ((threadIdx.x & 63) == 0) {
+    s[threadIdx.x >> 6] = lo;
+    s[NT / 64 + (threadIdx.x >> 6)] = hi;
+  }
+  __syncthreads();
+  for (int k = 0; k < NT / 64; k++) {
+    lo = min(lo, s[k]);
+    hi = max(hi, s[NT / 64 + k]);
+  }
+  __syncthreads();
+}
+
+// A value that is the same in every lane, kept in scalar registers.
+__device__ __forceinline__ double scalar_of(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readfirstlane(static_cast<int>(b));
+  const int hi = __builtin_amdgcn_readfirstlane(static_cast<int>(b >> 32));
+  return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// The rows a workgroup gathers, numbered without gaps: `mark` a bit per row
+// of its range, `base` the marked rows before each 32-bit word.
+constexpr uint32_t kResRange = 65536;  // rows its columns may span (16-bit local numbers)
+constexpr uint32_t kResWords = kResRange / 32;
+struct Gathered {
+  uint32_t* mark;
+  uint16_t* base;
+  __device__ __forceinline__ void set(uint32_t j) const { atomicOr(&mark[j >> 5], 1u << (j & 31u)); }
+  __device__ __forceinline__ uint32_t at(uint32_t j) const {
+    return base[j >> 5] + __popc(mark[j >> 5] & ((1u << (j & 31u)) - 1u));
+  }
+};
+// base from mark; returns the number of marked rows (block-uniform)
+__device__ __forceinline__ uint32_t number_marked(const Gathered& g) {
+  __shared__ uint32_t s[NT / 64];
+  constexpr int PER = kResWords / NT;
+  const uint32_t w0 = threadIdx.x * PER;
+  uint32_t mine = 0;
+#pragma unroll
+  for (int u = 0; u < PER; u++) mine += __popc(g.mark[w0 + u]);
+  uint32_t inc = mine;
+  const uint32_t lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(inc, o, 64);
+    if (lane >= static_cast<uint32_t>(o)) inc += t;
+  }
+  if (lane == 63) s[threadIdx.x >> 6] = inc;
+  __syncthreads();
+  uint32_t before = inc - mine, total = 0;
+  for (uint32_t k = 0; k < NT / 64; k++) {
+    if (k < (threadIdx.x >> 6)) before += s[k];
+    total += s[k];
+  }
+  // (numbers past 16 bits: the caller refuses such a total)
+#pragma unroll
+  for (int u = 0; u < PER; u++) {
+    g.base[w0 + u] = static_cast<uint16_t>(before);
+    before += __popc(g.mark[w0 + u]);
+  }
+  __syncthreads();
+  return total;
+}
+
+// The sum of the workgroups' partial sums of generation gen, in the order in
+// which block_sum<NT> adds one per thread; up to 64 of them by one wavefront.
+__device__ __forceinline__ double resident_sum(ResidentCtl* ctl, unsigned gen, unsigned idx, unsigned G, double* lds,
+                                               bool& ok) {
+  double v = 0.0;
+  if (threadIdx.x < 64 || G > 64) v = resident_poll(ctl, gen, G, ok);
+  if (G <= 64) {
+    v = wave_sum(v);
+    if (threadIdx.x == 0) lds[0] = v;
+    ok = __syncthreads_and(ok) != 0;
+    resident_empty(ctl, gen, idx);
+    v = lds[0];
+    __syncthreads();
+  } else {
+    ok = __syncthreads_and(ok) != 0;
+    resident_empty(ctl, gen, idx);
+    v = block_sum<NT>(v, lds);
+  }
+  return scalar_of(v);
+}
+
+// Dynamic LDS (bytes): first the gathered r (before the iterations, the marks
+// and their numbers), then the gathered rows' list and the matrix entries from
+// REG on that fit.
+template <class M, int REG, int WAVES>
+__global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restrict__ x, double* r,
+                                                           double* __restrict__ p, double* __restrict__ q,
+                                                           const double* __restrict__ part_rr,
+                                                           const double* __restrict__ part_bb, CgStatus* st,
+                                                           StopRule sr, long long max_iter, ResidentCtl* ctl,
+                                                           uint32_t bytes) {
+  extern __shared__ double win[];
+  __shared__ double lds[NT / 64];
+  const unsigned G = gridDim.x, idx = blockIdx.x;
+  const Rows rw = block_rows(A.n, A.rpb);
+  const size_t i = rw.lo + threadIdx.x;
+  const bool in = i < rw.hi;
+  const auto row = row_of(A, i, in);
+  const uint32_t m = row.m;
+  uint32_t lo = in ? static_cast<uint32_t>(i) : 0xffffffffu, hi = in ? static_cast<uint32_t>(i) : 0u;
+  for (uint32_t k = 0; k < m; k++) {
+    const uint32_t j = row.col(k);
+    lo = min(lo, j);
+    hi = max(hi, j);
+  }
+  block_range(lo, hi);
+  const bool narrow = hi - lo < kResRange;
+  const Gathered ga{reinterpret_cast<uint32_t*>(win), reinterpret_cast<uint16_t*>(win) + 2 * kResWords};
+  constexpr uint32_t kMarkBytes = 6 * kResWords;
+  for (uint32_t k = threadIdx.x; k < kResWords; k += NT) ga.mark[k] = 0u;
+  __syncthreads();
+  // the row's first entries: values, and columns as 16-bit numbers from lo, two a register
+  double a[REG];
+  uint32_t off[REG / 2];
+  if (narrow && in) ga.set(static_cast<uint32_t>(i) - lo);
+#pragma unroll
+  for (int k = 0; k < REG; k++) {
+    a[k] = 0.0;
+    uint32_t d = in ? (static_cast<uint32_t>(i) - lo) & 0xffffu : 0u;  // past the row's end: its own r, value 0
+    if (static_cast<uint32_t>(k) < m) {
+      a[k] = row.val(k);
+      if (narrow) {
+        d = row.col(k) - lo;
+        ga.set(d);
+      }
+    }
+    if (k & 1) off[k >> 1] |= d << 16;
+    else off[k >> 1] = d;
+  }
+  if (narrow)
+    for (uint32_t k = REG; k < m; k++) ga.set(row.col(k) - lo);
+  __syncthreads();
+  const uint32_t wn = number_marked(ga);
+  // LDS behind the gathered r: the list of its rows, entries of the matrix
+  const uint32_t list_at = max(wn * 8u, kMarkBytes), mat_at = (list_at + 2 * wn + 15u) & ~15u;
+  const bool ok_lds = narrow && wn < kResRange && mat_at <= bytes;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(win) + list_at);
+  const uint32_t lrows = ok_lds ? min((bytes - mat_at) / (10u * NT), 64u) : 0u;
+  double* const lval = reinterpret_cast<double*>(reinterpret_cast<char*>(win) + mat_at);
+  uint16_t* const lcol = reinterpret_cast<uint16_t*>(lval + static_cast<size_t>(lrows) * NT);
+  const uint32_t own = (ok_lds && in) ? ga.at(static_cast<uint32_t>(i) - lo) : 0u;
+  const uint32_t kl = min(m, static_cast<uint32_t>(REG) + lrows);  // entries in registers and LDS
+  if (ok_lds) {
+#pragma unroll
+    for (int k = 0; k < REG / 2; k++)
+      off[k] = in ? (ga.at(off[k] & 0xffffu) | (ga.at(off[k] >> 16) << 16)) : 0u;
+    for (uint32_t k = REG; k < kl; k++) {
+      lval[(k - REG) * NT + threadIdx.x] = row.val(k);
+      lcol[(k - REG) * NT + threadIdx.x] = static_cast<uint16_t>(ga.at(row.col(k) - lo));
+    }
+    for (uint32_t w = threadIdx.x; w < kResWords; w += NT) {
+      uint32_t bits = ga.mark[w], at = ga.base[w];
+      for (; bits; bits &= bits - 1) list[at++] = static_cast<uint16_t>(32 * w + __ffs(bits) - 1);
+    }
+  }
+  const double dg = in ? row.diag() : 0.0;
+  double ri = in ? r[i] : 0.0, xi = in ? x[i] : 0.0, pi = 0.0, qi = 0.0;
+  double rr = scalar_of(block_sum<NT>(threadIdx.x < G ? part_rr[threadIdx.x] : 0.0, lds));
+  double rr_prev = 0.0, bb = 0.0, tol = 0.0;
+  if (sr.rule == MPS_STOP_RHS_NORM) bb = scalar_of(block_sum<NT>(threadIdx.x < G ? part_bb[threadIdx.x] : 0.0, lds));
+  const double rr0 = rr;
+  if (!resident_start(ctl, ok_lds)) return;
+  unsigned gen = 0;
+  long long it = 1;
+  bool conv = false, ok = true;
+  for (;; it++) {
+    if (it == 1) {
+      if (sr.rule == MPS_STOP_RHS_NORM) {
+        tol = (sr.tol * sr.tol) * bb;
+        conv = (rr <= tol);
+      } else {
+        tol = rr * sr.tol * sr.tol;  // residual0, Computer.hpp:1386
+        conv = (tol == 0);
+      }
+    } else {
+      conv = (sr.rule == MPS_STOP_RHS_NORM) ? (rr <= tol) : (rr < tol);  // :1408
+    }
+    if (conv || it > max_iter) break;
+    // r of the gathered rows (complete: r.r was collected)
+    for (uint32_t k0 = threadIdx.x; k0 < wn; k0 += 4 * NT) {
+      double t[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) t[u] = (k0 + u * NT < wn) ? agent_load(r + lo + list[k0 + u * NT]) : 0.0;
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+        if (k0 + u * NT < wn) win[k0 + u * NT] = t[u];
+    }
+    __syncthreads();
+    double s = dg * ri;
+#pragma unroll
+    for (int g = 0; g < REG / 4; g++)
+      if (static_cast<uint32_t>(4 * g) < m) {
+        // (opaque: unpacked per iteration, not kept unpacked across them)
+        uint32_t o0 = off[2 * g], o1 = off[2 * g + 1];
+        asm volatile("" : "+v"(o0), "+v"(o1));
+        const double x0 = win[o0 & 0xffffu], x1 = win[o0 >> 16], x2 = win[o1 & 0xffffu], x3 = win[o1 >> 16];
+        s = fma(a[4 * g], x0, s);
+        s = fma(a[4 * g + 1], x1, s);
+        s = fma(a[4 * g + 2], x2, s);
+        s = fma(a[4 * g + 3], x3, s);
+      }
+    for (uint32_t k = REG; k < kl; k++)
+      s = fma(lval[(k - REG) * NT + threadIdx.x], win[lcol[(k - REG) * NT + threadIdx.x]], s);
+    for (uint32_t k = kl; k < m; k++) s = fma(row.val(k), agent_load(r + row.col(k)), s);
+    if (it == 1) {
+      pi = ri;
+      qi = s;
+    } else {
+      const double beta = scalar_of(rr / rr_prev);
+      pi = fma(beta, pi, ri);
+      qi = fma(beta, qi, s);
+    }
+    const double sp = block_sum<NT>(in ? fma(pi, qi, 0.0) : 0.0, lds);
+    if (threadIdx.x == 0) resident_publish(ctl, gen, idx, sp);
+    const double alpha = scalar_of(rr / resident_sum(ctl, gen, idx, G, lds, ok));
+    gen++;
+    if (!ok) return;
+    xi = fma(alpha, pi, xi);
+    ri = fma(-alpha, qi, ri);
+    if (in) agent_store(r + i, ri);
+    const double ww = wave_sum(in ? fma(ri, ri, 0.0) : 0.0);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = ww;
+    stores_done();  // every wavefront's r is out before the block publishes its r.r
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = lds[0];
+#pragma unroll
+      for (int k = 1; k < NT / 64; k++) t += lds[k];
+      resident_publish(ctl, gen, idx, t);
+    }
+    rr_prev = rr;
+    rr = resident_sum(ctl, gen, idx, G, lds, ok);
+    gen++;
+    if (!ok) return;
+  }
+  if (in) {
+    x[i] = xi;
+    p[i] = pi;
+    q[i] = qi;
+  }
+  if (lead()) {
+    st->rr[it & 1] = rr;
+    st->rr[(it & 1) ^ 1] = rr_prev;
+    st->tol = tol;
+    st->rr0 = rr0;
+    st->b2 = bb;
+    st->converged = conv ? 1 : 0;
+    st->iterations = it - 1;
   }
 }
 
@@ -2123,58 +2435,179 @@ double spmv_bytes(const Context& c, int vbytes, double extra_per_row) {
   return nnz * vbytes + cols + c.ppe_n * (vbytes + extra_per_row) + c.nslices * 13.0;
 }
 
-// Plain FP64 CG (the reference algorithm); x = c.sol holds the warm start.
-void solve_cg64(Context& c, const StopRule& sr, long long max_iter) {
-  const size_t n = c.ppe_n;
-  const Launch L = cg_grid(n);
-  const Sell<double> A = sell<double>(c, c.sval, c.diag, L.rpb);
-  MPS_HIP(hipMemsetAsync(c.st, 0, sizeof(CgStatus), c.stream));
-  c.replay_ready = MPS_K_CG_SPMV;
+// ---- resident solves (mps_resident.hpp) ----
+//
+// One resident solve at a time per device and process: two that each held
+// part of the compute units would wait for the rest until the start limit.
+// A solve that finds another one running takes the launched kernels.
+constexpr int kMaxDevices = 64;
+std::atomic<int> g_resident_busy[kMaxDevices];
+struct ResidentTurn {
+  int dev = -1;
+  explicit ResidentTurn(int d) {
+    int idle = 0;
+    if (d >= 0 && d < kMaxDevices && g_resident_busy[d].compare_exchange_strong(idle, 1)) dev = d;
+  }
+  ~ResidentTurn() {
+    if (dev >= 0) g_resident_busy[dev].store(0);
+  }
+  ResidentTurn(const ResidentTurn&) = delete;
+  ResidentTurn& operator=(const ResidentTurn&) = delete;
+  explicit operator bool() const { return dev >= 0; }
+};
+
+// Which systems: one row a thread (launch shapes up to 512k rows) and at most two
+// workgroups of 512 a compute unit, i.e. up to 262144 rows on 256 compute units:
+// with more the matrix no longer stays on the chip.  Up to there the resident
+// CG is the faster at every size measured (k_cg_resident).  Systems whose
+// workgroups span 65536 rows or more, or gather more rows than their LDS holds
+// (shuffled orders), are refused on the device.
+//
+// The dynamic LDS of a resident launch of `grid` workgroups of `kernel`, per_cu
+// of them on a compute unit (the more LDS the longer the range of rows a
+// workgroup may span), or 0 if the current device cannot hold them all at once.
+template <class K>
+size_t resident_lds(K kernel, int grid, int per_cu) {
+  int dev = 0, cus = 0;
+  if (grid > kResSlots || hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 0;
+  const size_t bytes = per_cu == 1 ? 144 * 1024 : 72 * 1024;
+  int fit = 0;
+  if ((grid + cus - 1) / cus > per_cu ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, kernel, NT, bytes) != hipSuccess || fit < per_cu) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return bytes;
+}
+
+// Launches the resident CG on stream s (r, the partial sums of r.r and b.b
+// from k_cg_init already enqueued; ctl and st cleared by it); false if it
+// cannot run.  The result is in st (ctl->abort: nothing was solved).
+template <class M>
+bool resident_cg_launch(const M& A, const Launch& L, double* x, double* r, double* p, double* q, const double* part_rr,
+                        const double* part_bb, CgStatus* st, const StopRule& sr, long long max_iter, ResidentCtl* ctl,
+                        hipStream_t s) {
+  if (L.rpb != static_cast<size_t>(NT)) return false;  // one row per thread
+  auto kernel = k_cg_resident<M, 32, 2>;
+  size_t lds = resident_lds(kernel, L.grid, 1);
+  if (lds == 0) {
+    kernel = k_cg_resident<M, 20, 4>;
+    lds = resident_lds(kernel, L.grid, 2);
+  }
+  if (lds == 0) return false;
+  hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, s, ctl, st);
+  hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(NT), lds, s, A, x, r, p, q, part_rr, part_bb, st, sr, max_iter, ctl,
+                     static_cast<uint32_t>(lds));
+  check_launch();
+  return true;
+}
+
+// The start of the FP64 CG: r = b - A x and the partial sums of r.r and b.b.
+void cg64_init(Context& c, const Sell<double>& A, const Launch& L) {
   tracked(c, MPS_K_CG_INIT, spmv_bytes(c, 8, 8.0 + 8 + 8), [&] {
     hipLaunchKernelGGL(k_cg_init<Sell<double>>, dim3(L.grid), dim3(NT), 0, c.stream, A, static_cast<const double*>(c.b),
                        static_cast<const double*>(c.sol), c.r, c.partB, c.partC);
   });
   check_launch();
-  long long it = 1;
+}
+
+// A refusal (a workgroup's columns span too many rows, or the workgroups did
+// not get onto the device together) is remembered for this many solves.
+constexpr int kResSkip = 64;
+
+// The FP64 CG with resident workgroups; false: the launched kernels have to
+// run (nothing was solved).  The FP64 residual of the returned x rides on the
+// same synchronisation as the status.
+bool resident_cg64(Context& c, const Sell<double>& A, const Launch& L, const StopRule& sr, long long max_iter,
+                   double b_iter) {
+  if (c.ppe_col16 && c.mf_nnz_wide > 0) return false;  // columns beyond 16-bit offsets
+  if (c.res_skip > 0) {
+    c.res_skip--;
+    return false;
+  }
+  if (L.rpb != static_cast<size_t>(NT) || L.grid > kResSlots) return false;
+  ResidentTurn turn(c.device);
+  if (!turn) return false;
+  if (!c.res_ctl) c.res_ctl = dalloc<ResidentCtl>(1);
+  cg64_init(c, A, L);
+  bool launched = false;
+  tracked(c, MPS_K_CG_SPMV, 0.0, [&] {
+    launched = resident_cg_launch(A, L, c.sol, c.r, c.pa, c.q, static_cast<const double*>(c.partB),
+                                  static_cast<const double*>(c.partC), c.st, sr, max_iter, c.res_ctl, c.stream);
+  });
+  if (!launched) {
+    c.res_skip = kResSkip;
+    return false;
+  }
+  MPS_HIP(hipEventRecord(c.solve_b, c.stream));
+  residual64_launch(c);
+  check_launch();
+  MPS_HIP(hipMemcpyAsync(c.res_host, c.res_ctl, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, c.stream));
+  MPS_HIP(hipMemcpyAsync(c.red_host, c.red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  read_status(c, c.st, c.st_host);
+  if (c.res_host[1]) {
+    c.res_skip = kResSkip;
+    return false;
+  }
+  add_bytes(c, MPS_K_CG_SPMV, b_iter * static_cast<double>(c.st_host->iterations));
+  c.solve_ended = true;
+  c.final_rr = c.red_host[0];
+  c.final_bb = c.red_host[1];
+  return true;
+}
+
+// Plain FP64 CG (the reference algorithm); x = c.sol holds the warm start.
+void solve_cg64(Context& c, const StopRule& sr, long long max_iter) {
+  const size_t n = c.ppe_n;
+  const Launch L = cg_grid(n);
+  const Sell<double> A = sell<double>(c, c.sval, c.diag, L.rpb);
+  c.replay_ready = MPS_K_CG_SPMV;
   // reads r (own row and gathered), reads and writes p and q (the diagonal
   // is in spmv_bytes)
   const double b_spmv = spmv_bytes(c, 8, 8.0 * 5);
   const double b_upd = c.ppe_n * 48.0;
-  while (true) {
-    const long long chunk = next_chunk(it - 1, c.last_iters);
-    for (long long m = 0; m < chunk && it <= max_iter; m++, it++) {
-      tracked(c, MPS_K_CG_SPMV, b_spmv, [&] {
-        if (it == 1)
-          hipLaunchKernelGGL((k_cg_spmv<true, Sell<double>>), dim3(L.grid), dim3(NT), 0, c.stream, A,
-                             static_cast<const double*>(c.r), c.pa, c.q,
-                             static_cast<const double*>(c.partB), static_cast<const double*>(c.partC),
-                             L.grid, c.partA, c.st, sr, it);
-        else
-          hipLaunchKernelGGL((k_cg_spmv<false, Sell<double>>), dim3(L.grid), dim3(NT), 0, c.stream, A,
-                             static_cast<const double*>(c.r), c.pa, c.q,
-                             static_cast<const double*>(c.partB), static_cast<const double*>(c.partC),
-                             L.grid, c.partA, c.st, sr, it);
-      }, it);
-      tracked(c, MPS_K_CG_UPDATE, b_upd, [&] {
-        hipLaunchKernelGGL(k_cg_update, dim3(L.grid), dim3(NT), 0, c.stream, n, L.rpb, c.sol, c.r,
-                           static_cast<const double*>(c.pa), static_cast<const double*>(c.q),
-                           static_cast<const double*>(c.partA), L.grid, c.partB, c.st, it);
-      }, it);
-    }
-    check_launch();
-    if (it > max_iter) {
-      hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, c.stream, static_cast<const double*>(c.partB),
-                         L.grid, c.st, sr, it);
+  if (!resident_cg64(c, A, L, sr, max_iter, b_spmv + b_upd)) {
+    MPS_HIP(hipMemsetAsync(c.st, 0, sizeof(CgStatus), c.stream));
+    cg64_init(c, A, L);
+    long long it = 1;
+    while (true) {
+      const long long chunk = next_chunk(it - 1, c.last_iters);
+      for (long long m = 0; m < chunk && it <= max_iter; m++, it++) {
+        tracked(c, MPS_K_CG_SPMV, b_spmv, [&] {
+          if (it == 1)
+            hipLaunchKernelGGL((k_cg_spmv<true, Sell<double>>), dim3(L.grid), dim3(NT), 0, c.stream, A,
+                               static_cast<const double*>(c.r), c.pa, c.q,
+                               static_cast<const double*>(c.partB), static_cast<const double*>(c.partC),
+                               L.grid, c.partA, c.st, sr, it);
+          else
+            hipLaunchKernelGGL((k_cg_spmv<false, Sell<double>>), dim3(L.grid), dim3(NT), 0, c.stream, A,
+                               static_cast<const double*>(c.r), c.pa, c.q,
+                               static_cast<const double*>(c.partB), static_cast<const double*>(c.partC),
+                               L.grid, c.partA, c.st, sr, it);
+        }, it);
+        tracked(c, MPS_K_CG_UPDATE, b_upd, [&] {
+          hipLaunchKernelGGL(k_cg_update, dim3(L.grid), dim3(NT), 0, c.stream, n, L.rpb, c.sol, c.r,
+                             static_cast<const double*>(c.pa), static_cast<const double*>(c.q),
+                             static_cast<const double*>(c.partA), L.grid, c.partB, c.st, it);
+        }, it);
+      }
       check_launch();
+      if (it > max_iter) {
+        hipLaunchKernelGGL(k_cg_check, dim3(1), dim3(NT), 0, c.stream, static_cast<const double*>(c.partB),
+                           L.grid, c.st, sr, it);
+        check_launch();
+        read_status(c, c.st, c.st_host);
+        break;
+      }
       read_status(c, c.st, c.st_host);
-      break;
+      if (c.st_host->converged) break;
     }
-    read_status(c, c.st, c.st_host);
-    if (c.st_host->converged) break;
+    const long long launched = std::min(it - 1, max_iter);
+    uncount(c, MPS_K_CG_SPMV, launched - c.st_host->iterations, b_spmv);
+    uncount(c, MPS_K_CG_UPDATE, launched - c.st_host->iterations, b_upd);
   }
-  const long long launched = std::min(it - 1, max_iter);
-  uncount(c, MPS_K_CG_SPMV, launched - c.st_host->iterations, b_spmv);
-  uncount(c, MPS_K_CG_UPDATE, launched - c.st_host->iterations, b_upd);
   c.stats.iterations = c.st_host->iterations;
   c.stats.outer_iterations = 1;
   c.stats.rr0 = c.st_host->rr0;
@@ -3583,6 +4016,7 @@ void ppe_solve(Context& c) {
   c.stats = mps_solve_stats{};
   c.replay_ready = 0;
   c.final_rr = -1;
+  c.solve_ended = false;
   c.learned_pending = false;
   if (n == 0) return;
   StopRule sr;
@@ -3611,7 +4045,7 @@ void ppe_solve(Context& c) {
     rc = f.code;
     msg = f.msg;
   }
-  MPS_HIP(hipEventRecord(c.solve_b, c.stream));
+  if (!c.solve_ended) MPS_HIP(hipEventRecord(c.solve_b, c.stream));
   c.solve_pending = true;
   c.solve_pending_auto = false;
   // true FP64 residual of the returned x (reported, not part of the solve;
@@ -3933,11 +4367,12 @@ namespace {
 
 constexpr size_t kNoAllocMaxRows = MPS_NOALLOC_MAX_ROWS;
 constexpr size_t kStatusDoubles = (sizeof(CgStatus) + 7) / 8;
-constexpr size_t kScratchDoubles = 3 * kNoAllocMaxRows + 3 * static_cast<size_t>(kRedBlocks) + kStatusDoubles;
+constexpr size_t kResidentDoubles = (sizeof(ResidentCtl) + 7) / 8;
+constexpr size_t kScratchDoubles =
+    3 * kNoAllocMaxRows + 3 * static_cast<size_t>(kRedBlocks) + kResidentDoubles + kStatusDoubles;
 
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 double* g_scratch_dev[kMaxDevices] = {};
 
@@ -3959,17 +4394,41 @@ __global__ void k_status_clear(CgStatus* st) {
 }
 
 void csr_solve(size_t n, const uint64_t* rowptr, const uint32_t* col, const double* val, const double* b,
-               double* x, double eps, long long max_iter, hipStream_t s, double* work, long long* iters_out) {
+               double* x, double eps, long long max_iter, hipStream_t s, int dev, double* work, long long* iters_out) {
   double* r = work;
   double* p = r + kNoAllocMaxRows;
   double* q = p + kNoAllocMaxRows;
   double* partA = q + kNoAllocMaxRows;
   double* partB = partA + kRedBlocks;
   double* partC = partB + kRedBlocks;
-  CgStatus* st = reinterpret_cast<CgStatus*>(partC + kRedBlocks);
+  ResidentCtl* ctl = reinterpret_cast<ResidentCtl*>(partC + kRedBlocks);
+  CgStatus* st = reinterpret_cast<CgStatus*>(partC + kRedBlocks + kResidentDoubles);
   const Launch L = cg_grid(n);
   const Csr A{rowptr, col, val, n, L.rpb};
   const StopRule sr{MPS_STOP_INITIAL_RESIDUAL, eps};
+  CgStatus hs{};
+  {
+    // resident workgroups, if the system fits them
+    ResidentTurn turn(dev);
+    if (turn && L.rpb == static_cast<size_t>(NT) && L.grid <= kResSlots) {
+      hipLaunchKernelGGL(k_cg_init<Csr>, dim3(L.grid), dim3(NT), 0, s, A, b, static_cast<const double*>(x), r, partB,
+                         partC);
+      if (resident_cg_launch(A, L, x, r, p, q, static_cast<const double*>(partB), static_cast<const double*>(partC),
+                             st, sr, max_iter, ctl, s)) {
+        unsigned head[2] = {0, 0};
+        MPS_HIP(hipMemcpyAsync(head, ctl, sizeof head, hipMemcpyDeviceToHost, s));
+        MPS_HIP(hipMemcpyAsync(&hs, st, sizeof(CgStatus), hipMemcpyDeviceToHost, s));
+        MPS_HIP(hipStreamSynchronize(s));
+        if (!head[1]) {
+          if (iters_out) *iters_out = hs.iterations;
+          if (!hs.converged)
+            throw Failure{MPS_ERR_CG_NOT_CONVERGED, "Conjugate Gradient method couldn't solve Pressure Poison Equation"};
+          return;
+        }
+        hs = CgStatus{};
+      }
+    }
+  }
   // every value the iterations read is written first: the status by the clear
   // kernel, r and the partial slots by k_cg_init, p and q by the first
   // iteration (FIRST: p = r, q = A r)
@@ -3977,7 +4436,6 @@ void csr_solve(size_t n, const uint64_t* rowptr, const uint32_t* col, const doub
   hipLaunchKernelGGL(k_cg_init<Csr>, dim3(L.grid), dim3(NT), 0, s, A, b, static_cast<const double*>(x), r, partB,
                      partC);
   check_launch();
-  CgStatus hs{};
   long long it = 1;
   while (true) {
     const long long chunk = next_chunk(it - 1, 0);
@@ -4039,7 +4497,7 @@ extern "C" int mps_cg_solve_csr_noalloc(int device, size_t n, const uint64_t* ro
     MPS_HIP(hipSetDevice(device));
     double* work = scratch_ptr(device);
     csr_solve(n, rowptr, col, val, b, x, allowable_residual, max_iter > 0 ? max_iter : static_cast<long long>(n),
-              static_cast<hipStream_t>(stream), work, reinterpret_cast<long long*>(iterations));
+              static_cast<hipStream_t>(stream), device, work, reinterpret_cast<long long*>(iterations));
   } catch (Failure& f) {
     if (f.code == MPS_ERR_HIP) (void)hipGetLastError();
     put_err(err, err_len, f.msg.c_str());

@@ -48,6 +48,8 @@ struct IrStatus {
   int pad;
 };
 
+struct ResidentCtl;  // mps_resident.hpp
+
 constexpr int kAmgMaxLevels = 20;  // grid levels of the cell-grid multigrid
 
 constexpr int kFeat = 132;     // warm-start feature width
@@ -293,6 +295,12 @@ struct Context {
   IrStatus* ir = nullptr;
   IrStatus* ir_host = nullptr;
   long long last_iters = 0;
+  // resident solves: their control block, its head on the host ([1]: given
+  // up), and how many solves not to try after one was refused
+  ResidentCtl* res_ctl = nullptr;
+  unsigned* res_host = nullptr;  // pinned
+  int res_skip = 0;
+  bool solve_ended = false;  // solve_b was recorded by the solver (a residual follows it)
 
   mps_solver_opts solver{};
   mps_solve_stats stats{};

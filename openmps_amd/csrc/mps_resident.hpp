@@ -1,0 +1,139 @@
+// Workgroups that stay on the chip for a whole solve and exchange data
+// between themselves without ending the kernel.
+//
+// A solver iteration of a small system is two to nine launches of 4-8 us each,
+// of which the arithmetic is a fraction of a microsecond: the launches, the
+// ramp of every kernel and the reload of the matrix cost the rest.  A resident
+// kernel keeps one workgroup per block of rows for all iterations.  What a
+// workgroup hands to the others (vector entries, partial sums) is written and
+// read with relaxed agent-scope atomics, which bypass the caches that are not
+// coherent between XCDs; the writer waits for its stores to complete
+// (s_waitcnt vmcnt(0)) before it publishes the partial sum that says so.
+// Nothing is fenced: an agent-scope fence writes back or invalidates whole
+// caches.  Measured for one exchange among resident workgroups (32 / 64 / 128 /
+// 256 of them): 1.5 / 1.9 / 2.6 / 4.2 us this way, 4 / 7 / 13 / 28 us with
+// release and acquire fences.
+//
+// A reduction is also the barrier: each workgroup publishes its partial sum in
+// its own slot and every workgroup polls all slots until none holds the empty
+// mark, then adds them in the fixed order of the launched kernels (1.8 / 2.2 /
+// 2.4 / 2.8 us for 5 / 64 / 128 / 256 workgroups, both block sums included; 4.0
+// for 256 with the slots side by side; 3.5-3.6 through one reducing workgroup
+// that hands the total on).  Slots are used in a ring of kResRing generations.  Emptying: once generation g is
+// complete everyone has published g and so has finished reading g - 1; the
+// owner then empties its slot of g - 1, and that store completes before its
+// publication of g + 1, hence before anyone polls g + 3 (the same ring entry).
+//
+// Every wait is bounded.  Before the first iteration the workgroups wait until
+// all of them have started (they might not fit beside other work on the GPU)
+// or the time limit has passed; then they all leave without having written
+// anything, and the caller runs the launched kernels instead.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "mps_device.hpp"
+
+namespace mps {
+
+constexpr int kResRing = 4;
+constexpr int kResSlots = 512;  // partial sums of one generation (one per workgroup)
+constexpr int kResPitch = 8;    // a slot per 64-byte line: polls of one slot do not hold up a store to another
+constexpr unsigned long long kResEmpty = ~0ull;  // no partial sum: NaNs are published as one quiet pattern
+
+struct ResidentCtl {
+  unsigned started;
+  unsigned abort;
+  unsigned pad[30];
+  unsigned long long slot[kResRing][kResSlots * kResPitch];
+};
+
+// Limits of the waits, in ticks of the constant 100 MHz clock: for the start
+// (5 ms: other work on the GPU may hold the compute units) and for one
+// generation (2 s: only a lost workgroup gets there).
+constexpr long long kResStartTicks = 500000;
+constexpr long long kResWaitTicks = 200000000;
+
+template <class T>
+__device__ __forceinline__ T agent_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void agent_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The wavefront's stores have completed at their destination.
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Block-uniform; every thread calls it.  True once all workgroups of the grid
+// have started and none has refused (ok == false).
+__device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok) {
+  __shared__ int s_go;
+  if (threadIdx.x == 0) {
+    if (!ok) {
+      agent_store(&c->abort, 1u);
+      stores_done();
+    }
+    __hip_atomic_fetch_add(&c->started, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const long long t0 = wall_clock64();
+    int go = 1;
+    while (agent_load(&c->started) < gridDim.x) {
+      if (agent_load(&c->abort) || wall_clock64() - t0 > kResStartTicks) {
+        agent_store(&c->abort, 1u);
+        go = 0;
+        break;
+      }
+    }
+    if (agent_load(&c->abort)) go = 0;
+    s_go = go;
+  }
+  __syncthreads();
+  return s_go != 0;
+}
+
+// One thread: the workgroup's partial sum of generation g (after the emptying
+// of an older slot, and whatever else this thread's wavefront stored, is done).
+__device__ __forceinline__ void resident_publish(ResidentCtl* c, unsigned g, unsigned idx, double v) {
+  if (v != v) v = __builtin_nan("");  // never the empty mark
+  stores_done();
+  agent_store(&c->slot[g % kResRing][idx * kResPitch], static_cast<unsigned long long>(__double_as_longlong(v)));
+}
+
+// Threads t < count: slot t of generation g once it is published (0 on the
+// others); ok: false on a thread whose wait was given up.
+__device__ __forceinline__ double resident_poll(ResidentCtl* c, unsigned g, unsigned count, bool& ok) {
+  if (threadIdx.x >= count) return 0.0;
+  const unsigned long long* s = &c->slot[g % kResRing][threadIdx.x * kResPitch];
+  unsigned long long b = agent_load(s);
+  if (b == kResEmpty) {
+    const long long t0 = wall_clock64();
+    do {
+      b = agent_load(s);
+      if (b == kResEmpty && (agent_load(&c->abort) || wall_clock64() - t0 > kResWaitTicks)) {
+        agent_store(&c->abort, 1u);
+        ok = false;
+        break;
+      }
+    } while (b == kResEmpty);
+  }
+  return __longlong_as_double(static_cast<long long>(b));
+}
+
+// After the whole workgroup has seen generation g complete: its slot of
+// generation g - 1 is emptied.
+__device__ __forceinline__ void resident_empty(ResidentCtl* c, unsigned g, unsigned idx) {
+  if (threadIdx.x == 0) agent_store(&c->slot[(g + kResRing - 1) % kResRing][idx * kResPitch], kResEmpty);
+}
+
+// Clears the control block (and whatever `extra` words of a status) before a
+// resident launch: one launch of kResSlots threads.
+__device__ __forceinline__ void resident_clear(ResidentCtl* c) {
+  if (threadIdx.x == 0) {
+    c->started = 0;
+    c->abort = 0;
+  }
+  for (int g = 0; g < kResRing; g++)
+    for (int k = threadIdx.x; k < kResSlots; k += blockDim.x) c->slot[g][k * kResPitch] = kResEmpty;
+}
+
+}  // namespace mps
