@@ -414,7 +414,7 @@ int mps_create(const mps_env* env, double allowable_residual, int device, mps_ct
     mps::pinned(c.st_host, 1);
     mps::pinned(c.st32_host, 1);
     mps::pinned(c.ir_host, 1);
-    mps::pinned(c.res_host, 2);
+    mps::pinned(c.res_host, mps::kResHead / sizeof(unsigned));
     MPS_HIP(hipEventCreate(&c.solve_a));
     MPS_HIP(hipEventCreate(&c.solve_b));
   } catch (Failure& f) {

@@ -695,12 +695,63 @@ __device__ __forceinline__ uint32_t number_marked(const Gathered& g) {
   return total;
 }
 
+// Marks and numbers the rows that a workgroup gathers: the columns col(k), k < m,
+// of every thread's row i and the row itself (in: the thread has a row).  lo:
+// the lowest of them, wn: their number.  Block-uniform; false: they span too
+// many rows.
+template <class Col>
+__device__ __forceinline__ bool gather_rows(const Gathered& ga, bool in, uint32_t i, uint32_t m, Col col, uint32_t& lo,
+                                            uint32_t& wn) {
+  lo = in ? i : 0xffffffffu;
+  uint32_t hi = in ? i : 0u;
+  for (uint32_t k = 0; k < m; k++) {
+    const uint32_t j = col(k);
+    lo = min(lo, j);
+    hi = max(hi, j);
+  }
+  for (uint32_t k = threadIdx.x; k < kResWords; k += NT) ga.mark[k] = 0u;
+  block_range(lo, hi);
+  wn = 0;
+  if (hi < lo) {  // no rows at all
+    lo = 0;
+    return true;
+  }
+  if (hi - lo >= kResRange) return false;
+  if (in) ga.set(i - lo);
+  for (uint32_t k = 0; k < m; k++) ga.set(col(k) - lo);
+  __syncthreads();
+  wn = number_marked(ga);
+  return wn < kResRange;
+}
+// The numbered rows (less lo) into list.
+__device__ __forceinline__ void gather_list(const Gathered& ga, uint16_t* list) {
+  for (uint32_t w = threadIdx.x; w < kResWords; w += NT) {
+    uint32_t bits = ga.mark[w], at = ga.base[w];
+    for (; bits; bits &= bits - 1) list[at++] = static_cast<uint16_t>(32 * w + __ffs(bits) - 1);
+  }
+}
+constexpr uint32_t kMarkBytes = 6 * kResWords;  // marks and numbers, at the start of the dynamic LDS
+
+// The gathered entries of a vector into LDS, as they were published.
+template <class T>
+__device__ __forceinline__ void gather_values(T* __restrict__ to, const T* from, const uint16_t* __restrict__ list,
+                                              uint32_t wn) {
+  for (uint32_t k0 = threadIdx.x; k0 < wn; k0 += 4 * NT) {
+    T t[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) t[u] = (k0 + u * NT < wn) ? agent_load(from + list[k0 + u * NT]) : T(0);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (k0 + u * NT < wn) to[k0 + u * NT] = t[u];
+  }
+}
+
 // The sum of the workgroups' partial sums of generation gen, in the order in
 // which block_sum<NT> adds one per thread; up to 64 of them by one wavefront.
 __device__ __forceinline__ double resident_sum(ResidentCtl* ctl, unsigned gen, unsigned idx, unsigned G, double* lds,
                                                bool& ok) {
   double v = 0.0;
-  if (threadIdx.x < 64 || G > 64) v = resident_poll(ctl, gen, G, ok);
+  if (threadIdx.x < G) v = resident_word(ctl, gen, threadIdx.x, 0, ok);
   if (G <= 64) {
     v = wave_sum(v);
     if (threadIdx.x == 0) lds[0] = v;
@@ -733,62 +784,39 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   const size_t i = rw.lo + threadIdx.x;
   const bool in = i < rw.hi;
   const auto row = row_of(A, i, in);
-  const uint32_t m = row.m;
-  uint32_t lo = in ? static_cast<uint32_t>(i) : 0xffffffffu, hi = in ? static_cast<uint32_t>(i) : 0u;
-  for (uint32_t k = 0; k < m; k++) {
-    const uint32_t j = row.col(k);
-    lo = min(lo, j);
-    hi = max(hi, j);
-  }
-  block_range(lo, hi);
-  const bool narrow = hi - lo < kResRange;
+  const uint32_t m = row.m, self = static_cast<uint32_t>(i);
   const Gathered ga{reinterpret_cast<uint32_t*>(win), reinterpret_cast<uint16_t*>(win) + 2 * kResWords};
-  constexpr uint32_t kMarkBytes = 6 * kResWords;
-  for (uint32_t k = threadIdx.x; k < kResWords; k += NT) ga.mark[k] = 0u;
-  __syncthreads();
-  // the row's first entries: values, and columns as 16-bit numbers from lo, two a register
-  double a[REG];
-  uint32_t off[REG / 2];
-  if (narrow && in) ga.set(static_cast<uint32_t>(i) - lo);
-#pragma unroll
-  for (int k = 0; k < REG; k++) {
-    a[k] = 0.0;
-    uint32_t d = in ? (static_cast<uint32_t>(i) - lo) & 0xffffu : 0u;  // past the row's end: its own r, value 0
-    if (static_cast<uint32_t>(k) < m) {
-      a[k] = row.val(k);
-      if (narrow) {
-        d = row.col(k) - lo;
-        ga.set(d);
-      }
-    }
-    if (k & 1) off[k >> 1] |= d << 16;
-    else off[k >> 1] = d;
-  }
-  if (narrow)
-    for (uint32_t k = REG; k < m; k++) ga.set(row.col(k) - lo);
-  __syncthreads();
-  const uint32_t wn = number_marked(ga);
+  uint32_t lo, wn;
+  const bool narrow = gather_rows(ga, in, self, m, [&](uint32_t k) { return row.col(k); }, lo, wn);
   // LDS behind the gathered r: the list of its rows, entries of the matrix
   const uint32_t list_at = max(wn * 8u, kMarkBytes), mat_at = (list_at + 2 * wn + 15u) & ~15u;
-  const bool ok_lds = narrow && wn < kResRange && mat_at <= bytes;
+  const bool ok_lds = narrow && mat_at <= bytes;
   uint16_t* const list = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(win) + list_at);
   const uint32_t lrows = ok_lds ? min((bytes - mat_at) / (10u * NT), 64u) : 0u;
   double* const lval = reinterpret_cast<double*>(reinterpret_cast<char*>(win) + mat_at);
   uint16_t* const lcol = reinterpret_cast<uint16_t*>(lval + static_cast<size_t>(lrows) * NT);
-  const uint32_t own = (ok_lds && in) ? ga.at(static_cast<uint32_t>(i) - lo) : 0u;
   const uint32_t kl = min(m, static_cast<uint32_t>(REG) + lrows);  // entries in registers and LDS
-  if (ok_lds) {
+  // the row's first entries: values, and columns as their numbers, two a register
+  double a[REG];
+  uint32_t off[REG / 2];
+  const uint32_t own = (ok_lds && in) ? ga.at(self - lo) : 0u;  // past the row's end: its own r, value 0
 #pragma unroll
-    for (int k = 0; k < REG / 2; k++)
-      off[k] = in ? (ga.at(off[k] & 0xffffu) | (ga.at(off[k] >> 16) << 16)) : 0u;
+  for (int k = 0; k < REG; k++) {
+    a[k] = 0.0;
+    uint32_t d = own;
+    if (static_cast<uint32_t>(k) < m) {
+      a[k] = row.val(k);
+      if (ok_lds) d = ga.at(row.col(k) - lo);
+    }
+    if (k & 1) off[k >> 1] |= d << 16;
+    else off[k >> 1] = d;
+  }
+  if (ok_lds) {
     for (uint32_t k = REG; k < kl; k++) {
       lval[(k - REG) * NT + threadIdx.x] = row.val(k);
       lcol[(k - REG) * NT + threadIdx.x] = static_cast<uint16_t>(ga.at(row.col(k) - lo));
     }
-    for (uint32_t w = threadIdx.x; w < kResWords; w += NT) {
-      uint32_t bits = ga.mark[w], at = ga.base[w];
-      for (; bits; bits &= bits - 1) list[at++] = static_cast<uint16_t>(32 * w + __ffs(bits) - 1);
-    }
+    gather_list(ga, list);
   }
   const double dg = in ? row.diag() : 0.0;
   double ri = in ? r[i] : 0.0, xi = in ? x[i] : 0.0, pi = 0.0, qi = 0.0;
@@ -813,15 +841,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
       conv = (sr.rule == MPS_STOP_RHS_NORM) ? (rr <= tol) : (rr < tol);  // :1408
     }
     if (conv || it > max_iter) break;
-    // r of the gathered rows (complete: r.r was collected)
-    for (uint32_t k0 = threadIdx.x; k0 < wn; k0 += 4 * NT) {
-      double t[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) t[u] = (k0 + u * NT < wn) ? agent_load(r + lo + list[k0 + u * NT]) : 0.0;
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-        if (k0 + u * NT < wn) win[k0 + u * NT] = t[u];
-    }
+    gather_values(win, static_cast<const double*>(r + lo), list, wn);  // complete: r.r was collected
     __syncthreads();
     double s = dg * ri;
 #pragma unroll
@@ -1093,6 +1113,13 @@ __device__ __forceinline__ BlockLane block_lane(const CellGrid& G, uint32_t b) {
 }
 __device__ __forceinline__ bool in_agg(uint8_t t) { return t != kDummy && t != kDisabled; }
 
+// Sum of v over the four lanes (l, l ^ 16, l ^ 32, l ^ 48) of one cell.
+__device__ __forceinline__ float cell_sum(float v) {
+  PairU32 p = pair16(__float_as_uint(v));
+  v = __uint_as_float(p.a) + __uint_as_float(p.b);
+  p = pair32(__float_as_uint(v));
+  return __uint_as_float(p.a) + __uint_as_float(p.b);
+}
 // Sums of v over the lanes of one cell, of one 2x2 block and of the 4x4 block.
 template <class T>
 __device__ __forceinline__ void agg_sums(T v, T& y0, T& y1, T& y2) {
@@ -1406,29 +1433,34 @@ __device__ __forceinline__ void amg_down_point(const AmgGrid& g, const AmgVec& v
 
 // Level l + 1 -> l: one thread per point p of level l: x = x_pre + corr e(parent),
 // then e_p = x_p + omega (r_p - (S x)_p) / S_pp.
-template <class SV>
+// SKIP: nothing is read for empty points (a whole box of cells, mostly empty).
+template <bool SKIP = true, class SV>
 __device__ __forceinline__ float amg_up_value(const AmgGrid& g, const AmgVec& v, const SV& sten, int l, uint32_t p) {
   const AmgLevel F = g.L[l], C = g.L[l + 1];
   const uint32_t ix = p / F.nz, iz = p % F.nz;
   const uint32_t fo = F.off - v.base, co = C.off - v.base;
   const float di = v.dinv[fo + p];
-  if (di == 0.0f) return 0.0f;  // empty point
-  float xq[9], sv[9];
+  if (SKIP && di == 0.0f) return 0.0f;  // empty point
+  // every load first, unconditionally (neighbours outside: the point itself)
+  float ev[9], xv[9], sv[9];
+  bool in[9];
 #pragma unroll
-  for (int dx = -1; dx <= 1; dx++)
+  for (int k = 0; k < 9; k++) {
+    const int jx = static_cast<int>(ix) + k / 3 - 1, jz = static_cast<int>(iz) + k % 3 - 1;
+    in[k] = jx >= 0 && jz >= 0 && jx < static_cast<int>(F.nx) && jz < static_cast<int>(F.nz);
+    const uint32_t ux = in[k] ? static_cast<uint32_t>(jx) : ix, uz = in[k] ? static_cast<uint32_t>(jz) : iz;
+    ev[k] = v.e[co + (ux >> 1) * C.nz + (uz >> 1)];
+    xv[k] = v.x[fo + ux * F.nz + uz];
+    sv[k] = sten(l, k, p);
+  }
+  const float rp = v.r[fo + p];
+  float xq[9], sum = 0.0f;
 #pragma unroll
-    for (int dz = -1; dz <= 1; dz++) {
-      const int k = 3 * (dx + 1) + dz + 1;
-      const int jx = static_cast<int>(ix) + dx, jz = static_cast<int>(iz) + dz;
-      const bool in = jx >= 0 && jz >= 0 && jx < static_cast<int>(F.nx) && jz < static_cast<int>(F.nz);
-      const uint32_t ux = static_cast<uint32_t>(in ? jx : 0), uz = static_cast<uint32_t>(in ? jz : 0);
-      xq[k] = in ? fmaf(g.corr, v.e[co + (ux >> 1) * C.nz + (uz >> 1)], v.x[fo + ux * F.nz + uz]) : 0.0f;
-      sv[k] = in ? sten(l, k, p) : 0.0f;
-    }
-  float sum = 0.0f;
-#pragma unroll
-  for (int k = 0; k < 9; k++) sum = fmaf(sv[k], xq[k], sum);
-  return fmaf(g.omega * di, v.r[fo + p] - sum, xq[4]);
+  for (int k = 0; k < 9; k++) {
+    xq[k] = in[k] ? fmaf(g.corr, ev[k], xv[k]) : 0.0f;
+    sum = fmaf(in[k] ? sv[k] : 0.0f, xq[k], sum);
+  }
+  return (di == 0.0f) ? 0.0f : fmaf(g.omega * di, rp - sum, xq[4]);
 }
 
 // Level l + 1 -> l: one thread per point p of level l: x = x_pre + e(parent),
@@ -1624,23 +1656,25 @@ __global__ void __launch_bounds__(kAmgChainThreads) k_amg_up_chain(AmgGrid g, in
         const uint32_t p = static_cast<uint32_t>(px) * F.nz + static_cast<uint32_t>(pz);
         const float di = g.dinv[F.off + p];
         if (di != 0.0f) {
-          float xq[9], sv[9];
+          // every load first, unconditionally (neighbours outside: the point itself)
+          float xv[9], ev[9], sv[9];
+          bool in[9];
 #pragma unroll
-          for (int dx = -1; dx <= 1; dx++)
+          for (int kk = 0; kk < 9; kk++) {
+            const int jx = px + kk / 3 - 1, jz = pz + kk % 3 - 1;
+            in[kk] = amg_in(F, jx, jz);
+            xv[kk] = g.x[F.off + (in[kk] ? static_cast<uint32_t>(jx) * F.nz + static_cast<uint32_t>(jz) : p)];
+            ev[kk] = ce[((jx >> 1) - cox) * sc + ((jz >> 1) - coz)];
+            sv[kk] = g.S[9ull * F.off + static_cast<size_t>(kk) * amg_npts(F) + p];
+          }
+          const float rp = g.r[F.off + p];
+          float xq[9], sum = 0.0f;
 #pragma unroll
-            for (int dz = -1; dz <= 1; dz++) {
-              const int kk = 3 * (dx + 1) + dz + 1;
-              const int jx = px + dx, jz = pz + dz;
-              const bool in = amg_in(F, jx, jz);
-              const uint32_t q = F.off + static_cast<uint32_t>(in ? jx : 0) * F.nz + static_cast<uint32_t>(in ? jz : 0);
-              const float ep = ce[((jx >> 1) - cox) * sc + ((jz >> 1) - coz)];
-              xq[kk] = in ? fmaf(g.corr, ep, g.x[q]) : 0.0f;
-              sv[kk] = in ? g.S[9ull * F.off + static_cast<size_t>(kk) * amg_npts(F) + p] : 0.0f;
-            }
-          float sum = 0.0f;
-#pragma unroll
-          for (int kk = 0; kk < 9; kk++) sum = fmaf(sv[kk], xq[kk], sum);
-          val = fmaf(g.omega * di, g.r[F.off + p] - sum, xq[4]);
+          for (int kk = 0; kk < 9; kk++) {
+            xq[kk] = in[kk] ? fmaf(g.corr, ev[kk], xv[kk]) : 0.0f;
+            sum = fmaf(in[kk] ? sv[kk] : 0.0f, xq[kk], sum);
+          }
+          val = fmaf(g.omega * di, rp - sum, xq[4]);
         }
         if (k == 0) g.e[F.off + p] = val;
       }
@@ -1931,8 +1965,7 @@ __device__ __forceinline__ void ml_prec_body(const PrecArgs& a, long long it, co
       const int pt = L.valid ? amg_point(a, L.cell, G.gnz) : -1;
 #pragma unroll
       for (int e = 0; e < 9; e++) {
-        float t = t9[e] + __shfl_xor(t9[e], 16, 64);
-        t = t + __shfl_xor(t, 32, 64);
+        const float t = cell_sum(t9[e]);
         if (pt >= 0 && L.sub == 0) a.tq[static_cast<size_t>(e) * a.tq_stride + static_cast<uint32_t>(pt)] = t;
       }
     } else if (MODE == 2) {
@@ -1949,7 +1982,7 @@ __device__ __forceinline__ void ml_prec_body(const PrecArgs& a, long long it, co
         const int cz = static_cast<int>(4 * (b % G.bnz)) - 1 + static_cast<int>(lane % 6) - static_cast<int>(a.bz0);
         float val = 0.0f;
         if (lane < 36 && cx >= 0 && cz >= 0 && cx < static_cast<int>(a.bnx) && cz < static_cast<int>(a.bnz))
-          val = amg_up_value(*amg, amg_global(*amg), AmgStenGlobal{amg}, 0,
+          val = amg_up_value<false>(*amg, amg_global(*amg), AmgStenGlobal{amg}, 0,
                              static_cast<uint32_t>(cx) * a.bnz + static_cast<uint32_t>(cz));
         const int ux = static_cast<int>((lane & 15u) >> 2), uz = static_cast<int>(lane & 3u);
 #pragma unroll
@@ -2058,17 +2091,29 @@ __global__ void __launch_bounds__(256) k_amg_q(size_t nslots, const uint32_t* __
 // Level 0's right-hand side P_s^T r from pass 1's direction sums:
 // r0(p) = sum_d T_d(p - off(d)), T_d(c) the share of cell c's rows for the
 // cell c + off(d) (off(d) = (d / 3 - 1, d % 3 - 1)).
-__device__ __forceinline__ void amg_rfix_point(const float* __restrict__ tq, size_t stride, uint32_t nx,
-                                               uint32_t nz, float* __restrict__ r0, uint32_t p) {
-  const int x = static_cast<int>(p / nz), zc = static_cast<int>(p % nz);
-  float s = 0.0f;
+// (Out-of-range terms read the point's own sum and count as 0: a load in its own
+// branch, with the addition, would wait for every term in turn.)
+template <bool SHARED = false>
+__device__ __forceinline__ float amg_rfix_at(const float* tq, size_t stride, uint32_t nx, uint32_t nz, int x, int zc) {
+  const uint32_t p = static_cast<uint32_t>(x) * nz + static_cast<uint32_t>(zc);
+  float t[9];
+  bool in[9];
 #pragma unroll
   for (int e = 0; e < 9; e++) {
     const int sx = x - (e / 3 - 1), sz = zc - (e % 3 - 1);
-    if (sx >= 0 && sz >= 0 && sx < static_cast<int>(nx) && sz < static_cast<int>(nz))
-      s += tq[static_cast<size_t>(e) * stride + static_cast<uint32_t>(sx) * nz + static_cast<uint32_t>(sz)];
+    in[e] = sx >= 0 && sz >= 0 && sx < static_cast<int>(nx) && sz < static_cast<int>(nz);
+    const float* a = tq + static_cast<size_t>(e) * stride +
+                     (in[e] ? static_cast<uint32_t>(sx) * nz + static_cast<uint32_t>(sz) : p);
+    t[e] = SHARED ? agent_load(a) : *a;
   }
-  r0[p] = s;
+  float s = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 9; e++) s += in[e] ? t[e] : 0.0f;
+  return s;
+}
+__device__ __forceinline__ void amg_rfix_point(const float* __restrict__ tq, size_t stride, uint32_t nx,
+                                               uint32_t nz, float* __restrict__ r0, uint32_t p) {
+  r0[p] = amg_rfix_at(tq, stride, nx, nz, static_cast<int>(p / nz), static_cast<int>(p % nz));
 }
 __global__ void __launch_bounds__(256) k_amg_rfix(const float* __restrict__ tq, size_t stride, uint32_t nx,
                                                   uint32_t nz, float* __restrict__ r0, const CgStatus* st,
@@ -2384,6 +2429,997 @@ __global__ void __launch_bounds__(256) k_jacobi_inv(size_t n, const double* __re
   if (i < n) {
     const double d = diag[i];
     dinv[i] = (d != 0.0) ? static_cast<float>(1.0 / d) : 1.0f;
+  }
+}
+
+// ---- the mixed solve with resident workgroups ----
+//
+// The whole refinement of a small scene in one launch: FP64 residual, FP32
+// sweeps (multilevel or multigrid preconditioned CG), correction, until the
+// target is met or the host has to decide (stall).  Launched, an iteration is
+// two to nine kernels of 4-9 us and every sweep ends in two host round trips.
+//
+// A workgroup has two roles.  Rows, one per thread: x, d, p, q and the row's
+// FP32 coefficients (the matrix-free terms c0 / r^3, computed once: the
+// positions do not move during a solve) in registers and LDS, z gathered from
+// an LDS copy of exactly the rows its columns name.  Cells, one listed 4x4
+// block of cells per wavefront: r and the Jacobi factors of the block's
+// particles in registers, P_s's rows loaded while the workgroup waits for the
+// others.  q goes from rows to cells and z from cells to rows through global
+// memory (agent-scope, mps_resident.hpp), as do the multigrid's direction sums.
+//
+// The cycle is bound by its chain of levels, each a few hundred points or
+// less, and by the exchanges between them (2-3 us apiece): levels from l0 on
+// (kResLevelBytes) are computed by every workgroup alike, in its own LDS, so
+// that the chain down and up costs no exchange at all; above l0 a workgroup
+// takes tiles of the coarser level, two levels in one step from the cells
+// down, and the way back up through levels 1 and 0 is computed by the
+// wavefronts that need it.  Exchanges per iteration: q with p.q; z with r.z
+// and r.r; the multigrid adds the direction sums, and one for l0 = 1 or 2.
+//
+// Time of an iteration, launched and resident, in us:
+//   multilevel   0.7k particles 18.3 / 8.2, 12k 19.1 / 9.3, 63k 19.8 / 10.9, 95k 20.4 / 12.0, 177k 23.7 / 20.6
+//   multigrid    0.7k 44.2 / 21.9, 6k 55 / 28, 25k 68.5 / 36.8, 36k 77 / 41, 63k 81.0 / 45.3, 95k 82.9 / 51.7
+// What is left of it: the exchanges (2-6 us each with the wait for the
+// slowest), the dependent loads of q, z and the sums after them, and for the
+// multigrid the levels' chain (about 0.5 us a level and direction).
+//
+// Every value and every sum is computed as the launched kernels compute it, in
+// their order (partial sums per 512 rows and per 4 blocks of cells), and the
+// refinement's decisions are those of refine and run_inner: the two agree bit
+// for bit.
+//
+// What does not change between iterations but is cheap to form (addresses,
+// unpacked numbers) is formed where it is used: opaque() keeps the compiler
+// from holding it in registers across the whole solve.
+template <class T>
+__device__ __forceinline__ T opaque(T v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+struct MixedResult {
+  double rr0, rr, bb;
+  long long total;
+  long long pred[Context::kSweepPred];
+  int outer, done, stalled, pad;
+};
+static_assert(sizeof(MixedResult) <= sizeof(ResidentCtl::out), "results in the control block");
+
+struct MixedArgs {
+  size_t n;
+  unsigned rows;  // workgroups that have rows
+  Sell<double> A;
+  const double* b;
+  double *x, *r64;
+  const uint32_t* len;
+  const uint2* pos;
+  const float* ghost;
+  float c0;
+  float *z, *q, *p, *d;
+  PrecArgs a;
+  AmgGrid g;
+  int l0;         // first level held in LDS
+  uint32_t lvp;   // points and places of the levels held in LDS
+  uint32_t lvq;
+  uint16_t place[kAmgMaxLevels];  // start of each level's bordered grid
+  StopRule sr;
+  double inner_tol;
+  long long total_cap, limit;
+  long long pred[Context::kSweepPred];
+  int have_r;  // r64 and rr, bb hold the first residual
+  double rr, bb;
+  ResidentCtl* ctl;
+  uint32_t bytes;  // dynamic LDS
+};
+
+// The levels l0 .. of the cycle in a workgroup's LDS: the stencils as in global
+// memory, r, x, e and 1 / S_center on grids with a border of zeros (a neighbour
+// is a fixed distance away and needs no range test), and per point its place,
+// its first child's and its parent's.
+struct LdsLevels {
+  const float* s;      // 9 stencil coefficients per point, as in global memory from level l0 on
+  const uint2* meta;   // per point: place | first child's place << 16; parent's place | odd row << 16 | odd column << 17
+  float *r, *x, *e, *d;
+  const float* inv;    // inverse of the coarsest level
+  float* last;         // the coarsest right-hand side, in point order
+};
+struct LdsLevel {
+  uint32_t nx, nz, first, pitch, place;  // points before it (from l0 on), row pitch and start of the bordered grid
+};
+// Levels as the kernel's arguments give them (scalar registers).
+template <class Args>
+__device__ __forceinline__ LdsLevel lds_level(const Args& A, int l) {
+  const AmgLevel L = A.g.L[l];
+  return LdsLevel{L.nx, L.nz, L.off - A.g.L[A.l0].off, L.nz + 2, A.place[l]};
+}
+// amg_down_point, one thread per child (its residual to e, unused on the way
+// down), then the parents' sums.
+__device__ __forceinline__ void lds_down(const LdsLevels& v, const LdsLevel& F, const LdsLevel& C, float omega,
+                                         bool last) {
+  const uint32_t nf = F.nx * F.nz, nc = C.nx * C.nz;
+  const float* __restrict__ st = v.s + 9u * F.first;
+  for (uint32_t p = threadIdx.x; p < nf; p += NT) {
+    const uint32_t at = v.meta[F.first + p].x & 0xffffu;
+    float rr[9], dd[9], sv[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      const uint32_t q = at + (k / 3) * F.pitch + k % 3 - F.pitch - 1;
+      rr[k] = v.r[q];
+      dd[k] = v.d[q];
+      sv[k] = st[static_cast<uint32_t>(k) * nf + p];
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 9; k++) sum = fmaf(sv[k], omega * dd[k] * rr[k], sum);
+    v.x[at] = omega * dd[4] * rr[4];
+    v.e[at] = rr[4] - sum;
+  }
+  __syncthreads();
+  for (uint32_t P = threadIdx.x; P < nc; P += NT) {
+    const uint32_t m = v.meta[C.first + P].x, c = m >> 16;
+    float rc = 0.0f;
+    rc += v.e[c];
+    rc += v.e[c + 1];
+    rc += v.e[c + F.pitch];
+    rc += v.e[c + F.pitch + 1];
+    if (last) v.last[P] = rc;
+    else v.r[m & 0xffffu] = rc;
+  }
+}
+// amg_up_point.
+__device__ __forceinline__ void lds_up(const LdsLevels& v, const LdsLevel& F, const LdsLevel& C, float omega, float corr) {
+  const uint32_t nf = F.nx * F.nz;
+  const float* __restrict__ st = v.s + 9u * F.first;
+  for (uint32_t p = threadIdx.x; p < nf; p += NT) {
+    const uint2 m = v.meta[F.first + p];
+    const uint32_t at = m.x & 0xffffu, up = m.y & 0xffffu;
+    const uint32_t ox = (m.y >> 16) & 1u, oz = (m.y >> 17) & 1u;
+    // rows and columns of the parents of the neighbours on either side
+    const uint32_t ra = ox ? up : up - C.pitch, rb = up, rc = ox ? up + C.pitch : up;
+    const uint32_t ca = oz ? 0u : 0xffffffffu, cc = oz ? 1u : 0u;
+    float xv[9], ev[9], sv[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      xv[k] = v.x[at + (k / 3) * F.pitch + k % 3 - F.pitch - 1];
+      ev[k] = v.e[(k / 3 == 0 ? ra : k / 3 == 1 ? rb : rc) + (k % 3 == 0 ? ca : k % 3 == 1 ? 0u : cc)];
+      sv[k] = st[static_cast<uint32_t>(k) * nf + p];
+    }
+    const float di = v.d[at], rp = v.r[at];
+    float xq[9], sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+      xq[k] = fmaf(corr, ev[k], xv[k]);
+      sum = fmaf(sv[k], xq[k], sum);
+    }
+    v.e[at] = (di == 0.0f) ? 0.0f : fmaf(omega * di, rp - sum, xq[4]);
+  }
+}
+
+// Bytes of LDS for levels of lvp points on bordered grids of lvq places, with the inverse of nb coarsest points.
+__host__ __device__ constexpr uint32_t lds_level_bytes(uint32_t lvp, uint32_t lvq, uint32_t nb) {
+  return 4 * (11 * lvp + 4 * lvq + nb * nb + nb) + 8;
+}
+// amg_up_value at point (ix, iz) of level c < l0, whose vectors are shared
+// between the workgroups; ev: e of the parents of its 3x3 neighbourhood.
+template <class Args>
+__device__ __forceinline__ float up_with(const Args& A, int c, int ix, int iz, const float ev[9]) {
+  const AmgLevel F = A.g.L[c];
+  const uint32_t np = amg_npts(F), p = static_cast<uint32_t>(ix) * F.nz + static_cast<uint32_t>(iz);
+  float xv[9], sv[9];
+  bool in[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const int jx = ix + k / 3 - 1, jz = iz + k % 3 - 1;
+    in[k] = amg_in(F, jx, jz);
+    xv[k] = agent_load(A.g.x + F.off + (in[k] ? static_cast<uint32_t>(jx) * F.nz + static_cast<uint32_t>(jz) : p));
+    sv[k] = A.g.S[9ull * F.off + static_cast<size_t>(k) * np + p];
+  }
+  const float rp = agent_load(A.g.r + F.off + p), di = A.g.dinv[F.off + p];
+  float xq[9], sum = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    xq[k] = in[k] ? fmaf(A.g.corr, ev[k], xv[k]) : 0.0f;
+    sum = fmaf(in[k] ? sv[k] : 0.0f, xq[k], sum);
+  }
+  return (di == 0.0f) ? 0.0f : fmaf(A.g.omega * di, rp - sum, xq[4]);
+}
+// The parents' e for it, from LDS where level c + 1 is level l0.
+template <class Args>
+__device__ __forceinline__ void up_parents(const Args& A, const LdsLevels& v, int c, int ix, int iz, float ev[9]) {
+  const AmgLevel F = A.g.L[c], C = A.g.L[c + 1];
+  const bool lds = c + 1 == A.l0;
+  const uint32_t place = A.place[c + 1];
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const int jx = ix + k / 3 - 1, jz = iz + k % 3 - 1;
+    const bool in = amg_in(F, jx, jz);
+    const uint32_t ux = static_cast<uint32_t>(in ? jx : ix) >> 1, uz = static_cast<uint32_t>(in ? jz : iz) >> 1;
+    ev[k] = lds ? v.e[place + (ux + 1) * (C.nz + 2) + uz + 1] : agent_load(A.g.e + C.off + ux * C.nz + uz);
+  }
+}
+
+// A step of the cycle down by tiles: kTile x kTile points of the coarser level,
+// the finer points with the halo of their residuals.
+constexpr int kTile = 8;
+constexpr int kTileF = 2 * kTile + 2;
+// Two steps (levels 0, 1, 2) by tiles of kTile2 x kTile2 points of level 2:
+// their children, those with the residuals' halo, and the same a level below.
+constexpr int kTile2 = 4;
+constexpr int kC1 = 2 * kTile2, kF1 = kC1 + 2, kC0 = 2 * kF1, kF0 = kC0 + 2;
+static_assert(kF0 * kF0 <= NT && kTileF * kTileF <= kF0 * kF0 && 4 * kTile * kTile <= kC0 * kC0, "one point a thread");
+
+template <bool AMG, int REG, int WAVES>
+__global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
+  extern __shared__ double win[];
+  __shared__ double lds[2 * (NT / 64)];
+  __shared__ float tile_r[AMG ? kF0 * kF0 : 1], tile_d[AMG ? kF0 * kF0 : 1], tile_c[AMG ? kC0 * kC0 : 1];
+  __shared__ float tile1_r[AMG ? kF1 * kF1 : 1], tile1_d[AMG ? kF1 * kF1 : 1], tile1_c[AMG ? kC1 * kC1 : 1];
+  const unsigned G = gridDim.x, idx = blockIdx.x, tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const PrecArgs& a = A.a;
+  ResidentCtl* const ctl = A.ctl;
+
+  // ---- rows ----
+  const bool has_rows = idx < A.rows;
+  const Rows rw = has_rows ? block_rows(A.n, NT, Frame{idx, A.rows, true}) : Rows{0, 0};
+  const size_t i = rw.lo + tid;
+  const bool in = has_rows && i < rw.hi;
+  const uint32_t self = static_cast<uint32_t>(i), m = in ? A.len[i] : 0u;
+  const SellRow<double> row(A.A, i, in);
+  const Gathered ga{reinterpret_cast<uint32_t*>(win), reinterpret_cast<uint16_t*>(win) + 2 * kResWords};
+  uint32_t lo, wn;
+  const bool narrow = gather_rows(ga, in, self, m, [&](uint32_t k) { return row.col(k); }, lo, wn);
+  // dynamic LDS: the gathered vector (first the marks), the list of its rows, the cycle's levels, matrix entries
+  const uint32_t list_at = max(wn * 8u, kMarkBytes), lev_at = (list_at + 2 * wn + 15u) & ~15u;
+  const uint32_t mat_at = lev_at + (AMG ? lds_level_bytes(A.lvp, A.lvq, amg_npts(A.g.L[A.g.levels - 1])) : 0u);
+  const bool ok_lds = narrow && mat_at <= A.bytes;
+  uint16_t* const list = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(win) + list_at);
+  const uint32_t lrows = ok_lds ? min((A.bytes - mat_at) / (6u * NT), 64u) & ~3u : 0u;
+  float* const lval = reinterpret_cast<float*>(reinterpret_cast<char*>(win) + mat_at);
+  uint16_t* const lcol = reinterpret_cast<uint16_t*>(lval + static_cast<size_t>(lrows) * NT);
+  const uint32_t kl = min(m, static_cast<uint32_t>(REG) + lrows);
+  const uint2 qi = in ? A.pos[i] : make_uint2(0u, 0u);
+  auto coef = [&](uint32_t j) {  // rec_sum's factor of column j
+    const uint2 qj = A.pos[j];
+    const float fx = static_cast<float>(static_cast<int>(qj.x - qi.x));
+    const float fz = static_cast<float>(static_cast<int>(qj.y - qi.y));
+    const float t = __builtin_amdgcn_rsqf(fmaf(fx, fx, fz * fz));
+    return A.c0 * (t * t * t);
+  };
+  const uint32_t own = (ok_lds && in) ? ga.at(self - lo) : 0u;
+  float cf[REG];
+  uint32_t off[REG / 2];
+#pragma unroll
+  for (int k = 0; k < REG; k++) {
+    cf[k] = 0.0f;
+    uint32_t e = own;
+    if (static_cast<uint32_t>(k) < m) {
+      const uint32_t j = row.col(k);
+      cf[k] = coef(j);
+      if (ok_lds) e = ga.at(j - lo);
+    }
+    if (k & 1) off[k >> 1] |= e << 16;
+    else off[k >> 1] = e;
+  }
+  if (ok_lds) {
+    for (uint32_t k = REG; k < REG + lrows; k++) {  // (past the row's end: factor 0, its own z)
+      const uint32_t j = k < m ? row.col(k) : 0u;
+      lval[(k - REG) * NT + tid] = k < m ? coef(j) : 0.0f;
+      lcol[(k - REG) * NT + tid] = static_cast<uint16_t>(k < m ? ga.at(j - lo) : own);
+    }
+    gather_list(ga, list);
+  }
+  const float ghost = in ? A.ghost[i] : 0.0f;
+  double x = in ? A.x[i] : 0.0;
+  if (in) agent_store(A.z + i, 0.0f);  // rows outside every cell keep z = 0
+
+  // ---- cells ----
+  const uint32_t w = idx * (NT / 64) + wv;
+  const bool active = w < a.nact;
+  uint32_t id[kPerLane];
+  float rv[kPerLane], dv[kPerLane];
+  uint4 q9[AMG ? kPerLane : 1];  // P_s's rows, read again for every pass over the cells
+  uint16_t q9c[AMG ? kPerLane : 1];
+  float4 scl = make_float4(0.f, 0.f, 0.f, 0.f);
+  int pt = -1;
+  uint32_t sub = 0, blk = 0;
+#pragma unroll
+  for (int u = 0; u < kPerLane; u++) {
+    id[u] = kNoSlot;
+    rv[u] = dv[u] = 0.0f;
+  }
+  if (active) {
+    blk = a.list[w];
+    scl = a.sc[static_cast<size_t>(w) * 64 + lane];
+#pragma unroll
+    for (int u = 0; u < kPerLane; u++) {
+      const size_t o = (static_cast<size_t>(w) * kPerLane + u) * 64 + lane;
+      id[u] = a.pid[o];
+      dv[u] = a.dvp[o];
+    }
+    const BlockLane L = block_lane(a.G, blk);
+    sub = L.sub;
+    if (AMG) pt = L.valid ? amg_point(a, L.cell, a.G.gnz) : -1;
+  }
+  auto load_q9s = [&]() {
+    if (AMG && active) {
+      const size_t o0 = static_cast<size_t>(w) * kPerLane * 64 + opaque(lane);
+#pragma unroll
+      for (int u = 0; u < kPerLane; u++) {
+        q9[u] = a.q9[o0 + 64 * u];
+        q9c[u] = a.q9c[o0 + 64 * u];
+      }
+    }
+  };
+  auto row9 = [&](int u, float out[9]) {  // P_s's row of slot u
+    const uint32_t h[4] = {q9[u].x, q9[u].y, q9[u].z, q9[u].w};
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+      out[e] = static_cast<float>(
+          __builtin_bit_cast(_Float16, static_cast<uint16_t>((h[e >> 1] >> (16 * (e & 1))) & 0xffffu)));
+    out[8] = static_cast<float>(__builtin_bit_cast(_Float16, q9c[u]));
+  };
+
+  // ---- the cycle's levels from l0 on, in every workgroup's LDS ----
+  const AmgGrid& g = A.g;
+  LdsLevels lv{};
+  if (AMG && ok_lds) {
+    float* f = reinterpret_cast<float*>(reinterpret_cast<char*>(win) + lev_at);
+    uint2* meta = reinterpret_cast<uint2*>(f);
+    f += 2 * A.lvp;
+    float* st = f;
+    f += 9 * A.lvp;
+    lv.r = f;
+    lv.x = f + A.lvq;
+    lv.e = f + 2 * A.lvq;
+    lv.d = f + 3 * A.lvq;
+    f += 4 * A.lvq;
+    float* inv = f;
+    const uint32_t nb = amg_npts(g.L[g.levels - 1]);
+    lv.last = f + nb * nb;
+    lv.s = st;
+    lv.meta = meta;
+    lv.inv = inv;
+    for (uint32_t k = tid; k < 4 * A.lvq; k += NT) lv.r[k] = 0.0f;
+    for (uint32_t k = tid; k < nb * nb; k += NT) inv[k] = g.inv[k];
+    __syncthreads();
+    for (int l = A.l0; l < g.levels; l++) {
+      const LdsLevel L = lds_level(A, l);
+      const uint32_t n = L.nx * L.nz;
+      for (uint32_t p = tid; p < n; p += NT) {
+        const uint32_t ix = p / L.nz, iz = p % L.nz;
+        const uint32_t at = L.place + (ix + 1) * L.pitch + iz + 1;
+        uint32_t child = 0, up = 0;
+        if (l > A.l0) {
+          const LdsLevel F = lds_level(A, l - 1);
+          child = F.place + (2 * ix + 1) * F.pitch + 2 * iz + 1;
+        }
+        if (l + 1 < g.levels) {
+          const LdsLevel C = lds_level(A, l + 1);
+          up = C.place + ((ix >> 1) + 1) * C.pitch + (iz >> 1) + 1;
+        }
+        meta[L.first + p] = make_uint2(at | (child << 16), up | ((ix & 1u) << 16) | ((iz & 1u) << 17));
+        lv.d[at] = g.dinv[g.L[l].off + p];
+        for (int k = 0; k < 9; k++)  // (no coefficient leads out of the level)
+          st[9u * L.first + static_cast<uint32_t>(k) * n + p] =
+              amg_in(g.L[l], static_cast<int>(ix) + k / 3 - 1, static_cast<int>(iz) + k % 3 - 1)
+                  ? g.S[9ull * g.L[l].off + static_cast<size_t>(k) * n + p] : 0.0f;
+      }
+    }
+  }
+
+  stores_done();
+  __syncthreads();
+  if (!resident_start(ctl, ok_lds)) return;
+
+  unsigned gen = 0;
+  bool ok = true;
+  // Generation gen is complete: everyone's value 0 is there.
+  auto arrive = [&](double v) {  // after every thread's stores: publishes one value
+    stores_done();
+    __syncthreads();
+    if (tid == 0) resident_publish(ctl, gen, idx, v);
+  };
+  auto passed = [&]() {
+    ok = __syncthreads_and(ok) != 0;
+    resident_empty(ctl, gen, idx, kResWords64);
+    gen++;
+    return ok;
+  };
+  auto barrier = [&]() {
+    arrive(0.0);
+    if (tid < G) (void)resident_word(ctl, gen, tid, 0, ok);
+    return passed();
+  };
+  auto here = [](uint32_t v) { return opaque(v) & ~kOutAgg; };  // the row of a slot
+  // (sum over threads t of va, vb) in the order of block_sum2<NT>, when only
+  // threads t < used have values
+  auto sum2 = [&](double va, double vb, unsigned used, double& sa, double& sb) {
+    va = wave_sum(va);
+    vb = wave_sum(vb);
+    if (lane == 0) {
+      lds[wv] = va;
+      lds[NT / 64 + wv] = vb;
+    }
+    __syncthreads();
+    sa = lds[0];
+    sb = lds[NT / 64];
+    for (unsigned k = 1; 64 * k < used && k < NT / 64; k++) {
+      sa += lds[k];
+      sb += lds[NT / 64 + k];
+    }
+    __syncthreads();
+    sa = scalar_of(sa);
+    sb = scalar_of(sb);
+  };
+
+  long long pred[Context::kSweepPred];
+#pragma unroll
+  for (int k = 0; k < Context::kSweepPred; k++) pred[k] = A.pred[k];
+  double rr = A.rr, bb = A.bb, rr0 = 0.0, rr_prev = 0.0;
+  float p = 0.0f, q = 0.0f, d = 0.0f;
+  long long total = 0;
+  int outer = 0;
+  bool done = false, stalled = false;
+  for (;; outer++) {
+    if (!(outer == 0 && A.have_r)) {
+      // r = b - A x in FP64 (cg_init_body)
+      gather_values(win, static_cast<const double*>(A.x + lo), list, wn);
+      __syncthreads();
+      double ri = 0.0, bi = 0.0;
+      if (in) {
+        double s = A.A.diag[i] * x;
+        const double* vp = A.A.val + row.base;
+#pragma unroll
+        for (int g4 = 0; g4 < REG / 4; g4++)
+          if (static_cast<uint32_t>(4 * g4) < m) {
+            // (addresses and numbers formed here, not kept over the sweeps)
+            vp = opaque(vp);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+              const int k = 4 * g4 + u;
+              const uint32_t o = opaque(off[k >> 1]);
+              if (static_cast<uint32_t>(k) < m) s = fma(vp[64 * k], win[(o >> (16 * (k & 1))) & 0xffffu], s);
+            }
+          }
+        for (uint32_t k = REG; k < kl; k++) s = fma(row.val(k), win[lcol[(k - REG) * NT + tid]], s);
+        for (uint32_t k = kl; k < m; k++) s = fma(row.val(k), agent_load(A.x + row.col(k)), s);
+        bi = A.b[i];
+        ri = bi - s;
+        agent_store(A.r64 + i, ri);
+      }
+      double sr_ = wave_sum(in ? fma(ri, ri, 0.0) : 0.0), sb_ = wave_sum(in ? fma(bi, bi, 0.0) : 0.0);
+      if (lane == 0) {
+        lds[wv] = sr_;
+        lds[NT / 64 + wv] = sb_;
+      }
+      stores_done();
+      __syncthreads();
+      if (tid == 0) {
+        double t = lds[0], v = lds[NT / 64];
+#pragma unroll
+        for (int k = 1; k < NT / 64; k++) {
+          t += lds[k];
+          v += lds[NT / 64 + k];
+        }
+        resident_publish(ctl, gen, idx, t, v);
+      }
+      double va = 0.0, vb = 0.0;
+      if (tid < G) resident_words(ctl, gen, tid, 0, ok, va, vb);
+      if (!passed()) return;
+      sum2(va, vb, G, rr, bb);
+    }
+    // refine's decisions
+    if (outer == 0) rr0 = rr;
+    stalled = outer > 0 && !(rr < 0.5 * rr_prev);
+    rr_prev = rr;
+    double target;
+    if (A.sr.rule == MPS_STOP_RHS_NORM) {
+      target = (A.sr.tol * A.sr.tol) * bb;
+      done = rr <= target;
+    } else {
+      target = rr0 * A.sr.tol * A.sr.tol;
+      done = (outer == 0) ? (target == 0) : (rr < target);
+    }
+    if (done || stalled || outer >= 64 || total >= A.total_cap || !(rr == rr)) break;
+    const double norm = sqrt(rr), inv_norm = 1.0 / norm;
+    const double need = 0.5 * sqrt(target / rr);
+    const double tol_rel = (A.inner_tol < need) ? need : A.inner_tol;
+
+    // ---- one FP32 sweep ----
+    const int sw = outer < Context::kSweepPred - 1 ? outer : Context::kSweepPred - 1;
+    d = p = q = 0.0f;
+    float alpha = 0.0f;
+    double rho = 0.0, rho_prev = 0.0, rr32 = 0.0, h1 = 0.0, h2 = 0.0, tol = 0.0;  // h1, h2: older r.r
+    long long predicted = 0;
+#pragma unroll
+    for (int k = 0; k < Context::kSweepPred; k++)
+      if (k == sw) predicted = pred[k];
+    long long inner = 0, chunk_end = predicted > 0 ? predicted + 2 : 32;
+    double rr_last = -1.0;
+    int flat = 0;
+    for (long long it = 0;; it++) {
+      if (it > 0) {
+        // k_ml_spmv(it): r.z and r.r of the preconditioner's last pass
+        double va = 0.0, vb = 0.0;
+        if ((tid >> 1) < G) resident_words(ctl, gen, tid >> 1, 2 * (tid & 1), ok, va, vb);
+        if (((tid + NT) >> 1) < G) {
+          double vc, vd;
+          resident_words(ctl, gen, (tid + NT) >> 1, 2 * (tid & 1), ok, vc, vd);
+          va += vc;
+          vb += vd;
+        }
+        if (!passed()) return;
+        rho_prev = rho;
+        h2 = h1;
+        h1 = rr32;
+        sum2(va, vb, 2 * G, rho, rr32);
+        // run_inner's checks, where the launched solve would have read the status
+        // (after the iterations up to it - 1: their r.r up to it - 2)
+        if (it - 1 >= A.limit) {
+          inner = A.limit;
+          d = fmaf(alpha, p, d);
+          break;
+        }
+        if (it - 1 == chunk_end) {
+          const bool even = (it & 1) == 0;  // r.r of even iterations in rr[0]
+          const double e0 = even ? h1 : h2, e1 = even ? h2 : h1;
+          const double now = (e1 < e0) ? e1 : e0;
+          flat = (rr_last > 0 && !(now < 0.81 * rr_last)) ? flat + 1 : 0;
+          rr_last = now;
+          if (flat >= 2) {
+            inner = it - 1;
+            d = fmaf(alpha, p, d);
+            break;
+          }
+          const long long c4 = (it - 1) / 4;
+          chunk_end = it - 1 + (c4 < 8 ? 8 : (c4 > 256 ? 256 : c4));
+        }
+        if (it == 1) tol = rr32 * tol_rel * tol_rel;
+        if ((it == 1) ? (tol == 0) : (rr32 < tol)) {
+          inner = it - 1;
+          if (it > 1) d = fmaf(alpha, p, d);
+          break;
+        }
+        // q = A z + beta q, p = z + beta p
+        float* const zl = reinterpret_cast<float*>(win);
+        gather_values(zl, static_cast<const float*>(A.z + lo), list, wn);
+        __syncthreads();
+        if (in) {
+          const float zi = zl[own];
+          float s = ghost * zi;
+#pragma unroll
+          for (int g = 0; g < REG / 4; g++)
+            if (static_cast<uint32_t>(4 * g) < m) {
+              const uint32_t o0 = opaque(off[2 * g]), o1 = opaque(off[2 * g + 1]);
+              // entries past the row's end: factor 0, the row's own z
+              const float x0 = zl[o0 & 0xffffu], x1 = zl[o0 >> 16], x2 = zl[o1 & 0xffffu], x3 = zl[o1 >> 16];
+              s = fmaf(cf[4 * g], x0 - zi, s);
+              s = fmaf(cf[4 * g + 1], x1 - zi, s);
+              s = fmaf(cf[4 * g + 2], x2 - zi, s);
+              s = fmaf(cf[4 * g + 3], x3 - zi, s);
+            }
+          for (uint32_t k = 0; k + REG < kl; k += 4) {
+            float c4[4], x4[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+              c4[u] = lval[(k + u) * NT + tid];
+              x4[u] = zl[lcol[(k + u) * NT + tid]];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) s = fmaf(c4[u], x4[u] - zi, s);
+          }
+          for (uint32_t k = kl; k < m; k++) {
+            const uint32_t j = row.col(k);
+            s = fmaf(coef(j), agent_load(A.z + j) - zi, s);
+          }
+          if (it == 1) {
+            p = zi;
+            q = s;
+          } else {
+            const float beta = static_cast<float>(rho / rho_prev);
+            d = fmaf(alpha, p, d);
+            p = fmaf(beta, p, zi);
+            q = fmaf(beta, q, s);
+          }
+          agent_store(A.q + i, q);
+        }
+        const double pq1 = wave_sum(in ? fma(static_cast<double>(p), static_cast<double>(q), 0.0) : 0.0);
+        if (lane == 0) lds[wv] = pq1;
+        stores_done();
+        __syncthreads();
+        if (tid == 0) {
+          double t = lds[0];
+#pragma unroll
+          for (int k = 1; k < NT / 64; k++) t += lds[k];
+          resident_publish(ctl, gen, idx, t);
+        }
+        load_q9s();
+        // alpha, as k_ml_prec's blocks of NTP threads sum it
+        double v = 0.0;
+        if (tid < NTP) {
+          if (tid < G) v = resident_word(ctl, gen, tid, 0, ok);
+          if (tid + NTP < G) v += resident_word(ctl, gen, tid + NTP, 0, ok);
+        }
+        if (!passed()) return;
+        v = wave_sum(v);
+        if (lane == 0) lds[wv] = v;
+        __syncthreads();
+        double pq = lds[0];
+        for (unsigned k = 1; k < NTP / 64 && 64 * k < G; k++) pq += lds[k];
+        __syncthreads();
+        alpha = static_cast<float>(scalar_of(rho / pq));
+      }
+
+      // ---- the preconditioner's pass it ----
+      if (it == 0) load_q9s();
+      float s = 0.0f;
+      double prho = 0.0, prr = 0.0;
+      if (active) {
+        if (it == 0) {
+          double t[kPerLane];
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++) t[u] = id[u] != kNoSlot ? agent_load(A.r64 + here(id[u])) : 0.0;
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++) rv[u] = static_cast<float>(t[u] * inv_norm);
+        } else {
+          float t[kPerLane];
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++) t[u] = id[u] != kNoSlot ? agent_load(A.q + here(id[u])) : 0.0f;
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++) rv[u] = fmaf(-alpha, t[u], rv[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kPerLane; u++)
+          if (id[u] != kNoSlot) {
+            if (!(id[u] & kOutAgg)) s += rv[u];
+            prr = fma(static_cast<double>(rv[u]), static_cast<double>(rv[u]), prr);
+          }
+      }
+      if constexpr (!AMG) {
+        if (active) {
+          float y0, y1, y2;
+          agg_sums(s, y0, y1, y2);
+          const float corr = y0 * scl.x + y1 * scl.y + y2 * scl.z;
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++)
+            if (id[u] != kNoSlot) {
+              const float zi = (id[u] & kOutAgg) ? dv[u] * rv[u] : fmaf(dv[u], rv[u], corr);
+              agent_store(A.z + here(id[u]), zi);
+              prho = fma(static_cast<double>(rv[u]), static_cast<double>(zi), prho);
+            }
+        }
+      } else {
+        // pass 1: the cells' direction sums of P_s^T r
+        if (active) {
+          float t9[9];
+#pragma unroll
+          for (int e = 0; e < 9; e++) t9[e] = 0.0f;
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++)
+            if (id[u] != kNoSlot && !(id[u] & kOutAgg)) {
+              float qv9[9];
+              row9(u, qv9);
+#pragma unroll
+              for (int e = 0; e < 9; e++) t9[e] = fmaf(qv9[e], rv[u], t9[e]);
+            }
+          t9[4] += 0.0f;  // (no members beyond the registers)
+#pragma unroll
+          for (int e = 0; e < 9; e++) {
+            const float t = cell_sum(t9[e]);
+            if (pt >= 0 && sub == 0)
+              agent_store(a.tq + static_cast<size_t>(e) * a.tq_stride + static_cast<uint32_t>(opaque(pt)), t);
+          }
+        }
+        if (!barrier()) return;
+        // the cycle: down to level l0, spread over the workgroups
+        const AmgLevel F = g.L[0];
+        int l = 0;
+        if (A.l0 >= 2) {
+          const AmgLevel L1 = g.L[1], L2 = g.L[2];
+          const uint32_t tnz = (L2.nz + kTile2 - 1) / kTile2, nt = ((L2.nx + kTile2 - 1) / kTile2) * tnz;
+          for (uint32_t t = idx; t < nt; t += G) {
+            const int X2 = static_cast<int>(t / tnz) * kTile2, Z2 = static_cast<int>(t % tnz) * kTile2;
+            const int x1 = 2 * X2 - 1, z1 = 2 * Z2 - 1;  // level-1 region with halo: kF1 x kF1 from here
+            const int x0 = 2 * x1, z0 = 2 * z1;          // its children: kC0 x kC0
+            const int th = opaque(static_cast<int>(tid));
+            // level 0's right-hand side with halo
+            if (th < kF0 * kF0) {
+              const int ix = x0 - 1 + th / kF0, iz = z0 - 1 + th % kF0;
+              const bool inside = amg_in(F, ix, iz);
+              const int jx = inside ? ix : 0, jz = inside ? iz : 0;
+              const float r = amg_rfix_at<true>(a.tq, a.tq_stride, F.nx, F.nz, jx, jz);
+              const float di = g.dinv[static_cast<uint32_t>(jx) * F.nz + static_cast<uint32_t>(jz)];
+              tile_r[th] = inside ? r : 0.0f;
+              tile_d[th] = inside ? di : 0.0f;
+            }
+            __syncthreads();
+            if (th < kC0 * kC0) {
+              const int cx = th / kC0, cz = th % kC0, ix = x0 + cx, iz = z0 + cz;
+              float c = 0.0f;
+              if (amg_in(F, ix, iz)) {
+                const uint32_t p0 = static_cast<uint32_t>(ix) * F.nz + static_cast<uint32_t>(iz), np = amg_npts(F);
+                float sv[9], sum = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 9; e++) sv[e] = g.S[static_cast<size_t>(e) * np + p0];
+#pragma unroll
+                for (int e = 0; e < 9; e++) {
+                  const int o = (cx + e / 3) * kF0 + cz + e % 3;
+                  sum = fmaf(sv[e], g.omega * tile_d[o] * tile_r[o], sum);
+                }
+                const int o = (cx + 1) * kF0 + cz + 1;
+                if (cx >= 2 && cx < kC0 - 2 && cz >= 2 && cz < kC0 - 2) {  // this tile's own
+                  agent_store(g.x + p0, g.omega * tile_d[o] * tile_r[o]);
+                  agent_store(g.r + p0, tile_r[o]);
+                }
+                c = tile_r[o] - sum;
+              }
+              tile_c[th] = c;
+            }
+            __syncthreads();
+            if (th < kF1 * kF1) {
+              const int px = th / kF1, pz = th % kF1, ix = x1 + px, iz = z1 + pz;
+              float rc = 0.0f, di = 0.0f;
+              if (amg_in(L1, ix, iz)) {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                  if (amg_in(F, 2 * ix + e / 2, 2 * iz + e % 2)) rc += tile_c[(2 * px + e / 2) * kC0 + 2 * pz + e % 2];
+                const uint32_t p1 = L1.off + static_cast<uint32_t>(ix) * L1.nz + static_cast<uint32_t>(iz);
+                di = g.dinv[p1];
+                if (px >= 1 && px < kF1 - 1 && pz >= 1 && pz < kF1 - 1) agent_store(g.r + p1, rc);
+              }
+              tile1_r[th] = rc;
+              tile1_d[th] = di;
+            }
+            __syncthreads();
+            if (th < kC1 * kC1) {
+              const int cx = th / kC1, cz = th % kC1, ix = 2 * X2 + cx, iz = 2 * Z2 + cz;
+              float c = 0.0f;
+              if (amg_in(L1, ix, iz)) {
+                const uint32_t p1 = static_cast<uint32_t>(ix) * L1.nz + static_cast<uint32_t>(iz), np = amg_npts(L1);
+                float sv[9], sum = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 9; e++) sv[e] = g.S[9ull * L1.off + static_cast<size_t>(e) * np + p1];
+#pragma unroll
+                for (int e = 0; e < 9; e++) {
+                  const int o = (cx + e / 3) * kF1 + cz + e % 3;
+                  sum = fmaf(sv[e], g.omega * tile1_d[o] * tile1_r[o], sum);
+                }
+                const int o = (cx + 1) * kF1 + cz + 1;
+                agent_store(g.x + L1.off + p1, g.omega * tile1_d[o] * tile1_r[o]);
+                c = tile1_r[o] - sum;
+              }
+              tile1_c[th] = c;
+            }
+            __syncthreads();
+            if (th < kTile2 * kTile2) {
+              const int px = th / kTile2, pz = th % kTile2, ix = X2 + px, iz = Z2 + pz;
+              if (amg_in(L2, ix, iz)) {
+                float rc = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                  if (amg_in(L1, 2 * ix + e / 2, 2 * iz + e % 2)) rc += tile1_c[(2 * px + e / 2) * kC1 + 2 * pz + e % 2];
+                agent_store(g.r + L2.off + static_cast<uint32_t>(ix) * L2.nz + static_cast<uint32_t>(iz), rc);
+              }
+            }
+            __syncthreads();
+          }
+          if (!barrier()) return;
+          l = 2;
+        }
+        for (; l < A.l0; l++) {
+          const AmgLevel D = g.L[l], C = g.L[l + 1];
+          const uint32_t tnz = (C.nz + kTile - 1) / kTile, nt = ((C.nx + kTile - 1) / kTile) * tnz;
+          for (uint32_t t = idx; t < nt; t += G) {
+            const int X0 = static_cast<int>(t / tnz) * kTile, Z0 = static_cast<int>(t % tnz) * kTile;
+            const int th = opaque(static_cast<int>(tid));
+            if (th < kTileF * kTileF) {
+              const int ix = 2 * X0 - 1 + th / kTileF, iz = 2 * Z0 - 1 + th % kTileF;
+              const bool inside = amg_in(D, ix, iz);
+              const int jx = inside ? ix : 0, jz = inside ? iz : 0;
+              const uint32_t pc = D.off + static_cast<uint32_t>(jx) * D.nz + static_cast<uint32_t>(jz);
+              const float r = l == 0 ? amg_rfix_at<true>(a.tq, a.tq_stride, D.nx, D.nz, jx, jz) : agent_load(g.r + pc);
+              const float di = g.dinv[pc];
+              tile_r[th] = inside ? r : 0.0f;
+              tile_d[th] = inside ? di : 0.0f;
+            }
+            __syncthreads();
+            if (th < 4 * kTile * kTile) {
+              const int cx = th / (2 * kTile), cz = th % (2 * kTile), ix = 2 * X0 + cx, iz = 2 * Z0 + cz;
+              float c = 0.0f;
+              if (amg_in(D, ix, iz)) {
+                const uint32_t pc = static_cast<uint32_t>(ix) * D.nz + static_cast<uint32_t>(iz), np = amg_npts(D);
+                float sv[9], sum = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 9; e++) sv[e] = g.S[9ull * D.off + static_cast<size_t>(e) * np + pc];
+#pragma unroll
+                for (int e = 0; e < 9; e++) {
+                  const int o = (cx + e / 3) * kTileF + cz + e % 3;
+                  sum = fmaf(sv[e], g.omega * tile_d[o] * tile_r[o], sum);
+                }
+                const int o = (cx + 1) * kTileF + cz + 1;
+                agent_store(g.x + D.off + pc, g.omega * tile_d[o] * tile_r[o]);
+                if (l == 0) agent_store(g.r + pc, tile_r[o]);
+                c = tile_r[o] - sum;
+              }
+              tile_c[th] = c;
+            }
+            __syncthreads();
+            if (th < kTile * kTile) {
+              const int px = th / kTile, pz = th % kTile, X = X0 + px, Z = Z0 + pz;
+              if (amg_in(C, X, Z)) {
+                float rc = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                  if (amg_in(D, 2 * X + e / 2, 2 * Z + e % 2)) rc += tile_c[(2 * px + e / 2) * 2 * kTile + 2 * pz + e % 2];
+                agent_store(g.r + C.off + static_cast<uint32_t>(X) * C.nz + static_cast<uint32_t>(Z), rc);
+              }
+            }
+            __syncthreads();
+          }
+          if (!barrier()) return;
+        }
+        // levels l0 .. in LDS, in every workgroup alike
+        {
+          const int levels = g.levels;
+          const LdsLevel T = lds_level(A, A.l0);
+          const uint32_t n0 = T.nx * T.nz;
+          const bool one = A.l0 == levels - 1;
+          for (uint32_t k = tid; k < n0; k += NT) {
+            const float r = A.l0 >= 1 ? agent_load(g.r + g.L[A.l0].off + k)
+                                      : amg_rfix_at<true>(a.tq, a.tq_stride, F.nx, F.nz, static_cast<int>(k / F.nz),
+                                                        static_cast<int>(k % F.nz));
+            if (one) lv.last[k] = r;
+            else lv.r[lv.meta[k].x & 0xffffu] = r;
+          }
+          __syncthreads();
+          for (int c = A.l0; c + 1 < levels; c++) {
+            lds_down(lv, lds_level(A, c), lds_level(A, c + 1), g.omega, c + 2 == levels);
+            __syncthreads();
+          }
+          const LdsLevel B = lds_level(A, levels - 1);
+          const uint32_t nb = B.nx * B.nz;
+          for (uint32_t r0 = tid >> 4; r0 < nb; r0 += NT / 16) {  // 16 lanes per row of the coarsest inverse
+            const uint32_t part = tid & 15;
+            float t = 0.0f;
+            for (uint32_t k = part; k < nb; k += 16) t = fmaf(lv.inv[r0 * nb + k], lv.last[k], t);
+#pragma unroll
+            for (int o = 8; o >= 1; o >>= 1) t += __shfl_xor(t, o, 16);
+            if (part == 0) lv.e[lv.meta[B.first + r0].x & 0xffffu] = t;
+          }
+          __syncthreads();
+          for (int c = levels - 2; c >= A.l0; c--) {
+            lds_up(lv, lds_level(A, c), lds_level(A, c + 1), g.omega, g.corr);
+            __syncthreads();
+          }
+        }
+        // up from level l0 - 1 to 2, spread over the workgroups
+        for (int c = A.l0 - 1; c >= 2; c--) {
+          const AmgLevel D = g.L[c];
+          const uint32_t nl = amg_npts(D);
+          for (uint32_t k = idx * NT + tid; k < nl; k += G * NT) {
+            const int ix = static_cast<int>(k / D.nz), iz = static_cast<int>(k % D.nz);
+            float ev[9];
+            up_parents(A, lv, c, ix, iz, ev);
+            agent_store(g.e + D.off + k, up_with(A, c, ix, iz, ev));
+          }
+          if (!barrier()) return;
+        }
+        // pass 2, with the up steps of levels 1 and 0 where those are not in LDS:
+        // lanes 0 .. 35 take the wavefront's 6x6 cells (its 4x4 block and their
+        // neighbours), lanes 0 .. 24 the 5x5 points of level 1 that the up step
+        // of those cells may ask for
+        if (active) {
+          float e9[9];
+          const int ln = static_cast<int>(opaque(lane));
+          const int cx0 = static_cast<int>(4 * (blk / a.G.bnz)) - 1 - static_cast<int>(a.bx0);
+          const int cz0 = static_cast<int>(4 * (blk % a.G.bnz)) - 1 - static_cast<int>(a.bz0);
+          if (A.l0 >= 1) {
+            const int cx = cx0 + ln / 6, cz = cz0 + ln % 6;
+            const bool mine = ln < 36 && amg_in(F, cx, cz);
+            float ev[9];
+            if (A.l0 >= 2) {
+              const int px0 = (cx0 - 1) >> 1, pz0 = (cz0 - 1) >> 1;  // floors, also below 0
+              const int X = px0 + ln / 5, Z = pz0 + ln % 5;
+              float e1 = 0.0f;
+              if (ln < 25 && amg_in(g.L[1], X, Z)) {
+                float ew[9];
+                up_parents(A, lv, 1, X, Z, ew);
+                e1 = up_with(A, 1, X, Z, ew);
+              }
+#pragma unroll
+              for (int e = 0; e < 9; e++) {
+                const int ux = ((cx + e / 3 - 1) >> 1) - px0, uz = ((cz + e % 3 - 1) >> 1) - pz0;
+                ev[e] = __shfl(e1, 5 * ux + uz, 64);  // (lanes past the 36 take some lane's)
+              }
+            } else if (mine) {
+              up_parents(A, lv, 0, cx, cz, ev);
+            }
+            const float val = mine ? up_with(A, 0, cx, cz, ev) : 0.0f;
+            const int ux = (ln & 15) >> 2, uz = ln & 3;
+#pragma unroll
+            for (int e = 0; e < 9; e++) e9[e] = __shfl(val, (ux + e / 3) * 6 + (uz + e % 3), 64);
+          } else {
+            const LdsLevel T = lds_level(A, 0);
+            const int ux = (ln & 15) >> 2, uz = ln & 3;
+            // the lane's cell and its neighbours on the bordered grid; cells further out are empty
+            const int cx = cx0 + 1 + ux, cz = cz0 + 1 + uz;
+#pragma unroll
+            for (int e = 0; e < 9; e++) {
+              const int X = cx + e / 3 - 1, Z = cz + e % 3 - 1;
+              const bool inside = pt >= 0 && amg_in(F, X, Z);
+              e9[e] = lv.e[T.place + (inside ? static_cast<uint32_t>(X + 1) * T.pitch + static_cast<uint32_t>(Z + 1) : 0u)];
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < kPerLane; u++)
+            if (id[u] != kNoSlot) {
+              float zi;
+              if (id[u] & kOutAgg) {
+                zi = dv[u] * rv[u];
+              } else {
+                float qv9[9];
+                row9(u, qv9);
+                float ez = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 9; e++) ez = fmaf(qv9[e], e9[e], ez);
+                zi = fmaf(a.omega * dv[u], rv[u], ez);
+              }
+              agent_store(A.z + here(id[u]), zi);
+              prho = fma(static_cast<double>(rv[u]), static_cast<double>(zi), prho);
+            }
+        }
+      }
+      // z is out: r.z and r.r of each 4 blocks of cells (k_ml_prec's blocks)
+      prho = wave_sum(prho);
+      prr = wave_sum(prr);
+      if (lane == 0) {
+        lds[wv] = prho;
+        lds[NT / 64 + wv] = prr;
+      }
+      stores_done();
+      __syncthreads();
+      if (tid == 0) {
+        double t[2], v[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          t[h] = lds[4 * h];
+          v[h] = lds[NT / 64 + 4 * h];
+#pragma unroll
+          for (int k = 1; k < 4; k++) {
+            t[h] += lds[4 * h + k];
+            v[h] += lds[NT / 64 + 4 * h + k];
+          }
+        }
+        resident_publish(ctl, gen, idx, t[0], v[0], t[1], v[1]);
+      }
+    }
+    // x += |r| d, visible to everyone before the next residual
+#pragma unroll
+    for (int k = 0; k < Context::kSweepPred; k++)
+      if (k == sw) pred[k] = inner;
+    total += inner;
+    if (in) {
+      x = fma(static_cast<double>(d), norm, x);
+      agent_store(A.x + i, x);
+    }
+    if (!barrier()) return;
+  }
+  if (in) {  // what the launched solve leaves in its vectors
+    A.p[i] = p;
+    A.d[i] = d;
+  }
+  if (idx == 0 && tid == 0) {
+    MixedResult* o = reinterpret_cast<MixedResult*>(ctl->out);
+    o->rr0 = rr0;
+    o->rr = rr;
+    o->bb = bb;
+    o->total = total;
+#pragma unroll
+    for (int k = 0; k < Context::kSweepPred; k++) o->pred[k] = pred[k];
+    o->outer = outer;
+    o->done = done ? 1 : 0;
+    o->stalled = stalled ? 1 : 0;
   }
 }
 
@@ -2722,6 +3758,35 @@ namespace {
 // adds |r| d to x in FP64 and recomputes r = b - A x in FP64.
 long long max_iter_fallback(const Context& c) { return static_cast<long long>(c.ppe_n); }
 
+// The FP32 sweeps no longer make progress: the plain FP64 CG (the reference
+// algorithm) finishes from the current x, to the same target.
+void refine_fallback(Context& c, const StopRule& sr, double rr0, double rr, long long total, int outer) {
+  StopRule rest = sr;
+  if (sr.rule == MPS_STOP_INITIAL_RESIDUAL) rest.tol = sr.tol * std::sqrt(rr0 / rr);
+  const long long cap = c.solver.max_iter > 0 ? c.solver.max_iter - total : max_iter_fallback(c);
+  solve_cg64(c, rest, cap);
+  c.stats.iterations += total;
+  c.stats.outer_iterations = outer + 1;
+  c.stats.rr0 = rr0;
+  c.stats.fallback = 1;
+}
+
+// What a refinement that did not fall back leaves in the context; throws if
+// the target was not met.
+void refine_finished(Context& c, bool done, long long total, int outer, double rr0, double rr, double bb) {
+  c.stats.iterations = total;
+  c.stats.outer_iterations = outer;
+  c.stats.rr0 = rr0;
+  c.stats.rr = rr;
+  c.last_iters = total;
+  // rr, bb: the FP64 residual of the returned x
+  c.final_rr = rr;
+  c.final_bb = bb;
+  if (!done)
+    throw Failure{MPS_ERR_CG_NOT_CONVERGED,
+                  "Conjugate Gradient method couldn't solve Pressure Poison Equation"};
+}
+
 template <class Sweep, class Correct>
 void refine(Context& c, const StopRule& sr, Sweep sweep, Correct correct) {
   const double inner_tol = c.solver.inner_tol > 0 ? c.solver.inner_tol : 1e-4;
@@ -2750,16 +3815,7 @@ void refine(Context& c, const StopRule& sr, Sweep sweep, Correct correct) {
       done = (outer == 0) ? (target == 0) : (rr < target);
     }
     if (stalled && !done && rr == rr && total < total_cap) {
-      // the FP32 sweeps no longer make progress: the plain FP64 CG (the
-      // reference algorithm) finishes from the current x, to the same target
-      StopRule rest = sr;
-      if (sr.rule == MPS_STOP_INITIAL_RESIDUAL) rest.tol = sr.tol * std::sqrt(rr0 / rr);
-      const long long cap = c.solver.max_iter > 0 ? c.solver.max_iter - total : max_iter_fallback(c);
-      solve_cg64(c, rest, cap);
-      c.stats.iterations += total;
-      c.stats.outer_iterations = outer + 1;
-      c.stats.rr0 = rr0;
-      c.stats.fallback = 1;
+      refine_fallback(c, sr, rr0, rr, total, outer);
       return;
     }
     if (done || stalled || outer >= max_outer || total >= total_cap || !(rr == rr)) break;
@@ -2774,17 +3830,7 @@ void refine(Context& c, const StopRule& sr, Sweep sweep, Correct correct) {
     correct(norm);
     check_launch();
   }
-  c.stats.iterations = total;
-  c.stats.outer_iterations = outer;
-  c.stats.rr0 = rr0;
-  c.stats.rr = rr;
-  c.last_iters = total;
-  // rr, bb: the FP64 residual of the returned x, computed above
-  c.final_rr = rr;
-  c.final_bb = bb;
-  if (!done)
-    throw Failure{MPS_ERR_CG_NOT_CONVERGED,
-                  "Conjugate Gradient method couldn't solve Pressure Poison Equation"};
+  refine_finished(c, done, total, outer, rr0, rr, bb);
 }
 
 long long inner_limit(const Context& c, long long max_iter) {
@@ -2914,6 +3960,32 @@ CellGrid ml_grid(const Context& c, const MlGeom& g) {
                   g.off1, g.off2};
 }
 
+// The list of the 4x4 blocks of cells that hold particles, from the search's
+// cell counts, and its length on its way to the host, on c.stream.
+}  // namespace
+void enqueue_block_list(Context& c) {
+  const MlGeom g = ml_geom(c);
+  if (c.ml_blk_cap < g.nblk) {
+    dfree(c.ml_flag);
+    dfree(c.ml_off);
+    dfree(c.ml_list);
+    c.ml_flag = dalloc<uint32_t>(g.nblk);
+    c.ml_off = dalloc<uint32_t>(g.nblk);
+    c.ml_list = dalloc<uint32_t>(g.nblk);
+    c.ml_blk_cap = g.nblk;
+  }
+  if (!c.ml_active) c.ml_active = dalloc<uint64_t>(1);
+  hipLaunchKernelGGL(k_ml_active, dim3(grid_for(g.nblk)), dim3(256), 0, c.stream, ml_grid(c, g), c.ml_flag);
+  scan_counts(c, c.ml_flag, g.nblk, c.ml_off, c.ml_active);
+  hipLaunchKernelGGL(k_ml_compact, dim3(grid_for(g.nblk)), dim3(256), 0, c.stream, static_cast<uint32_t>(g.nblk),
+                     static_cast<const uint32_t*>(c.ml_flag), static_cast<const uint32_t*>(c.ml_off), c.ml_list);
+  MPS_HIP(hipMemcpyAsync(c.ml_active_host, c.ml_active, sizeof(uint64_t), hipMemcpyDeviceToHost, c.stream));
+  check_launch();
+  c.ml_list_serial = c.search_serial;
+}
+namespace {
+bool block_list_ready(const Context& c) { return c.ml_list_serial == c.search_serial; }
+
 // The multilevel solver's set-up on c.stream, which does not depend on the
 // initial guess: Jacobi factors, the aggregate sums of A from the FP64 system
 // (row sums in z, r, d as scratch, unless the fill of this system summed the
@@ -2935,21 +4007,10 @@ void ml_setup(Context& c) {
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
   }
-  if (c.ml_blk_cap < g.nblk) {
-    dfree(c.ml_flag);
-    dfree(c.ml_off);
-    dfree(c.ml_list);
-    c.ml_flag = dalloc<uint32_t>(g.nblk);
-    c.ml_off = dalloc<uint32_t>(g.nblk);
-    c.ml_list = dalloc<uint32_t>(g.nblk);
-    c.ml_blk_cap = g.nblk;
-  }
-  if (!c.ml_active) c.ml_active = dalloc<uint64_t>(1);
   const CellGrid G = ml_grid(c, g);
   const bool sums = c.ml_rowsums_ready;
   c.ml_rowsums_ready = false;
-  tracked(c, MPS_K_ML_SETUP, (sums ? 0.0 : c.nnz_offdiag * 12.0 + n * 17.0) + n * 20.0 + g.total_aggs * 4.0 +
-                                 g.nblk * 12.0, [&] {
+  tracked(c, MPS_K_ML_SETUP, (sums ? 0.0 : c.nnz_offdiag * 12.0 + n * 17.0) + n * 20.0 + g.total_aggs * 4.0, [&] {
     if (!sums)
       hipLaunchKernelGGL(k_ml_rowsum, dim3(L.grid), dim3(NT), 0, c.stream,
                          sell<double>(c, c.sval, c.diag, L.rpb), static_cast<const uint32_t*>(c.row_len),
@@ -2958,99 +4019,9 @@ void ml_setup(Context& c) {
     hipLaunchKernelGGL(k_ml_setup, dim3(static_cast<unsigned>(g.sgrid)), dim3(NTP), 0, c.stream, G,
                        static_cast<const float*>(c.z32), static_cast<const float*>(c.r32),
                        static_cast<const float*>(c.d32), c.agg_inv);
-    hipLaunchKernelGGL(k_ml_active, dim3(grid_for(g.nblk)), dim3(256), 0, c.stream, G, c.ml_flag);
-    scan_counts(c, c.ml_flag, g.nblk, c.ml_off, c.ml_active);
-    hipLaunchKernelGGL(k_ml_compact, dim3(grid_for(g.nblk)), dim3(256), 0, c.stream, static_cast<uint32_t>(g.nblk),
-                       static_cast<const uint32_t*>(c.ml_flag), static_cast<const uint32_t*>(c.ml_off),
-                       c.ml_list);
   });
-  MPS_HIP(hipMemcpyAsync(c.ml_active_host, c.ml_active, sizeof(uint64_t), hipMemcpyDeviceToHost, c.stream));
   check_launch();
-}
-
-void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max_iter) {
-  const size_t n = c.ppe_n;
-  const Launch L = cg_grid(n);
-  ensure_zrec(c, n);
-  const MatFreeRec A = matfree_rec(c, L.rpb);
-  float* const zval = reinterpret_cast<float*>(c.zrec) + 2;  // z_i at zval[4 i]
-  if (!join_ml_setup(c)) ml_setup(c);  // enqueued ahead on the auxiliary stream, or now
-  const MlGeom g = ml_geom(c);
-  const size_t stride = c.part_ml_cap;
-  const CellGrid G = ml_grid(c, g);
-  // rows outside every cell keep r = d = z = 0; the records take the positions
-  hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
-                     c.zrec, c.r32, c.d32);
-  check_launch();
-  double* p_pq = c.part3b;
-  const long long limit = inner_limit(c, max_iter);
-  // per particle: r (read, written), q, z; per slot of the packed layout: id
-  // and Jacobi factor; per lane: the aggregate scales (set once nact is known)
-  double b_prec = n * 16.0;
-  uint32_t nact = 0;
-  size_t pgrid = 1;
-  bool packed = false;
-  auto prec = [&](double norm, long long it) {
-    const PrecArgs a{G,      c.ml_list, nact,   c.ml_pid, c.ml_dv, c.ml_sc,   c.r,       1.0 / norm,
-                     c.r32,  c.d32,     c.q32,  c.dinv32, zval,    4u,        p_pq,      L.grid,
-                     c.part_ml, stride, c.st32};
-    hipLaunchKernelGGL(k_ml_prec<0>, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, a, it);
-  };
-  double b_spmv = b_base;
-  c.replay_ready = MPS_K_CG_SPMV32;
-  refine(c, sr, [&](double norm, double sweep_tol) {
-    // refine() has synchronised the stream (residual) before every sweep: the
-    // block count and the wide nnz are on the host
-    nact = static_cast<uint32_t>(*c.ml_active_host);
-    b_spmv = b_base + 2.0 * mf_nnz_wide(c);
-    pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
-    b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
-    if (!packed) {
-      const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
-      if (c.ml_pack_cap < slots) {
-        dfree(c.ml_pid);
-        dfree(c.ml_dv);
-        dfree(c.ml_sc);
-        c.ml_pid = dalloc<uint32_t>(slots * kPerLane);
-        c.ml_dv = dalloc<float>(slots * kPerLane);
-        c.ml_sc = dalloc<float4>(slots);
-        c.ml_pack_cap = slots;
-      }
-      tracked(c, MPS_K_ML_SETUP, n * 13.0 + slots * (8.0 * kPerLane + 16), [&] {
-        hipLaunchKernelGGL(k_ml_pack, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, G,
-                           static_cast<const uint32_t*>(c.ml_list), nact, static_cast<const float*>(c.agg_inv),
-                           static_cast<const float*>(c.dinv32), c.ml_pid, c.ml_dv, c.ml_sc,
-                           static_cast<const uint32_t*>(nullptr));
-      });
-      packed = true;
-    }
-    MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
-    tracked(c, MPS_K_CG_INIT32, n * 25.0, [&] { prec(norm, 0); });
-    long long launched = 0;
-    const long long inner = run_inner(c, limit, [&](long long it) {
-      tracked(c, MPS_K_CG_SPMV32, b_spmv, [&] {
-        const SpmvArgs<MatFreeRec> a{A,      nullptr, c.pa32,  c.q32, c.d32, c.part_ml, stride,
-                                     static_cast<int>(pgrid), p_pq, c.st32, sweep_tol};
-        if (it == 1)
-          hipLaunchKernelGGL((k_ml_spmv<true, MatFreeRec>), dim3(L.grid), dim3(NT), 0, c.stream, a, it);
-        else
-          hipLaunchKernelGGL((k_ml_spmv<false, MatFreeRec>), dim3(L.grid), dim3(NT), 0, c.stream, a, it);
-      }, it);
-      tracked(c, MPS_K_ML_PREC, b_prec, [&] { prec(norm, it); }, it);
-      launched = it;
-    });
-    if (!c.st32_host->converged && launched > 0)
-      hipLaunchKernelGGL(k_ml_finish, dim3(grid_for(n)), dim3(256), 0, c.stream, n,
-                         static_cast<const CgStatus*>(c.st32), static_cast<const float*>(c.pa32), c.d32);
-    // launches after the stop did no work: count them out (k_ml_spmv(inner + 1)
-    // only finished d)
-    uncount(c, MPS_K_CG_SPMV32, launched - inner, b_spmv);
-    uncount(c, MPS_K_ML_PREC, launched - inner, b_prec);
-    return inner;
-  }, [&](double norm) {
-    hipLaunchKernelGGL(k_ir_correct, dim3(grid_for(n)), dim3(256), 0, c.stream, n, c.sol,
-                       static_cast<const float*>(c.d32), norm);
-  });
+  if (!block_list_ready(c)) enqueue_block_list(c);
 }
 
 // ---- cell-grid multigrid (MPS_PRECOND_AMG) ----
@@ -3101,19 +4072,6 @@ void amg_setup(Context& c) {
   const Launch L = cg_grid(n);
   hipLaunchKernelGGL(k_jacobi_inv, dim3(grid_for(n)), dim3(256), 0, c.stream, n,
                      static_cast<const double*>(c.diag), c.dinv32);
-  // the occupied 4x4 blocks of cells, as the multilevel set-up lists them
-  const MlGeom mg = ml_geom(c);
-  if (c.ml_blk_cap < mg.nblk) {
-    dfree(c.ml_flag);
-    dfree(c.ml_off);
-    dfree(c.ml_list);
-    c.ml_flag = dalloc<uint32_t>(mg.nblk);
-    c.ml_off = dalloc<uint32_t>(mg.nblk);
-    c.ml_list = dalloc<uint32_t>(mg.nblk);
-    c.ml_blk_cap = mg.nblk;
-  }
-  if (!c.ml_active) c.ml_active = dalloc<uint64_t>(1);
-  const CellGrid G = ml_grid(c, mg);
   // level shapes
   amg_box(c);
   int lv = 0;
@@ -3156,10 +4114,6 @@ void amg_setup(Context& c) {
   const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
   tracked(c, MPS_K_ML_SETUP, (rows_ready ? 0.0 : c.nnz_offdiag * 16.0 + n * 17.0) + n * 72.0 + npts0 * 8.0 +
                                  off * 9 * 12.0, [&] {
-    hipLaunchKernelGGL(k_ml_active, dim3(grid_for(mg.nblk)), dim3(256), 0, c.stream, G, c.ml_flag);
-    scan_counts(c, c.ml_flag, mg.nblk, c.ml_off, c.ml_active);
-    hipLaunchKernelGGL(k_ml_compact, dim3(grid_for(mg.nblk)), dim3(256), 0, c.stream, static_cast<uint32_t>(mg.nblk),
-                       static_cast<const uint32_t*>(c.ml_flag), static_cast<const uint32_t*>(c.ml_off), c.ml_list);
     if (!rows_ready)
       hipLaunchKernelGGL(k_amg_rows, dim3(L.grid), dim3(NT), 0, c.stream, sell<double>(c, c.sval, c.diag, L.rpb),
                          static_cast<const uint32_t*>(c.row_len), static_cast<const uint32_t*>(c.key),
@@ -3181,8 +4135,58 @@ void amg_setup(Context& c) {
     // (level 0's right-hand side needs no clearing: k_amg_rfix writes every
     // level-0 point each cycle, from direction sums cleared per solve)
   });
-  MPS_HIP(hipMemcpyAsync(c.ml_active_host, c.ml_active, sizeof(uint64_t), hipMemcpyDeviceToHost, c.stream));
   check_launch();
+  if (!block_list_ready(c)) enqueue_block_list(c);
+}
+
+// The packed slots of the listed blocks (k_ml_pack) and, for the multigrid,
+// P_s's rows in their order; the list's length must be on the host.
+void pack_slots(Context& c, bool amg) {
+  const size_t n = c.ppe_n;
+  const MlGeom g = ml_geom(c);
+  const uint32_t nact = static_cast<uint32_t>(*c.ml_active_host);
+  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
+  const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
+  if (c.ml_pack_cap < slots) {
+    dfree(c.ml_pid);
+    dfree(c.ml_dv);
+    dfree(c.ml_sc);
+    c.ml_pid = dalloc<uint32_t>(slots * kPerLane);
+    c.ml_dv = dalloc<float>(slots * kPerLane);
+    c.ml_sc = dalloc<float4>(slots);
+    c.ml_pack_cap = slots;
+  }
+  // the multigrid's rules: no aggregate scales, rows without stored
+  // off-diagonals outside every aggregate
+  tracked(c, MPS_K_ML_SETUP, n * (amg ? 17.0 : 13.0) + slots * (8.0 * kPerLane + 16), [&] {
+    hipLaunchKernelGGL(k_ml_pack, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, ml_grid(c, g),
+                       static_cast<const uint32_t*>(c.ml_list), nact,
+                       static_cast<const float*>(amg ? nullptr : c.agg_inv), static_cast<const float*>(c.dinv32),
+                       c.ml_pid, c.ml_dv, c.ml_sc, static_cast<const uint32_t*>(amg ? c.row_len : nullptr));
+  });
+  if (amg) {
+    const size_t nslots = static_cast<size_t>(nact) * kPerLane * 64;
+    ensure_q9(c, nslots);
+    if (nslots > 0)
+      tracked(c, MPS_K_ML_SETUP, nslots * (4.0 + 18.0) + n * 80.0, [&] {
+        hipLaunchKernelGGL(k_amg_q, dim3(grid_for(nslots)), dim3(256), 0, c.stream, nslots,
+                           static_cast<const uint32_t*>(c.ml_pid), static_cast<const double*>(c.amg_rows),
+                           static_cast<const double*>(c.diag), kAmgOmegaP, c.amg_q9, c.amg_q9c);
+      });
+  }
+  check_launch();
+}
+
+// Pass 1's direction sums, cleared (those of cells in unlisted blocks stay zero).
+void clear_direction_sums(Context& c) {
+  const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
+  c.amg_tq_stride = (npts0 + 63) & ~static_cast<size_t>(63);
+  if (c.amg_tq_cap < 9 * c.amg_tq_stride) {
+    dfree(c.amg_tq);
+    c.amg_tq = dalloc<float>(9 * c.amg_tq_stride);
+    c.amg_tq_cap = 9 * c.amg_tq_stride;
+  }
+  MPS_HIP(hipMemsetAsync(c.amg_tq, 0, 9 * c.amg_tq_stride * sizeof(float), c.stream));
 }
 
 // One V-cycle on the cell-grid levels: level 0's right-hand side in, its
@@ -3217,29 +4221,232 @@ bool amg_cycle(Context& c, bool fold0, const CgStatus* st, long long it) {
   return left;
 }
 
+// LDS for the levels that every workgroup holds: of its 144 KB the gathered z
+// takes up to 25 and the matrix entries beyond the registers' 32 a row 3 KB each.
+constexpr uint32_t kResLevelBytes = 64 * 1024;
+
+// The mixed solve with resident workgroups (set-up enqueued, slots packed);
+// false: the launched solve has to run (nothing was solved).  Which scenes:
+// no cell with more particles than its wavefront's registers, columns within
+// 16-bit offsets, one row a thread, at most 512 workgroups (kResSlots), two a
+// compute unit.
+template <bool AMG>
+bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
+  const size_t n = c.ppe_n;
+  const Launch L = cg_grid(n);
+  const uint32_t nact = static_cast<uint32_t>(*c.ml_active_host);
+  const int grid = std::max(L.grid, static_cast<int>((nact + NT / 64 - 1) / (NT / 64)));
+  if (L.rpb != static_cast<size_t>(NT) || c.cap > 4u * kPerLane || mf_nnz_wide(c) > 0 || grid > kResSlots) return false;
+  if (c.res_skip > 0) {
+    c.res_skip--;
+    return false;
+  }
+  ResidentTurn turn(c.device);
+  if (!turn) return false;
+  auto kernel = k_mixed_resident<AMG, 32, 2>;
+  size_t lds = resident_lds(kernel, grid, 1);
+  if (lds == 0 && !AMG) {
+    kernel = k_mixed_resident<false, 16, 4>;
+    lds = resident_lds(kernel, grid, 2);
+  }
+  if (lds == 0) return false;
+  if (!c.res_ctl) c.res_ctl = dalloc<ResidentCtl>(1);
+  MixedArgs A{};
+  A.n = n;
+  A.rows = static_cast<unsigned>(L.grid);
+  A.A = sell<double>(c, c.sval, c.diag, L.rpb);
+  A.b = c.b;
+  A.x = c.sol;
+  A.r64 = c.r;
+  A.len = c.row_len;
+  A.pos = c.qpos;
+  A.ghost = c.ghost32;
+  A.c0 = matfree_rec(c, L.rpb).c0;
+  A.z = c.z32;
+  A.q = c.q32;
+  A.p = c.pa32;
+  A.d = c.d32;
+  A.a.G = ml_grid(c, ml_geom(c));
+  A.a.list = c.ml_list;
+  A.a.nact = nact;
+  A.a.pid = c.ml_pid;
+  A.a.dvp = c.ml_dv;
+  A.a.sc = c.ml_sc;
+  if (AMG) {
+    A.a.omega = kAmgOmegaRows;
+    A.a.bx0 = c.amg_box[0];
+    A.a.bz0 = c.amg_box[1];
+    A.a.bnx = c.amg_box[2];
+    A.a.bnz = c.amg_box[3];
+    A.a.q9 = c.amg_q9;
+    A.a.q9c = c.amg_q9c;
+    A.a.tq = c.amg_tq;
+    A.a.tq_stride = c.amg_tq_stride;
+    A.g = amg_grid(c);
+    // the levels that every workgroup holds in LDS
+    const int end = c.amg_levels;
+    const uint32_t last = c.amg_nx[end - 1] * c.amg_nz[end - 1];
+    auto levels_from = [&](int l) {  // {points, places} of levels l .. end - 1
+      uint32_t pts = c.amg_off[end - 1] + last - c.amg_off[l], places = 0;
+      for (int k = l; k < end; k++) places += (c.amg_nx[k] + 2) * (c.amg_nz[k] + 2);
+      return std::pair<uint32_t, uint32_t>(pts, places);
+    };
+    int l0 = end - 1;
+    while (l0 > 0) {
+      const auto v = levels_from(l0 - 1);
+      if (lds_level_bytes(v.first, v.second, last) > kResLevelBytes) break;
+      l0--;
+    }
+    const auto v = levels_from(l0);
+    A.lvp = v.first;
+    A.lvq = v.second;
+    uint32_t place = 0;
+    for (int k = l0; k < end; k++) {
+      A.place[k] = static_cast<uint16_t>(place);
+      place += (c.amg_nx[k] + 2) * (c.amg_nz[k] + 2);
+    }
+    A.l0 = l0;
+  }
+  A.sr = sr;
+  A.inner_tol = c.solver.inner_tol > 0 ? c.solver.inner_tol : 1e-4;
+  A.total_cap = c.solver.max_iter > 0 ? c.solver.max_iter : LLONG_MAX;
+  A.limit = inner_limit(c, max_iter);
+  for (int k = 0; k < Context::kSweepPred; k++) A.pred[k] = c.pred(k);
+  A.have_r = (c.learned_pending && learned_resolve(c, A.rr, A.bb)) ? 1 : 0;
+  A.ctl = c.res_ctl;
+  A.bytes = static_cast<uint32_t>(lds);
+  hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, c.stream, c.res_ctl, c.st32);
+  tracked(c, MPS_K_CG_SPMV32, 0.0, [&] {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), lds, c.stream, A);
+  });
+  check_launch();
+  MPS_HIP(hipEventRecord(c.solve_b, c.stream));
+  MPS_HIP(hipMemcpyAsync(c.res_host, c.res_ctl, kResHead, hipMemcpyDeviceToHost, c.stream));
+  MPS_HIP(hipStreamSynchronize(c.stream));
+  collect_events(c);
+  c.rec_ready = false;
+  if (c.res_host[1]) {
+    c.res_skip = kResSkip;
+    return false;
+  }
+  c.solve_ended = true;
+  c.replay_ready = MPS_K_CG_SPMV32;
+  MixedResult r;
+  std::memcpy(&r, reinterpret_cast<const char*>(c.res_host) + offsetof(ResidentCtl, out), sizeof r);
+  for (int k = 0; k < Context::kSweepPred; k++) c.pred(k) = r.pred[k];
+  if (r.stalled && !r.done && r.rr == r.rr && r.total < A.total_cap)
+    refine_fallback(c, sr, r.rr0, r.rr, r.total, r.outer);
+  else
+    refine_finished(c, r.done != 0, r.total, r.outer, r.rr0, r.rr, r.bb);
+  return true;
+}
+
+void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max_iter) {
+  const size_t n = c.ppe_n;
+  const Launch L = cg_grid(n);
+  ensure_zrec(c, n);
+  const MatFreeRec A = matfree_rec(c, L.rpb);
+  float* const zval = reinterpret_cast<float*>(c.zrec) + 2;  // z_i at zval[4 i]
+  const bool listed = block_list_ready(c);  // the search listed the blocks
+  if (!join_ml_setup(c)) ml_setup(c);  // enqueued ahead on the auxiliary stream, or now
+  if (listed) {
+    pack_slots(c, false);
+    if (resident_mixed<false>(c, sr, max_iter)) return;
+  }
+  const MlGeom g = ml_geom(c);
+  const size_t stride = c.part_ml_cap;
+  const CellGrid G = ml_grid(c, g);
+  // rows outside every cell keep r = d = z = 0; the records take the positions
+  hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
+                     c.zrec, c.r32, c.d32);
+  c.rec_ready = true;
+  check_launch();
+  double* p_pq = c.part3b;
+  const long long limit = inner_limit(c, max_iter);
+  // per particle: r (read, written), q, z; per slot of the packed layout: id
+  // and Jacobi factor; per lane: the aggregate scales (set once nact is known)
+  double b_prec = n * 16.0;
+  uint32_t nact = 0;
+  size_t pgrid = 1;
+  bool packed = listed;
+  auto prec = [&](double norm, long long it) {
+    const PrecArgs a{G,      c.ml_list, nact,   c.ml_pid, c.ml_dv, c.ml_sc,   c.r,       1.0 / norm,
+                     c.r32,  c.d32,     c.q32,  c.dinv32, zval,    4u,        p_pq,      L.grid,
+                     c.part_ml, stride, c.st32};
+    hipLaunchKernelGGL(k_ml_prec<0>, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, a, it);
+  };
+  double b_spmv = b_base;
+  c.replay_ready = MPS_K_CG_SPMV32;
+  refine(c, sr, [&](double norm, double sweep_tol) {
+    // refine() has synchronised the stream (residual) before every sweep: the
+    // block count and the wide nnz are on the host
+    nact = static_cast<uint32_t>(*c.ml_active_host);
+    b_spmv = b_base + 2.0 * mf_nnz_wide(c);
+    pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
+    b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
+    if (!packed) {
+      pack_slots(c, false);
+      packed = true;
+    }
+    MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
+    tracked(c, MPS_K_CG_INIT32, n * 25.0, [&] { prec(norm, 0); });
+    long long launched = 0;
+    const long long inner = run_inner(c, limit, [&](long long it) {
+      tracked(c, MPS_K_CG_SPMV32, b_spmv, [&] {
+        const SpmvArgs<MatFreeRec> a{A,      nullptr, c.pa32,  c.q32, c.d32, c.part_ml, stride,
+                                     static_cast<int>(pgrid), p_pq, c.st32, sweep_tol};
+        if (it == 1)
+          hipLaunchKernelGGL((k_ml_spmv<true, MatFreeRec>), dim3(L.grid), dim3(NT), 0, c.stream, a, it);
+        else
+          hipLaunchKernelGGL((k_ml_spmv<false, MatFreeRec>), dim3(L.grid), dim3(NT), 0, c.stream, a, it);
+      }, it);
+      tracked(c, MPS_K_ML_PREC, b_prec, [&] { prec(norm, it); }, it);
+      launched = it;
+    });
+    if (!c.st32_host->converged && launched > 0)
+      hipLaunchKernelGGL(k_ml_finish, dim3(grid_for(n)), dim3(256), 0, c.stream, n,
+                         static_cast<const CgStatus*>(c.st32), static_cast<const float*>(c.pa32), c.d32);
+    // launches after the stop did no work: count them out (k_ml_spmv(inner + 1)
+    // only finished d)
+    uncount(c, MPS_K_CG_SPMV32, launched - inner, b_spmv);
+    uncount(c, MPS_K_ML_PREC, launched - inner, b_prec);
+    return inner;
+  }, [&](double norm) {
+    hipLaunchKernelGGL(k_ir_correct, dim3(grid_for(n)), dim3(256), 0, c.stream, n, c.sol,
+                       static_cast<const float*>(c.d32), norm);
+  });
+}
+
 void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long max_iter) {
   const size_t n = c.ppe_n;
   const Launch L = cg_grid(n);
   ensure_zrec(c, n);
   const MatFreeRec A = matfree_rec(c, L.rpb);
   float* const zval = reinterpret_cast<float*>(c.zrec) + 2;  // z_i at zval[4 i]
+  const bool listed = block_list_ready(c);  // the search listed the blocks
   amg_setup(c);
+  clear_direction_sums(c);
   const MlGeom g = ml_geom(c);
   if (c.part_ml_cap < g.sgrid) {
     dfree(c.part_ml);
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
   }
+  if (listed) {
+    pack_slots(c, true);
+    if (resident_mixed<true>(c, sr, max_iter)) return;
+  }
   const size_t stride = c.part_ml_cap;
   const CellGrid G = ml_grid(c, g);
   hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
                      c.zrec, c.r32, c.d32);
+  c.rec_ready = true;
   check_launch();
   double* p_pq = c.part3b;
   const long long limit = inner_limit(c, max_iter);
   uint32_t nact = 0;
   size_t pgrid = 1;
-  bool packed = false;
+  bool packed = listed;
   // per pass over the particles (k_ml_prec<1>, then k_ml_prec<2>): r, q or z
   // per particle, the packed ids and Jacobi factors per slot, P_s's rows (18
   // bytes per particle); the cycle: level 0's direction sums written and
@@ -3248,14 +4455,7 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   double b_pass = n * 30.0;
   const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
   const double b_cycle = static_cast<double>(c.amg_pts) * 2 * (36 + 16) + npts0 * 19.0 * 4;
-  const size_t tq_stride = (npts0 + 63) & ~static_cast<size_t>(63);
-  if (c.amg_tq_cap < 9 * tq_stride) {
-    dfree(c.amg_tq);
-    c.amg_tq = dalloc<float>(9 * tq_stride);
-    c.amg_tq_cap = 9 * tq_stride;
-  }
-  // the direction sums of cells in unlisted (empty) blocks stay zero
-  MPS_HIP(hipMemsetAsync(c.amg_tq, 0, 9 * tq_stride * sizeof(float), c.stream));
+  const size_t tq_stride = c.amg_tq_stride;
   // it == 0 (the sweep's start) is accounted as a whole by the caller
   auto prec = [&](double norm, long long it) {
     PrecArgs a{G,         c.ml_list, nact,  c.ml_pid, c.ml_dv,    c.ml_sc, c.r,   1.0 / norm, c.r32,
@@ -3300,31 +4500,7 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
     pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
     b_pass = n * 30.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 8);
     if (!packed) {
-      const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
-      if (c.ml_pack_cap < slots) {
-        dfree(c.ml_pid);
-        dfree(c.ml_dv);
-        dfree(c.ml_sc);
-        c.ml_pid = dalloc<uint32_t>(slots * kPerLane);
-        c.ml_dv = dalloc<float>(slots * kPerLane);
-        c.ml_sc = dalloc<float4>(slots);
-        c.ml_pack_cap = slots;
-      }
-      tracked(c, MPS_K_ML_SETUP, n * 17.0 + slots * (8.0 * kPerLane + 16), [&] {
-        hipLaunchKernelGGL(k_ml_pack, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, G,
-                           static_cast<const uint32_t*>(c.ml_list), nact, static_cast<const float*>(nullptr),
-                           static_cast<const float*>(c.dinv32), c.ml_pid, c.ml_dv, c.ml_sc,
-                           static_cast<const uint32_t*>(c.row_len));
-      });
-      // P_s's rows in the same slot order
-      const size_t nslots = static_cast<size_t>(nact) * kPerLane * 64;
-      ensure_q9(c, nslots);
-      if (nslots > 0)
-        tracked(c, MPS_K_ML_SETUP, nslots * (4.0 + 18.0) + n * 80.0, [&] {
-          hipLaunchKernelGGL(k_amg_q, dim3(grid_for(nslots)), dim3(256), 0, c.stream, nslots,
-                             static_cast<const uint32_t*>(c.ml_pid), static_cast<const double*>(c.amg_rows),
-                             static_cast<const double*>(c.diag), kAmgOmegaP, c.amg_q9, c.amg_q9c);
-        });
+      pack_slots(c, true);
       packed = true;
     }
     MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
@@ -3924,6 +5100,12 @@ double replay_spmv(Context& c, int kid, int reps) {
   s.tol = -1.0;
   MPS_HIP(hipMemcpyAsync(c.st_replay, &s, sizeof(s), hipMemcpyHostToDevice, c.stream));
   const Launch L = cg_grid(c.ppe_n);
+  if (kid == MPS_K_CG_SPMV32 && !c.rec_ready) {  // a resident solve keeps no records
+    ensure_zrec(c, c.ppe_n);
+    hipLaunchKernelGGL(k_rec_init, dim3(grid_for(c.ppe_n)), dim3(256), 0, c.stream, c.ppe_n,
+                       static_cast<const uint2*>(c.qpos), c.zrec, c.r32, c.d32);
+    c.rec_ready = true;
+  }
   const size_t pgrid = std::max<size_t>(1, (*c.ml_active_host + NTP / 64 - 1) / (NTP / 64));
   auto launch = [&] {
     if (kid == MPS_K_CG_SPMV32)
@@ -4185,6 +5367,7 @@ bool batch_amg(const Context& c) { return c.solver.precond == MPS_PRECOND_AMG; }
 void amg_prepare(Context& c) {
   const size_t n = c.ppe_n;
   ensure_zrec(c, n);
+  const bool listed = block_list_ready(c);
   amg_setup(c);
   const MlGeom g = ml_geom(c);
   if (c.part_ml_cap < g.sgrid) {
@@ -4192,71 +5375,25 @@ void amg_prepare(Context& c) {
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
   }
-  MPS_HIP(hipStreamSynchronize(c.stream));  // the count of occupied cell blocks
-  const CellGrid G = ml_grid(c, g);
-  const uint32_t nact = static_cast<uint32_t>(*c.ml_active_host);
-  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
-  const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
-  if (c.ml_pack_cap < slots) {
-    dfree(c.ml_pid);
-    dfree(c.ml_dv);
-    dfree(c.ml_sc);
-    c.ml_pid = dalloc<uint32_t>(slots * kPerLane);
-    c.ml_dv = dalloc<float>(slots * kPerLane);
-    c.ml_sc = dalloc<float4>(slots);
-    c.ml_pack_cap = slots;
-  }
-  // the multigrid's rules: no aggregate scales, rows without stored
-  // off-diagonals outside every aggregate (as solve_mixed_amg packs)
-  hipLaunchKernelGGL(k_ml_pack, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, G,
-                     static_cast<const uint32_t*>(c.ml_list), nact, static_cast<const float*>(nullptr),
-                     static_cast<const float*>(c.dinv32), c.ml_pid, c.ml_dv, c.ml_sc,
-                     static_cast<const uint32_t*>(c.row_len));
-  const size_t nslots = static_cast<size_t>(nact) * kPerLane * 64;
-  ensure_q9(c, nslots);
-  if (nslots > 0)
-    hipLaunchKernelGGL(k_amg_q, dim3(grid_for(nslots)), dim3(256), 0, c.stream, nslots,
-                       static_cast<const uint32_t*>(c.ml_pid), static_cast<const double*>(c.amg_rows),
-                       static_cast<const double*>(c.diag), kAmgOmegaP, c.amg_q9, c.amg_q9c);
-  const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
-  const size_t tq_stride = (npts0 + 63) & ~static_cast<size_t>(63);
-  if (c.amg_tq_cap < 9 * tq_stride) {
-    dfree(c.amg_tq);
-    c.amg_tq = dalloc<float>(9 * tq_stride);
-    c.amg_tq_cap = 9 * tq_stride;
-  }
-  c.amg_tq_stride = tq_stride;
-  MPS_HIP(hipMemsetAsync(c.amg_tq, 0, 9 * tq_stride * sizeof(float), c.stream));
+  if (!listed) MPS_HIP(hipStreamSynchronize(c.stream));  // the count of occupied cell blocks
+  pack_slots(c, true);
+  clear_direction_sums(c);
   hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
                      c.zrec, c.r32, c.d32);
+  c.rec_ready = true;
   check_launch();
 }
 
 void ml_prepare(Context& c) {
   const size_t n = c.ppe_n;
   ensure_zrec(c, n);
+  const bool listed = block_list_ready(c);
   if (!join_ml_setup(c)) ml_setup(c);
-  MPS_HIP(hipStreamSynchronize(c.stream));  // the count of occupied cell blocks
-  const MlGeom g = ml_geom(c);
-  const CellGrid G = ml_grid(c, g);
-  const uint32_t nact = static_cast<uint32_t>(*c.ml_active_host);
-  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
-  const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
-  if (c.ml_pack_cap < slots) {
-    dfree(c.ml_pid);
-    dfree(c.ml_dv);
-    dfree(c.ml_sc);
-    c.ml_pid = dalloc<uint32_t>(slots * kPerLane);
-    c.ml_dv = dalloc<float>(slots * kPerLane);
-    c.ml_sc = dalloc<float4>(slots);
-    c.ml_pack_cap = slots;
-  }
-  hipLaunchKernelGGL(k_ml_pack, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, G,
-                     static_cast<const uint32_t*>(c.ml_list), nact, static_cast<const float*>(c.agg_inv),
-                     static_cast<const float*>(c.dinv32), c.ml_pid, c.ml_dv, c.ml_sc,
-                     static_cast<const uint32_t*>(nullptr));
+  if (!listed) MPS_HIP(hipStreamSynchronize(c.stream));  // the count of occupied cell blocks
+  pack_slots(c, false);
   hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
                      c.zrec, c.r32, c.d32);
+  c.rec_ready = true;
   check_launch();
 }
 

@@ -49,6 +49,7 @@ struct IrStatus {
 };
 
 struct ResidentCtl;  // mps_resident.hpp
+constexpr size_t kResHead = 384;  // its head and results, read by the host after a solve
 
 constexpr int kAmgMaxLevels = 20;  // grid levels of the cell-grid multigrid
 
@@ -268,6 +269,8 @@ struct Context {
   float* ml_dv = nullptr;
   float4* ml_sc = nullptr;
   size_t ml_pack_cap = 0;      // lanes (64 per listed block)
+  long long ml_list_serial = -1;       // search whose cells the list is of
+  bool rec_ready = false;              // zrec holds the installed system's positions
   uint64_t* ml_active = nullptr;       // count of such blocks
   uint64_t* ml_active_host = nullptr;  // pinned
   size_t agg_cap = 0;
@@ -298,7 +301,7 @@ struct Context {
   // resident solves: their control block, its head on the host ([1]: given
   // up), and how many solves not to try after one was refused
   ResidentCtl* res_ctl = nullptr;
-  unsigned* res_host = nullptr;  // pinned
+  unsigned* res_host = nullptr;  // pinned, kResHead bytes
   int res_skip = 0;
   bool solve_ended = false;  // solve_b was recorded by the solver (a residual follows it)
 
@@ -514,6 +517,10 @@ void ensure_amg_rows(Context& c, size_t n);
 // the particles (MPS_PRECOND_AUTO picks it; mps_cg.hip), and the one in force.
 int precond_for_system(Context& c);
 int effective_precond(const Context& c);
+// The occupied 4x4 blocks of cells, for the mixed solvers' preconditioners
+// (mps_cg.hip): enqueued by the search so that their count is on the host
+// with the search's own synchronisation.
+void enqueue_block_list(Context& c);
 double replay_spmv(Context& c, int kid, int reps);  // mps_cg.hip: mean ms of one launch
 // exclusive scan of n u32 counts into out, grand total to *total (device); mps_search.hip
 void scan_counts(Context& c, const uint32_t* in, size_t n, uint32_t* out, uint64_t* total);

@@ -19,10 +19,11 @@
 // mark, then adds them in the fixed order of the launched kernels (1.8 / 2.2 /
 // 2.4 / 2.8 us for 5 / 64 / 128 / 256 workgroups, both block sums included; 4.0
 // for 256 with the slots side by side; 3.5-3.6 through one reducing workgroup
-// that hands the total on).  Slots are used in a ring of kResRing generations.  Emptying: once generation g is
-// complete everyone has published g and so has finished reading g - 1; the
-// owner then empties its slot of g - 1, and that store completes before its
-// publication of g + 1, hence before anyone polls g + 3 (the same ring entry).
+// that hands the total on).  Slots are used in a ring of kResRing generations.
+// Emptying: once generation g is complete everyone has published g and so has
+// finished reading g - 1; the owner then empties its slot of g - 1, and that
+// store completes before its publication of g + 1, hence before anyone polls
+// g + 3 (the same ring entry).
 //
 // Every wait is bounded.  Before the first iteration the workgroups wait until
 // all of them have started (they might not fit beside other work on the GPU)
@@ -32,7 +33,10 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+
 #include "mps_device.hpp"
+#include "mps_internal.hpp"
 
 namespace mps {
 
@@ -41,12 +45,16 @@ constexpr int kResSlots = 512;  // partial sums of one generation (one per workg
 constexpr int kResPitch = 8;    // a slot per 64-byte line: polls of one slot do not hold up a store to another
 constexpr unsigned long long kResEmpty = ~0ull;  // no partial sum: NaNs are published as one quiet pattern
 
+constexpr int kResWords64 = 4;  // values of one slot at most (a line holds 8)
 struct ResidentCtl {
   unsigned started;
   unsigned abort;
   unsigned pad[30];
+  long long out[32];  // results of a solve (read by the host together with the head)
   unsigned long long slot[kResRing][kResSlots * kResPitch];
 };
+
+static_assert(offsetof(ResidentCtl, slot) == kResHead, "what the host reads");
 
 // Limits of the waits, in ticks of the constant 100 MHz clock: for the start
 // (5 ms: other work on the GPU may hold the compute units) and for one
@@ -91,19 +99,23 @@ __device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok) {
   return s_go != 0;
 }
 
-// One thread: the workgroup's partial sum of generation g (after the emptying
-// of an older slot, and whatever else this thread's wavefront stored, is done).
-__device__ __forceinline__ void resident_publish(ResidentCtl* c, unsigned g, unsigned idx, double v) {
-  if (v != v) v = __builtin_nan("");  // never the empty mark
+// One thread: the workgroup's values of generation g (after the emptying of an
+// older slot, and whatever else this thread's wavefront stored, is done).
+template <class... V>
+__device__ __forceinline__ void resident_publish(ResidentCtl* c, unsigned g, unsigned idx, V... values) {
+  const double v[] = {values...};
   stores_done();
-  agent_store(&c->slot[g % kResRing][idx * kResPitch], static_cast<unsigned long long>(__double_as_longlong(v)));
+#pragma unroll
+  for (unsigned k = 0; k < sizeof...(V); k++) {
+    const double t = (v[k] != v[k]) ? __builtin_nan("") : v[k];  // never the empty mark
+    agent_store(&c->slot[g % kResRing][idx * kResPitch + k], static_cast<unsigned long long>(__double_as_longlong(t)));
+  }
 }
 
-// Threads t < count: slot t of generation g once it is published (0 on the
-// others); ok: false on a thread whose wait was given up.
-__device__ __forceinline__ double resident_poll(ResidentCtl* c, unsigned g, unsigned count, bool& ok) {
-  if (threadIdx.x >= count) return 0.0;
-  const unsigned long long* s = &c->slot[g % kResRing][threadIdx.x * kResPitch];
+// Value `word` of workgroup k's slot of generation g once it is published; ok:
+// false if the wait was given up.
+__device__ __forceinline__ double resident_word(ResidentCtl* c, unsigned g, unsigned k, int word, bool& ok) {
+  const unsigned long long* s = &c->slot[g % kResRing][k * kResPitch + word];
   unsigned long long b = agent_load(s);
   if (b == kResEmpty) {
     const long long t0 = wall_clock64();
@@ -119,10 +131,33 @@ __device__ __forceinline__ double resident_poll(ResidentCtl* c, unsigned g, unsi
   return __longlong_as_double(static_cast<long long>(b));
 }
 
+// Values word and word + 1 of workgroup k's slot, polled together.
+__device__ __forceinline__ void resident_words(ResidentCtl* c, unsigned g, unsigned k, int word, bool& ok, double& v0,
+                                               double& v1) {
+  const unsigned long long* s = &c->slot[g % kResRing][k * kResPitch + word];
+  unsigned long long a = agent_load(s), b = agent_load(s + 1);
+  if (a == kResEmpty || b == kResEmpty) {
+    const long long t0 = wall_clock64();
+    do {
+      a = agent_load(s);
+      b = agent_load(s + 1);
+      if ((a == kResEmpty || b == kResEmpty) &&
+          (agent_load(&c->abort) || wall_clock64() - t0 > kResWaitTicks)) {
+        agent_store(&c->abort, 1u);
+        ok = false;
+        break;
+      }
+    } while (a == kResEmpty || b == kResEmpty);
+  }
+  v0 = __longlong_as_double(static_cast<long long>(a));
+  v1 = __longlong_as_double(static_cast<long long>(b));
+}
+
 // After the whole workgroup has seen generation g complete: its slot of
-// generation g - 1 is emptied.
-__device__ __forceinline__ void resident_empty(ResidentCtl* c, unsigned g, unsigned idx) {
-  if (threadIdx.x == 0) agent_store(&c->slot[(g + kResRing - 1) % kResRing][idx * kResPitch], kResEmpty);
+// generation g - 1 is emptied (the first `words` values).
+__device__ __forceinline__ void resident_empty(ResidentCtl* c, unsigned g, unsigned idx, unsigned words = 1) {
+  if (threadIdx.x < words)
+    agent_store(&c->slot[(g + kResRing - 1) % kResRing][idx * kResPitch + threadIdx.x], kResEmpty);
 }
 
 // Clears the control block (and whatever `extra` words of a status) before a
@@ -133,7 +168,8 @@ __device__ __forceinline__ void resident_clear(ResidentCtl* c) {
     c->abort = 0;
   }
   for (int g = 0; g < kResRing; g++)
-    for (int k = threadIdx.x; k < kResSlots; k += blockDim.x) c->slot[g][k * kResPitch] = kResEmpty;
+    for (int k = threadIdx.x; k < kResSlots; k += blockDim.x)
+      for (int w = 0; w < kResWords64; w++) c->slot[g][k * kResPitch + w] = kResEmpty;
 }
 
 }  // namespace mps

@@ -551,6 +551,10 @@ void search(Context& c) {
                        c.nbr_total_dev);
   });
   check_launch();
+  if (c.solver.kind == MPS_SOLVER_MIXED_IR &&
+      (c.solver.precond == MPS_PRECOND_MULTILEVEL || c.solver.precond == MPS_PRECOND_AMG ||
+       c.solver.precond == MPS_PRECOND_AUTO))
+    enqueue_block_list(c);
   MPS_HIP(hipMemcpyAsync(c.flags_host, c.flags, 4 * sizeof(int), hipMemcpyDeviceToHost, c.stream));
   MPS_HIP(hipMemcpyAsync(c.nbr_total_host, c.nbr_total_dev, sizeof(unsigned long long),
                          hipMemcpyDeviceToHost, c.stream));
