@@ -147,6 +147,23 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v) {
   return wave_fold_u32(v, [](unsigned a, unsigned b) { return b > a ? b : a; });
 }
 
+// Adds the sum of v over the block (THREADS threads, every one calls it) to
+// *total: one atomic a block.  One a wavefront, 16k of them to one address at
+// 1.05M particles, took a third of the passes that count: the search 237 -> 151
+// us, the density and count pass 230 -> 153.
+template <int THREADS>
+__device__ __forceinline__ void block_count(uint32_t v, unsigned long long* total) {
+  __shared__ unsigned part[THREADS / 64];
+  const unsigned w = wave_fold_u32(v, [](unsigned a, unsigned b) { return a + b; });
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = w;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (int k = 0; k < THREADS / 64; k++) t += part[k];
+    if (t > 0) atomicAdd(total, t);
+  }
+}
+
 // Deterministic block sum of one double per thread (blockDim.x == NT):
 // fixed wavefront butterflies, then the NT/64 wavefront sums in order.
 template <int NT>

@@ -54,14 +54,16 @@ __device__ __forceinline__ void count_slice(size_t n, size_t sl, uint32_t cnt, b
                                             uint32_t* __restrict__ slice_width, uint8_t* __restrict__ slice_wide,
                                             unsigned long long* nnz_total, unsigned long long* nnz_wide) {
   const unsigned wmax = wave_max_u32(cnt);
-  const unsigned long long wsum = static_cast<unsigned long long>(wave_sum(static_cast<double>(cnt)));
   const unsigned long long far = __ballot(!fits);
+  if (far) {  // rare
+    const unsigned long long wsum = static_cast<unsigned long long>(wave_sum(static_cast<double>(cnt)));
+    if ((threadIdx.x & 63) == 0) atomicAdd(nnz_wide, wsum);
+  }
   if ((threadIdx.x & 63) == 0 && sl * 64 < n) {
     slice_width[sl] = wmax;
     slice_wide[sl] = static_cast<uint8_t>(far != 0);
-    atomicAdd(nnz_total, wsum);
-    if (far) atomicAdd(nnz_wide, wsum);
   }
+  block_count<kBlock>(cnt, nnz_total);
 }
 
 // b and x0 (Computer.hpp:1185-1221), row lengths and slice widths.

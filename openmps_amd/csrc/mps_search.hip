@@ -309,18 +309,25 @@ __global__ void __launch_bounds__(kBlock) k_cell_pos(size_t n, const uint64_t* _
 // IDENT: the particles are stored in cell order (slot k holds particle k),
 // so the candidate ids are the slots themselves and are not loaded.
 //
-// A lane's found neighbours form groups of four slots (16 bytes, the list
-// layout's unit).  Stored by each lane as it completes them, the groups of a
-// wavefront reach a cache line at different times and the lines are written
-// back part-filled (2.2x the list bytes).  Instead each lane keeps its last
-// kRing completed groups in a ring in LDS, and after each batch of
-// candidates (the batch loop is uniform for the wavefront) the groups every
-// lane has completed are stored together: one 1-KB coalesced store per group
-// index.  A lane more than kRing groups ahead of the slowest stores its
-// oldest ring group directly to make room; the end of the walk stores the
-// rest.
-constexpr int kRing = 4;
-constexpr int kNbrBatch = 4;  // candidates per lane per round trip to memory
+// A lane's candidates are one sequence over its three ranges; the positions of
+// the next kNbrBatch of them are loaded before the current ones are tested.
+// Found neighbours go to the lane's ring of kRing slots in LDS ([slot][thread]:
+// no bank conflicts whatever slots the lanes are at), one store and an
+// increment each.  The list's unit is a group of four slots (16 bytes).
+// Stored by each lane as it completes them, the groups of a wavefront reach a
+// cache line at different times and the lines are written back part-filled
+// (2.2x the list bytes); instead the groups that every lane has completed are
+// stored together after a batch (the batch loop is uniform for the wavefront):
+// one 1-KB coalesced store per group index.  A lane whose ring is full stores
+// its oldest group itself; the end of the walk stores the rest.
+//
+// Bound by instruction issue from about 100k particles on (87% of the cycles at
+// 1.05M) and by the latency of a wavefront's own chain below.  Against one range
+// after the other, a branch per candidate and one atomic a wavefront: 2k
+// particles 46 -> 24 us, 33k 48 -> 25, 131k 65 -> 38, 1.05M 251 -> 147.
+// Batches of 4 instead of 8: 27, 27, 40, 152.
+constexpr uint32_t kRing = 32;
+constexpr int kNbrBatch = 8;  // candidates per lane per round trip to memory
 template <bool IDENT>
 __global__ void __launch_bounds__(kBlock) k_neighbors(GridParams g, size_t n, const double* __restrict__ x,
                                                       const double* __restrict__ z,
@@ -332,98 +339,113 @@ __global__ void __launch_bounds__(kBlock) k_neighbors(GridParams g, size_t n, co
                                                       uint32_t kstride, uint32_t* __restrict__ nbr,
                                                       uint32_t* __restrict__ ncount, int* flags,
                                                       unsigned long long* total) {
-  __shared__ uint4 ring[kRing][kBlock];
+  __shared__ uint32_t ring[kRing][kBlock];
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
   const size_t i = blk * static_cast<size_t>(blockDim.x) + threadIdx.x;
   const bool active = i < n && type[i] != kDisabled;
-  uint32_t cnt = 0;
-  // complete groups of this lane (those whose last slot is below kmax);
-  // groups below `flushed` (a wavefront value) are stored, and of the others
-  // the last kRing are in ring[group % kRing], the older ones stored
-  uint32_t ngrp = 0, flushed = 0;
-  uint4 grp = make_uint4(0u, 0u, 0u, 0u);
+  // found neighbours; groups of them stored by this lane and by every lane
+  uint32_t cnt = 0, mine = 0, flushed = 0;
   uint4* const out = reinterpret_cast<uint4*>(nbr);
   const uint32_t self = static_cast<uint32_t>(i);
-  auto store = [&](uint32_t gi, const uint4& v) { out[nbr_slot(self, 4 * gi, kstride) >> 2] = v; };
+  auto store = [&](uint32_t gi) {
+    if (4 * gi >= kstride) return;  // beyond the list's capacity: counted only
+    const uint32_t k = 4 * gi % kRing;
+    out[nbr_slot(self, 4 * gi, kstride) >> 2] =
+        make_uint4(ring[k][threadIdx.x], ring[k + 1][threadIdx.x], ring[k + 2][threadIdx.x], ring[k + 3][threadIdx.x]);
+  };
   double xi = 0, zi = 0;
-  long long bx = 0, bz = 0;
+  // the candidates: those below to0, to1 and total_m are in the first, second
+  // and third column of cells, candidate t in slot t + o0 (+ o1 (+ o2))
+  uint32_t to0 = 0, to1 = 0, total_m = 0, o0 = 0, o1 = 0, o2 = 0;
   if (active) {
     xi = x[i];
     zi = z[i];
+    long long bx = 0, bz = 0;
     cell_of(g, xi, zi, bx, bz);  // in the grid: the others are disabled
+    uint32_t s[3], m[3];
+#pragma unroll
+    for (int ox = 0; ox < 3; ox++) {
+      const long long cx = bx + ox - 1;
+      const bool inside = cx >= 0 && cx < g.gnx;
+      const long long cc = inside ? cx : bx;
+      const size_t c0 = static_cast<size_t>(cc * g.gnz + (bz > 0 ? bz - 1 : 0));
+      const size_t c1 = static_cast<size_t>(cc * g.gnz + (bz + 1 < g.gnz ? bz + 1 : bz));
+      s[ox] = cell_start[c0];
+      m[ox] = inside ? cell_start[c1] + cell_count[c1] - s[ox] : 0u;
+    }
+    to0 = m[0];
+    to1 = to0 + m[1];
+    total_m = to1 + m[2];
+    o0 = s[0];
+    o1 = s[1] - s[0] - to0;
+    o2 = s[2] - s[1] - m[1];
   }
   const double nl = g.nl;
-  auto test = [&](bool valid, uint32_t j, double xj, double zj) {
-    if (!valid || j == i) return;
-    const double rx = xi - xj, rz = zi - zj;
-    // Computer::R, Computer.hpp:568-572: sqrt(r.r) < NL.  sqrt is correctly
-    // rounded, so the test only depends on r.r near NL^2: outside the
-    // narrow band [lo, hi] the comparison of r.r decides it exactly.
-    const double q = rx * rx + rz * rz;
-    bool within = q < g.lo;
-    // the band is a few ulps of NL^2 wide: its square root is taken on its
-    // own branch, which a wavefront almost never enters (evaluated beside
-    // the comparisons it costs every candidate beyond lo twenty FP64
-    // instructions)
-    if (q >= g.lo && q <= g.hi) within = sqrt(q) < nl;
-    if (within) {
-      const uint32_t lane = cnt & 3u;
-      grp.x = (lane == 0) ? j : grp.x;
-      grp.y = (lane == 1) ? j : grp.y;
-      grp.z = (lane == 2) ? j : grp.z;
-      grp.w = (lane == 3) ? j : grp.w;
-      if (lane == 3 && cnt < kmax) {
-        // group ngrp is complete; a full ring gives up its oldest group
-        if (ngrp >= flushed + kRing) store(ngrp - kRing, ring[ngrp % kRing][threadIdx.x]);
-        ring[ngrp % kRing][threadIdx.x] = grp;
-        ngrp++;
-      }
-      cnt++;
+  const uint32_t rounds = wave_max_u32(total_m);
+  uint32_t jj[kNbrBatch];
+  double2 pj[kNbrBatch];
+  auto load = [&](uint32_t t0, uint32_t(&j)[kNbrBatch], double2(&p)[kNbrBatch]) {
+#pragma unroll
+    for (int v = 0; v < kNbrBatch; v++) {
+      const uint32_t t = t0 + v;
+      const uint32_t s = t + o0 + (t < to0 ? 0u : o1) + (t < to1 ? 0u : o2);
+      const uint32_t k = (t < total_m) ? s : 0u;  // past the end: slot 0 (in the arrays, not tested)
+      j[v] = IDENT ? k : sorted[k];
+      p[v] = pos[k];
     }
   };
-  for (int ox = -1; ox <= 1; ox++) {
-    const long long cx = bx + ox;
-    uint32_t s = 0, m = 0;
-    if (active && cx >= 0 && cx < g.gnx) {
-      const size_t c0 = static_cast<size_t>(cx * g.gnz + (bz > 0 ? bz - 1 : 0));
-      const size_t c1 = static_cast<size_t>(cx * g.gnz + (bz + 1 < g.gnz ? bz + 1 : bz));
-      s = cell_start[c0];
-      m = cell_start[c1] + cell_count[c1] - s;
+  load(0, jj, pj);
+  for (uint32_t t0 = 0; t0 < rounds; t0 += kNbrBatch) {
+    uint32_t jn[kNbrBatch];
+    double2 pn[kNbrBatch];
+    load(t0 + kNbrBatch, jn, pn);
+    // room in the ring for a batch (a lane without a particle finds nothing:
+    // cnt = 0, while mine follows flushed)
+    while (active && cnt > 4 * mine + (kRing - kNbrBatch)) {
+      store(mine);
+      mine++;
     }
-    // a batch loop uniform for the wavefront (lanes past their range skip
-    // the tests), so that the completed groups can be stored after a batch
-    const uint32_t mw = wave_max_u32(m);
-    for (uint32_t l = 0; l < mw; l += kNbrBatch) {
-      uint32_t jj[kNbrBatch];
-      double2 pj[kNbrBatch];
-      bool ok[kNbrBatch];
+    // Computer::R, Computer.hpp:568-572: sqrt(r.r) < NL.  sqrt is correctly
+    // rounded, so the test only depends on r.r near NL^2: outside the narrow
+    // band [lo, hi] the comparison of r.r decides it exactly.  The band is a
+    // few ulps of NL^2 wide: its square roots are taken on a branch of their
+    // own, which a wavefront almost never enters.
+    double q[kNbrBatch];
+    bool within[kNbrBatch], band = false;
 #pragma unroll
-      for (int v = 0; v < kNbrBatch; v++) {
-        ok[v] = l + v < m;
-        const uint32_t k = s + (ok[v] ? l + v : 0u);  // a valid slot (unused when !ok)
-        jj[v] = IDENT ? k : (ok[v] ? sorted[k] : 0u);
-        pj[v] = ok[v] ? pos[k] : make_double2(0.0, 0.0);
-      }
+    for (int v = 0; v < kNbrBatch; v++) {
+      const double rx = xi - pj[v].x, rz = zi - pj[v].y;
+      q[v] = rx * rx + rz * rz;
+      within[v] = q[v] < g.lo;
+      band = band || (!within[v] && q[v] <= g.hi);
+    }
+    if (band) {
 #pragma unroll
-      for (int v = 0; v < kNbrBatch; v++) test(ok[v], jj[v], pj[v].x, pj[v].y);
-      // the groups every active lane has completed
-      const uint32_t upto = wave_min_u32(active ? ngrp : 0xffffffffu);
-      if (upto != 0xffffffffu) {
-        for (uint32_t gi = flushed; gi < upto; gi++)
-          if (active && gi + kRing >= ngrp) store(gi, ring[gi % kRing][threadIdx.x]);
-        flushed = upto > flushed ? upto : flushed;
-      }
+      for (int v = 0; v < kNbrBatch; v++) within[v] = sqrt(q[v]) < nl;
+    }
+#pragma unroll
+    for (int v = 0; v < kNbrBatch; v++) {
+      ring[cnt % kRing][threadIdx.x] = jj[v];  // (overwritten by the next one found if it does not count)
+      cnt += (within[v] && t0 + v < total_m && jj[v] != self) ? 1u : 0u;
+    }
+    // the groups every active lane has completed
+    const uint32_t upto = wave_min_u32(active ? cnt >> 2 : 0xffffffffu);
+    if (upto != 0xffffffffu) {
+      for (; flushed < upto; flushed++)
+        if (active && flushed >= mine) store(flushed);
+      mine = mine > flushed ? mine : flushed;
+    }
+#pragma unroll
+    for (int v = 0; v < kNbrBatch; v++) {
+      jj[v] = jn[v];
+      pj[v] = pn[v];
     }
   }
-  // the rest: the complete groups still in the ring and the last, partial
-  // one (its slots past the count are never read)
-  const bool partial = active && (cnt & 3u) && cnt <= kmax;
-  const uint32_t mine = active ? ngrp + (partial ? 1u : 0u) : 0u;
-  const uint32_t last = wave_max_u32(mine);
-  for (uint32_t gi = flushed; gi < last; gi++) {
-    if (gi < ngrp && gi + kRing >= ngrp) store(gi, ring[gi % kRing][threadIdx.x]);
-    if (partial && gi == ngrp) store(gi, grp);
-  }
+  // the rest, the last of them partial (its slots past the count are never read)
+  const uint32_t groups = active ? (cnt + 3) >> 2 : 0u;
+  const uint32_t last = wave_max_u32(groups);
+  for (uint32_t gi = flushed; gi < last; gi++)
+    if (gi < groups && gi >= mine) store(gi);
   if (active) {
     if (cnt > kmax) {
       flags[1] = 1;
@@ -431,8 +453,7 @@ __global__ void __launch_bounds__(kBlock) k_neighbors(GridParams g, size_t n, co
     }
     ncount[i] = cnt;
   }
-  const double ws = wave_sum(static_cast<double>(cnt));
-  if ((threadIdx.x & 63) == 0 && ws > 0) atomicAdd(total, static_cast<unsigned long long>(ws));
+  block_count<kBlock>(cnt, total);
 }
 
 }  // namespace
