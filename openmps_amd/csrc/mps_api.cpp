@@ -234,8 +234,8 @@ void forward(Context& c, double dt) {
   density_save_and_assemble(c);
   ppe_solve(c);
   pressure_writeback(c);
-  pressure_gradient(c);
-  dynamic_stabilize(c);
+  pressure_gradient(c, true);
+  dynamic_stabilize(c, true);
   sync(c);
 }
 
@@ -719,14 +719,14 @@ int mps_stage_pressure_writeback(mps_ctx* ctx) {
 int mps_stage_pressure_gradient(mps_ctx* ctx) {
   return mps::guard(ctx, [&](Context& c) {
     mps::require_neighbors(c);
-    mps::pressure_gradient(c);
+    mps::pressure_gradient(c, false);
     mps::sync(c);
   });
 }
 int mps_stage_dynamic_stabilize(mps_ctx* ctx) {
   return mps::guard(ctx, [&](Context& c) {
     mps::require_neighbors(c);
-    mps::dynamic_stabilize(c);
+    mps::dynamic_stabilize(c, false);
     mps::sync(c);
   });
 }

@@ -230,8 +230,8 @@ void batch_forward(mps_batch& b, double dt_fixed, double* dt_out) {
     try {
       if (joined[s]) MPS_HIP(hipStreamWaitEvent(c.stream, b.ev_solved, 0));
       pressure_writeback(c);
-      pressure_gradient(c);
-      dynamic_stabilize(c);
+      pressure_gradient(c, true);
+      dynamic_stabilize(c, true);
       MPS_HIP(hipStreamSynchronize(c.stream));
       collect_events(c);
     } catch (Failure& f) {

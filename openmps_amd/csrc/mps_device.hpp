@@ -42,36 +42,146 @@ __device__ __forceinline__ bool ghost_pos(double xi, double zi, double sx, doubl
   return true;
 }
 
-// Walks particle i's m-entry neighbour list in list order, U neighbours per
-// round trip to memory: the U ids, then load(j) for all U of them (the
-// gathered fields of neighbour j, returned as a T), then use(j, T) in list
-// order.  A walk that issues each neighbour's loads only after the previous
-// one's arithmetic pays a full memory latency per neighbour.
-template <int U, class T, class Load, class Use>
+// Walks particle i's m-entry neighbour list in list order, four neighbours (one
+// group of slots) at a time: use(j, f, in) gets the group's ids, load(j) of each
+// (the gathered fields, as a T) and which of them are in the list (the last
+// group's rest holds particle i itself).
+//
+// `use` computes all four neighbours' terms first, without branches, and then
+// adds those that count in list order.  A term is a chain of a dozen to thirty
+// dependent FP64 instructions (square root, division): behind a branch per
+// neighbour, which some lane of a wavefront nearly always takes, the four
+// chains run one after the other; without it they overlap.  The next group's
+// ids and fields are loaded before the current group's arithmetic.  (Density
+// and acceleration pass, bound by FP64 issue: 2k particles 23 -> 16 us, 131k 46
+// -> 37, 1.05M 215 -> 180.)
+template <class T, class Load, class Use>
 __device__ __forceinline__ void walk_list(uint32_t i, uint32_t m, const uint32_t* __restrict__ ids, uint32_t kmax,
                                           Load load, Use use) {
-  static_assert(U % 4 == 0, "whole slot groups");
-  uint32_t q = 0;
-  for (; q + U <= m; q += U) {
-    uint32_t jj[U];
+  if (m == 0) return;
+  auto group = [&](uint32_t q, uint32_t j[4]) {
+    const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, q, kmax));
+    j[0] = g.x;
+    j[1] = (q + 1 < m) ? g.y : i;
+    j[2] = (q + 2 < m) ? g.z : i;
+    j[3] = (q + 3 < m) ? g.w : i;
+  };
+  uint32_t j[4], jn[4];
+  T f[4];
+  group(0, j);
+  group(m > 4 ? 4u : 0u, jn);
 #pragma unroll
-    for (int v = 0; v < U; v += 4) {
-      const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, q + v, kmax));
-      jj[v] = g.x;
-      jj[v + 1] = g.y;
-      jj[v + 2] = g.z;
-      jj[v + 3] = g.w;
+  for (int v = 0; v < 4; v++) f[v] = load(j[v]);
+  for (uint32_t q = 0; q < m; q += 4) {
+    T fn[4];
+    uint32_t j2[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) fn[v] = load(jn[v]);
+    group(q + 8 < m ? q + 8 : 0u, j2);
+    bool in[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) in[v] = q + v < m;
+    use(j, f, in);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      j[v] = jn[v];
+      jn[v] = j2[v];
+      f[v] = fn[v];
     }
-    T f[U];
-#pragma unroll
-    for (int v = 0; v < U; v++) f[v] = load(jj[v]);
-#pragma unroll
-    for (int v = 0; v < U; v++) use(jj[v], f[v]);
   }
-  for (; q < m; q++) {
-    const uint32_t j = ids[nbr_slot(i, q, kmax)];
-    use(j, load(j));
+}
+
+// The walk of a pass whose expensive terms only count for the nearer neighbours
+// (r < r_e, while the list reaches r_lap): far(j, p, f1, in, e) gets four
+// neighbours' positions p and fields f1 (load1), adds the terms of all of them
+// and sets e[v] for the nearer ones; near(p, f2, e) gets those with the fields
+// f2 (load2) and adds their terms, in list order.
+//
+// NEAR: a lane first collects its nearer neighbours in its column of `queue`
+// (LDS, kNearQueue slots, [slot][thread]), then computes their terms, so that a
+// wavefront goes through the expensive instructions as often as its lanes have
+// near neighbours (about 14 times, for r_e = 2.1 and r_lap = 3.1) and not once
+// per list entry (37): gradient of 1.05M particles 147 -> 97 us, density and
+// count pass 153 -> 137; 131k 32 -> 19 and 33 -> 25.  Otherwise (the radii are
+// alike and nearly every neighbour is near: collecting would only add a pass;
+// 6k particles at r_e = r_lap = 2.4: gradient 9.9, count 12.1 us) the terms are
+// computed on the way.  The line (near_pays): near neighbours below three
+// quarters of the list.
+constexpr uint32_t kNearQueue = 24;
+inline bool near_pays(double re, double rl) { return re * re < 0.75 * rl * rl; }
+template <bool NEAR, int THREADS, class F1, class F2, class Load1, class Load2, class Far, class Near>
+__device__ __forceinline__ void walk_near(uint32_t i, uint32_t m, const uint32_t* __restrict__ ids, uint32_t kmax,
+                                          const double2* __restrict__ xz, uint32_t (*queue)[THREADS], Load1 load1,
+                                          Load2 load2, Far far, Near near) {
+  if (m == 0) return;
+  auto group = [&](uint32_t q, uint32_t j[4]) {
+    const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, q, kmax));
+    j[0] = g.x;
+    j[1] = (q + 1 < m) ? g.y : i;
+    j[2] = (q + 2 < m) ? g.z : i;
+    j[3] = (q + 3 < m) ? g.w : i;
+  };
+  uint32_t j[4], jn[4];
+  double2 p[4], pn[4];
+  F1 f[4], fn[4];
+  F2 g[4], gn[4];
+  group(0, j);
+  group(m > 4 ? 4u : 0u, jn);
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    p[v] = xz[j[v]];
+    f[v] = load1(j[v]);
+    if (!NEAR) g[v] = load2(j[v]);
   }
+  uint32_t q = 0;
+  do {
+    uint32_t found = 0;
+    for (; q < m && (!NEAR || found + 4 <= kNearQueue); q += 4) {
+      uint32_t j2[4];
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        pn[v] = xz[jn[v]];
+        fn[v] = load1(jn[v]);
+        if (!NEAR) gn[v] = load2(jn[v]);
+      }
+      group(q + 8 < m ? q + 8 : 0u, j2);
+      bool in[4], e[4];
+#pragma unroll
+      for (int v = 0; v < 4; v++) in[v] = q + v < m;
+      far(j, p, f, in, e);
+      if (NEAR) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          queue[found][threadIdx.x] = j[v];  // (overwritten by the next near one if it is not)
+          found += e[v] ? 1u : 0u;
+        }
+      } else {
+        near(p, g, e);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        j[v] = jn[v];
+        jn[v] = j2[v];
+        p[v] = pn[v];
+        f[v] = fn[v];
+        if (!NEAR) g[v] = gn[v];
+      }
+    }
+    if (NEAR)
+      for (uint32_t k = 0; k < found; k += 4) {
+        double2 pk[4];
+        F2 gk[4];
+        bool e[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          e[v] = k + v < found;
+          const uint32_t jk = e[v] ? queue[k + v < kNearQueue ? k + v : 0u][threadIdx.x] : i;
+          pk[v] = xz[jk];
+          gk[v] = load2(jk);
+        }
+        near(pk, gk, e);
+      }
+  } while (NEAR && q < m);
 }
 
 // XCD-aware block order: hardware hands consecutive workgroups to the 8 XCDs

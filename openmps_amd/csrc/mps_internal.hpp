@@ -499,8 +499,9 @@ void density_and_explicit(Context& c);
 void explicit_update(Context& c);  // wall targets and the integration of the explicit stage
 void wall_targets_from_callback(Context& c);
 void pressure_writeback(Context& c);
-void pressure_gradient(Context& c);
-void dynamic_stabilize(Context& c);
+// packed: xz holds the current positions (in a step, after the explicit update)
+void pressure_gradient(Context& c, bool packed);
+void dynamic_stabilize(Context& c, bool packed);
 void ppe_assemble(Context& c);           // mps_ppe.hip
 void pack_state(Context& c);             // mps_particles.hip: xz, uw from x, z, u, w
 // density(c, false, true, true) followed by ppe_assemble(c), the density walk

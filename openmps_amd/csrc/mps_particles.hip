@@ -28,8 +28,6 @@ struct Consts {
   double re, re2, rl, rl2, n0, n0l, nu, rho, dt, gx, gz, d2;
 };
 
-constexpr int kWalk = 4;  // neighbours whose loads are issued together (walk_list)
-
 Consts consts(const Context& c) {
   Consts k;
   k.re = c.env.r_e;
@@ -87,27 +85,33 @@ __global__ void __launch_bounds__(kBlock) k_density(size_t n, const double* __re
   struct F {
     double x, z, u, w;
   };
-  walk_list<kWalk, F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-                      [&](uint32_t j) {
-                        F f{x[j], z[j], 0.0, 0.0};
-                        if (ECS) {
-                          f.u = u[j];
-                          f.w = w[j];
-                        }
-                        return f;
-                      },
-                      [&](uint32_t, const F& f) {
-                        const double dx = f.x - xi, dz = f.z - zi;
-                        const double r2 = dx * dx + dz * dz;
-                        if (r2 < k.re2) {
-                          const double r = sqrt(r2);
-                          if (DENS) s += weight(r, k.re);
-                          if (ECS) {
-                            const double du = f.u - ui, dw = f.w - wi;
-                            h += (dx * du + dz * dw) / (r * r * r);
-                          }
-                        }
-                      });
+  walk_list<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
+               [&](uint32_t j) {
+                 F f{x[j], z[j], 0.0, 0.0};
+                 if (ECS) {
+                   f.u = u[j];
+                   f.w = w[j];
+                 }
+                 return f;
+               },
+               [&](const uint32_t*, const F* f, const bool* in) {
+                 double wg[4], hs[4];
+                 bool e[4];
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   const double dx = f[v].x - xi, dz = f[v].z - zi;
+                   const double r2 = dx * dx + dz * dz;
+                   e[v] = in[v] && r2 < k.re2;
+                   const double r = sqrt(r2);
+                   wg[v] = weight(r, k.re);
+                   hs[v] = (dx * (f[v].u - ui) + dz * (f[v].w - wi)) / (r * r * r);
+                 }
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   if (DENS) s = e[v] ? s + wg[v] : s;
+                   if (ECS) h = e[v] ? h + hs[v] : h;
+                 }
+               });
   double thisNws, thisN;
   if (DENS) {
     thisNws = s;
@@ -168,23 +172,33 @@ __global__ void __launch_bounds__(kBlock) k_explicit(size_t n, const double* __r
     double x, z, u, w;
     uint8_t t;
   };
-  walk_list<kWalk, F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-                      [&](uint32_t j) { return F{x[j], z[j], u[j], w[j], type[j]}; },
-                      [&](uint32_t, const F& f) {
-                        const double dx = f.x - xi, dz = f.z - zi;
-                        const double r2 = dx * dx + dz * dz;
-                        if (r2 < k.rl2 && f.t != kDummy) {
-                          const double r = sqrt(r2);
-                          const double c = k.nu * 3.0 * k.rl / k.n0l / (r * r * r);
-                          vx += c * (f.u - ui);
-                          vz += c * (f.w - wi);
-                        }
-                        if (r2 < k.re2) {
-                          const double wg = weight(sqrt(r2), k.re);
-                          sx += wg * dx;
-                          sz += wg * dz;
-                        }
-                      });
+  walk_list<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
+               [&](uint32_t j) { return F{x[j], z[j], u[j], w[j], type[j]}; },
+               [&](const uint32_t*, const F* f, const bool* in) {
+                 double tx[4], tz[4], cx[4], cz[4];
+                 bool e[4], l[4];
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   const double dx = f[v].x - xi, dz = f[v].z - zi;
+                   const double r2 = dx * dx + dz * dz;
+                   e[v] = in[v] && r2 < k.re2;
+                   l[v] = in[v] && r2 < k.rl2 && f[v].t != kDummy;
+                   const double r = sqrt(r2);
+                   const double c = k.nu * 3.0 * k.rl / k.n0l / (r * r * r);
+                   tx[v] = c * (f[v].u - ui);
+                   tz[v] = c * (f[v].w - wi);
+                   const double wg = weight(r, k.re);
+                   cx[v] = wg * dx;
+                   cz[v] = wg * dz;
+                 }
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   vx = l[v] ? vx + tx[v] : vx;
+                   vz = l[v] ? vz + tz[v] : vz;
+                   sx = e[v] ? sx + cx[v] : sx;
+                   sz = e[v] ? sz + cz[v] : sz;
+                 }
+               });
   double gxp, gzp;
   if (ghost_pos(xi, zi, sx, sz, nws[i], k.n0, k.re, gxp, gzp)) {
     const double rx = xi - gxp, rz = zi - gzp;
@@ -233,39 +247,44 @@ __global__ void __launch_bounds__(kBlock) k_density_explicit(size_t n, const dou
   const bool fluid = (ti == kFluid);
   const double xi = x[i], zi = z[i], ui = u[i], wi = w[i];
   double s = 0.0, h = 0.0;                     // density, HS
-  double vx = 0, vz = 0, sx = 0, sz = 0;       // viscosity, ghost direction (fluid)
+  double vx = 0, vz = 0, sx = 0, sz = 0;       // viscosity, ghost direction (used for fluid particles only)
   struct F {
-    double x, z, u, w;
+    double2 xz, uw;
     uint8_t t;
   };
-  walk_list<kWalk, F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-                      [&](uint32_t j) {
-                        const double2 pj = xz[j], vj = uw[j];
-                        return F{pj.x, pj.y, vj.x, vj.y, type[j]};
-                      },
-                      [&](uint32_t, const F& f) {
-                        const double dx = f.x - xi, dz = f.z - zi;
-                        const double r2 = dx * dx + dz * dz;
-                        if (r2 < k.re2) {
-                          const double r = sqrt(r2);
-                          s += weight(r, k.re);
-                          const double du = f.u - ui, dw = f.w - wi;
-                          h += (dx * du + dz * dw) / (r * r * r);
-                        }
-                        if (fluid) {
-                          if (r2 < k.rl2 && f.t != kDummy) {
-                            const double r = sqrt(r2);
-                            const double c = k.nu * 3.0 * k.rl / k.n0l / (r * r * r);
-                            vx += c * (f.u - ui);
-                            vz += c * (f.w - wi);
-                          }
-                          if (r2 < k.re2) {
-                            const double wg = weight(sqrt(r2), k.re);
-                            sx += wg * dx;
-                            sz += wg * dz;
-                          }
-                        }
-                      });
+  // (collecting the r_e neighbours first, as walk_near does, gains nothing here: most
+  // of the arithmetic is the viscosity's, over all of them; 186 us instead of 179)
+  walk_list<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
+               [&](uint32_t j) { return F{xz[j], uw[j], type[j]}; },
+               [&](const uint32_t*, const F* f, const bool* in) {
+                 double wg[4], hs[4], tx[4], tz[4], cx[4], cz[4];
+                 bool e[4], l[4];
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   const double dx = f[v].xz.x - xi, dz = f[v].xz.y - zi;
+                   const double r2 = dx * dx + dz * dz;
+                   e[v] = in[v] && r2 < k.re2;
+                   l[v] = in[v] && r2 < k.rl2 && f[v].t != kDummy;
+                   const double r = sqrt(r2);
+                   const double du = f[v].uw.x - ui, dw = f[v].uw.y - wi;
+                   wg[v] = weight(r, k.re);
+                   hs[v] = (dx * du + dz * dw) / (r * r * r);
+                   const double c = k.nu * 3.0 * k.rl / k.n0l / (r * r * r);
+                   tx[v] = c * du;
+                   tz[v] = c * dw;
+                   cx[v] = wg[v] * dx;
+                   cz[v] = wg[v] * dz;
+                 }
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   s = e[v] ? s + wg[v] : s;
+                   h = e[v] ? h + hs[v] : h;
+                   vx = l[v] ? vx + tx[v] : vx;
+                   vz = l[v] ? vz + tz[v] : vz;
+                   sx = e[v] ? sx + cx[v] : sx;
+                   sz = e[v] ? sz + cz[v] : sz;
+                 }
+               });
   const double thisN = (s < k.n0) ? k.n0 : s;
   nws[i] = s;
   nd[i] = thisN;
@@ -345,8 +364,8 @@ __global__ void __launch_bounds__(kBlock) k_writeback(size_t n, const uint8_t* _
 }
 
 // ModifyByPressureGradient, midpoint form (Computer.hpp:1501-1521).
-__global__ void __launch_bounds__(kBlock) k_gradient(size_t n, const double* __restrict__ x,
-                                                     const double* __restrict__ z,
+template <bool NEAR>
+__global__ void __launch_bounds__(kBlock) k_gradient(size_t n, const double2* __restrict__ xz,
                                                      const double* __restrict__ p,
                                                      const uint8_t* __restrict__ type, NV nb, Consts k,
                                                      const double* __restrict__ nws,
@@ -354,28 +373,47 @@ __global__ void __launch_bounds__(kBlock) k_gradient(size_t n, const double* __r
   const size_t i = thread_particle();
   if (i >= n) return;
   if (type[i] != kFluid) return;
-  const double xi = x[i], zi = z[i], pi = p[i];
+  const double2 xzi = xz[i];
+  const double xi = xzi.x, zi = xzi.y, pi = p[i];
   double fx = 0, fz = 0, sx = 0, sz = 0;
+  struct None {};
   struct F {
-    double x, z, p;
+    double p;
     uint8_t t;
   };
-  walk_list<kWalk, F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-                      [&](uint32_t j) { return F{x[j], z[j], p[j], type[j]}; },
-                      [&](uint32_t, const F& f) {
-                        const double dx = f.x - xi, dz = f.z - zi;
-                        const double r2 = dx * dx + dz * dz;
-                        if (r2 < k.re2) {
-                          const double wg = weight(sqrt(r2), k.re);
-                          sx += wg * dx;
-                          sz += wg * dz;
-                          if (f.t != kDummy) {
-                            const double s = (f.p + pi) / r2 * wg;
-                            fx += s * dx;
-                            fz += s * dz;
-                          }
-                        }
-                      });
+  __shared__ uint32_t queue[NEAR ? kNearQueue : 1][kBlock];
+  walk_near<NEAR, kBlock, None, F>(
+      static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax, xz, queue, [&](uint32_t) { return None{}; },
+      [&](uint32_t j) { return F{p[j], type[j]}; },
+      [&](const uint32_t*, const double2* q, const None*, const bool* in, bool* e) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const double dx = q[v].x - xi, dz = q[v].y - zi;
+          e[v] = in[v] && dx * dx + dz * dz < k.re2;
+        }
+      },
+      [&](const double2* q, const F* f, const bool* e) {
+        double tx[4], tz[4], cx[4], cz[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const double dx = q[v].x - xi, dz = q[v].y - zi;
+          const double r2 = dx * dx + dz * dz;
+          const double wg = weight(sqrt(r2), k.re);
+          cx[v] = wg * dx;
+          cz[v] = wg * dz;
+          const double s = (f[v].p + pi) / r2 * wg;
+          tx[v] = s * dx;
+          tz[v] = s * dz;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const bool g = e[v] && f[v].t != kDummy;
+          sx = e[v] ? sx + cx[v] : sx;
+          sz = e[v] ? sz + cz[v] : sz;
+          fx = g ? fx + tx[v] : fx;
+          fz = g ? fz + tz[v] : fz;
+        }
+      });
   double gxp, gzp;
   if (ghost_pos(xi, zi, sx, sz, nws[i], k.n0, k.re, gxp, gzp)) {
     const double dx = gxp - xi, dz = gzp - zi;
@@ -389,9 +427,10 @@ __global__ void __launch_bounds__(kBlock) k_gradient(size_t n, const double* __r
   duz[i] = coef * fz;
 }
 
-// DynamicStabilize first pass (Computer.hpp:1576-1635).
-__global__ void __launch_bounds__(kBlock) k_ds(size_t n, const double* __restrict__ x,
-                                               const double* __restrict__ z,
+// DynamicStabilize first pass (Computer.hpp:1576-1635).  Bound by the gathers:
+// one 16-byte one per neighbour, where two coordinates and a type apart took
+// 102 us for 1.05M particles and 19 for 131k (now 64 and 11).
+__global__ void __launch_bounds__(kBlock) k_ds(size_t n, const double2* __restrict__ xz,
                                                const double* __restrict__ ox,
                                                const double* __restrict__ oz,
                                                const uint8_t* __restrict__ type, NV nb, Consts k,
@@ -399,30 +438,29 @@ __global__ void __launch_bounds__(kBlock) k_ds(size_t n, const double* __restric
   const size_t i = thread_particle();
   if (i >= n) return;
   if (type[i] != kFluid) return;
-  const double xi = x[i], zi = z[i], oxi = ox[i], ozi = oz[i];
+  const double2 xzi = xz[i];
+  const double xi = xzi.x, zi = xzi.y, oxi = ox[i], ozi = oz[i];
   double fx = 0, fz = 0;
-  // X0 is read only for the few neighbours closer than d = (1 - C) l0
-  struct F {
-    double x, z;
-    uint8_t t;
-  };
-  walk_list<kWalk, F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-                      [&](uint32_t j) { return F{x[j], z[j], type[j]}; },
-                      [&](uint32_t j, const F& f) {
-    const double dx = f.x - xi, dz = f.z - zi;
-    const double r2 = dx * dx + dz * dz;
-    if (r2 < k.re2 && f.t != kDummy && r2 < k.d2) {
-      const double e0x = ox[j] - oxi, e0z = oz[j] - ozi;
-      const double nrm = sqrt(e0x * e0x + e0z * e0z);
-      const double ex = e0x / nrm, ez = e0z / nrm;
-      const double rpar = dx * ex + dz * ez;
-      const double px = dx - rpar * ex, pz = dz - rpar * ez;
-      const double rperp2 = px * px + pz * pz;
-      const double m = sqrt(k.d2 - rperp2) - rpar;
-      fx += m * ex;
-      fz += m * ez;
-    }
-                      });
+  // X0 and the type are read only for the few neighbours closer than d = (1 - C) l0
+  walk_list<double2>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
+                     [&](uint32_t j) { return xz[j]; },
+                     [&](const uint32_t* j, const double2* f, const bool* in) {
+#pragma unroll
+                 for (int v = 0; v < 4; v++) {
+                   const double dx = f[v].x - xi, dz = f[v].y - zi;
+                   const double r2 = dx * dx + dz * dz;
+                   if (!(in[v] && r2 < k.re2 && r2 < k.d2) || type[j[v]] == kDummy) continue;
+                   const double e0x = ox[j[v]] - oxi, e0z = oz[j[v]] - ozi;
+                   const double nrm = sqrt(e0x * e0x + e0z * e0z);
+                   const double ex = e0x / nrm, ez = e0z / nrm;
+                   const double rpar = dx * ex + dz * ez;
+                   const double px = dx - rpar * ex, pz = dz - rpar * ez;
+                   const double rperp2 = px * px + pz * pz;
+                   const double m = sqrt(k.d2 - rperp2) - rpar;
+                   fx += m * ex;
+                   fz += m * ez;
+                 }
+               });
   const double coef = -1.0 / (2 * k.dt * k.n0);
   dux[i] = coef * fx;
   duz[i] = coef * fz;
@@ -435,15 +473,18 @@ __global__ void __launch_bounds__(kBlock) k_apply_du(size_t n, double* __restric
                                                      double* __restrict__ w,
                                                      const uint8_t* __restrict__ type,
                                                      const double* __restrict__ dux,
-                                                     const double* __restrict__ duz, double dt) {
+                                                     const double* __restrict__ duz, double dt,
+                                                     double2* __restrict__ xz) {
   const size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
   if (i >= n) return;
   if (type[i] != kFluid) return;
   const double ax = dux[i], az = duz[i];
+  const double xn = x[i] + ax * dt, zn = z[i] + az * dt;
   u[i] = u[i] + ax;
   w[i] = w[i] + az;
-  x[i] = x[i] + ax * dt;
-  z[i] = z[i] + az * dt;
+  x[i] = xn;
+  z[i] = zn;
+  if (xz) xz[i] = make_double2(xn, zn);
 }
 
 // The API's per-particle arrays between the caller's order and storage order:
@@ -719,36 +760,39 @@ void pressure_writeback(Context& c) {
   check_launch();
 }
 
-void pressure_gradient(Context& c) {
+void pressure_gradient(Context& c, bool packed) {
   const size_t n = c.n;
   if (n == 0) return;
+  if (!packed) pack_state(c);
   const Consts k = consts(c);
   tracked(c, MPS_K_GRADIENT, n * (24.0 + 1 + 4 + 8 + 16) + 4.0 * c.nbr_total, [&] {
-    hipLaunchKernelGGL(k_gradient, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.p,
-                       static_cast<const uint8_t*>(c.type), nview(c), k,
-                       static_cast<const double*>(c.nws), c.dux, c.duz);
+    hipLaunchKernelGGL(near_pays(k.re, k.rl) ? k_gradient<true> : k_gradient<false>, dim3(grid_for(n)), dim3(kBlock), 0,
+                       c.stream, n, static_cast<const double2*>(c.xz), static_cast<const double*>(c.p),
+                       static_cast<const uint8_t*>(c.type), nview(c), k, static_cast<const double*>(c.nws), c.dux,
+                       c.duz);
   });
-  tracked(c, MPS_K_UPDATE, n * (32.0 + 1 + 16 + 32), [&] {
+  tracked(c, MPS_K_UPDATE, n * (32.0 + 1 + 16 + 32 + 16), [&] {
     hipLaunchKernelGGL(k_apply_du, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w,
                        static_cast<const uint8_t*>(c.type), static_cast<const double*>(c.dux),
-                       static_cast<const double*>(c.duz), c.dt);
+                       static_cast<const double*>(c.duz), c.dt, c.xz);
   });
   check_launch();
 }
 
-void dynamic_stabilize(Context& c) {
+void dynamic_stabilize(Context& c, bool packed) {
   const size_t n = c.n;
   if (n == 0) return;
+  if (!packed) pack_state(c);
   const Consts k = consts(c);
   tracked(c, MPS_K_DS, n * (32.0 + 1 + 4 + 16) + 4.0 * c.nbr_total, [&] {
-    hipLaunchKernelGGL(k_ds, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z,
+    hipLaunchKernelGGL(k_ds, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, static_cast<const double2*>(c.xz),
                        static_cast<const double*>(c.ox), static_cast<const double*>(c.oz),
                        static_cast<const uint8_t*>(c.type), nview(c), k, c.dux, c.duz);
   });
   tracked(c, MPS_K_UPDATE, n * (32.0 + 1 + 16 + 32), [&] {
     hipLaunchKernelGGL(k_apply_du, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w,
                        static_cast<const uint8_t*>(c.type), static_cast<const double*>(c.dux),
-                       static_cast<const double*>(c.duz), c.dt);
+                       static_cast<const double*>(c.duz), c.dt, static_cast<double2*>(nullptr));
   });
   check_launch();
 }

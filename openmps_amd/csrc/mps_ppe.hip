@@ -39,8 +39,6 @@ struct PpeConsts {
   double qx0, qz0, qinv;  // fixed-point positions: q = (x - x0) * qinv mod 2^32
 };
 
-constexpr int kWalk = 4;  // neighbours whose loads are issued together (walk_list)
-
 // Column j of row i fits the 16-bit offset j - i.
 __device__ __forceinline__ bool offset16(uint32_t j, size_t i) {
   const long long off = static_cast<long long>(j) - static_cast<long long>(i);
@@ -66,7 +64,20 @@ __device__ __forceinline__ void count_slice(size_t n, size_t sl, uint32_t cnt, b
   block_count<kBlock>(cnt, nnz_total);
 }
 
-// b and x0 (Computer.hpp:1185-1221), row lengths and slice widths.
+// The SPP ghost's share of a row's diagonal (Computer.hpp:1232-1328), 0 without a
+// ghost: from the sums over the r_e neighbours that the count passes have in
+// hand, left in diag for the fill.
+__device__ __forceinline__ double ghost_entry(const PpeConsts& k, double xi, double zi, double sx, double sz,
+                                              double nws_i) {
+  double gxp, gzp;
+  if (!ghost_pos(xi, zi, sx, sz, nws_i, k.n0, k.re, gxp, gzp)) return 0.0;
+  const double rx = xi - gxp, rz = zi - gzp;
+  const double r = sqrt(rx * rx + rz * rz);
+  const double a = 3 * k.rl / k.n0l / (r * r * r);
+  return -a;
+}
+
+// b and x0 (Computer.hpp:1185-1221), row lengths, slice widths and the ghosts' shares.
 __global__ void __launch_bounds__(kBlock) k_ppe_count(size_t n, const double* __restrict__ x,
                                                       const double* __restrict__ z,
                                                       const double* __restrict__ u,
@@ -81,7 +92,7 @@ __global__ void __launch_bounds__(kBlock) k_ppe_count(size_t n, const double* __
                                                       uint8_t* __restrict__ slice_wide,
                                                       uint2* __restrict__ qpos,
                                                       unsigned long long* nnz_total,
-                                                      unsigned long long* nnz_wide) {
+                                                      unsigned long long* nnz_wide, double* __restrict__ diag) {
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
   const size_t i = blk * static_cast<size_t>(blockDim.x) + threadIdx.x;
   uint32_t cnt = 0;
@@ -97,26 +108,38 @@ __global__ void __launch_bounds__(kBlock) k_ppe_count(size_t n, const double* __
       sol[i] = 0;
     } else {
       const double xi = x[i], zi = z[i], ui = u[i], wi = w[i];
-      double h = 0.0;
+      double h = 0.0, sx = 0.0, sz = 0.0;
       struct F {
         double x, z, u, w;
         uint8_t t;
       };
-      walk_list<kWalk, F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-                          [&](uint32_t j) { return F{x[j], z[j], u[j], w[j], type[j]}; },
-                          [&](uint32_t j, const F& f) {
-                            const double dx = f.x - xi, dz = f.z - zi;
-                            const double r2 = dx * dx + dz * dz;
-                            if (r2 < k.re2) {
-                              const double r = sqrt(r2);
-                              const double du = f.u - ui, dw = f.w - wi;
-                              h += (dx * du + dz * dw) / (r * r * r);
-                            }
-                            if (r2 < k.rl2 && f.t != kDummy) {
-                              cnt++;
-                              fits = fits && offset16(j, i);
-                            }
-                          });
+      walk_list<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
+                   [&](uint32_t j) { return F{x[j], z[j], u[j], w[j], type[j]}; },
+                   [&](const uint32_t* j, const F* f, const bool* in) {
+                     double hs[4], tx[4], tz[4];
+                     bool e[4];
+#pragma unroll
+                     for (int v = 0; v < 4; v++) {
+                       const double dx = f[v].x - xi, dz = f[v].z - zi;
+                       const double r2 = dx * dx + dz * dz;
+                       e[v] = in[v] && r2 < k.re2;
+                       const double r = sqrt(r2);
+                       hs[v] = (dx * (f[v].u - ui) + dz * (f[v].w - wi)) / (r * r * r);
+                       const double wg = weight(r, k.re);
+                     tx[v] = wg * dx;
+                     tz[v] = wg * dz;
+                     const bool l = in[v] && r2 < k.rl2 && f[v].t != kDummy;
+                       cnt += l ? 1u : 0u;
+                       fits = fits && (!l || offset16(j[v], i));
+                     }
+#pragma unroll
+                     for (int v = 0; v < 4; v++) {
+                       h = e[v] ? h + hs[v] : h;
+                     sx = e[v] ? sx + tx[v] : sx;
+                     sz = e[v] ? sz + tz[v] : sz;
+                     }
+                   });
+      diag[i] = ghost_entry(k, xi, zi, sx, sz, nws[i]);
       const double speed = (nws[i] < k.n0) ? 0.0 : -k.re * h;  // HS, :838-872
       b[i] = -k.rho / (k.n0 * k.dt) * (speed + ecs[i]);
       sol[i] = (k.warm == MPS_WARM_ZERO) ? 0.0 : p[i];
@@ -131,6 +154,7 @@ __global__ void __launch_bounds__(kBlock) k_ppe_count(size_t n, const double* __
 // moves between the two stages, so the RHS reads the positions, velocities
 // and nWithoutSpp the density pass has in hand.  Every value is computed as
 // the two separate kernels compute it (same expressions, same list order).
+template <bool NEAR>
 __global__ void __launch_bounds__(kBlock) k_density_ppe_count(size_t n, const double* __restrict__ x,
                                                               const double* __restrict__ z,
                                                               const double* __restrict__ u,
@@ -149,7 +173,9 @@ __global__ void __launch_bounds__(kBlock) k_density_ppe_count(size_t n, const do
                                                               unsigned long long* nnz_total,
                                                               unsigned long long* nnz_wide,
                                                               const double2* __restrict__ xz,
-                                                              const double2* __restrict__ uw) {
+                                                              const double2* __restrict__ uw,
+                                                              double* __restrict__ diag) {
+  __shared__ uint32_t queue[NEAR ? kNearQueue : 1][kBlock];
   const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
   const size_t i = blk * static_cast<size_t>(blockDim.x) + threadIdx.x;
   uint32_t cnt = 0;
@@ -167,45 +193,42 @@ __global__ void __launch_bounds__(kBlock) k_density_ppe_count(size_t n, const do
       ox[i] = xi;
       oz[i] = zi;
       const double ui = u[i], wi = w[i];
-      double s = 0.0, h = 0.0;
-      const uint32_t m = nb.count[i];
-      auto use = [&](uint32_t j, double xj, double zj, double uj, double wj, uint8_t tj) {
-        const double dx = xj - xi, dz = zj - zi;
-        const double r2 = dx * dx + dz * dz;
-        if (r2 < k.re2) {
-          const double r = sqrt(r2);
-          s += weight(r, k.re);
-          const double du = uj - ui, dw = wj - wi;
-          h += (dx * du + dz * dw) / (r * r * r);
-        }
-        if (r2 < k.rl2 && tj != kDummy) {
-          cnt++;
-          fits = fits && offset16(j, i);
-        }
-      };
-      // kWalk neighbours per round trip: their ids, then all their fields,
-      // loaded before any is used; the sums still run in list order
-      uint32_t q = 0;
-      for (; q + kWalk <= m; q += kWalk) {
-        uint32_t jj[kWalk];
+      double s = 0.0, h = 0.0, sx = 0.0, sz = 0.0;
+      walk_near<NEAR, kBlock, uint8_t, double2>(
+          static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax, xz, queue, [&](uint32_t j) { return type[j]; },
+          [&](uint32_t j) { return uw[j]; },
+          [&](const uint32_t* j, const double2* q, const uint8_t* tj, const bool* in, bool* e) {
 #pragma unroll
-        for (int v = 0; v < kWalk; v++) jj[v] = nb.ids[nbr_slot(static_cast<uint32_t>(i), q + v, nb.kmax)];
-        double2 pj[kWalk], vj[kWalk];
-        uint8_t tj[kWalk];
+            for (int v = 0; v < 4; v++) {
+              const double dx = q[v].x - xi, dz = q[v].y - zi;
+              const double r2 = dx * dx + dz * dz;
+              e[v] = in[v] && r2 < k.re2;
+              const bool l = in[v] && r2 < k.rl2 && tj[v] != kDummy;
+              cnt += l ? 1u : 0u;
+              fits = fits && (!l || offset16(j[v], i));
+            }
+          },
+          [&](const double2* q, const double2* f, const bool* e) {
+            double wg[4], hs[4], tx[4], tz[4];
 #pragma unroll
-        for (int v = 0; v < kWalk; v++) {
-          pj[v] = xz[jj[v]];
-          vj[v] = uw[jj[v]];
-          tj[v] = type[jj[v]];
-        }
+            for (int v = 0; v < 4; v++) {
+              const double dx = q[v].x - xi, dz = q[v].y - zi;
+              const double r2 = dx * dx + dz * dz;
+              const double r = sqrt(r2);
+              wg[v] = weight(r, k.re);
+              hs[v] = (dx * (f[v].x - ui) + dz * (f[v].y - wi)) / (r * r * r);
+              tx[v] = wg[v] * dx;
+              tz[v] = wg[v] * dz;
+            }
 #pragma unroll
-        for (int v = 0; v < kWalk; v++) use(jj[v], pj[v].x, pj[v].y, vj[v].x, vj[v].y, tj[v]);
-      }
-      for (; q < m; q++) {
-        const uint32_t j = nb.ids[nbr_slot(static_cast<uint32_t>(i), q, nb.kmax)];
-        const double2 pj = xz[j], vj = uw[j];
-        use(j, pj.x, pj.y, vj.x, vj.y, type[j]);
-      }
+            for (int v = 0; v < 4; v++) {
+              s = e[v] ? s + wg[v] : s;
+              h = e[v] ? h + hs[v] : h;
+              sx = e[v] ? sx + tx[v] : sx;
+              sz = e[v] ? sz + tz[v] : sz;
+            }
+          });
+      diag[i] = ghost_entry(k, xi, zi, sx, sz, s);
       nws[i] = s;
       nd[i] = (s < k.n0) ? k.n0 : s;
       const double speed = (s < k.n0) ? 0.0 : -k.re * h;  // HS, :838-872
@@ -300,7 +323,7 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
     g = 1.0;
   } else {
     const double xi = x[i], zi = z[i];
-    double s = 0.0, sx = 0, sz = 0;
+    double s = 0.0;
     const uint32_t m = nb.count[i];
     // the emitted columns (r < r_lap, not dummy) form at most 9 ascending
     // runs, one per cell: their starts, for the merge below
@@ -312,46 +335,51 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
       double x, z;
       uint8_t t;
     };
-    walk_list<kWalk, F>(self, m, nb.ids, nb.kmax,
-                        [&](uint32_t j) {
-                          const double2 pj = xz[j];
-                          return F{pj.x, pj.y, type[j]};
-                        },
-                        [&](uint32_t j, const F& f) {
-      const double dx = f.x - xi, dz = f.z - zi;
-      const double r2 = dx * dx + dz * dz;
-      if (r2 < k.rl2 && f.t != kDummy) {
-        const double r = sqrt(r2);
-        s += -(3 * k.rl / k.n0l / (r * r * r));
-        if (ne == 0 || j < prev) {
-          if (nr < kRuns) {
+    walk_list<F>(self, m, nb.ids, nb.kmax,
+                 [&](uint32_t j) {
+                   const double2 pj = xz[j];
+                   return F{pj.x, pj.y, type[j]};
+                 },
+                 [&](const uint32_t* j, const F* f, const bool* in) {
+                   double a[4];
+                   bool l[4];
 #pragma unroll
-            for (int u = 0; u < kRuns; u++)
-              if (u == nr) er[u] = ne;
-            nr++;
-          } else {
-            staged = false;  // not a cell-ordered list: store in list order
-          }
-        }
-        prev = j;
-        if (ne < kStage) stage[ne][t] = j;
-        else staged = false;
-        ne++;
-      }
-      if (r2 < k.re2) {
-        const double wg = weight(sqrt(r2), k.re);
-        sx += wg * dx;
-        sz += wg * dz;
-      }
-                        });
-    double gxp, gzp;
-    if (ghost_pos(xi, zi, sx, sz, nws[i], k.n0, k.re, gxp, gzp)) {
-      const double rx = xi - gxp, rz = zi - gzp;
-      const double r = sqrt(rx * rx + rz * rz);
-      const double a = 3 * k.rl / k.n0l / (r * r * r);
-      s += -a;
-      g = -a;
-    }
+                   for (int v = 0; v < 4; v++) {
+                     const double dx = f[v].x - xi, dz = f[v].z - zi;
+                     const double r2 = dx * dx + dz * dz;
+                     l[v] = in[v] && r2 < k.rl2 && f[v].t != kDummy;
+                     const double r = sqrt(r2);
+                     a[v] = 3 * k.rl / k.n0l / (r * r * r);
+                   }
+#pragma unroll
+                   for (int v = 0; v < 4; v++) {
+                     s = l[v] ? s + -a[v] : s;
+                     if (l[v]) {
+                       // stored at once, in list order; the merge below writes rows whose
+                       // list is not ascending again
+                       const size_t o = base + static_cast<size_t>(ne) * 64;
+                       val[o] = a[v];
+                       if (wide) col[o] = j[v];
+                       col16[o] = static_cast<int16_t>(static_cast<long long>(j[v]) - static_cast<long long>(self));
+                       if (ne == 0 || j[v] < prev) {
+                         if (nr < kRuns) {
+#pragma unroll
+                           for (int u = 0; u < kRuns; u++)
+                             if (u == nr) er[u] = ne;
+                           nr++;
+                         } else {
+                           staged = false;  // not a cell-ordered list: store in list order
+                         }
+                       }
+                       prev = j[v];
+                       if (ne < kStage) stage[ne][t] = j[v];
+                       else staged = false;
+                       ne++;
+                     }
+                   }
+                 });
+    g = diag[i];  // the ghost's share, from the count pass
+    if (g != 0.0) s += g;
     d = s;
     const uint32_t ki = ag.s0 ? ag.key[i] : kNoCell;
     const uint32_t cx = ki / ag.gnz, cz = ki % ag.gnz;
@@ -359,17 +387,8 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
     // ROWS9: the row's cell when it takes part (its row length is known from the count pass)
     const uint32_t k9 = ROWS9 ? ag.aggkey[i] : kNoCell;
     const int c9x = static_cast<int>(k9 / ag.gnz), c9z = static_cast<int>(k9 % ag.gnz);
-    // value of an emitted column j in slot kk (and its share of the aggregate row sums)
-    auto emit = [&](uint32_t j) {
-      const double2 pj = xz[j];
-      const double dx = pj.x - xi, dz = pj.y - zi;
-      const double r = sqrt(dx * dx + dz * dz);
-      const size_t o = base + static_cast<size_t>(kk) * 64;
-      const double a = 3 * k.rl / k.n0l / (r * r * r);
-      val[o] = a;
-      if (wide) col[o] = j;
-      col16[o] = static_cast<int16_t>(static_cast<long long>(j) - static_cast<long long>(self));
-      kk++;
+    // the share of a stored entry in the aggregate row sums
+    auto share = [&](uint32_t j, double a) {
       if (ki != kNoCell) {
         const uint32_t kj = ag.key[j];
         if (kj != kNoCell) {
@@ -389,6 +408,19 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
         if (kj != kNoCell) dir = 3 * (static_cast<int>(kj / ag.gnz) - c9x + 1) + static_cast<int>(kj % ag.gnz) - c9z + 1;
       }
       return make_pair_da(dir, a);
+    };
+    // value of an emitted column j in slot kk (and its share)
+    auto emit = [&](uint32_t j) {
+      const double2 pj = xz[j];
+      const double dx = pj.x - xi, dz = pj.y - zi;
+      const double r = sqrt(dx * dx + dz * dz);
+      const size_t o = base + static_cast<size_t>(kk) * 64;
+      const double a = 3 * k.rl / k.n0l / (r * r * r);
+      val[o] = a;
+      if (wide) col[o] = j;
+      col16[o] = static_cast<int16_t>(static_cast<long long>(j) - static_cast<long long>(self));
+      kk++;
+      return share(j, a);
     };
     // consecutive columns of one direction are summed in a run and the run
     // added to its direction's sum when the direction changes (in cell order
@@ -414,10 +446,13 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
     };
     if (staged && nr <= 1) {
       // one ascending run (the particles in cell order: the list visits the
-      // cells, and each cell's members, in ascending index order): the
-      // staged columns in their order
+      // cells, and each cell's members, in ascending index order): stored by
+      // the walk; the sums need the diagonal first, so they read the values back
+      kk = ne;
+      if (ki != kNoCell || k9 != kNoCell) {
 #pragma unroll 4
-      for (uint32_t v = 0; v < ne; v++) add9(emit(stage[v][t]));
+        for (uint32_t v = 0; v < ne; v++) add9(share(stage[v][t], val[base + static_cast<size_t>(v) * 64]));
+      }
     } else if (staged) {
       // 9-way merge of the staged runs (LDS only on its dependency chain),
       // the ascending columns written first, the values computed after
@@ -742,7 +777,7 @@ void ppe_assemble(Context& c) {
     hipLaunchKernelGGL(k_ppe_count, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w,
                        c.p, static_cast<const uint8_t*>(c.type), nb, k, static_cast<const double*>(c.nws),
                        static_cast<const double*>(c.ecs), c.b, c.sol, c.row_len, c.slice_width,
-                       c.slice_wide, c.qpos, c.ppe_counters, c.ppe_counters + 1);
+                       c.slice_wide, c.qpos, c.ppe_counters, c.ppe_counters + 1, c.diag);
   });
   check_launch();
   pack_state(c);  // the fill gathers the packed positions
@@ -757,12 +792,12 @@ void density_save_and_assemble(Context& c) {
   // the second density pass's bytes and the count pass's (x, z, u, w, p, type,
   // ecs read; n, nWithoutSpp, X0, b, x0, row length, position written)
   tracked(c, MPS_K_DENSITY_SAVE, n * (40.0 + 1 + 8 + 4 + 16 + 16 + 16 + 4 + 8) + 4.0 * c.nbr_total, [&] {
-    hipLaunchKernelGGL(k_density_ppe_count, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u,
-                       c.w, c.p, static_cast<const uint8_t*>(c.type), nb, k, c.nd, c.nws,
+    hipLaunchKernelGGL(near_pays(k.re, k.rl) ? k_density_ppe_count<true> : k_density_ppe_count<false>,
+                       dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w, c.p, static_cast<const uint8_t*>(c.type), nb, k, c.nd, c.nws,
                        static_cast<const double*>(c.ecs), c.ox, c.oz, c.b, c.sol, c.row_len, c.slice_width,
                        c.slice_wide, c.qpos, c.ppe_counters, c.ppe_counters + 1,
                        static_cast<const double2*>(c.xz),
-                       static_cast<const double2*>(c.uw));
+                       static_cast<const double2*>(c.uw), c.diag);
   });
   check_launch();
   ppe_finish(c, k);

@@ -1,0 +1,65 @@
+"""The neighbour search and the list walks on uneven neighbourhoods: cells from
+one to the most particles a cell may hold, so that the lanes of a wavefront
+find very different numbers of neighbours (rings that fill before the others
+complete a group, near neighbours in several portions, lists from empty to the
+longest), particle counts around a wavefront's and a block's, radii far apart
+and equal.  Lists, densities, accelerations, the assembled system, gradient and
+stabilisation are the oracle's bit for bit; a whole step, whose passes are
+fused, assembles the system of the separate stages."""
+import numpy as np
+import pytest
+
+import cases
+from openmps_amd import ComputerException
+from test_gpu_parity import compare_stage
+
+pytestmark = pytest.mark.gpu
+L0 = 0.01
+
+
+def cloud(n, nl, side, cap, seed):
+    """n particles in random cells of size nl (at most cap in one)."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    cells = rng.permutation(side * side)
+    x, z, k = [], [], 0
+    while len(x) < n:
+        m = min(n - len(x), int(rng.integers(1, cap + 1)) if k % 3 else 1)
+        c = cells[k]
+        x.extend((c // side + rng.uniform(0.02, 0.98, m)) * nl)
+        z.extend((c % side + rng.uniform(0.02, 0.98, m)) * nl)
+        k += 1
+    t = rng.choice(np.array([0, 0, 0, 0, 1, 2], np.uint8), n)
+    f = [rng.standard_normal(n) * 1e-2 for _ in range(2)] + [rng.uniform(0, 100, n)]
+    return dict(x=np.array(x), z=np.array(z), u=f[0], w=f[1], p=f[2], n=np.zeros(n), type=t)
+
+
+@pytest.mark.parametrize("r_e,r_lap", [(2.1, 3.1), (2.4, 2.4), (3.1, 2.1)])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 257, 1500])
+def test_uneven_neighbourhoods(n, r_e, r_lap):
+    probe = cases.make("gpu", cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, r_e, L0, 0, 0, 1, 1, r_lap), 1e-9)
+    nl, cap = probe.env()["neighbor_length"], probe.grid()["cap"]
+    side = max(2, int(np.ceil(np.sqrt(n / (cap / 4)))) + 1)
+    env = cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, r_e, L0, 0.0, 0.0, side * nl, side * nl, r_lap)
+    parts = cloud(n, nl, side, cap, 7 * n + int(10 * r_e))
+    g, o, whole = cases.make("gpu", env, 1e-9), cases.make("oracle", env, 1e-9), cases.make("gpu", env, 1e-9)
+    for c in (g, o, whole):
+        c.add_particles(parts)
+        c.set_time(1e-4, 1e-4)
+    for st in ("search", "density", "error_correction", "explicit", "density", "save_x", "ppe_assemble"):
+        g.stage(st)
+        o.stage(st)
+        compare_stage(g, o, st)
+    count = g.neighbors()[0]
+    print(f"  {n} particles, r {r_e}/{r_lap}: {count.min()} to {count.max()} neighbours, {cap} a cell", flush=True)
+    A = g.ppe()
+    for st in ("pressure_gradient", "dynamic_stabilize"):
+        g.stage(st)
+        o.stage(st)
+        compare_stage(g, o, st)
+    whole.set_time(0.0, 0.0)
+    try:
+        whole.forward_time(1e-4)
+    except ComputerException:  # (a random cloud's system need not be solvable)
+        pass
+    for a, b in zip(A[:4], whole.ppe()[:4]):
+        assert np.array_equal(a, b)
