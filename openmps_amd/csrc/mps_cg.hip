@@ -582,19 +582,22 @@ __global__ void __launch_bounds__(NT) k_cg_check(const double* __restrict__ part
 // rows fit one per thread of the workgroups that the chip holds at once: each
 // thread keeps x, r, p, q and its row's first REG matrix entries in registers,
 // the next entries (10 bytes each) in LDS as far as it goes, and streams the
-// rest.  A workgroup gathers r from an LDS copy of exactly the rows its columns
-// name, reloaded every iteration (cell-ordered rows couple to three short
-// ranges of rows, far apart: copying the whole span took 2 us more per
-// iteration at 131k rows).  Two exchanges per iteration (p.q, then r with
-// r.r).  Every value and every sum is computed in the order of the launched
-// kernels, so the two agree bit for bit.  REG = 32 (170 VGPRs) with one
-// workgroup per compute unit, 20 (128 VGPRs) with two.
+// rest.  A workgroup gathers r into an LDS copy of exactly the rows its columns
+// name, every iteration (cell-ordered rows couple to three short ranges of rows,
+// far apart: copying the whole span took 2 us more per iteration at 131k rows).
+// Two exchanges per iteration: p.q, and r.r while the gather waits for the
+// entries of r themselves (flagged, in two buffers: r and p, which the launched
+// solve's p replaces at the end).  Every value and every sum is computed in the
+// order of the launched kernels, so the two agree bit for bit.  REG = 32 (168
+// VGPRs) with one workgroup per compute unit, 20 (128 VGPRs) with two.
 //
-// It is bound by the two exchanges (1.8 us each for 5 workgroups, 2.8 for 256)
-// and the round trip of the gather; launched, by the two launches and, from
-// 100k rows on, by the matrix streams.  Per iteration (dam breaks, 28 entries a
-// row; launched -> resident): 1.5k rows 12.0 -> 4.7 us, 12k 13.0 -> 5.9, 50k
-// 13.7 -> 6.9, 131k 17.9 -> 9.8, 191k 24.0 -> 13.6, 257k 26.5 -> 16.0.
+// It is bound by the two exchanges and, with two workgroups a compute unit, by
+// the LDS reads of the products; launched, by the two launches and, from 100k
+// rows on, by the matrix streams.  Per iteration (dam breaks, 28 entries a row;
+// launched -> resident, in brackets with r stored, waited for and gathered after
+// the sum): 1.5k rows 12.2 -> 4.5 us (4.7), 12k 12.8 -> 4.8 (5.9), 50k 13.9 ->
+// 5.5 (6.9), 125k 17.5 -> 6.5 (8.0), 134k 18.1 -> 9.2 (9.8), 191k 24.1 -> 11.8
+// (13.6), 257k 26.5 -> 14.2 (16.0).
 __global__ void __launch_bounds__(NT) k_resident_clear(ResidentCtl* ctl, CgStatus* st) {
   resident_clear(ctl);
   if (threadIdx.x == 0) *st = CgStatus{};
@@ -746,12 +749,51 @@ __device__ __forceinline__ void gather_values(T* __restrict__ to, const T* from,
   }
 }
 
-// The sum of the workgroups' partial sums of generation gen, in the order in
-// which block_sum<NT> adds one per thread; up to 64 of them by one wavefront.
+// The same of a vector whose entries say that they are there (mps_resident.hpp).
+// Returns thread k's look at workgroup k's partial sum of generation gen, waited
+// for with the first entries when the workgroups are few (5: 0.25 us less an
+// iteration than after them) and after them otherwise (polling more words than
+// needed holds up the stores: 262 workgroups 9.1 instead of 9.9 us).
+__device__ __forceinline__ double gather_flagged(ResidentCtl* ctl, double* __restrict__ to, const double* from,
+                                                 const uint16_t* __restrict__ list, uint32_t wn, unsigned gen,
+                                                 unsigned idx, unsigned G, bool& ok) {
+  double sum = 0.0;
+  uint32_t k0 = threadIdx.x;
+  if (G <= 64) {
+    const double* at[5];
+    double t[5];
+    at[4] = resident_slot(ctl, gen, threadIdx.x < G ? threadIdx.x : idx, 0);
+#pragma unroll
+    for (int u = 0; u < 4; u++) at[u] = k0 + u * NT < wn ? from + list[k0 + u * NT] : at[4];
+    flag_wait(ctl, at, t, ok);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (k0 + u * NT < wn) to[k0 + u * NT] = t[u];
+    sum = threadIdx.x < G ? t[4] : 0.0;
+    k0 += 4 * NT;
+  }
+  for (; k0 < wn; k0 += 4 * NT) {
+    const double* at[4];
+    double t[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) at[u] = from + list[k0 + u * NT < wn ? k0 + u * NT : k0];
+    flag_wait(ctl, at, t, ok);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (k0 + u * NT < wn) to[k0 + u * NT] = t[u];
+  }
+  if (G > 64) {
+    __syncthreads();
+    if (threadIdx.x < G) sum = resident_word(ctl, gen, threadIdx.x, 0, ok);
+  }
+  return sum;
+}
+
+// The sum of the workgroups' partial sums of generation gen (v: thread k's of
+// workgroup k) in the order in which block_sum<NT> adds one per thread; up to 64
+// of them by one wavefront.
 __device__ __forceinline__ double resident_sum(ResidentCtl* ctl, unsigned gen, unsigned idx, unsigned G, double* lds,
-                                               bool& ok) {
-  double v = 0.0;
-  if (threadIdx.x < G) v = resident_word(ctl, gen, threadIdx.x, 0, ok);
+                                               double v, bool& ok) {
   if (G <= 64) {
     v = wave_sum(v);
     if (threadIdx.x == 0) lds[0] = v;
@@ -771,8 +813,8 @@ __device__ __forceinline__ double resident_sum(ResidentCtl* ctl, unsigned gen, u
 // and their numbers), then the gathered rows' list and the matrix entries from
 // REG on that fit.
 template <class M, int REG, int WAVES>
-__global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restrict__ x, double* r,
-                                                           double* __restrict__ p, double* __restrict__ q,
+__global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restrict__ x, double* r, double* p,
+                                                           double* __restrict__ q,
                                                            const double* __restrict__ part_rr,
                                                            const double* __restrict__ part_bb, CgStatus* st,
                                                            StopRule sr, long long max_iter, ResidentCtl* ctl,
@@ -824,10 +866,17 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   double rr_prev = 0.0, bb = 0.0, tol = 0.0;
   if (sr.rule == MPS_STOP_RHS_NORM) bb = scalar_of(block_sum<NT>(threadIdx.x < G ? part_bb[threadIdx.x] : 0.0, lds));
   const double rr0 = rr;
+  // r's two buffers: r, which holds the first one, and p
+  if (in) flag_clear(p + i);
+  stores_done();
+  __syncthreads();
   if (!resident_start(ctl, ok_lds)) return;
   unsigned gen = 0;
   long long it = 1;
   bool conv = false, ok = true;
+  double *cur = r, *next = p;
+  gather_values(win, static_cast<const double*>(r + lo), list, wn);
+  __syncthreads();
   for (;; it++) {
     if (it == 1) {
       if (sr.rule == MPS_STOP_RHS_NORM) {
@@ -841,24 +890,45 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
       conv = (sr.rule == MPS_STOP_RHS_NORM) ? (rr <= tol) : (rr < tol);  // :1408
     }
     if (conv || it > max_iter) break;
-    gather_values(win, static_cast<const double*>(r + lo), list, wn);  // complete: r.r was collected
-    __syncthreads();
     double s = dg * ri;
+    // (opaque: unpacked per iteration, not kept unpacked across them)
+    if constexpr (REG % 8 == 0) {  // eight LDS reads go out together
 #pragma unroll
-    for (int g = 0; g < REG / 4; g++)
-      if (static_cast<uint32_t>(4 * g) < m) {
-        // (opaque: unpacked per iteration, not kept unpacked across them)
-        uint32_t o0 = off[2 * g], o1 = off[2 * g + 1];
-        asm volatile("" : "+v"(o0), "+v"(o1));
-        const double x0 = win[o0 & 0xffffu], x1 = win[o0 >> 16], x2 = win[o1 & 0xffffu], x3 = win[o1 >> 16];
-        s = fma(a[4 * g], x0, s);
-        s = fma(a[4 * g + 1], x1, s);
-        s = fma(a[4 * g + 2], x2, s);
-        s = fma(a[4 * g + 3], x3, s);
-      }
+      for (int g = 0; g < REG / 8; g++)
+        if (static_cast<uint32_t>(8 * g) < m) {
+          uint32_t o[4];
+          double xv[8];
+#pragma unroll
+          for (int u = 0; u < 4; u++) {
+            o[u] = off[4 * g + u];
+            asm volatile("" : "+v"(o[u]));
+          }
+#pragma unroll
+          for (int u = 0; u < 8; u++) xv[u] = win[(u & 1) ? o[u / 2] >> 16 : o[u / 2] & 0xffffu];
+#pragma unroll
+          for (int u = 0; u < 8; u++) s = fma(a[8 * g + u], xv[u], s);
+        }
+    } else {
+#pragma unroll
+      for (int g = 0; g < REG / 4; g++)
+        if (static_cast<uint32_t>(4 * g) < m) {
+          uint32_t o0 = off[2 * g], o1 = off[2 * g + 1];
+          asm volatile("" : "+v"(o0), "+v"(o1));
+          const double x0 = win[o0 & 0xffffu], x1 = win[o0 >> 16], x2 = win[o1 & 0xffffu], x3 = win[o1 >> 16];
+          s = fma(a[4 * g], x0, s);
+          s = fma(a[4 * g + 1], x1, s);
+          s = fma(a[4 * g + 2], x2, s);
+          s = fma(a[4 * g + 3], x3, s);
+        }
+    }
     for (uint32_t k = REG; k < kl; k++)
       s = fma(lval[(k - REG) * NT + threadIdx.x], win[lcol[(k - REG) * NT + threadIdx.x]], s);
-    for (uint32_t k = kl; k < m; k++) s = fma(row.val(k), agent_load(r + row.col(k)), s);
+    for (uint32_t k = kl; k < m; k++) {
+      const double* const at[1] = {cur + row.col(k)};
+      double t[1] = {agent_load(at[0])};
+      if (it > 1) flag_wait(ctl, at, t, ok);
+      s = fma(row.val(k), t[0], s);
+    }
     if (it == 1) {
       pi = ri;
       qi = s;
@@ -867,29 +937,39 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
       pi = fma(beta, pi, ri);
       qi = fma(beta, qi, s);
     }
+    stores_done();  // the entries and slots emptied since the last exchange
     const double sp = block_sum<NT>(in ? fma(pi, qi, 0.0) : 0.0, lds);
-    if (threadIdx.x == 0) resident_publish(ctl, gen, idx, sp);
-    const double alpha = scalar_of(rr / resident_sum(ctl, gen, idx, G, lds, ok));
+    if (threadIdx.x == 0) resident_put(ctl, gen, idx, sp);
+    const double pq1 = threadIdx.x < G ? resident_word(ctl, gen, threadIdx.x, 0, ok) : 0.0;
+    const double pq = resident_sum(ctl, gen, idx, G, lds, pq1, ok);
+    const double alpha = scalar_of(rr / pq);
     gen++;
     if (!ok) return;
     xi = fma(alpha, pi, xi);
     ri = fma(-alpha, qi, ri);
-    if (in) agent_store(r + i, ri);
     const double ww = wave_sum(in ? fma(ri, ri, 0.0) : 0.0);
     if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = ww;
-    stores_done();  // every wavefront's r is out before the block publishes its r.r
     __syncthreads();
+    if (in) {
+      flag_store(next + i, ri);
+      flag_clear(cur + i);  // everyone has published a p.q, so has gathered it
+    }
     if (threadIdx.x == 0) {
       double t = lds[0];
 #pragma unroll
       for (int k = 1; k < NT / 64; k++) t += lds[k];
-      resident_publish(ctl, gen, idx, t);
+      resident_put(ctl, gen, idx, t);
     }
+    double* const swap = cur;
+    cur = next;
+    next = swap;
+    const double rr1 = gather_flagged(ctl, win, static_cast<const double*>(cur + lo), list, wn, gen, idx, G, ok);
     rr_prev = rr;
-    rr = resident_sum(ctl, gen, idx, G, lds, ok);
+    rr = resident_sum(ctl, gen, idx, G, lds, rr1, ok);
     gen++;
     if (!ok) return;
   }
+  if (in) r[i] = ri;
   if (in) {
     x[i] = xi;
     p[i] = pi;

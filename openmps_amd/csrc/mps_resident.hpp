@@ -22,8 +22,8 @@
 // that hands the total on).  Slots are used in a ring of kResRing generations.
 // Emptying: once generation g is complete everyone has published g and so has
 // finished reading g - 1; the owner then empties its slot of g - 1, and that
-// store completes before its publication of g + 1, hence before anyone polls
-// g + 3 (the same ring entry).
+// store completes before its publication of g + 2 (it waits at every second one
+// at least), hence before anyone polls g + 3 (the same ring entry).
 //
 // Every wait is bounded.  Before the first iteration the workgroups wait until
 // all of them have started (they might not fit beside other work on the GPU)
@@ -99,21 +99,30 @@ __device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok) {
   return s_go != 0;
 }
 
-// One thread: the workgroup's values of generation g (after the emptying of an
-// older slot, and whatever else this thread's wavefront stored, is done).
+// One thread: the workgroup's values of generation g.  Every wavefront has waited
+// for its stores of older generations (slots and vector entries emptied) before
+// the workgroup's last __syncthreads.
 template <class... V>
-__device__ __forceinline__ void resident_publish(ResidentCtl* c, unsigned g, unsigned idx, V... values) {
+__device__ __forceinline__ void resident_put(ResidentCtl* c, unsigned g, unsigned idx, V... values) {
   const double v[] = {values...};
-  stores_done();
 #pragma unroll
   for (unsigned k = 0; k < sizeof...(V); k++) {
     const double t = (v[k] != v[k]) ? __builtin_nan("") : v[k];  // never the empty mark
     agent_store(&c->slot[g % kResRing][idx * kResPitch + k], static_cast<unsigned long long>(__double_as_longlong(t)));
   }
 }
+// The same after this thread's own wavefront's stores.
+template <class... V>
+__device__ __forceinline__ void resident_publish(ResidentCtl* c, unsigned g, unsigned idx, V... values) {
+  stores_done();
+  resident_put(c, g, idx, values...);
+}
 
-// Value `word` of workgroup k's slot of generation g once it is published; ok:
-// false if the wait was given up.
+// Value `word` of workgroup k's slot of generation g.
+__device__ __forceinline__ const double* resident_slot(const ResidentCtl* c, unsigned g, unsigned k, int word) {
+  return reinterpret_cast<const double*>(&c->slot[g % kResRing][k * kResPitch + word]);
+}
+// It once it is published; ok: false if the wait was given up.
 __device__ __forceinline__ double resident_word(ResidentCtl* c, unsigned g, unsigned k, int word, bool& ok) {
   const unsigned long long* s = &c->slot[g % kResRing][k * kResPitch + word];
   unsigned long long b = agent_load(s);
@@ -151,6 +160,44 @@ __device__ __forceinline__ void resident_words(ResidentCtl* c, unsigned g, unsig
   }
   v0 = __longlong_as_double(static_cast<long long>(a));
   v1 = __longlong_as_double(static_cast<long long>(b));
+}
+
+// Vectors whose entries say themselves that they are there: two buffers taken in
+// turn, an entry is empty (all ones, a NaN that is never stored) until its owner
+// has written it, and a reader polls the entries it needs.  So neither does the
+// owner wait for its stores before it publishes the partial sum that goes with
+// them, nor the reader for everyone's partial sum before it loads (the CG's
+// iteration in k_cg_resident: 0.2 us less with 3 workgroups, 1.1-1.5 with 24 to
+// 250).  Emptying: the exchange after the readers have used generation g
+// (they publish theirs after it) tells the owner that all of them have; it then
+// empties its entries, and that completes before it publishes again, hence
+// before anyone polls the buffer for generation g + 2.
+__device__ __forceinline__ bool flag_empty(double v) {
+  return static_cast<unsigned long long>(__double_as_longlong(v)) == kResEmpty;
+}
+__device__ __forceinline__ void flag_clear(double* p) {
+  agent_store(reinterpret_cast<unsigned long long*>(p), kResEmpty);
+}
+__device__ __forceinline__ void flag_store(double* p, double v) { agent_store(p, v != v ? __builtin_nan("") : v); }
+// Entries p[0 .. N) once they are there; ok: false if the wait was given up.
+template <int N, class T>
+__device__ __forceinline__ void flag_wait(ResidentCtl* c, const T* const (&p)[N], T (&v)[N], bool& ok) {
+  auto look = [&] {
+    bool there = true;
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = agent_load(p[k]);
+#pragma unroll
+    for (int k = 0; k < N; k++) there = there && !flag_empty(v[k]);
+    return there;
+  };
+  if (look()) return;
+  const long long t0 = wall_clock64();
+  while (!look())
+    if (agent_load(&c->abort) || wall_clock64() - t0 > kResWaitTicks) {
+      agent_store(&c->abort, 1u);
+      ok = false;
+      return;
+    }
 }
 
 // After the whole workgroup has seen generation g complete: its slot of
