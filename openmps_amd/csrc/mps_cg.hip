@@ -2523,9 +2523,8 @@ __global__ void __launch_bounds__(256) k_jacobi_inv(size_t n, const double* __re
 // FP32 coefficients (the matrix-free terms c0 / r^3, computed once: the
 // positions do not move during a solve) in registers and LDS, z gathered from
 // an LDS copy of exactly the rows its columns name.  Cells, one listed 4x4
-// block of cells per wavefront: r and the Jacobi factors of the block's
-// particles in registers, P_s's rows loaded while the workgroup waits for the
-// others.  q goes from rows to cells and z from cells to rows through global
+// block of cells per wavefront, the block's particles' r in registers (see
+// load_cells for the rest).  q goes from rows to cells and z from cells to rows through global
 // memory (agent-scope, mps_resident.hpp), as do the multigrid's direction sums.
 //
 // The cycle is bound by its chain of levels, each a few hundred points or
@@ -2539,7 +2538,7 @@ __global__ void __launch_bounds__(256) k_jacobi_inv(size_t n, const double* __re
 //
 // Time of an iteration, launched and resident, in us:
 //   multilevel   0.7k particles 18.3 / 8.2, 12k 19.1 / 9.3, 63k 19.8 / 10.9, 95k 20.4 / 12.0, 177k 23.7 / 20.6
-//   multigrid    0.7k 44.2 / 21.9, 6k 55 / 28, 25k 68.5 / 36.8, 36k 77 / 41, 63k 81.0 / 45.3, 95k 82.9 / 51.7
+//   multigrid    0.7k 44.2 / 19.7, 6k 55 / 27, 25k 68.5 / 35.7, 36k 77 / 38, 63k 81.0 / 41.3, 95k 82.9 / 49.1
 // What is left of it: the exchanges (2-6 us each with the wait for the
 // slowest), the dependent loads of q, z and the sums after them, and for the
 // multigrid the levels' chain (about 0.5 us a level and direction).
@@ -2810,27 +2809,31 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
   }
   if (active) {
     blk = a.list[w];
-    scl = a.sc[static_cast<size_t>(w) * 64 + lane];
-#pragma unroll
-    for (int u = 0; u < kPerLane; u++) {
-      const size_t o = (static_cast<size_t>(w) * kPerLane + u) * 64 + lane;
-      id[u] = a.pid[o];
-      dv[u] = a.dvp[o];
-    }
     const BlockLane L = block_lane(a.G, blk);
     sub = L.sub;
     if (AMG) pt = L.valid ? amg_point(a, L.cell, a.G.gnz) : -1;
   }
-  auto load_q9s = [&]() {
-    if (AMG && active) {
+  // What the cells' passes read and never changes: ids, Jacobi factors and the
+  // aggregates' scales or P_s's rows.  The multigrid kernel, which has no
+  // registers for them over the rows' part of an iteration, loads them for every
+  // pass while the workgroup waits for the others (38.9 -> 38.2 us an iteration at
+  // 36k particles; for the multilevel one it costs 0.2).
+  auto load_cells = [&]() {
+    if (active) {
       const size_t o0 = static_cast<size_t>(w) * kPerLane * 64 + opaque(lane);
 #pragma unroll
       for (int u = 0; u < kPerLane; u++) {
-        q9[u] = a.q9[o0 + 64 * u];
-        q9c[u] = a.q9c[o0 + 64 * u];
+        id[u] = a.pid[o0 + 64 * u];
+        dv[u] = a.dvp[o0 + 64 * u];
+        if (AMG) {
+          q9[u] = a.q9[o0 + 64 * u];
+          q9c[u] = a.q9c[o0 + 64 * u];
+        }
       }
+      if (!AMG) scl = a.sc[static_cast<size_t>(w) * 64 + opaque(lane)];
     }
   };
+  if (!AMG) load_cells();
   auto row9 = [&](int u, float out[9]) {  // P_s's row of slot u
     const uint32_t h[4] = {q9[u].x, q9[u].y, q9[u].z, q9[u].w};
 #pragma unroll
@@ -2948,6 +2951,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
       __syncthreads();
       double ri = 0.0, bi = 0.0;
       if (in) {
+        const size_t i = opaque(self);  // (addresses formed here: see above)
         double s = A.A.diag[i] * x;
         const double* vp = A.A.val + row.base;
 #pragma unroll
@@ -3102,7 +3106,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
             p = fmaf(beta, p, zi);
             q = fmaf(beta, q, s);
           }
-          agent_store(A.q + i, q);
+          agent_store(A.q + opaque(self), q);
         }
         const double pq1 = wave_sum(in ? fma(static_cast<double>(p), static_cast<double>(q), 0.0) : 0.0);
         if (lane == 0) lds[wv] = pq1;
@@ -3114,7 +3118,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
           for (int k = 1; k < NT / 64; k++) t += lds[k];
           resident_publish(ctl, gen, idx, t);
         }
-        load_q9s();
+        if (AMG) load_cells();
         // alpha, as k_ml_prec's blocks of NTP threads sum it
         double v = 0.0;
         if (tid < NTP) {
@@ -3132,7 +3136,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
       }
 
       // ---- the preconditioner's pass it ----
-      if (it == 0) load_q9s();
+      if (AMG && it == 0) load_cells();
       float s = 0.0f;
       double prho = 0.0, prr = 0.0;
       if (active) {
@@ -3481,7 +3485,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
     total += inner;
     if (in) {
       x = fma(static_cast<double>(d), norm, x);
-      agent_store(A.x + i, x);
+      agent_store(A.x + opaque(self), x);
     }
     if (!barrier()) return;
   }
@@ -4301,9 +4305,12 @@ bool amg_cycle(Context& c, bool fold0, const CgStatus* st, long long it) {
   return left;
 }
 
-// LDS for the levels that every workgroup holds: of its 144 KB the gathered z
-// takes up to 25 and the matrix entries beyond the registers' 32 a row 3 KB each.
-constexpr uint32_t kResLevelBytes = 64 * 1024;
+// LDS for the levels that every workgroup holds.  Of its 144 KB the gathered z
+// takes up to 25 and the matrix entries beyond the registers' 20 a row 3 KB each:
+// 36 entries fit beside the largest levels, 28-33 are usual.  (36k particles,
+// 64 KB: 43.0 us an iteration, one level and its two exchanges more than with 96
+// KB: 39.0; 32 entries in registers instead of 20 spill 44 of them: 0.6 more.)
+constexpr uint32_t kResLevelBytes = 96 * 1024;
 
 // The mixed solve with resident workgroups (set-up enqueued, slots packed);
 // false: the launched solve has to run (nothing was solved).  Which scenes:
@@ -4323,7 +4330,7 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   }
   ResidentTurn turn(c.device);
   if (!turn) return false;
-  auto kernel = k_mixed_resident<AMG, 32, 2>;
+  auto kernel = k_mixed_resident<AMG, AMG ? 20 : 32, 2>;
   size_t lds = resident_lds(kernel, grid, 1);
   if (lds == 0 && !AMG) {
     kernel = k_mixed_resident<false, 16, 4>;
