@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -88,6 +89,9 @@ struct Model {
   float *tb = nullptr, *z1 = nullptr, *z2 = nullptr, *a2 = nullptr, *y = nullptr, *dy = nullptr,
         *dh1 = nullptr;
   uint32_t* idx = nullptr;
+  float* part = nullptr;  // parts of a weight gradient
+  float* xf = nullptr;    // rows from the host, before packing
+  size_t xf_cap = 0;
   std::string err;
   static size_t param_count(int k);
   void init(int seed);

@@ -12,10 +12,10 @@
 // correction p - p_prev in units of s_d = s_r l0^2 / 5 (the size of A^-1 r0
 // for HL coefficients ~ 5 / l0^2 on the diagonal).
 //
-// GEMM: C = op(A) op(B), BF16 operands with arbitrary strides staged through
-// LDS in 64 x 32 tiles, v_mfma_f32_16x16x32_bf16 (each wave owns a 32 x 32
-// quarter of the 64 x 64 block tile), FP32 accumulation, optional split-K with
-// FP32 atomic accumulation for the weight gradients (reduction over the batch).
+// GEMM: C = op(A) op(B), BF16 operands contiguous along K or along M / N,
+// staged through LDS in 64 x 64 tiles, v_mfma_f32_16x16x32_bf16 (each wave owns a
+// 32 x 32 quarter of the 64 x 64 block tile), FP32 accumulation, optional split-K
+// for the weight gradients (reduction over the batch), whose parts k_sum_parts adds.
 #include <cmath>
 #include <random>
 
@@ -51,48 +51,94 @@ __device__ __forceinline__ float gelu_grad_f(float z) {
 struct GemmArgs {
   int M, N, K;
   const __bf16* A;
-  long long sam, sak;  // A(m, k) = A[m * sam + k * sak]
+  long long as;  // K contiguous: A(m, k) = A[m * as + k], else A[k * as + m]
   const __bf16* B;
-  long long sbk, sbn;  // B(k, n) = B[k * sbk + n * sbn]
-  float* C;
-  long long scm, scn;  // C(m, n)
-  int atomic;          // 1: C += (split-K partials, FP32 atomics)
-  int ksplit;          // K range per blockIdx.z
+  long long bs;  // K contiguous: B(k, n) = B[n * bs + k], else B[k * bs + n]
+  float* C;      // row-major, N columns
+  const float* bias;  // GELU: C + bias is stored, and h = bf16(gelu(it))
+  __bf16* h;
+  int ksplit;  // K range per blockIdx.z: its product at C + z M N
 };
 
+// Half a block (128 threads, th) stages one operand's 64 x kStep tile (64 rows of M
+// or N from r0, K from k0): four 16-byte loads per thread, held in registers until
+// the tile's LDS buffer is free.  Entries outside (row >= rows, k >= kend) are 0.
+// KC: K contiguous (rows' stride s; K a multiple of 32): 32 consecutive k of one
+// row.  Otherwise eight rows at four consecutive k, stored as quads of k.  Both
+// strides and `rows` are multiples of 8, the bases 16-byte aligned.
+constexpr int kStep = 64;
+constexpr int kStepLds = kStep + 8;  // (16-byte rows, neighbouring rows on other banks)
+template <bool KC>
+struct Stage {
+  bf16x8 v[4];
+  __device__ __forceinline__ void load(const __bf16* __restrict__ p, long long s, int r0, int rows, int k0, int kend,
+                                       int th) {
+    const bf16x8 zero = {};
+    const int r = r0 + (KC ? th >> 1 : (th & 7) * 8), k = k0 + (KC ? (th & 1) * 32 : (th >> 3) * 4);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const bool in = r < rows && k + (KC ? 0 : i) < kend;
+      const __bf16* q = KC ? p + r * s + k + 8 * i : p + (k + i) * s + r;
+      v[i] = in ? *reinterpret_cast<const bf16x8*>(q) : zero;
+    }
+  }
+  __device__ __forceinline__ void store(__bf16 (*t)[kStepLds], int th) const {
+    if (KC) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) *reinterpret_cast<bf16x8*>(&t[th >> 1][(th & 1) * 32 + 8 * i]) = v[i];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; e++)
+        *reinterpret_cast<bf16x4*>(&t[(th & 7) * 8 + e][(th >> 3) * 4]) = bf16x4{v[0][e], v[1][e], v[2][e], v[3][e]};
+    }
+  }
+};
+
+// Bound by latency (a block has 3 to 8 steps of 64 k and little to do in each): the
+// next step's tiles are in flight while the current one is multiplied, from two
+// LDS buffers.  The five products of a training step of 8192 rows: 79 us, 257 with
+// element-wise 2-byte loads and one buffer (the weight gradients 23 each, of which
+// the operands' re-reads by the tiles of one part are the largest share).
+template <bool AK, bool BK, bool GELU>
 __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) __bf16 As[64][40];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[64][40];  // Bs[n][k]
+  __shared__ __attribute__((aligned(16))) __bf16 As[2][64][kStepLds];
+  __shared__ __attribute__((aligned(16))) __bf16 Bs[2][64][kStepLds];  // [n][k]
   const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
   const int kbeg = blockIdx.z * g.ksplit;
   const int kend = (kbeg + g.ksplit < g.K) ? kbeg + g.ksplit : g.K;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const bool of_a = t < 128;
+  const int th = t & 127;
   f32x4 acc[2][2];
 #pragma unroll
   for (int a = 0; a < 2; a++)
 #pragma unroll
     for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int r = t >> 2, kc = (t & 3) * 8;
-  for (int k0 = kbeg; k0 < kend; k0 += 32) {
-    const int m = m0 + r, n = n0 + r;
+  Stage<AK> sa;
+  Stage<BK> sb;
+  auto load = [&](int k0) {
+    if (of_a) sa.load(g.A, g.as, m0, g.M, k0, kend, th);
+    else sb.load(g.B, g.bs, n0, g.N, k0, kend, th);
+  };
+  load(kbeg);
+  int buf = 0;
+  for (int k0 = kbeg; k0 < kend; k0 += kStep, buf ^= 1) {
+    if (of_a) sa.store(As[buf], th);
+    else sb.store(Bs[buf], th);
+    __syncthreads();  // (and the other buffer's readers are done before it is stored again)
+    if (k0 + kStep < kend) load(k0 + kStep);
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int k = k0 + kc + e;
-      As[r][kc + e] = (m < g.M && k < kend) ? g.A[m * g.sam + k * g.sak] : __bf16(0.0f);
-      Bs[r][kc + e] = (n < g.N && k < kend) ? g.B[k * g.sbk + n * g.sbn] : __bf16(0.0f);
-    }
-    __syncthreads();
+    for (int k = 0; k < kStep; k += 32)
 #pragma unroll
-    for (int a = 0; a < 2; a++) {
-      const bf16x8 af = *reinterpret_cast<const bf16x8*>(&As[wm + a * 16 + (lane & 15)][(lane >> 4) * 8]);
+      for (int a = 0; a < 2; a++) {
+        const bf16x8 af = *reinterpret_cast<const bf16x8*>(&As[buf][wm + a * 16 + (lane & 15)][k + (lane >> 4) * 8]);
 #pragma unroll
-      for (int b = 0; b < 2; b++) {
-        const bf16x8 bfv = *reinterpret_cast<const bf16x8*>(&Bs[wn + b * 16 + (lane & 15)][(lane >> 4) * 8]);
-        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfv, acc[a][b], 0, 0, 0);
+        for (int b = 0; b < 2; b++) {
+          const bf16x8 bfv = *reinterpret_cast<const bf16x8*>(&Bs[buf][wn + b * 16 + (lane & 15)][k + (lane >> 4) * 8]);
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bfv, acc[a][b], 0, 0, 0);
+        }
       }
-    }
-    __syncthreads();
   }
 #pragma unroll
   for (int a = 0; a < 2; a++)
@@ -103,21 +149,32 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
         const int m = m0 + wm + a * 16 + 4 * (lane >> 4) + v;
         const int n = n0 + wn + b * 16 + (lane & 15);
         if (m < g.M && n < g.N) {
-          float* c = g.C + m * g.scm + n * g.scn;
-          if (g.atomic) atomicAdd(c, acc[a][b][v]);
-          else *c = acc[a][b][v];
+          const size_t o = (static_cast<size_t>(blockIdx.z) * g.M + m) * g.N + n;
+          if (GELU) {
+            const float z = acc[a][b][v] + g.bias[n];
+            g.C[o] = z;
+            g.h[o] = __bf16(gelu_f(z));
+          } else {
+            g.C[o] = acc[a][b][v];
+          }
         }
       }
 }
 
-// z <- z + b (in place, FP32) and h = bf16(gelu(z)) (row-major M x N).
-__global__ void __launch_bounds__(256) k_bias_gelu(size_t total, int N, float* __restrict__ z,
-                                                   const float* __restrict__ b, __bf16* __restrict__ h) {
-  const size_t i = blockIdx.x * 256ull + threadIdx.x;
-  if (i >= total) return;
-  const float v = z[i] + b[i % N];
-  z[i] = v;
-  h[i] = __bf16(gelu_f(v));
+// out = the sum of `parts` products of n values, in order (23 + 6 us for the weight
+// gradient of 8192 rows in 32 parts; FP32 atomics into one result took as long and
+// left the order of the sums to chance).
+__global__ void __launch_bounds__(256) k_sum_parts(uint32_t n4, int parts, const float4* __restrict__ part,
+                                                   float4* __restrict__ out) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= n4) return;
+  float4 s = part[i];
+#pragma unroll 8
+  for (int k = 1; k < parts; k++) {
+    const float4 v = part[static_cast<size_t>(k) * n4 + i];
+    s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+  }
+  out[i] = s;
 }
 
 // y[m] = sum_n gelu(z2[m][n] + b2[n]) w3[n] + b3; one wavefront per row.
@@ -164,42 +221,95 @@ __global__ void __launch_bounds__(256) k_loss(int M, const float* __restrict__ y
   }
 }
 
-// Head backward over 64 rows per block, one thread per hidden column:
-// dW3[n] += sum h2 dy, da2 = dy w3 gelu'(a2) (FP32 + BF16), db2 += sum da2.
+// Column sums over a block: thread t has the sums s of columns 4 (t & 63) .. of its
+// quarter of the rows; the block's go to out[] with one atomic a column.
+__device__ __forceinline__ void add_columns(const float s[4], float (*part)[kHid], float* __restrict__ out) {
+#pragma unroll
+  for (int e = 0; e < 4; e++) part[threadIdx.x >> 6][4 * (threadIdx.x & 63) + e] = s[e];
+  __syncthreads();
+  const int n = threadIdx.x;
+  atomicAdd(&out[n], (part[0][n] + part[1][n]) + (part[2][n] + part[3][n]));
+  __syncthreads();
+}
+
+// Head backward, kBwdRows rows per block:
+// dW3[n] += sum h2 dy, da2 = dy w3 gelu'(a2) (BF16), db2 += sum da2.
+// A thread takes four columns of eight rows, all loads first (one column of 64
+// rows in turn waited for each: 25 us for 8192 rows, now 12; k_gelu_bwd 24, 12).
+constexpr int kBwdRows = 32;
 __global__ void __launch_bounds__(256) k_head_bwd(int M, const float* __restrict__ a2,
                                                   const float* __restrict__ dy,
                                                   const float* __restrict__ w3, float* __restrict__ dw3,
                                                   float* __restrict__ db2, __bf16* __restrict__ da2b) {
-  const int n = threadIdx.x;
-  const int r0 = blockIdx.x * 64;
-  float aw = 0, ab = 0;
-  const float wn = w3[n];
-  for (int r = r0; r < r0 + 64 && r < M; r++) {
-    const float a = a2[static_cast<size_t>(r) * kHid + n];
-    const float d = dy[r];
-    aw += gelu_f(a) * d;
-    const float g = d * wn * gelu_grad_f(a);
-    ab += g;
-    da2b[static_cast<size_t>(r) * kHid + n] = __bf16(g);
+  static_assert(kHid == 256, "four columns a thread");
+  __shared__ float part[4][kHid];
+  const int c = 4 * (threadIdx.x & 63), r0 = blockIdx.x * kBwdRows + (threadIdx.x >> 6) * 8;
+  float4 a[8];
+  float d[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int r = r0 + q < M ? r0 + q : M - 1;
+    a[q] = *reinterpret_cast<const float4*>(a2 + static_cast<size_t>(r) * kHid + c);
+    d[q] = dy[r];
   }
-  atomicAdd(&dw3[n], aw);
-  atomicAdd(&db2[n], ab);
+  const float4 wn = *reinterpret_cast<const float4*>(w3 + c);
+  const float w[4] = {wn.x, wn.y, wn.z, wn.w};
+  float aw[4] = {0, 0, 0, 0}, ab[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 8; q++)
+    if (r0 + q < M) {
+      const float v[4] = {a[q].x, a[q].y, a[q].z, a[q].w};
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        aw[e] += gelu_f(v[e]) * d[q];
+        const float g = d[q] * w[e] * gelu_grad_f(v[e]);
+        ab[e] += g;
+        o[e] = __bf16(g);
+      }
+      *reinterpret_cast<bf16x4*>(da2b + static_cast<size_t>(r0 + q) * kHid + c) = o;
+    }
+  add_columns(aw, part, dw3);
+  add_columns(ab, part, db2);
 }
 
-// da1 = dh1 gelu'(a1) (BF16), db1 += column sums; 64 rows per block.
+// da1 = dh1 gelu'(a1) (BF16), db1 += column sums; rows as in k_head_bwd.
 __global__ void __launch_bounds__(256) k_gelu_bwd(int M, const float* __restrict__ a1,
                                                   const float* __restrict__ dh1,
                                                   float* __restrict__ db1, __bf16* __restrict__ da1b) {
-  const int n = threadIdx.x;
-  const int r0 = blockIdx.x * 64;
-  float ab = 0;
-  for (int r = r0; r < r0 + 64 && r < M; r++) {
-    const size_t o = static_cast<size_t>(r) * kHid + n;
-    const float g = dh1[o] * gelu_grad_f(a1[o]);
-    ab += g;
-    da1b[o] = __bf16(g);
+  __shared__ float part[4][kHid];
+  const int c = 4 * (threadIdx.x & 63), r0 = blockIdx.x * kBwdRows + (threadIdx.x >> 6) * 8;
+  float4 a[8], h[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const size_t o = static_cast<size_t>(r0 + q < M ? r0 + q : M - 1) * kHid + c;
+    a[q] = *reinterpret_cast<const float4*>(a1 + o);
+    h[q] = *reinterpret_cast<const float4*>(dh1 + o);
   }
-  atomicAdd(&db1[n], ab);
+  float ab[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 8; q++)
+    if (r0 + q < M) {
+      const float v[4] = {a[q].x, a[q].y, a[q].z, a[q].w}, u[4] = {h[q].x, h[q].y, h[q].z, h[q].w};
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float g = u[e] * gelu_grad_f(v[e]);
+        ab[e] += g;
+        o[e] = __bf16(g);
+      }
+      *reinterpret_cast<bf16x4*>(da1b + static_cast<size_t>(r0 + q) * kHid + c) = o;
+    }
+  add_columns(ab, part, db1);
+}
+
+// The sums that k_loss, k_head_bwd and k_gelu_bwd add to, cleared in one launch.
+struct ClearArgs {
+  float *db1, *db2, *dw3, *db3, *loss;
+};
+__global__ void __launch_bounds__(kHid) k_clear_sums(ClearArgs a) {
+  a.db1[threadIdx.x] = a.db2[threadIdx.x] = a.dw3[threadIdx.x] = 0.0f;
+  if (threadIdx.x == 0) *a.db3 = *a.loss = 0.0f;
 }
 
 __global__ void __launch_bounds__(256) k_adam(size_t n, float* __restrict__ w, const float* __restrict__ g,
@@ -674,15 +784,30 @@ __global__ void __launch_bounds__(kMlpThreads) k_mlp_infer(size_t M, const __bf1
 
 unsigned blocks(size_t n) { return static_cast<unsigned>((n + 255) / 256); }
 
-void gemm(hipStream_t s, int M, int N, int K, const __bf16* A, long long sam, long long sak,
-          const __bf16* B, long long sbk, long long sbn, float* C, long long scm, long long scn,
-          int splits) {
-  GemmArgs g{M, N, K, A, sam, sak, B, sbk, sbn, C, scm, scn, splits > 1 ? 1 : 0, 0};
-  int ks = (K + splits - 1) / splits;
-  ks = (ks + 31) / 32 * 32;
-  g.ksplit = ks;
-  const int nz = (K + ks - 1) / ks;
-  hipLaunchKernelGGL(k_gemm_bf16, dim3((N + 63) / 64, (M + 63) / 64, nz), dim3(256), 0, s, g);
+template <bool AK, bool BK, bool GELU = false>
+void gemm(hipStream_t s, int M, int N, int K, const __bf16* A, long long as, const __bf16* B, long long bs, float* C,
+          const float* bias = nullptr, __bf16* h = nullptr) {
+  const GemmArgs g{M, N, K, A, as, B, bs, C, bias, h, K};
+  hipLaunchKernelGGL((k_gemm_bf16<AK, BK, GELU>), dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, g);
+}
+
+// Parts of a weight gradient's reduction over m rows: 32 give two blocks of 64 x 64
+// of the 256 x 256 result to a compute unit (8192 rows: 23 us, 16 parts 28; 64 parts
+// 21, but adding them up costs 2 more).
+int grad_parts(size_t m) { return static_cast<int>(std::max<size_t>(1, std::min<size_t>(32, m / 128))); }
+
+// out[n][k] = sum over m rows of a[m][n] b[m][k] (a: kHid wide, b: N wide), in parts.
+void weight_gradient(hipStream_t s, int m, const __bf16* a, const __bf16* b, int N, float* part, float* out) {
+  int ks = (m + grad_parts(m) - 1) / grad_parts(m);
+  ks = (ks + kStep - 1) / kStep * kStep;
+  const int nz = (m + ks - 1) / ks;
+  const GemmArgs g{kHid, N, m, a, kHid, b, N, nz > 1 ? part : out, nullptr, nullptr, ks};
+  hipLaunchKernelGGL((k_gemm_bf16<false, false, false>), dim3((N + 63) / 64, kHid / 64, nz), dim3(256), 0, s, g);
+  if (nz > 1) {
+    const uint32_t n4 = static_cast<uint32_t>(kHid) * N / 4;
+    hipLaunchKernelGGL(k_sum_parts, dim3((n4 + 255) / 256), dim3(256), 0, s, n4, nz,
+                       reinterpret_cast<const float4*>(part), reinterpret_cast<float4*>(out));
+  }
 }
 
 }  // namespace
@@ -711,6 +836,7 @@ void Model::ensure_batch(size_t m) {
   dh1 = dalloc<float>(m * kHid);
   da1b = dalloc<__bf16>(m * kHid);
   idx = dalloc<uint32_t>(m);
+  if (!part) part = dalloc<float>(static_cast<size_t>(grad_parts(~size_t(0))) * kHid * kHid);
   cap = m;
 }
 
@@ -765,7 +891,7 @@ void Model::release() {
   }
   dfree(w1b); dfree(w2b); dfree(w2p); dfree(loss);
   dfree(xb); dfree(tb); dfree(z1); dfree(z2); dfree(a2); dfree(h1b); dfree(y); dfree(dy);
-  dfree(da2b); dfree(dh1); dfree(da1b); dfree(idx);
+  dfree(da2b); dfree(dh1); dfree(da1b); dfree(idx); dfree(xf); dfree(part);
   if (stream) (void)hipStreamDestroy(stream);
   stream = nullptr;
 }
@@ -786,10 +912,9 @@ void Model::forward(hipStream_t s, size_t m, const __bf16* x, float* out, bool t
   }
   ensure_batch(m);
   const int M = static_cast<int>(m);
-  gemm(s, M, kHid, kFeatPad, x, kFeatPad, 1, w1b, 1, kFeatPad, z1, kHid, 1, 1);
-  hipLaunchKernelGGL(k_bias_gelu, dim3(blocks(m * kHid)), dim3(256), 0, s, m * kHid, kHid, z1,
-                     static_cast<const float*>(w[1]), h1b);
-  gemm(s, M, kHid, kHid, h1b, kHid, 1, w2b, 1, kHid, z2, kHid, 1, 1);
+  // z1 = x W1^T + b1 and h1 = gelu(z1), then z2 = h1 W2^T
+  gemm<true, true, true>(s, M, kHid, kFeatPad, x, kFeatPad, w1b, kFeatPad, z1, w[1], h1b);
+  gemm<true, true>(s, M, kHid, kHid, h1b, kHid, w2b, kHid, z2);
   hipLaunchKernelGGL(k_head, dim3((M + 3) / 4), dim3(256), 0, s, M, static_cast<const float*>(z2),
                      static_cast<const float*>(w[3]), static_cast<const float*>(w[4]),
                      static_cast<const float*>(w[5]), out, train ? a2 : static_cast<float*>(nullptr));
@@ -799,21 +924,19 @@ void Model::forward(hipStream_t s, size_t m, const __bf16* x, float* out, bool t
 // Gradients of the mean squared error for the batch in xb / tb (into g[]).
 void Model::backward(hipStream_t s, size_t m) {
   const int M = static_cast<int>(m);
-  for (int k = 0; k < 6; k++) MPS_HIP(hipMemsetAsync(g[k], 0, param_count(k) * 4, s));
-  MPS_HIP(hipMemsetAsync(loss, 0, 4, s));
+  hipLaunchKernelGGL(k_clear_sums, dim3(1), dim3(kHid), 0, s, ClearArgs{g[1], g[3], g[4], g[5], loss});
   hipLaunchKernelGGL(k_loss, dim3(blocks(m)), dim3(256), 0, s, M, static_cast<const float*>(y),
                      static_cast<const float*>(tb), dy, loss, g[5]);
-  hipLaunchKernelGGL(k_head_bwd, dim3((M + 63) / 64), dim3(256), 0, s, M, static_cast<const float*>(a2),
+  hipLaunchKernelGGL(k_head_bwd, dim3((M + kBwdRows - 1) / kBwdRows), dim3(256), 0, s, M, static_cast<const float*>(a2),
                      static_cast<const float*>(dy), static_cast<const float*>(w[4]), g[4], g[3], da2b);
-  const int splits = std::max(1, std::min(64, M / 512));
   // dW2[n][k] = sum_m da2[m][n] h1[m][k]
-  gemm(s, kHid, kHid, M, da2b, 1, kHid, h1b, kHid, 1, g[2], kHid, 1, splits);
+  weight_gradient(s, M, da2b, h1b, kHid, part, g[2]);
   // dh1[m][k] = sum_n da2[m][n] W2[n][k]
-  gemm(s, M, kHid, kHid, da2b, kHid, 1, w2b, kHid, 1, dh1, kHid, 1, 1);
-  hipLaunchKernelGGL(k_gelu_bwd, dim3((M + 63) / 64), dim3(256), 0, s, M, static_cast<const float*>(z1),
+  gemm<true, false>(s, M, kHid, kHid, da2b, kHid, w2b, kHid, dh1);
+  hipLaunchKernelGGL(k_gelu_bwd, dim3((M + kBwdRows - 1) / kBwdRows), dim3(256), 0, s, M, static_cast<const float*>(z1),
                      static_cast<const float*>(dh1), g[1], da1b);
   // dW1[n][k] = sum_m da1[m][n] x[m][k]
-  gemm(s, kHid, kFeatPad, M, da1b, 1, kHid, xb, kFeatPad, 1, g[0], kFeatPad, 1, splits);
+  weight_gradient(s, M, da1b, xb, kFeatPad, part, g[0]);
   check_launch();
 }
 
@@ -835,13 +958,15 @@ void Model::adam(hipStream_t s, float lr) {
 
 void Model::pack_host_rows(size_t m, const float* x_host) {
   ensure_batch(m);
-  float* tmp = dalloc<float>(m * kFeat);
-  MPS_HIP(hipMemcpyAsync(tmp, x_host, m * kFeat * 4, hipMemcpyHostToDevice, stream));
+  if (m > xf_cap) {
+    dfree(xf);
+    xf = dalloc<float>(m * kFeat);
+    xf_cap = m;
+  }
+  MPS_HIP(hipMemcpyAsync(xf, x_host, m * kFeat * 4, hipMemcpyHostToDevice, stream));
   hipLaunchKernelGGL(k_pack_rows, dim3(blocks(m * kFeatPad)), dim3(256), 0, stream, m,
-                     static_cast<const float*>(tmp), xb);
+                     static_cast<const float*>(xf), xb);
   check_launch();
-  MPS_HIP(hipStreamSynchronize(stream));
-  dfree(tmp);
 }
 
 // Epochs of shuffled mini-batches over the dataset; returns the mean loss of
