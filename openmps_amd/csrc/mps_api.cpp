@@ -927,18 +927,19 @@ void params_to_device(mps::Model& m, const float* const* src) {
   }
   m.refresh_bf16();
 }
-void params_to_host(float* const* base, float* const* dst) {
-  for (int k = 0; k < 6; k++) {
-    const size_t n = mps::Model::param_count(k);
-    std::vector<float> h(n);
-    MPS_HIP(hipMemcpy(h.data(), base[k], n * 4, hipMemcpyDeviceToHost));
-    if (k == 0) {
-      for (int r = 0; r < mps::kHid; r++)
-        for (int q = 0; q < mps::kFeat; q++) dst[0][r * mps::kFeat + q] = h[r * mps::kFeatPad + q];
-    } else {
-      std::memcpy(dst[k], h.data(), n * 4);
-    }
-  }
+// All copies go to a pinned buffer and are waited for once (one at a time into
+// pageable memory: 0.1 ms of a 0.45 ms call for the gradients of 8192 rows).
+void params_to_host(mps::Model& m, float* const* base, float* const* dst) {
+  std::lock_guard<std::mutex> turn(m.staging_turn);
+  size_t at[7] = {0};
+  for (int k = 0; k < 6; k++) at[k + 1] = at[k] + mps::Model::param_count(k);
+  if (!m.staging) mps::pinned(m.staging, at[6]);
+  for (int k = 0; k < 6; k++)
+    MPS_HIP(hipMemcpyAsync(m.staging + at[k], base[k], (at[k + 1] - at[k]) * 4, hipMemcpyDeviceToHost, m.stream));
+  MPS_HIP(hipStreamSynchronize(m.stream));
+  for (int r = 0; r < mps::kHid; r++)
+    std::memcpy(dst[0] + r * mps::kFeat, m.staging + static_cast<size_t>(r) * mps::kFeatPad, mps::kFeat * 4);
+  for (int k = 1; k < 6; k++) std::memcpy(dst[k], m.staging + at[k], (at[k + 1] - at[k]) * 4);
 }
 }  // namespace
 }  // namespace mps
@@ -978,7 +979,7 @@ int mps_model_get_params(mps_model* m, float* w1, float* b1, float* w2, float* b
     float* dst[6] = {w1, b1, w2, b2, w3, b3};
     for (float* p : dst)
       if (!p) throw Failure{MPS_ERR_BAD_ARG, "null parameter array"};
-    mps::params_to_host(m->m.w, dst);
+    mps::params_to_host(m->m, m->m.w, dst);
   });
 }
 
@@ -1005,7 +1006,7 @@ int mps_model_gradients(mps_model* m, size_t rows, const float* x, const float* 
     if (rows == 0) throw Failure{MPS_ERR_BAD_ARG, "no rows"};
     mps::model_grads_host(m->m, rows, x, t, loss);
     float* dst[6] = {g_w1, g_b1, g_w2, g_b2, g_w3, g_b3};
-    mps::params_to_host(m->m.g, dst);
+    mps::params_to_host(m->m, m->m.g, dst);
   });
 }
 

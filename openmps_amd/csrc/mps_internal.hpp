@@ -92,6 +92,8 @@ struct Model {
   float* part = nullptr;  // parts of a weight gradient
   float* xf = nullptr;    // rows from the host, before packing
   size_t xf_cap = 0;
+  float* staging = nullptr;  // pinned: parameters or gradients on their way to the host
+  std::mutex staging_turn;
   std::string err;
   static size_t param_count(int k);
   void init(int seed);

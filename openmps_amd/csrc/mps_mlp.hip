@@ -892,6 +892,8 @@ void Model::release() {
   dfree(w1b); dfree(w2b); dfree(w2p); dfree(loss);
   dfree(xb); dfree(tb); dfree(z1); dfree(z2); dfree(a2); dfree(h1b); dfree(y); dfree(dy);
   dfree(da2b); dfree(dh1); dfree(da1b); dfree(idx); dfree(xf); dfree(part);
+  if (staging) (void)hipHostFree(staging);
+  staging = nullptr;
   if (stream) (void)hipStreamDestroy(stream);
   stream = nullptr;
 }
