@@ -928,7 +928,7 @@ void params_to_device(mps::Model& m, const float* const* src) {
   m.refresh_bf16();
 }
 // All copies go to a pinned buffer and are waited for once (one at a time into
-// pageable memory: 0.1 ms of a 0.45 ms call for the gradients of 8192 rows).
+// pageable memory: 0.06 ms of a 0.45 ms call for the gradients of 8192 rows).
 void params_to_host(mps::Model& m, float* const* base, float* const* dst) {
   std::lock_guard<std::mutex> turn(m.staging_turn);
   size_t at[7] = {0};

@@ -2195,6 +2195,108 @@ __device__ __forceinline__ void amg_rfix_point(const float* __restrict__ tq, siz
                                                uint32_t nz, float* __restrict__ r0, uint32_t p) {
   r0[p] = amg_rfix_at(tq, stride, nx, nz, static_cast<int>(p / nz), static_cast<int>(p % nz));
 }
+// The first steps of the cycle in one launch: level 0's right-hand side from the
+// direction sums, levels 0 -> 1 -> 2.  A block takes kDownT x kDownT points of level
+// 2, their children with the halo of the residuals and the same a level below
+// (r and 1 / S_pp in LDS), each point as the level kernels compute it; r and x of
+// levels 0 and 1 and r of level 2 are written by the block that owns the point.
+// Bound by the chain of three dependent reads and the launch.  With it and chains
+// of two levels, an iteration of 189k particles in motion takes 87.6 us (96.1 with
+// a launch per level), 419k 106.9 (126.8), 515k at rest 94.8 (106.8), 1.05M 148
+// (149: its chain of three levels began at level 1).
+constexpr int kDownT = 8;
+struct AmgDownTile {
+  static constexpr int c1 = 2 * kDownT, f1 = c1 + 2;  // level 1: the children, with halo
+  static constexpr int c0 = 2 * f1, f0 = c0 + 2;      // level 0: theirs
+};
+__global__ void __launch_bounds__(kAmgChainThreads) k_amg_down_tiles(AmgGrid g, const float* __restrict__ tq,
+                                                                     size_t stride) {
+  if (amg_skip(g)) return;
+  using D = AmgDownTile;
+  __shared__ float r0[D::f0 * D::f0], d0[D::f0 * D::f0], e0[D::c0 * D::c0];
+  __shared__ float r1[D::f1 * D::f1], d1[D::f1 * D::f1], e1[D::c1 * D::c1];
+  const AmgLevel F = g.L[0], M = g.L[1], C = g.L[2];
+  const uint32_t tnz = (C.nz + kDownT - 1) / kDownT;
+  const int X2 = static_cast<int>(blockIdx.x / tnz) * kDownT, Z2 = static_cast<int>(blockIdx.x % tnz) * kDownT;
+  const int x1 = 2 * X2 - 1, z1 = 2 * Z2 - 1, x0 = 2 * x1, z0 = 2 * z1;  // origins of the regions f1 and c0
+  for (int i = threadIdx.x; i < D::f0 * D::f0; i += kAmgChainThreads) {
+    const int ix = x0 - 1 + i / D::f0, iz = z0 - 1 + i % D::f0;
+    const bool in = amg_in(F, ix, iz);
+    const int jx = in ? ix : 0, jz = in ? iz : 0;
+    const float r = amg_rfix_at(tq, stride, F.nx, F.nz, jx, jz);
+    const float d = g.dinv[static_cast<uint32_t>(jx) * F.nz + static_cast<uint32_t>(jz)];
+    r0[i] = in ? r : 0.0f;
+    d0[i] = in ? d : 0.0f;
+  }
+  __syncthreads();
+  // a point's residual after the first smoothing, from the region with halo
+  auto resid = [&](const AmgLevel& L, const float* r, const float* d, int side, int cx, int cz, uint32_t p, float& x) {
+    float sv[9], sum = 0.0f;
+    const uint32_t np = amg_npts(L);
+#pragma unroll
+    for (int e = 0; e < 9; e++) sv[e] = g.S[9ull * L.off + static_cast<size_t>(e) * np + p];
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+      const int o = (cx + e / 3) * side + cz + e % 3;
+      sum = fmaf(sv[e], g.omega * d[o] * r[o], sum);
+    }
+    const int o = (cx + 1) * side + cz + 1;
+    x = g.omega * d[o] * r[o];
+    return r[o] - sum;
+  };
+  for (int i = threadIdx.x; i < D::c0 * D::c0; i += kAmgChainThreads) {
+    const int cx = i / D::c0, cz = i % D::c0, ix = x0 + cx, iz = z0 + cz;
+    float e = 0.0f;
+    if (amg_in(F, ix, iz)) {
+      const uint32_t p = static_cast<uint32_t>(ix) * F.nz + static_cast<uint32_t>(iz);
+      float x;
+      e = resid(F, r0, d0, D::f0, cx, cz, p, x);
+      if (cx >= 2 && cx < D::c0 - 2 && cz >= 2 && cz < D::c0 - 2) {  // this block's own
+        g.x[p] = x;
+        g.r[p] = r0[(cx + 1) * D::f0 + cz + 1];
+      }
+    }
+    e0[i] = e;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < D::f1 * D::f1; i += kAmgChainThreads) {
+    const int px = i / D::f1, pz = i % D::f1, ix = x1 + px, iz = z1 + pz;
+    float rc = 0.0f, d = 0.0f;
+    if (amg_in(M, ix, iz)) {
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (amg_in(F, 2 * ix + e / 2, 2 * iz + e % 2)) rc += e0[(2 * px + e / 2) * D::c0 + 2 * pz + e % 2];
+      const uint32_t p = M.off + static_cast<uint32_t>(ix) * M.nz + static_cast<uint32_t>(iz);
+      d = g.dinv[p];
+      if (px >= 1 && px < D::f1 - 1 && pz >= 1 && pz < D::f1 - 1) g.r[p] = rc;
+    }
+    r1[i] = rc;
+    d1[i] = d;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < D::c1 * D::c1; i += kAmgChainThreads) {
+    const int cx = i / D::c1, cz = i % D::c1, ix = x1 + 1 + cx, iz = z1 + 1 + cz;
+    float e = 0.0f;
+    if (amg_in(M, ix, iz)) {
+      const uint32_t p = static_cast<uint32_t>(ix) * M.nz + static_cast<uint32_t>(iz);
+      float x;
+      e = resid(M, r1, d1, D::f1, cx, cz, p, x);
+      g.x[M.off + p] = x;
+    }
+    e1[i] = e;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kDownT * kDownT; i += kAmgChainThreads) {
+    const int px = i / kDownT, pz = i % kDownT, ix = X2 + px, iz = Z2 + pz;
+    if (!amg_in(C, ix, iz)) continue;
+    float rc = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+      if (amg_in(M, 2 * ix + e / 2, 2 * iz + e % 2)) rc += e1[(2 * px + e / 2) * D::c1 + 2 * pz + e % 2];
+    g.r[C.off + static_cast<uint32_t>(ix) * C.nz + static_cast<uint32_t>(iz)] = rc;
+  }
+}
+
 __global__ void __launch_bounds__(256) k_amg_rfix(const float* __restrict__ tq, size_t stride, uint32_t nx,
                                                   uint32_t nz, float* __restrict__ r0, const CgStatus* st,
                                                   long long it) {
@@ -4273,35 +4375,51 @@ void clear_direction_sums(Context& c) {
   MPS_HIP(hipMemsetAsync(c.amg_tq, 0, 9 * c.amg_tq_stride * sizeof(float), c.stream));
 }
 
-// One V-cycle on the cell-grid levels: level 0's right-hand side in, its
+// One V-cycle on the cell-grid levels: pass 1's direction sums in, level 0's
 // result (the correction per cell) out.  The level-0 up-pass is left to the
 // caller when `fold0` (k_ml_prec_up does it) and the cycle has a level below
 // the cells' outside the single-workgroup kernel; returns whether it was left.
 // The cycle of inner iteration `it` of the solve with status `st` does
 // nothing once that solve has stopped before it (launches past the stop).
-bool amg_cycle(Context& c, bool fold0, const CgStatus* st, long long it) {
+bool amg_cycle(Context& c, bool fold0, const float* tq, const CgStatus* st, long long it) {
   AmgGrid g = amg_grid(c);
   g.st = st;
   g.it = it;
   const int l0 = amg_block_level(c);
-  // the kAmgChainLevels levels above the single-workgroup ones in one launch
-  // each way (level 0 keeps its own kernels)
-  const int l1 = (l0 - kAmgChainLevels >= 1) ? l0 - kAmgChainLevels : l0;
-  const unsigned tiles = ((c.amg_nx[l0] + kAmgChainT - 1) / kAmgChainT) * ((c.amg_nz[l0] + kAmgChainT - 1) / kAmgChainT);
-  for (int l = 0; l < l1; l++)
-    hipLaunchKernelGGL(k_amg_down, dim3(grid_for(static_cast<size_t>(c.amg_nx[l + 1]) * c.amg_nz[l + 1])),
-                       dim3(256), 0, c.stream, g, l);
-  if (l1 < l0)
-    hipLaunchKernelGGL((k_amg_down_chain<kAmgChainT, kAmgChainLevels>), dim3(tiles), dim3(kAmgChainThreads), 0,
-                       c.stream, g, l1);
+  auto tiles = [&](int l, int t) {  // of t x t points of level l
+    return dim3(((c.amg_nx[l] + t - 1) / t) * ((c.amg_nz[l] + t - 1) / t));
+  };
+  auto points = [&](int l) { return dim3(grid_for(static_cast<size_t>(c.amg_nx[l]) * c.amg_nz[l])); };
+  // down: the first two levels in one launch, the last two or three above the
+  // single-workgroup ones in another, any between them one by one
+  int l = 0;
+  if (l0 >= 2) {
+    hipLaunchKernelGGL(k_amg_down_tiles, tiles(2, kDownT), dim3(kAmgChainThreads), 0, c.stream, g, tq, c.amg_tq_stride);
+    l = 2;
+  } else {
+    hipLaunchKernelGGL(k_amg_rfix, points(0), dim3(256), 0, c.stream, tq, c.amg_tq_stride, c.amg_box[2], c.amg_box[3],
+                       c.amg_r, st, it);
+  }
+  const int nd = std::min(kAmgChainLevels, l0 - l);
+  for (; l < (nd >= 2 ? l0 - nd : l0); l++) hipLaunchKernelGGL(k_amg_down, points(l + 1), dim3(256), 0, c.stream, g, l);
+  if (nd == 3)
+    hipLaunchKernelGGL((k_amg_down_chain<kAmgChainT, 3>), tiles(l0, kAmgChainT), dim3(kAmgChainThreads), 0, c.stream, g,
+                       l);
+  else if (nd == 2)
+    hipLaunchKernelGGL((k_amg_down_chain<kAmgChainT, 2>), tiles(l0, kAmgChainT), dim3(kAmgChainThreads), 0, c.stream, g,
+                       l);
   hipLaunchKernelGGL(k_amg_block, dim3(1), dim3(kAmgBlockThreads), 0, c.stream, g, l0);
-  if (l1 < l0)
-    hipLaunchKernelGGL((k_amg_up_chain<kAmgChainT, kAmgChainLevels>), dim3(tiles), dim3(kAmgChainThreads), 0,
-                       c.stream, g, l1);
+  // up to level 1 (or 0)
   const bool left = fold0 && l0 >= 1;
-  for (int l = l1 - 1; l >= (left ? 1 : 0); l--)
-    hipLaunchKernelGGL(k_amg_up, dim3(grid_for(static_cast<size_t>(c.amg_nx[l]) * c.amg_nz[l])), dim3(256), 0,
-                       c.stream, g, l);
+  const int last = left ? 1 : 0, nu = std::min(kAmgChainLevels, l0 - last);
+  if (nu == 3)
+    hipLaunchKernelGGL((k_amg_up_chain<kAmgChainT, 3>), tiles(l0, kAmgChainT), dim3(kAmgChainThreads), 0, c.stream, g,
+                       l0 - nu);
+  else if (nu == 2)
+    hipLaunchKernelGGL((k_amg_up_chain<kAmgChainT, 2>), tiles(l0, kAmgChainT), dim3(kAmgChainThreads), 0, c.stream, g,
+                       l0 - nu);
+  for (l = (nu >= 2 ? l0 - nu : l0) - 1; l >= last; l--)
+    hipLaunchKernelGGL(k_amg_up, points(l), dim3(256), 0, c.stream, g, l);
   return left;
 }
 
@@ -4564,10 +4682,7 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
     });
     bool left = false;
     track(MPS_K_AMG_CYCLE, b_cycle, [&] {
-      hipLaunchKernelGGL(k_amg_rfix, dim3(grid_for(npts0)), dim3(256), 0, c.stream,
-                         static_cast<const float*>(c.amg_tq), tq_stride, c.amg_box[2], c.amg_box[3], c.amg_r,
-                         static_cast<const CgStatus*>(c.st32), it);
-      left = amg_cycle(c, true, c.st32, it);
+      left = amg_cycle(c, true, c.amg_tq, c.st32, it);
     });
     track(MPS_K_ML_PREC, b_pass, [&] {
       if (left)
