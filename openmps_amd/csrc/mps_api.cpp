@@ -122,12 +122,11 @@ void free_all(Context& c) {
   for (auto& d : c.spare_d) dfree(d);
   dfree(c.spare_type); dfree(c.spare_group); dfree(c.spare_orig); dfree(c.spare_key);
   dfree(c.key); dfree(c.sorted); dfree(c.pos_sorted); dfree(c.in_cells); dfree(c.nbr); dfree(c.ncount);
-  dfree(c.cell_count); dfree(c.cell_start); dfree(c.cell_fill); dfree(c.scan_tmp); dfree(c.flags);
-  dfree(c.nbr_total_dev); dfree(c.ppe_counters);
+  dfree(c.cell_count); dfree(c.cell_start); dfree(c.cell_fill); dfree(c.scan_tmp); dfree(c.counters);
   dfree(c.row_len); dfree(c.slice_width); dfree(c.slice_off); dfree(c.sval); dfree(c.sval32);
   dfree(c.scol); dfree(c.diag); dfree(c.diag32); dfree(c.b); dfree(c.sol);
   dfree(c.r); dfree(c.pa); dfree(c.q); dfree(c.partA); dfree(c.partB); dfree(c.partC);
-  dfree(c.red_out); dfree(c.st); dfree(c.st32); dfree(c.ir);
+  dfree(c.red_out); dfree(c.st32); dfree(c.ir);
   dfree(c.pa32); dfree(c.d32); dfree(c.dinv32);
   if (!c.feats_borrowed) {
     dfree(c.feats);
@@ -137,17 +136,13 @@ void free_all(Context& c) {
   dfree(c.ghost32); dfree(c.qpos); dfree(c.slice_wide); dfree(c.col16);
   dfree(c.g32a); dfree(c.g32b); dfree(c.part3a); dfree(c.part3b);
   dfree(c.r32); dfree(c.z32); dfree(c.q32); dfree(c.agg_inv); dfree(c.part_ml);
-  dfree(c.ml_flag); dfree(c.ml_off); dfree(c.ml_list); dfree(c.ml_active); dfree(c.st_replay);
+  dfree(c.ml_flag); dfree(c.ml_off); dfree(c.ml_list); dfree(c.st_replay);
   dfree(c.ml_pid); dfree(c.ml_dv); dfree(c.ml_sc); dfree(c.zrec);
   dfree(c.amg_S64); dfree(c.amg_S); dfree(c.amg_dinv); dfree(c.amg_r); dfree(c.amg_x); dfree(c.amg_e);
   dfree(c.res_ctl);
   dfree(c.amg_inv); dfree(c.amg_rows); dfree(c.box_part); dfree(c.amg_q9); dfree(c.amg_tq);
-  if (c.flags_host) (void)hipHostFree(c.flags_host);
-  if (c.nbr_total_host) (void)hipHostFree(c.nbr_total_host);
-  if (c.ppe_counters_host) (void)hipHostFree(c.ppe_counters_host);
+  if (c.counters_host) (void)hipHostFree(c.counters_host);
   if (c.red_host) (void)hipHostFree(c.red_host);
-  if (c.ml_active_host) (void)hipHostFree(c.ml_active_host);
-  if (c.st_host) (void)hipHostFree(c.st_host);
   if (c.st32_host) (void)hipHostFree(c.st32_host);
   if (c.ir_host) (void)hipHostFree(c.ir_host);
   if (c.res_host) (void)hipHostFree(c.res_host);
@@ -393,25 +388,22 @@ int mps_create(const mps_env* env, double allowable_residual, int device, mps_ct
     c.cell_start = mps::dalloc<uint32_t>(c.ncells);
     c.cell_fill = mps::dalloc<uint32_t>(c.ncells);
     c.scan_tmp = mps::dalloc<uint64_t>(c.ncells / 2048 + 4096);
-    c.flags = mps::dalloc<int>(4);
-    c.nbr_total_dev = mps::dalloc<unsigned long long>(1);
+    c.counters = mps::dalloc<mps::Counters>(1);
     c.in_cells = mps::dalloc<uint64_t>(1);
-    c.ppe_counters = mps::dalloc<unsigned long long>(8);
     c.partA = mps::dalloc<double>(mps::kRedBlocks);
     c.partB = mps::dalloc<double>(mps::kRedBlocks);
     c.partC = mps::dalloc<double>(mps::kRedBlocks);
     c.part3a = mps::dalloc<double>(3 * mps::kRedBlocks);
     c.part3b = mps::dalloc<double>(3 * mps::kRedBlocks);
-    c.red_out = mps::dalloc<double>(mps::kRedOut);
-    c.st = mps::dalloc<mps::CgStatus>(1);
+    // the solve's reduced scalars and status side by side: one copy to the host
+    constexpr size_t kScalars = mps::kRedOut + sizeof(mps::CgStatus) / sizeof(double);
+    c.red_out = mps::dalloc<double>(kScalars);
+    c.st = reinterpret_cast<mps::CgStatus*>(c.red_out + mps::kRedOut);
     c.st32 = mps::dalloc<mps::CgStatus>(1);
     c.ir = mps::dalloc<mps::IrStatus>(1);
-    mps::pinned(c.flags_host, 4);
-    mps::pinned(c.nbr_total_host, 1);
-    mps::pinned(c.ppe_counters_host, 8);
-    mps::pinned(c.red_host, mps::kRedOut);
-    mps::pinned(c.ml_active_host, 1);
-    mps::pinned(c.st_host, 1);
+    mps::pinned(c.counters_host, 1);
+    mps::pinned(c.red_host, kScalars);
+    c.st_host = reinterpret_cast<mps::CgStatus*>(c.red_host + mps::kRedOut);
     mps::pinned(c.st32_host, 1);
     mps::pinned(c.ir_host, 1);
     mps::pinned(c.res_host, mps::kResHead / sizeof(unsigned));

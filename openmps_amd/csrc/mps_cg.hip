@@ -982,6 +982,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
     st->rr0 = rr0;
     st->b2 = bb;
     st->converged = conv ? 1 : 0;
+    st->ran = 1;
     st->iterations = it - 1;
   }
 }
@@ -3766,10 +3767,11 @@ bool resident_cg64(Context& c, const Sell<double>& A, const Launch& L, const Sto
   MPS_HIP(hipEventRecord(c.solve_b, c.stream));
   residual64_launch(c);
   check_launch();
-  MPS_HIP(hipMemcpyAsync(c.res_host, c.res_ctl, 2 * sizeof(unsigned), hipMemcpyDeviceToHost, c.stream));
-  MPS_HIP(hipMemcpyAsync(c.red_host, c.red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  read_status(c, c.st, c.st_host);
-  if (c.res_host[1]) {
+  MPS_HIP(hipMemcpyAsync(c.red_host, c.red_out, kRedOut * sizeof(double) + sizeof(CgStatus), hipMemcpyDeviceToHost,
+                         c.stream));
+  MPS_HIP(hipStreamSynchronize(c.stream));
+  collect_events(c, c.st_host->converged ? c.st_host->iterations : 0x7fffffffffffffffLL);
+  if (!c.st_host->ran) {
     c.res_skip = kResSkip;
     return false;
   }
@@ -4149,7 +4151,7 @@ CellGrid ml_grid(const Context& c, const MlGeom& g) {
 // The list of the 4x4 blocks of cells that hold particles, from the search's
 // cell counts, and its length on its way to the host, on c.stream.
 }  // namespace
-void enqueue_block_list(Context& c) {
+void enqueue_block_list(Context& c, bool copy) {
   const MlGeom g = ml_geom(c);
   if (c.ml_blk_cap < g.nblk) {
     dfree(c.ml_flag);
@@ -4160,12 +4162,13 @@ void enqueue_block_list(Context& c) {
     c.ml_list = dalloc<uint32_t>(g.nblk);
     c.ml_blk_cap = g.nblk;
   }
-  if (!c.ml_active) c.ml_active = dalloc<uint64_t>(1);
   hipLaunchKernelGGL(k_ml_active, dim3(grid_for(g.nblk)), dim3(256), 0, c.stream, ml_grid(c, g), c.ml_flag);
-  scan_counts(c, c.ml_flag, g.nblk, c.ml_off, c.ml_active);
+  scan_counts(c, c.ml_flag, g.nblk, c.ml_off, &c.counters->ml_active);
   hipLaunchKernelGGL(k_ml_compact, dim3(grid_for(g.nblk)), dim3(256), 0, c.stream, static_cast<uint32_t>(g.nblk),
                      static_cast<const uint32_t*>(c.ml_flag), static_cast<const uint32_t*>(c.ml_off), c.ml_list);
-  MPS_HIP(hipMemcpyAsync(c.ml_active_host, c.ml_active, sizeof(uint64_t), hipMemcpyDeviceToHost, c.stream));
+  if (copy)
+    MPS_HIP(hipMemcpyAsync(&c.counters_host->ml_active, &c.counters->ml_active, sizeof(uint64_t),
+                           hipMemcpyDeviceToHost, c.stream));
   check_launch();
   c.ml_list_serial = c.search_serial;
 }
@@ -4207,7 +4210,7 @@ void ml_setup(Context& c) {
                        static_cast<const float*>(c.d32), c.agg_inv);
   });
   check_launch();
-  if (!block_list_ready(c)) enqueue_block_list(c);
+  if (!block_list_ready(c)) enqueue_block_list(c, true);
 }
 
 // ---- cell-grid multigrid (MPS_PRECOND_AMG) ----
@@ -4322,7 +4325,7 @@ void amg_setup(Context& c) {
     // level-0 point each cycle, from direction sums cleared per solve)
   });
   check_launch();
-  if (!block_list_ready(c)) enqueue_block_list(c);
+  if (!block_list_ready(c)) enqueue_block_list(c, true);
 }
 
 // The packed slots of the listed blocks (k_ml_pack) and, for the multigrid,
@@ -4330,7 +4333,7 @@ void amg_setup(Context& c) {
 void pack_slots(Context& c, bool amg) {
   const size_t n = c.ppe_n;
   const MlGeom g = ml_geom(c);
-  const uint32_t nact = static_cast<uint32_t>(*c.ml_active_host);
+  const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
   const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
   const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
   if (c.ml_pack_cap < slots) {
@@ -4439,7 +4442,7 @@ template <bool AMG>
 bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   const size_t n = c.ppe_n;
   const Launch L = cg_grid(n);
-  const uint32_t nact = static_cast<uint32_t>(*c.ml_active_host);
+  const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
   const int grid = std::max(L.grid, static_cast<int>((nact + NT / 64 - 1) / (NT / 64)));
   if (L.rpb != static_cast<size_t>(NT) || c.cap > 4u * kPerLane || mf_nnz_wide(c) > 0 || grid > kResSlots) return false;
   if (c.res_skip > 0) {
@@ -4585,7 +4588,7 @@ void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max
   refine(c, sr, [&](double norm, double sweep_tol) {
     // refine() has synchronised the stream (residual) before every sweep: the
     // block count and the wide nnz are on the host
-    nact = static_cast<uint32_t>(*c.ml_active_host);
+    nact = static_cast<uint32_t>(c.counters_host->ml_active);
     b_spmv = b_base + 2.0 * mf_nnz_wide(c);
     pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
     b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
@@ -4697,7 +4700,7 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   refine(c, sr, [&](double norm, double sweep_tol) {
     // refine() has synchronised the stream before every sweep: the block
     // count and the wide nnz are on the host
-    nact = static_cast<uint32_t>(*c.ml_active_host);
+    nact = static_cast<uint32_t>(c.counters_host->ml_active);
     b_spmv = b_base + 2.0 * mf_nnz_wide(c);
     pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
     b_pass = n * 30.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 8);
@@ -5019,7 +5022,7 @@ void batch_solve_run(std::vector<SceneRun>& sc, BatchWork& w) {
     rt[s] = ResidArgs{sell<double>(c, c.sval, c.diag, L.rpb), c.b, c.sol, c.r, c.partB, c.partC, red_dev + 2 * s,
                       L.grid};
     float* const zval = reinterpret_cast<float*>(c.zrec) + 2;
-    pt[s] = PrecArgs{ml_grid(c, g), c.ml_list, static_cast<uint32_t>(*c.ml_active_host), c.ml_pid, c.ml_dv,
+    pt[s] = PrecArgs{ml_grid(c, g), c.ml_list, static_cast<uint32_t>(c.counters_host->ml_active), c.ml_pid, c.ml_dv,
                      c.ml_sc, c.r, 1.0, c.r32, c.d32, c.q32, c.dinv32, zval, 4u, c.part3b, L.grid, c.part_ml,
                      c.part_ml_cap, w.st + s};
     st[s] = SpmvArgs<MatFreeRec>{matfree_rec(c, L.rpb), nullptr, c.pa32, c.q32, c.d32, c.part_ml, c.part_ml_cap,
@@ -5308,7 +5311,7 @@ double replay_spmv(Context& c, int kid, int reps) {
                        static_cast<const uint2*>(c.qpos), c.zrec, c.r32, c.d32);
     c.rec_ready = true;
   }
-  const size_t pgrid = std::max<size_t>(1, (*c.ml_active_host + NTP / 64 - 1) / (NTP / 64));
+  const size_t pgrid = std::max<size_t>(1, (c.counters_host->ml_active + NTP / 64 - 1) / (NTP / 64));
   auto launch = [&] {
     if (kid == MPS_K_CG_SPMV32)
       hipLaunchKernelGGL((k_ml_spmv<false, MatFreeRec>), dim3(L.grid), dim3(NT), 0, c.stream,
@@ -5607,7 +5610,7 @@ void batch_solve(std::vector<Context*>& scenes, BatchWork& w) {
     r.c = c;
     const size_t n = c->ppe_n;
     r.L = cg_grid(n);
-    const uint32_t nact = static_cast<uint32_t>(*c->ml_active_host);
+    const uint32_t nact = static_cast<uint32_t>(c->counters_host->ml_active);
     r.pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
     r.vgrid = grid_for(n);
     r.amg = batch_amg(*c);

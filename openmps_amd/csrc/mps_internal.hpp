@@ -35,7 +35,7 @@ struct CgStatus {
   double rr0;
   double b2;          // |b|^2 (stop rule on |b|)
   int converged;      // 1 once the stop rule holds
-  int pad;
+  int ran;            // resident solve: it was not refused or given up
   long long iterations;
   long long stop_mark;  // multilevel inner solver: 0 running, k + 1 once it stopped at iteration k
 };
@@ -47,6 +47,19 @@ struct IrStatus {
   double rr0;
   int done;
   int pad;
+};
+
+// What a step's kernels count and the host reads after its two synchronisations
+// before the solve, side by side: one copy each.  (A copy of a few bytes takes 3.5
+// us of the stream, whatever its size.)
+struct Counters {
+  int flags[4];                  // search: [0] cell overflow, [1] neighbour overflow, [2] a running count
+  unsigned long long nbr_total;  // search: entries of the neighbour lists
+  uint64_t ml_active;            // search: occupied 4x4 blocks of cells
+  // the pressure system: stored off-diagonals, those in slices with wide offsets,
+  // the cell box (amg_box_from_counters), slots
+  unsigned long long nnz, nnz_wide, box[4];
+  uint64_t slots;
 };
 
 struct ResidentCtl;  // mps_resident.hpp
@@ -144,8 +157,8 @@ struct Context {
   double2* pos_sorted = nullptr;  // (x, z) in cell order (the search's candidate ranges)
   uint64_t* in_cells = nullptr;    // particles in cells (device scalar, from the cell scan)
   uint64_t* scan_tmp = nullptr;   // block sums of the scans
-  int* flags = nullptr;           // [0] cell overflow, [1] neighbour overflow
-  int* flags_host = nullptr;      // pinned mirror
+  Counters* counters = nullptr;
+  Counters* counters_host = nullptr;  // pinned mirror
 
   // storage order: the particles are kept in cell order, permuted at every
   // neighbour search (cells in key order, ascending caller index inside a
@@ -168,8 +181,6 @@ struct Context {
   uint32_t *nbr = nullptr, *ncount = nullptr;
   bool have_neighbors = false;
   long long search_serial = 0;  // neighbour searches run so far (cells of the last one in key / sorted)
-  unsigned long long* nbr_total_dev = nullptr;
-  unsigned long long* nbr_total_host = nullptr;  // pinned
   double nbr_total = 0;                          // sum of list lengths (byte accounting)
 
   // PPE in sliced ELL (SELL-64): diagonal kept dense, off-diagonals of row i
@@ -206,11 +217,9 @@ struct Context {
   uint8_t* slice_wide = nullptr;
   int16_t* col16 = nullptr;  // sell_cap entries, beside scol
   double mf_nnz_wide = 0;
-  bool mf_wide_pending = false;  // mf_nnz_wide still in ppe_counters_host[2]
+  bool mf_wide_pending = false;  // mf_nnz_wide still in counters_host
   // [0] off-diagonal nnz, [1] wide nnz, [2..5] the cell box of the rows with
   // off-diagonals (gnx - 1 - min x, max x, gnz - 1 - min z, max z: atomic maxima)
-  unsigned long long* ppe_counters = nullptr;
-  unsigned long long* ppe_counters_host = nullptr;  // pinned: nnz, slots, wide nnz, cell box [3..6]
   uint32_t amg_box[4] = {0, 0, 0, 0};  // cells x0, z0, nx, nz of that box (the multigrid's level 0)
   bool amg_box_ready = false;          // the box belongs to the installed system
   uint4* box_part = nullptr;           // per-block partial boxes
@@ -219,8 +228,8 @@ struct Context {
   // CG work vectors
   double *r = nullptr, *pa = nullptr, *q = nullptr;  // residual, direction, A direction
   double *partA = nullptr, *partB = nullptr, *partC = nullptr;
-  double* red_out = nullptr;
-  double* red_host = nullptr;  // pinned, kRedOut entries (as red_out)
+  double* red_out = nullptr;   // kRedOut entries, then st
+  double* red_host = nullptr;  // pinned, as red_out (st_host after it)
   CgStatus* st = nullptr;
   CgStatus* st_host = nullptr;
   CgStatus* st32 = nullptr;
@@ -277,8 +286,6 @@ struct Context {
   size_t ml_pack_cap = 0;      // lanes (64 per listed block)
   long long ml_list_serial = -1;       // search whose cells the list is of
   bool rec_ready = false;              // zrec holds the installed system's positions
-  uint64_t* ml_active = nullptr;       // count of such blocks
-  uint64_t* ml_active_host = nullptr;  // pinned
   size_t agg_cap = 0;
   size_t agg_off[4] = {0, 0, 0, 0};  // level l at agg_inv + agg_off[l]
   float* dinv32 = nullptr;
@@ -526,8 +533,8 @@ int precond_for_system(Context& c);
 int effective_precond(const Context& c);
 // The occupied 4x4 blocks of cells, for the mixed solvers' preconditioners
 // (mps_cg.hip): enqueued by the search so that their count is on the host
-// with the search's own synchronisation.
-void enqueue_block_list(Context& c);
+// with the search's own synchronisation (copy: on its way by itself).
+void enqueue_block_list(Context& c, bool copy);
 double replay_spmv(Context& c, int kid, int reps);  // mps_cg.hip: mean ms of one launch
 // exclusive scan of n u32 counts into out, grand total to *total (device); mps_search.hip
 void scan_counts(Context& c, const uint32_t* in, size_t n, uint32_t* out, uint64_t* total);

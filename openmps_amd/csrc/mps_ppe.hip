@@ -23,7 +23,7 @@
 
 namespace mps {
 
-void scan_slices(Context& c, const uint32_t* widths, size_t nslices, uint64_t* offsets);
+void scan_slices(Context& c, const uint32_t* widths, size_t nslices, uint64_t* offsets, uint64_t* total);
 
 namespace {
 
@@ -594,7 +594,8 @@ PpeConsts ppe_prepare(Context& c) {
   PpeConsts k{c.env.r_e, c.env.r_e * c.env.r_e, c.env.r_lap, c.env.r_lap * c.env.r_lap, c.env.n0,
               c.env.n0_lap, c.env.rho, c.dt, c.solver.warm_start, c.env.min_x, c.env.min_z,
               c.qpos_inv_h};
-  if (n > 0) MPS_HIP(hipMemsetAsync(c.ppe_counters, 0, 6 * sizeof(unsigned long long), c.stream));
+  if (n > 0)
+    MPS_HIP(hipMemsetAsync(&c.counters->nnz, 0, sizeof(Counters) - offsetof(Counters, nnz), c.stream));
   return k;
 }
 
@@ -669,7 +670,7 @@ __global__ void __launch_bounds__(256) k_row_box_final(const uint4* __restrict__
   }
 }
 
-// Enqueues the two passes (box into ppe_counters[2..5]).
+// Enqueues the two passes (box into the counters).
 void row_box_launch(Context& c, size_t n) {
   if (!c.box_part) c.box_part = dalloc<uint4>(kBoxBlocks);
   const int nb = static_cast<int>(std::min<size_t>(kBoxBlocks, std::max<size_t>(1, (n + kBlock - 1) / kBlock)));
@@ -677,13 +678,13 @@ void row_box_launch(Context& c, size_t n) {
                      static_cast<const uint32_t*>(c.key), static_cast<uint32_t>(c.gnx),
                      static_cast<uint32_t>(c.gnz), c.box_part);
   hipLaunchKernelGGL(k_row_box_final, dim3(1), dim3(256), 0, c.stream, static_cast<const uint4*>(c.box_part), nb,
-                     c.ppe_counters + 2);
+                     c.counters->box);
 }
 
 // The box of cells of the rows with off-diagonals, from the counters k_row_box
-// left in ppe_counters_host[3..6].
+// left.
 void amg_box_from_counters(Context& c) {
-  const unsigned long long* h = c.ppe_counters_host + 3;
+  const unsigned long long* h = c.counters_host->box;
     if (h[1] == 0) {  // no row with off-diagonals: a one-cell level
       c.amg_box[0] = c.amg_box[1] = 0;
       c.amg_box[2] = c.amg_box[3] = 1;
@@ -702,25 +703,17 @@ void amg_box_from_counters(Context& c) {
 void ppe_finish(Context& c, const PpeConsts& k) {
   const size_t n = c.n;
   const NV nb{c.nbr, c.ncount, c.kstride};
-  scan_slices(c, c.slice_width, c.nslices, c.slice_off);
+  scan_slices(c, c.slice_width, c.nslices, c.slice_off, &c.counters->slots);
   const int pc = c.solver.kind == MPS_SOLVER_MIXED_IR ? precond_for_system(c) : MPS_PRECOND_NONE;
   const bool want_box = pc == MPS_PRECOND_AMG;
-  if (want_box) {
-    row_box_launch(c, n);
-    MPS_HIP(hipMemcpyAsync(c.ppe_counters_host + 3, c.ppe_counters + 2, 4 * sizeof(unsigned long long),
-                           hipMemcpyDeviceToHost, c.stream));
-  }
-  MPS_HIP(hipMemcpyAsync(c.ppe_counters_host, c.ppe_counters, sizeof(unsigned long long),
-                         hipMemcpyDeviceToHost, c.stream));
-  MPS_HIP(hipMemcpyAsync(c.ppe_counters_host + 1, c.slice_off + c.nslices, sizeof(uint64_t),
-                         hipMemcpyDeviceToHost, c.stream));
-  MPS_HIP(hipMemcpyAsync(c.ppe_counters_host + 2, c.ppe_counters + 1, sizeof(unsigned long long),
+  if (want_box) row_box_launch(c, n);
+  MPS_HIP(hipMemcpyAsync(&c.counters_host->nnz, &c.counters->nnz, sizeof(Counters) - offsetof(Counters, nnz),
                          hipMemcpyDeviceToHost, c.stream));
   MPS_HIP(hipStreamSynchronize(c.stream));
-  c.nnz_offdiag = c.ppe_counters_host[0];
-  c.sell_slots = c.ppe_counters_host[1];
+  c.nnz_offdiag = c.counters_host->nnz;
+  c.sell_slots = c.counters_host->slots;
   // the wide slices' stored count (byte accounting only), from the count pass
-  c.mf_nnz_wide = static_cast<double>(c.ppe_counters_host[2]);
+  c.mf_nnz_wide = static_cast<double>(c.counters_host->nnz_wide);
   c.mf_wide_pending = false;
   c.amg_box_ready = false;
   if (want_box) amg_box_from_counters(c);
@@ -777,7 +770,7 @@ void ppe_assemble(Context& c) {
     hipLaunchKernelGGL(k_ppe_count, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w,
                        c.p, static_cast<const uint8_t*>(c.type), nb, k, static_cast<const double*>(c.nws),
                        static_cast<const double*>(c.ecs), c.b, c.sol, c.row_len, c.slice_width,
-                       c.slice_wide, c.qpos, c.ppe_counters, c.ppe_counters + 1, c.diag);
+                       c.slice_wide, c.qpos, &c.counters->nnz, &c.counters->nnz_wide, c.diag);
   });
   check_launch();
   pack_state(c);  // the fill gathers the packed positions
@@ -795,7 +788,7 @@ void density_save_and_assemble(Context& c) {
     hipLaunchKernelGGL(near_pays(k.re, k.rl) ? k_density_ppe_count<true> : k_density_ppe_count<false>,
                        dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w, c.p, static_cast<const uint8_t*>(c.type), nb, k, c.nd, c.nws,
                        static_cast<const double*>(c.ecs), c.ox, c.oz, c.b, c.sol, c.row_len, c.slice_width,
-                       c.slice_wide, c.qpos, c.ppe_counters, c.ppe_counters + 1,
+                       c.slice_wide, c.qpos, &c.counters->nnz, &c.counters->nnz_wide,
                        static_cast<const double2*>(c.xz),
                        static_cast<const double2*>(c.uw), c.diag);
   });
@@ -807,15 +800,15 @@ void amg_box(Context& c) {
   if (c.amg_box_ready) return;
   row_box_launch(c, c.ppe_n);
   check_launch();
-  MPS_HIP(hipMemcpyAsync(c.ppe_counters_host + 3, c.ppe_counters + 2, 4 * sizeof(unsigned long long),
-                         hipMemcpyDeviceToHost, c.stream));
+  MPS_HIP(hipMemcpyAsync(c.counters_host->box, c.counters->box, sizeof c.counters->box, hipMemcpyDeviceToHost,
+                         c.stream));
   MPS_HIP(hipStreamSynchronize(c.stream));
   amg_box_from_counters(c);
 }
 
 double mf_nnz_wide(Context& c) {
   if (c.mf_wide_pending) {
-    c.mf_nnz_wide = static_cast<double>(c.ppe_counters_host[2]);
+    c.mf_nnz_wide = static_cast<double>(c.counters_host->nnz_wide);
     c.mf_wide_pending = false;
   }
   return c.mf_nnz_wide;

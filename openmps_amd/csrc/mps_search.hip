@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256) k_scan_reduce(const uint32_t* __restrict_
   if (threadIdx.x == 0) bsum[blockIdx.x] = s[0] + s[1] + s[2] + s[3];
 }
 
-// Inclusive scan of one value per thread across a 256-thread block.
+// Inclusive scan of one value per thread across a block (one word of lds a wavefront).
 __device__ __forceinline__ uint64_t block_inclusive_scan(uint64_t v, uint64_t* lds4) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
@@ -140,8 +140,9 @@ __device__ __forceinline__ uint64_t block_inclusive_scan(uint64_t v, uint64_t* l
   return v + off;
 }
 
-// Single block: exclusive scan of the block sums in place, grand total to *total.
-__global__ void __launch_bounds__(256) k_scan_top(uint64_t* bsum, int nb, uint64_t* total) {
+// Single block: exclusive scan of the block sums in place, grand total to *total
+// (and *copy).
+__global__ void __launch_bounds__(256) k_scan_top(uint64_t* bsum, int nb, uint64_t* total, uint64_t* copy) {
   __shared__ uint64_t lds4[4];
   __shared__ uint64_t tot;
   uint64_t carry = 0;
@@ -156,6 +157,37 @@ __global__ void __launch_bounds__(256) k_scan_top(uint64_t* bsum, int nb, uint64
     __syncthreads();
   }
   if (threadIdx.x == 0 && total) *total = carry;
+  if (threadIdx.x == 0 && copy) *copy = carry;
+}
+
+// The whole scan in one block, for up to kScanOne entries (one round): 3.5 us where
+// the three launches take 9.5.  (A second round would cost as much as they do: four,
+// for 33k cells, took 25 us instead of 12.)
+constexpr int kScanOneThreads = 1024;
+constexpr size_t kScanOne = kScanOneThreads * kScanItems;
+template <class TO>
+__global__ void __launch_bounds__(kScanOneThreads) k_scan_one(const uint32_t* __restrict__ in, size_t n,
+                                                              TO* __restrict__ out, uint64_t mult, uint64_t* total,
+                                                              uint64_t* copy) {
+  __shared__ uint64_t lds[kScanOneThreads / 64];
+  const size_t base = threadIdx.x * kScanItems;
+  uint64_t v[kScanItems], acc = 0;
+#pragma unroll
+  for (int k = 0; k < kScanItems; k++) {
+    v[k] = (base + k < n) ? static_cast<uint64_t>(in[base + k]) * mult : 0;
+    acc += v[k];
+  }
+  const uint64_t inc = block_inclusive_scan(acc, lds);
+  uint64_t run = inc - acc;
+#pragma unroll
+  for (int k = 0; k < kScanItems; k++) {
+    if (base + k < n) out[base + k] = static_cast<TO>(run);
+    run += v[k];
+  }
+  if (threadIdx.x == kScanOneThreads - 1) {
+    if (total) *total = inc;
+    if (copy) *copy = inc;
+  }
 }
 
 template <class TO>
@@ -458,13 +490,19 @@ __global__ void __launch_bounds__(kBlock) k_neighbors(GridParams g, size_t n, co
 
 }  // namespace
 
-// Exclusive scan out[k] = sum_{m<k} in[m] * mult over n entries; optional total.
+// Exclusive scan out[k] = sum_{m<k} in[m] * mult over n entries; optional total (and
+// a copy of it).
 template <class TO>
-static void scan_u32(Context& c, const uint32_t* in, size_t n, TO* out, uint64_t mult, uint64_t* total) {
+static void scan_u32(Context& c, const uint32_t* in, size_t n, TO* out, uint64_t mult, uint64_t* total,
+                     uint64_t* copy = nullptr) {
   const int nb = static_cast<int>((n + kScanChunk - 1) / kScanChunk);
   if (nb == 0) return;
+  if (n <= kScanOne) {
+    hipLaunchKernelGGL(k_scan_one<TO>, dim3(1), dim3(kScanOneThreads), 0, c.stream, in, n, out, mult, total, copy);
+    return;
+  }
   hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, c.stream, in, n, c.scan_tmp, mult);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, c.stream, c.scan_tmp, nb, total);
+  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, c.stream, c.scan_tmp, nb, total, copy);
   hipLaunchKernelGGL(k_scan_apply<TO>, dim3(nb), dim3(256), 0, c.stream, in, n,
                      static_cast<const uint64_t*>(c.scan_tmp), out, mult);
 }
@@ -473,8 +511,8 @@ void scan_counts(Context& c, const uint32_t* in, size_t n, uint32_t* out, uint64
   scan_u32<uint32_t>(c, in, n, out, 1, total);
 }
 
-void scan_slices(Context& c, const uint32_t* widths, size_t nslices, uint64_t* offsets) {
-  scan_u32<uint64_t>(c, widths, nslices, offsets, 64, offsets + nslices);
+void scan_slices(Context& c, const uint32_t* widths, size_t nslices, uint64_t* offsets, uint64_t* total) {
+  scan_u32<uint64_t>(c, widths, nslices, offsets, 64, offsets + nslices, total);
 }
 
 // Moves the particle state into the cell order the sort left in c.sorted.
@@ -527,7 +565,7 @@ void search(Context& c) {
   GridParams g{c.env.min_x, c.env.min_z, c.env.neighbor_length, c.gnx, c.gnz, c.cap,
                nl2 * (1.0 - 0x1p-48), nl2 * (1.0 + 0x1p-48)};
   hipLaunchKernelGGL(k_search_clear, dim3(grid_for(std::max<size_t>(c.ncells, 4))), dim3(kBlock), 0, c.stream,
-                     c.ncells, c.cell_count, c.cell_fill, c.flags, c.nbr_total_dev);
+                     c.ncells, c.cell_count, c.cell_fill, c.counters->flags, &c.counters->nbr_total);
   check_launch();
   if (n == 0) {
     c.have_neighbors = true;
@@ -535,7 +573,7 @@ void search(Context& c) {
   }
   tracked(c, MPS_K_CELL_KEYS, 26.0 * n, [&] {
     hipLaunchKernelGGL(k_cell_keys, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, g, n, c.x, c.z,
-                       c.type, c.key, c.cell_count, c.flags);
+                       c.type, c.key, c.cell_count, c.counters->flags);
   });
   tracked(c, MPS_K_CELL_SCAN, 8.0 * c.ncells, [&] {
     scan_u32<uint32_t>(c, c.cell_count, c.ncells, c.cell_start, 1, c.in_cells);
@@ -543,7 +581,7 @@ void search(Context& c) {
   tracked(c, MPS_K_CELL_SCATTER, 16.0 * n, [&] {
     hipLaunchKernelGGL(k_cell_scatter, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n,
                        static_cast<const uint32_t*>(c.key), static_cast<const uint32_t*>(c.cell_start),
-                       c.cell_fill, c.sorted, static_cast<const uint64_t*>(c.in_cells), c.flags);
+                       c.cell_fill, c.sorted, static_cast<const uint64_t*>(c.in_cells), c.counters->flags);
   });
   // sorted ids read and written, their caller indices gathered
   tracked(c, MPS_K_CELL_SORT, 12.0 * n + 8.0 * c.ncells, [&] {
@@ -568,22 +606,21 @@ void search(Context& c) {
     hipLaunchKernelGGL(walk, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, g, n, c.x, c.z,
                        static_cast<const uint8_t*>(c.type), static_cast<const uint32_t*>(c.cell_start),
                        static_cast<const uint32_t*>(c.cell_count), static_cast<const uint32_t*>(c.sorted),
-                       static_cast<const double2*>(c.pos_sorted), c.kmax, c.kstride, c.nbr, c.ncount, c.flags,
-                       c.nbr_total_dev);
+                       static_cast<const double2*>(c.pos_sorted), c.kmax, c.kstride, c.nbr, c.ncount,
+                       c.counters->flags, &c.counters->nbr_total);
   });
   check_launch();
   if (c.solver.kind == MPS_SOLVER_MIXED_IR &&
       (c.solver.precond == MPS_PRECOND_MULTILEVEL || c.solver.precond == MPS_PRECOND_AMG ||
        c.solver.precond == MPS_PRECOND_AUTO))
-    enqueue_block_list(c);
-  MPS_HIP(hipMemcpyAsync(c.flags_host, c.flags, 4 * sizeof(int), hipMemcpyDeviceToHost, c.stream));
-  MPS_HIP(hipMemcpyAsync(c.nbr_total_host, c.nbr_total_dev, sizeof(unsigned long long),
-                         hipMemcpyDeviceToHost, c.stream));
+    enqueue_block_list(c, false);
+  // flags, the lists' length and the block count in one copy (Counters)
+  MPS_HIP(hipMemcpyAsync(c.counters_host, c.counters, offsetof(Counters, nnz), hipMemcpyDeviceToHost, c.stream));
   MPS_HIP(hipStreamSynchronize(c.stream));
-  c.nbr_total = *c.nbr_total_host;
+  c.nbr_total = c.counters_host->nbr_total;
   add_bytes(c, MPS_K_NEIGHBORS, 4.0 * c.nbr_total);
   c.have_neighbors = true;
-  if (c.flags_host[0] || c.flags_host[1])
+  if (c.counters_host->flags[0] || c.counters_host->flags[1])
     throw Failure{MPS_ERR_CELL_OVERFLOW, "Too many particle in a block"};
 }
 

@@ -63,3 +63,24 @@ def test_uneven_neighbourhoods(n, r_e, r_lap):
         pass
     for a, b in zip(A[:4], whole.ppe()[:4]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nx,nz", [(1, 1), (40, 50), (61, 125), (62, 126), (128, 129), (181, 182)])
+def test_cell_counts(nx, nz):
+    """Grids around the size at which the scan of the cell counts goes from one
+    block (8192 cells) to several launches."""
+    nl = cases.make("gpu", cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, 2.1, L0, 0, 0, 1, 1, 3.1), 1e-9).env()["neighbor_length"]
+    env = cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, 2.1, L0, 0.0, 0.0, nx * nl, nz * nl, 3.1)
+    rng = np.random.Generator(np.random.PCG64(nx * nz))
+    n = min(2000, 4 * nx * nz)
+    at = rng.integers(0, nx * nz, n)
+    at[-1] = nx * nz - 1  # the last cell is occupied
+    zero = np.zeros(n)
+    parts = dict(x=(at // nz + rng.uniform(0.02, 0.98, n)) * nl, z=(at % nz + rng.uniform(0.02, 0.98, n)) * nl, u=zero,
+                 w=zero, p=zero, n=zero, type=np.zeros(n, np.uint8))
+    g, o = cases.make("gpu", env, 1e-9), cases.make("oracle", env, 1e-9)
+    print(f"  {g.grid()['nx']} x {g.grid()['nz']} cells", flush=True)
+    for c in (g, o):
+        c.add_particles(parts)
+        c.stage("search")
+    compare_stage(g, o, "search")
