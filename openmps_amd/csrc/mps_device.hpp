@@ -91,6 +91,43 @@ __device__ __forceinline__ void walk_list(uint32_t i, uint32_t m, const uint32_t
   }
 }
 
+// walk_list with the same number of groups for every lane of the wavefront (mw: the
+// longest list; m may be 0), so that `use` may work across lanes.
+template <class T, class Load, class Use>
+__device__ __forceinline__ void walk_uniform(uint32_t i, uint32_t m, uint32_t mw, const uint32_t* __restrict__ ids,
+                                             uint32_t kmax, Load load, Use use) {
+  auto group = [&](uint32_t q, uint32_t j[4]) {
+    const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, q < m ? q : 0u, kmax));
+    j[0] = (q < m) ? g.x : i;
+    j[1] = (q + 1 < m) ? g.y : i;
+    j[2] = (q + 2 < m) ? g.z : i;
+    j[3] = (q + 3 < m) ? g.w : i;
+  };
+  uint32_t j[4], jn[4];
+  T f[4];
+  group(0, j);
+  group(4, jn);
+#pragma unroll
+  for (int v = 0; v < 4; v++) f[v] = load(j[v]);
+  for (uint32_t q = 0; q < mw; q += 4) {
+    T fn[4];
+    uint32_t j2[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) fn[v] = load(jn[v]);
+    group(q + 8, j2);
+    bool in[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) in[v] = q + v < m;
+    use(j, f, in);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      j[v] = jn[v];
+      jn[v] = j2[v];
+      f[v] = fn[v];
+    }
+  }
+}
+
 // The walk of a pass whose expensive terms only count for the nearer neighbours
 // (r < r_e, while the list reaches r_lap): far(j, p, f1, in, e) gets four
 // neighbours' positions p and fields f1 (load1), adds the terms of all of them

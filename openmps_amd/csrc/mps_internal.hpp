@@ -179,6 +179,7 @@ struct Context {
   // neighbour lists: slot k of particle i at nbr_slot(i, k, kstride) (groups
   // of four slots per particle, a slice's 64 particles side by side)
   uint32_t *nbr = nullptr, *ncount = nullptr;
+  bool lists_ascending = false;  // the lists were made of particles in cell order
   bool have_neighbors = false;
   long long search_serial = 0;  // neighbour searches run so far (cells of the last one in key / sorted)
   double nbr_total = 0;                          // sum of list lengths (byte accounting)

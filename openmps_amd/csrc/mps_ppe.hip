@@ -554,6 +554,195 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 
                     stage, slice_wide[i >> 6] != 0, kk, xz);
 }
 
+// The fill for particles in cell order, whose lists are one ascending run: entries
+// are stored in list order as the walk finds them.  The rows of a wavefront reach a
+// slot at different times, and stored at once each of their 64 x 8 bytes is
+// written in several pieces (at 1.05M particles 23.7M write requests for 529 MB,
+// which bound the kernel): entries wait in a ring of kFillRing slots per lane in
+// LDS until every row has filled the slot, and the slot goes out in one store of
+// the wavefront; a lane further ahead stores its oldest itself.  The sums, which
+// need the diagonal first, read values and offsets back (from the cache); a
+// column's direction follows from the difference of the two cells' indices (they
+// are neighbours; the grid has a border, so dz + gnz dx is unique); the direction
+// sums are collected in LDS and stored together (72 bytes a row, one after the
+// other, touched 72 lines a store).
+// Every store is within the slice's `width` slots: a row's entries were counted
+// by the same test in the count pass.
+// k_ppe_fill on the same rows -> this kernel: 253 -> 187 us at 1.05M particles
+// (radii 2.1 / 3.1), with the nine direction sums 329 -> 273 us (2.1 / 3.1); 131k
+// particles of a settled column 47.6 -> 47.5 us, in motion 47 -> 36 us.
+constexpr uint32_t kFillRing = 8;
+template <bool ROWS9>
+__global__ void __launch_bounds__(kBlock) k_ppe_fill_cells(size_t n, const double* __restrict__ x,
+                                                           const double* __restrict__ z,
+                                                           const uint8_t* __restrict__ type, NV nb, PpeConsts k,
+                                                           const uint64_t* __restrict__ slice_off,
+                                                           const uint32_t* __restrict__ slice_width,
+                                                           double* __restrict__ val, uint32_t* __restrict__ col,
+                                                           int16_t* __restrict__ col16,
+                                                           const uint8_t* __restrict__ slice_wide,
+                                                           double* __restrict__ diag, float* __restrict__ ghost32,
+                                                           AggSums ag, const double2* __restrict__ xz) {
+  // a thread's column: the ring's values, later the direction sums
+  __shared__ double r9[9][kBlock];
+  __shared__ int16_t rc[kFillRing][kBlock];
+  const int t = threadIdx.x;
+  const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+  const size_t i = blk * static_cast<size_t>(blockDim.x) + t;
+  const size_t slice = (i < n ? i : n - 1) >> 6;
+  const size_t base = slice_off[slice] + (i & 63);
+  const uint32_t width = slice_width[slice], self = static_cast<uint32_t>(i < n ? i : n - 1);
+  const bool wide = slice_wide[slice] != 0;
+  const uint8_t ti = i < n ? type[i] : kDisabled;
+  const bool row = ti != kDummy && ti != kDisabled;
+  double s = 0.0;
+  // entries found; of them stored by this lane, and by every lane
+  uint32_t ne = 0, mine = 0, flushed = 0;
+  auto store = [&](uint32_t v) {
+    const size_t o = base + static_cast<size_t>(v) * 64;
+    val[o] = r9[v % kFillRing][t];
+    col16[o] = rc[v % kFillRing][t];
+  };
+  auto pad = [&](uint32_t v) {  // no entry: value 0, the row's own column
+    const size_t o = base + static_cast<size_t>(v) * 64;
+    val[o] = 0.0;
+    if (wide) col[o] = self;
+    col16[o] = 0;
+  };
+  // every slot v < width of every row i < n is written once: below `flushed` when
+  // the wavefront passes it (by row lanes, or earlier by themselves; padded by the
+  // lanes of dummy and disabled particles), the others at the end
+  {
+    const double xi = x[self], zi = z[self];
+    const uint32_t m = row ? nb.count[self] : 0u;
+    struct F {
+      double x, z;
+      uint8_t t;
+    };
+    walk_uniform<F>(self, m, wave_max_u32(m), nb.ids, nb.kmax,
+                    [&](uint32_t j) {
+                      const double2 pj = xz[j];
+                      return F{pj.x, pj.y, type[j]};
+                    },
+                    [&](const uint32_t* j, const F* f, const bool* in) {
+                      double a[4];
+                      bool l[4];
+#pragma unroll
+                      for (int v = 0; v < 4; v++) {
+                        const double dx = f[v].x - xi, dz = f[v].z - zi;
+                        const double r2 = dx * dx + dz * dz;
+                        l[v] = in[v] && r2 < k.rl2 && f[v].t != kDummy;
+                        const double r = sqrt(r2);
+                        a[v] = 3 * k.rl / k.n0l / (r * r * r);
+                      }
+                      while (ne + 4 > mine + kFillRing) {  // room for four
+                        if (mine >= flushed) store(mine);
+                        mine++;
+                      }
+#pragma unroll
+                      for (int v = 0; v < 4; v++) {
+                        s = l[v] ? s + -a[v] : s;
+                        r9[ne % kFillRing][t] = a[v];  // (overwritten by the next one that counts)
+                        rc[ne % kFillRing][t] = static_cast<int16_t>(static_cast<int>(j[v]) - static_cast<int>(self));
+                        if (wide && l[v]) col[base + static_cast<size_t>(ne) * 64] = j[v];
+                        ne += l[v] ? 1u : 0u;
+                      }
+                      const uint32_t upto = wave_min_u32(row ? ne : 0xffffffffu);
+                      if (upto != 0xffffffffu)
+                        for (; flushed < upto; flushed++) {
+                          if (!row) {
+                            if (i < n) pad(flushed);
+                          } else if (flushed >= mine) {
+                            store(flushed);
+                          }
+                        }
+                      if (row && mine < flushed) mine = flushed;
+                    });
+  }
+  // the rest, and the padding to the slice's width
+  if (i < n)
+    for (uint32_t v = flushed; v < width; v++) {
+      if (v >= ne) pad(v);
+      else if (v >= mine) store(v);
+    }
+  if (ROWS9)
+#pragma unroll
+    for (int u = 0; u < 9; u++) r9[u][t] = 0.0;
+  if (i < n) {
+    double d = 1.0, g = 1.0, a0 = 0, a1 = 0, a2 = 0;
+    if (row) {
+      g = diag[i];  // the ghost's share, from the count pass
+      if (g != 0.0) s += g;
+      d = s;
+      const uint32_t ki = ROWS9 ? ag.aggkey[i] : (ag.s0 ? ag.key[i] : kNoCell);
+      if (ki != kNoCell) {
+        const int gnz = static_cast<int>(ag.gnz);
+        const uint32_t cx = ki / ag.gnz, cz = ki % ag.gnz;
+        a0 = a1 = a2 = d;
+        // consecutive columns of one direction are summed in a run and the run
+        // added to its direction's sum when the direction changes; direction 4's
+        // first run starts from the diagonal
+        int cur = -1;
+        double run = 0.0;
+        bool seen4 = false;
+        for (uint32_t v0 = 0; v0 < ne; v0 += 4) {
+          double a[4];
+          uint32_t kj[4];
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const size_t o = base + static_cast<size_t>(v0 + v < ne ? v0 + v : v0) * 64;
+            a[v] = val[o];
+            const uint32_t j = wide ? col[o] : static_cast<uint32_t>(static_cast<int>(self) + col16[o]);
+            kj[v] = ROWS9 ? ag.aggkey[j] : ag.key[j];
+          }
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            if (v0 + v >= ne || kj[v] == kNoCell) continue;
+            const int diff = static_cast<int>(kj[v] - ki);
+            const int dx = diff > 1 ? 1 : (diff < -1 ? -1 : 0), dz = diff - dx * gnz;
+            if (ROWS9) {
+              const int dir = 3 * (dx + 1) + dz + 1;
+              if (dir != cur) {
+                if (cur >= 0) r9[cur][t] += run;
+                cur = dir;
+                run = (cur == 4 && !seen4) ? d : 0.0;
+                seen4 = seen4 || cur == 4;
+              }
+              run += a[v];
+            } else {
+              const uint32_t jx = cx + dx, jz = cz + dz;
+              if ((jx >> 2) == (cx >> 2) && (jz >> 2) == (cz >> 2)) {
+                a2 += a[v];
+                if ((jx >> 1) == (cx >> 1) && (jz >> 1) == (cz >> 1)) {
+                  a1 += a[v];
+                  if (dx == 0 && dz == 0) a0 += a[v];
+                }
+              }
+            }
+          }
+        }
+        if (ROWS9) {
+          if (cur >= 0) r9[cur][t] += run;
+          if (!seen4) r9[4][t] = d;
+        }
+      }
+    }
+    diag[i] = d;
+    ghost32[i] = static_cast<float>(g);
+    if (!ROWS9 && ag.s0) {
+      ag.s0[i] = static_cast<float>(a0);
+      ag.s1[i] = static_cast<float>(a1);
+      ag.s2[i] = static_cast<float>(a2);
+    }
+  }
+  if (ROWS9) {
+    __syncthreads();
+    const size_t first = blk * static_cast<size_t>(kBlock);
+    const uint32_t rows = first < n ? static_cast<uint32_t>(n - first < kBlock ? n - first : kBlock) : 0u;
+    for (uint32_t q = t; q < 9 * rows; q += kBlock) ag.rows9[9 * first + q] = r9[q % 9][q / 9];
+  }
+}
+
 __global__ void __launch_bounds__(kBlock) k_to_f32(size_t n, const double* __restrict__ a,
                                                    float* __restrict__ b) {
   const size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
@@ -736,6 +925,17 @@ void ppe_finish(Context& c, const PpeConsts& k) {
                        (want_sums ? n * 12.0 + c.nnz_offdiag * 4.0 : 0.0) +
                        (want9 ? n * (72.0 + 4) + c.nnz_offdiag * 4.0 : 0.0);  // k_agg_key's 13 N apart
   tracked(c, MPS_K_PPE_FILL, bytes, [&] {
+    // only lists of particles in cell order ascend; those of a kept storage order
+    // need k_ppe_fill's merge (in cell order it is never the faster: 253 vs 187 us
+    // at 1.05M particles, 47.6 vs 47.5 us at 131k, 18 vs 15 us at 2k)
+    if (c.lists_ascending) {
+      hipLaunchKernelGGL(want9 ? k_ppe_fill_cells<true> : k_ppe_fill_cells<false>, dim3(grid_for(n)), dim3(kBlock), 0,
+                         c.stream, n, c.x, c.z, static_cast<const uint8_t*>(c.type), nb, k,
+                         static_cast<const uint64_t*>(c.slice_off), static_cast<const uint32_t*>(c.slice_width), c.sval,
+                         c.scol, c.col16, static_cast<const uint8_t*>(c.slice_wide), c.diag, c.ghost32, ag,
+                         static_cast<const double2*>(c.xz));
+      return;
+    }
     if (want9)
       hipLaunchKernelGGL(k_ppe_fill<true>, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z,
                          static_cast<const uint8_t*>(c.type), nb, k, static_cast<const double*>(c.nws),

@@ -620,6 +620,7 @@ void search(Context& c) {
   c.nbr_total = c.counters_host->nbr_total;
   add_bytes(c, MPS_K_NEIGHBORS, 4.0 * c.nbr_total);
   c.have_neighbors = true;
+  c.lists_ascending = !c.keep_order;
   if (c.counters_host->flags[0] || c.counters_host->flags[1])
     throw Failure{MPS_ERR_CELL_OVERFLOW, "Too many particle in a block"};
 }
