@@ -4321,8 +4321,8 @@ void amg_setup(Context& c) {
     hipLaunchKernelGGL(k_amg_dense, dim3(1), dim3(1024), 0, c.stream,
                        static_cast<const double*>(c.amg_S64 + 9ull * c.amg_off[lv - 1]), c.amg_nx[lv - 1],
                        c.amg_nz[lv - 1], c.amg_inv);
-    // (level 0's right-hand side needs no clearing: k_amg_rfix writes every
-    // level-0 point each cycle, from direction sums cleared per solve)
+    // (level 0's right-hand side needs no clearing: k_amg_down_tiles or k_amg_rfix
+    // writes every level-0 point each cycle, from direction sums cleared per solve)
   });
   check_launch();
   if (!block_list_ready(c)) enqueue_block_list(c, true);

@@ -561,7 +561,8 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 
 // which bound the kernel): entries wait in a ring of kFillRing slots per lane in
 // LDS until every row has filled the slot, and the slot goes out in one store of
 // the wavefront; a lane further ahead stores its oldest itself.  The sums, which
-// need the diagonal first, read values and offsets back (from the cache); a
+// need the diagonal first, read values and offsets back (344 MB more fetched at
+// 1.05M particles, from the last-level cache); a
 // column's direction follows from the difference of the two cells' indices (they
 // are neighbours; the grid has a border, so dz + gnz dx is unique); the direction
 // sums are collected in LDS and stored together (72 bytes a row, one after the

@@ -32,15 +32,17 @@ KERNEL_IDS = {
     "k_density<true, false, true>": "density_save", "k_explicit": "explicit",
     "k_ppe_count": "ppe_count", "k_ppe_fill": "ppe_fill", "k_cg_init": "cg_init",
     "k_ppe_fill<true>": "ppe_fill", "k_ppe_fill<false>": "ppe_fill",
+    "k_ppe_fill_cells<true>": "ppe_fill", "k_ppe_fill_cells<false>": "ppe_fill",
     "k_cg_spmv<false>": "cg_spmv", "k_cg_spmv<true>": "cg_spmv", "k_cg_update": "cg_update",
     "k_cg_spmv<false, mps::(anonymous namespace)::Sell<double> >": "cg_spmv",
     "k_cg_spmv<true, mps::(anonymous namespace)::Sell<double> >": "cg_spmv",
-    "k_gradient": "gradient", "k_ds": "ds",
+    "k_gradient": "gradient", "k_gradient<true>": "gradient", "k_gradient<false>": "gradient", "k_ds": "ds",
     "k_ml_spmv<false, mps::(anonymous namespace)::MatFree>": "cg_spmv32",
     "k_ml_spmv<true, mps::(anonymous namespace)::MatFree>": "cg_spmv32",
     "k_ml_spmv<false, mps::(anonymous namespace)::MatFreeRec>": "cg_spmv32",
     "k_ml_spmv<true, mps::(anonymous namespace)::MatFreeRec>": "cg_spmv32",
     "k_density_explicit": "density_ecs", "k_density_ppe_count": "density_save",
+    "k_density_ppe_count<true>": "density_save", "k_density_ppe_count<false>": "density_save",
     "k_ml_prec": "ml_prec", "k_ml_prec<0>": "ml_prec", "k_ml_prec<1>": "ml_prec", "k_ml_prec<2>": "ml_prec",
     "k_ml_prec_up": "ml_prec",
     "k_cgf_iter<mps::(anonymous namespace)::MatFree>": "cg_iter32",
