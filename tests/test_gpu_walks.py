@@ -124,3 +124,29 @@ def test_cell_counts(nx, nz):
         c.add_particles(parts)
         c.stage("search")
     compare_stage(g, o, "search")
+
+
+@pytest.mark.parametrize("least", [0, 15])
+@pytest.mark.parametrize("most", [1, 2, 16, 17, 32, 33])
+def test_cell_sizes(most, least):
+    """Cells of `least` to `most` particles in random order: wavefronts whose cells all
+    fit the sort's smaller network (16), that need the larger (32), that mix them,
+    and cells beyond both."""
+    nl = cases.make("gpu", cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, 5.0, L0, 0, 0, 1, 1, 5.0), 1e-9).env()["neighbor_length"]
+    side = 13
+    env = cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, 5.0, L0, 0.0, 0.0, side * nl, side * nl, 5.0)
+    rng = np.random.Generator(np.random.PCG64(most))
+    cells = np.repeat(np.arange(side * side), rng.integers(min(least, most), most + 1, side * side))
+    cells = rng.permutation(np.append(cells, np.full(most, side * side // 2)))[:8000]
+    cells = cells[np.sort(np.concatenate([np.flatnonzero(cells == c)[:most] for c in range(side * side)]))]
+    n = len(cells)
+    zero = np.zeros(n)
+    parts = dict(x=(cells // side + rng.uniform(0.02, 0.98, n)) * nl, z=(cells % side + rng.uniform(0.02, 0.98, n)) * nl,
+                 u=zero, w=zero, p=zero, n=zero, type=np.zeros(n, np.uint8))
+    g, o = cases.make("gpu", env, 1e-9), cases.make("oracle", env, 1e-9)
+    assert g.grid()["cap"] >= most
+    print(f"  {n} particles, {np.bincount(cells).max()} in a cell at most", flush=True)
+    for c in (g, o):
+        c.add_particles(parts)
+        c.stage("search")
+    compare_stage(g, o, "search")
