@@ -598,8 +598,8 @@ __global__ void __launch_bounds__(NT) k_cg_check(const double* __restrict__ part
 // the sum): 1.5k rows 12.2 -> 4.5 us (4.7), 12k 12.8 -> 4.8 (5.9), 50k 13.9 ->
 // 5.5 (6.9), 125k 17.5 -> 6.5 (8.0), 134k 18.1 -> 9.2 (9.8), 191k 24.1 -> 11.8
 // (13.6), 257k 26.5 -> 14.2 (16.0).
-__global__ void __launch_bounds__(NT) k_resident_clear(ResidentCtl* ctl, CgStatus* st) {
-  resident_clear(ctl);
+__global__ void __launch_bounds__(NT) k_resident_clear(ResidentCtl* ctl, CgStatus* st, ResidentDrill drill) {
+  resident_clear(ctl, drill);
   if (threadIdx.x == 0) *st = CgStatus{};
 }
 
@@ -756,7 +756,7 @@ __device__ __forceinline__ void gather_values(T* __restrict__ to, const T* from,
 // needed holds up the stores: 262 workgroups 9.1 instead of 9.9 us).
 __device__ __forceinline__ double gather_flagged(ResidentCtl* ctl, double* __restrict__ to, const double* from,
                                                  const uint16_t* __restrict__ list, uint32_t wn, unsigned gen,
-                                                 unsigned idx, unsigned G, bool& ok) {
+                                                 unsigned idx, unsigned G, bool& ok, const Patience& w) {
   double sum = 0.0;
   uint32_t k0 = threadIdx.x;
   if (G <= 64) {
@@ -765,7 +765,7 @@ __device__ __forceinline__ double gather_flagged(ResidentCtl* ctl, double* __res
     at[4] = resident_slot(ctl, gen, threadIdx.x < G ? threadIdx.x : idx, 0);
 #pragma unroll
     for (int u = 0; u < 4; u++) at[u] = k0 + u * NT < wn ? from + list[k0 + u * NT] : at[4];
-    flag_wait(ctl, at, t, ok);
+    flag_wait(ctl, at, t, ok, w);
 #pragma unroll
     for (int u = 0; u < 4; u++)
       if (k0 + u * NT < wn) to[k0 + u * NT] = t[u];
@@ -777,14 +777,14 @@ __device__ __forceinline__ double gather_flagged(ResidentCtl* ctl, double* __res
     double t[4];
 #pragma unroll
     for (int u = 0; u < 4; u++) at[u] = from + list[k0 + u * NT < wn ? k0 + u * NT : k0];
-    flag_wait(ctl, at, t, ok);
+    flag_wait(ctl, at, t, ok, w);
 #pragma unroll
     for (int u = 0; u < 4; u++)
       if (k0 + u * NT < wn) to[k0 + u * NT] = t[u];
   }
   if (G > 64) {
     __syncthreads();
-    if (threadIdx.x < G) sum = resident_word(ctl, gen, threadIdx.x, 0, ok);
+    if (threadIdx.x < G) sum = resident_word(ctl, gen, threadIdx.x, 0, ok, w);
   }
   return sum;
 }
@@ -812,7 +812,7 @@ __device__ __forceinline__ double resident_sum(ResidentCtl* ctl, unsigned gen, u
 // Dynamic LDS (bytes): first the gathered r (before the iterations, the marks
 // and their numbers), then the gathered rows' list and the matrix entries from
 // REG on that fit.
-template <class M, int REG, int WAVES>
+template <class M, int REG, int WAVES, bool DRILL = false>
 __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restrict__ x, double* r, double* p,
                                                            double* __restrict__ q,
                                                            const double* __restrict__ part_rr,
@@ -870,7 +870,8 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   if (in) flag_clear(p + i);
   stores_done();
   __syncthreads();
-  if (!resident_start(ctl, ok_lds)) return;
+  const Patience patience = resident_patience<DRILL>(ctl);
+  if (!resident_start(ctl, ok_lds, patience)) return;
   unsigned gen = 0;
   long long it = 1;
   bool conv = false, ok = true;
@@ -926,7 +927,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
     for (uint32_t k = kl; k < m; k++) {
       const double* const at[1] = {cur + row.col(k)};
       double t[1] = {agent_load(at[0])};
-      if (it > 1) flag_wait(ctl, at, t, ok);
+      if (it > 1) flag_wait(ctl, at, t, ok, patience);
       s = fma(row.val(k), t[0], s);
     }
     if (it == 1) {
@@ -937,10 +938,11 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
       pi = fma(beta, pi, ri);
       qi = fma(beta, qi, s);
     }
+    resident_hold<DRILL>(ctl, gen, idx);
     stores_done();  // the entries and slots emptied since the last exchange
     const double sp = block_sum<NT>(in ? fma(pi, qi, 0.0) : 0.0, lds);
     if (threadIdx.x == 0) resident_put(ctl, gen, idx, sp);
-    const double pq1 = threadIdx.x < G ? resident_word(ctl, gen, threadIdx.x, 0, ok) : 0.0;
+    const double pq1 = threadIdx.x < G ? resident_word(ctl, gen, threadIdx.x, 0, ok, patience) : 0.0;
     const double pq = resident_sum(ctl, gen, idx, G, lds, pq1, ok);
     const double alpha = scalar_of(rr / pq);
     gen++;
@@ -950,6 +952,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
     const double ww = wave_sum(in ? fma(ri, ri, 0.0) : 0.0);
     if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = ww;
     __syncthreads();
+    resident_hold<DRILL>(ctl, gen, idx);
     if (in) {
       flag_store(next + i, ri);
       flag_clear(cur + i);  // everyone has published a p.q, so has gathered it
@@ -963,7 +966,8 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
     double* const swap = cur;
     cur = next;
     next = swap;
-    const double rr1 = gather_flagged(ctl, win, static_cast<const double*>(cur + lo), list, wn, gen, idx, G, ok);
+    const double rr1 = gather_flagged(ctl, win, static_cast<const double*>(cur + lo), list, wn, gen, idx, G, ok,
+                                      patience);
     rr_prev = rr;
     rr = resident_sum(ctl, gen, idx, G, lds, rr1, ok);
     gen++;
@@ -987,16 +991,19 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   }
 }
 
-// Final reduction of two partial arrays into out[0], out[1] (single block).
+// Final reduction of two partial arrays into out[0], out[1] (single block).  After a
+// resident solve (ctl): a solve that any workgroup gave up did not run, whatever the
+// leading one found.
 __global__ void __launch_bounds__(NT) k_reduce2(const double* __restrict__ a,
                                                 const double* __restrict__ b, int nparts,
-                                                double* __restrict__ out) {
+                                                double* __restrict__ out, const ResidentCtl* ctl, CgStatus* st) {
   __shared__ double lds[NT / 64];
   const double sa = reduce_partials<NT>(a, nparts, lds);
   const double sb = reduce_partials<NT>(b, nparts, lds);
   if (threadIdx.x == 0) {
     out[0] = sa;
     out[1] = sb;
+    if (ctl && ctl->abort) st->ran = 0;
   }
 }
 
@@ -2838,7 +2845,7 @@ constexpr int kTile2 = 4;
 constexpr int kC1 = 2 * kTile2, kF1 = kC1 + 2, kC0 = 2 * kF1, kF0 = kC0 + 2;
 static_assert(kF0 * kF0 <= NT && kTileF * kTileF <= kF0 * kF0 && 4 * kTile * kTile <= kC0 * kC0, "one point a thread");
 
-template <bool AMG, int REG, int WAVES>
+template <bool AMG, int REG, int WAVES, bool DRILL = false>
 __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
   extern __shared__ double win[];
   __shared__ double lds[2 * (NT / 64)];
@@ -3003,7 +3010,8 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
 
   stores_done();
   __syncthreads();
-  if (!resident_start(ctl, ok_lds)) return;
+  const Patience patience = resident_patience<DRILL>(ctl);
+  if (!resident_start(ctl, ok_lds, patience)) return;
 
   unsigned gen = 0;
   bool ok = true;
@@ -3020,8 +3028,9 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
     return ok;
   };
   auto barrier = [&]() {
+    resident_hold<DRILL>(ctl, gen, idx);
     arrive(0.0);
-    if (tid < G) (void)resident_word(ctl, gen, tid, 0, ok);
+    if (tid < G) (void)resident_word(ctl, gen, tid, 0, ok, patience);
     return passed();
   };
   auto here = [](uint32_t v) { return opaque(v) & ~kOutAgg; };  // the row of a slot
@@ -3057,6 +3066,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
   for (;; outer++) {
     if (!(outer == 0 && A.have_r)) {
       // r = b - A x in FP64 (cg_init_body)
+      resident_hold<DRILL>(ctl, gen, idx);
       gather_values(win, static_cast<const double*>(A.x + lo), list, wn);
       __syncthreads();
       double ri = 0.0, bi = 0.0;
@@ -3099,7 +3109,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
         resident_publish(ctl, gen, idx, t, v);
       }
       double va = 0.0, vb = 0.0;
-      if (tid < G) resident_words(ctl, gen, tid, 0, ok, va, vb);
+      if (tid < G) resident_words(ctl, gen, tid, 0, ok, va, vb, patience);
       if (!passed()) return;
       sum2(va, vb, G, rr, bb);
     }
@@ -3136,10 +3146,10 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
       if (it > 0) {
         // k_ml_spmv(it): r.z and r.r of the preconditioner's last pass
         double va = 0.0, vb = 0.0;
-        if ((tid >> 1) < G) resident_words(ctl, gen, tid >> 1, 2 * (tid & 1), ok, va, vb);
+        if ((tid >> 1) < G) resident_words(ctl, gen, tid >> 1, 2 * (tid & 1), ok, va, vb, patience);
         if (((tid + NT) >> 1) < G) {
           double vc, vd;
-          resident_words(ctl, gen, (tid + NT) >> 1, 2 * (tid & 1), ok, vc, vd);
+          resident_words(ctl, gen, (tid + NT) >> 1, 2 * (tid & 1), ok, vc, vd, patience);
           va += vc;
           vb += vd;
         }
@@ -3176,6 +3186,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
           break;
         }
         // q = A z + beta q, p = z + beta p
+        resident_hold<DRILL>(ctl, gen, idx);
         float* const zl = reinterpret_cast<float*>(win);
         gather_values(zl, static_cast<const float*>(A.z + lo), list, wn);
         __syncthreads();
@@ -3232,8 +3243,8 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
         // alpha, as k_ml_prec's blocks of NTP threads sum it
         double v = 0.0;
         if (tid < NTP) {
-          if (tid < G) v = resident_word(ctl, gen, tid, 0, ok);
-          if (tid + NTP < G) v += resident_word(ctl, gen, tid + NTP, 0, ok);
+          if (tid < G) v = resident_word(ctl, gen, tid, 0, ok, patience);
+          if (tid + NTP < G) v += resident_word(ctl, gen, tid + NTP, 0, ok, patience);
         }
         if (!passed()) return;
         v = wave_sum(v);
@@ -3565,6 +3576,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
         }
       }
       // z is out: r.z and r.r of each 4 blocks of cells (k_ml_prec's blocks)
+      resident_hold<DRILL>(ctl, gen, idx);
       prho = wave_sum(prho);
       prr = wave_sum(prr);
       if (lane == 0) {
@@ -3672,6 +3684,8 @@ double spmv_bytes(const Context& c, int vbytes, double extra_per_row) {
 // A solve that finds another one running takes the launched kernels.
 constexpr int kMaxDevices = 64;
 std::atomic<int> g_resident_busy[kMaxDevices];
+// solves ended and given up so far (read by tests)
+std::atomic<long long> g_resident_solved[kMaxDevices], g_resident_given_up[kMaxDevices];
 struct ResidentTurn {
   int dev = -1;
   explicit ResidentTurn(int d) {
@@ -3681,6 +3695,8 @@ struct ResidentTurn {
   ~ResidentTurn() {
     if (dev >= 0) g_resident_busy[dev].store(0);
   }
+  // what became of the launched solve
+  void ended(bool solved) const { (solved ? g_resident_solved : g_resident_given_up)[dev]++; }
   ResidentTurn(const ResidentTurn&) = delete;
   ResidentTurn& operator=(const ResidentTurn&) = delete;
   explicit operator bool() const { return dev >= 0; }
@@ -3718,16 +3734,16 @@ size_t resident_lds(K kernel, int grid, int per_cu) {
 template <class M>
 bool resident_cg_launch(const M& A, const Launch& L, double* x, double* r, double* p, double* q, const double* part_rr,
                         const double* part_bb, CgStatus* st, const StopRule& sr, long long max_iter, ResidentCtl* ctl,
-                        hipStream_t s) {
+                        const ResidentDrill* drill, hipStream_t s) {
   if (L.rpb != static_cast<size_t>(NT)) return false;  // one row per thread
-  auto kernel = k_cg_resident<M, 32, 2>;
+  auto kernel = drill ? k_cg_resident<M, 32, 2, true> : k_cg_resident<M, 32, 2>;
   size_t lds = resident_lds(kernel, L.grid, 1);
-  if (lds == 0) {
+  if (lds == 0 && !drill) {
     kernel = k_cg_resident<M, 20, 4>;
     lds = resident_lds(kernel, L.grid, 2);
   }
   if (lds == 0) return false;
-  hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, s, ctl, st);
+  hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, s, ctl, st, drill ? *drill : ResidentDrill{});
   hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(NT), lds, s, A, x, r, p, q, part_rr, part_bb, st, sr, max_iter, ctl,
                      static_cast<uint32_t>(lds));
   check_launch();
@@ -3765,19 +3781,21 @@ bool resident_cg64(Context& c, const Sell<double>& A, const Launch& L, const Sto
   bool launched = false;
   tracked(c, MPS_K_CG_SPMV, 0.0, [&] {
     launched = resident_cg_launch(A, L, c.sol, c.r, c.pa, c.q, static_cast<const double*>(c.partB),
-                                  static_cast<const double*>(c.partC), c.st, sr, max_iter, c.res_ctl, c.stream);
+                                  static_cast<const double*>(c.partC), c.st, sr, max_iter, c.res_ctl,
+                                  c.drilling ? &c.drill : nullptr, c.stream);
   });
   if (!launched) {
     c.res_skip = kResSkip;
     return false;
   }
   MPS_HIP(hipEventRecord(c.solve_b, c.stream));
-  residual64_launch(c);
+  residual64_launch(c, c.res_ctl);
   check_launch();
   MPS_HIP(hipMemcpyAsync(c.red_host, c.red_out, kRedOut * sizeof(double) + sizeof(CgStatus), hipMemcpyDeviceToHost,
                          c.stream));
   MPS_HIP(hipStreamSynchronize(c.stream));
   collect_events(c, c.st_host->converged ? c.st_host->iterations : 0x7fffffffffffffffLL);
+  turn.ended(c.st_host->ran != 0);
   if (!c.st_host->ran) {
     c.res_skip = kResSkip;
     return false;
@@ -3918,20 +3936,21 @@ __global__ void __launch_bounds__(1024) k_reduce5(const double* __restrict__ par
 
 // Single-block reduction of two partial arrays into c.red_host[0..1] (synchronous).
 void reduce2(Context& c, const double* a, const double* b, int nparts) {
-  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(NT), 0, c.stream, a, b, nparts, c.red_out);
+  hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(NT), 0, c.stream, a, b, nparts, c.red_out,
+                     static_cast<const ResidentCtl*>(nullptr), static_cast<CgStatus*>(nullptr));
   check_launch();
   MPS_HIP(hipMemcpyAsync(c.red_host, c.red_out, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
   MPS_HIP(hipStreamSynchronize(c.stream));
 }
 
 // FP64 residual |b - A x|^2 and |b|^2 (reuses the init kernel on scratch r).
-void residual64_launch(Context& c) {
+void residual64_launch(Context& c, const ResidentCtl* ctl) {
   const Launch L = cg_grid(c.ppe_n);
   const Sell<double> A = sell<double>(c, c.sval, c.diag, L.rpb);
   hipLaunchKernelGGL(k_cg_init<Sell<double>>, dim3(L.grid), dim3(NT), 0, c.stream, A, static_cast<const double*>(c.b),
                      static_cast<const double*>(c.sol), c.r, c.partB, c.partC);
   hipLaunchKernelGGL(k_reduce2, dim3(1), dim3(NT), 0, c.stream, static_cast<const double*>(c.partB),
-                     static_cast<const double*>(c.partC), L.grid, c.red_out);
+                     static_cast<const double*>(c.partC), L.grid, c.red_out, ctl, c.st);
 }
 
 void residual64(Context& c, double& rr, double& bb, bool track) {
@@ -4458,9 +4477,9 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   }
   ResidentTurn turn(c.device);
   if (!turn) return false;
-  auto kernel = k_mixed_resident<AMG, AMG ? 20 : 32, 2>;
+  auto kernel = c.drilling ? k_mixed_resident<AMG, AMG ? 20 : 32, 2, true> : k_mixed_resident<AMG, AMG ? 20 : 32, 2>;
   size_t lds = resident_lds(kernel, grid, 1);
-  if (lds == 0 && !AMG) {
+  if (lds == 0 && !AMG && !c.drilling) {
     kernel = k_mixed_resident<false, 16, 4>;
     lds = resident_lds(kernel, grid, 2);
   }
@@ -4530,7 +4549,7 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   A.have_r = (c.learned_pending && learned_resolve(c, A.rr, A.bb)) ? 1 : 0;
   A.ctl = c.res_ctl;
   A.bytes = static_cast<uint32_t>(lds);
-  hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, c.stream, c.res_ctl, c.st32);
+  hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, c.stream, c.res_ctl, c.st32, c.drill);
   tracked(c, MPS_K_CG_SPMV32, 0.0, [&] {
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(NT), lds, c.stream, A);
   });
@@ -4540,6 +4559,7 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   MPS_HIP(hipStreamSynchronize(c.stream));
   collect_events(c);
   c.rec_ready = false;
+  turn.ended(c.res_host[1] == 0);
   if (c.res_host[1]) {
     c.res_skip = kResSkip;
     return false;
@@ -5743,7 +5763,8 @@ __global__ void k_status_clear(CgStatus* st) {
 }
 
 void csr_solve(size_t n, const uint64_t* rowptr, const uint32_t* col, const double* val, const double* b,
-               double* x, double eps, long long max_iter, hipStream_t s, int dev, double* work, long long* iters_out) {
+               double* x, double eps, long long max_iter, hipStream_t s, int dev, double* work, const ResidentDrill* drill,
+               long long* iters_out) {
   double* r = work;
   double* p = r + kNoAllocMaxRows;
   double* q = p + kNoAllocMaxRows;
@@ -5763,11 +5784,12 @@ void csr_solve(size_t n, const uint64_t* rowptr, const uint32_t* col, const doub
       hipLaunchKernelGGL(k_cg_init<Csr>, dim3(L.grid), dim3(NT), 0, s, A, b, static_cast<const double*>(x), r, partB,
                          partC);
       if (resident_cg_launch(A, L, x, r, p, q, static_cast<const double*>(partB), static_cast<const double*>(partC),
-                             st, sr, max_iter, ctl, s)) {
+                             st, sr, max_iter, ctl, drill, s)) {
         unsigned head[2] = {0, 0};
         MPS_HIP(hipMemcpyAsync(head, ctl, sizeof head, hipMemcpyDeviceToHost, s));
         MPS_HIP(hipMemcpyAsync(&hs, st, sizeof(CgStatus), hipMemcpyDeviceToHost, s));
         MPS_HIP(hipStreamSynchronize(s));
+        turn.ended(head[1] == 0);
         if (!head[1]) {
           if (iters_out) *iters_out = hs.iterations;
           if (!hs.converged)
@@ -5819,10 +5841,9 @@ void put_err(char* err, size_t len, const char* msg) {
 }  // namespace
 }  // namespace mps
 
-extern "C" int mps_cg_solve_csr_noalloc(int device, size_t n, const uint64_t* rowptr, const uint32_t* col,
-                                        const double* val, const double* b, double* x,
-                                        double allowable_residual, int64_t max_iter, void* stream,
-                                        int64_t* iterations, char* err, size_t err_len) {
+static int csr_entry(int device, size_t n, const uint64_t* rowptr, const uint32_t* col, const double* val,
+                     const double* b, double* x, double allowable_residual, int64_t max_iter, void* stream,
+                     const mps::ResidentDrill* drill, int64_t* iterations, char* err, size_t err_len) {
   using namespace mps;
   put_err(err, err_len, "");
   if (iterations) *iterations = 0;
@@ -5846,7 +5867,7 @@ extern "C" int mps_cg_solve_csr_noalloc(int device, size_t n, const uint64_t* ro
     MPS_HIP(hipSetDevice(device));
     double* work = scratch_ptr(device);
     csr_solve(n, rowptr, col, val, b, x, allowable_residual, max_iter > 0 ? max_iter : static_cast<long long>(n),
-              static_cast<hipStream_t>(stream), device, work, reinterpret_cast<long long*>(iterations));
+              static_cast<hipStream_t>(stream), device, work, drill, reinterpret_cast<long long*>(iterations));
   } catch (Failure& f) {
     if (f.code == MPS_ERR_HIP) (void)hipGetLastError();
     put_err(err, err_len, f.msg.c_str());
@@ -5854,4 +5875,44 @@ extern "C" int mps_cg_solve_csr_noalloc(int device, size_t n, const uint64_t* ro
   }
   if (prev >= 0 && prev != device) (void)hipSetDevice(prev);
   return rc;
+}
+
+extern "C" int mps_cg_solve_csr_noalloc(int device, size_t n, const uint64_t* rowptr, const uint32_t* col,
+                                        const double* val, const double* b, double* x,
+                                        double allowable_residual, int64_t max_iter, void* stream,
+                                        int64_t* iterations, char* err, size_t err_len) {
+  return csr_entry(device, n, rowptr, col, val, b, x, allowable_residual, max_iter, stream, nullptr, iterations, err,
+                   err_len);
+}
+
+// ---- rehearsals of given-up resident solves (for tests; not in mps.h) ----
+//
+// d[0..4]: the limits of the wait for the start and of one exchange, the time a
+// workgroup holds back (ticks of 10 ns, at most the ordinary limit of an exchange),
+// the workgroup and the exchange before which it does.
+static mps::ResidentDrill resident_drill(const int64_t* d) {
+  auto ticks = [](int64_t t) { return static_cast<long long>(std::min<int64_t>(std::max<int64_t>(t, 0), mps::kResWaitTicks)); };
+  return mps::ResidentDrill{ticks(d[0]), ticks(d[1]), ticks(d[2]), static_cast<unsigned>(d[3]),
+                            static_cast<unsigned>(d[4])};
+}
+// The context's resident solves from now on (d null: the ordinary ones again, and no
+// solve left out because of an earlier refusal).
+extern "C" int mps_drill_resident(mps_ctx* ctx, const int64_t* d) {
+  if (!ctx) return MPS_ERR_BAD_ARG;
+  ctx->c.drilling = d != nullptr;
+  if (d) ctx->c.drill = resident_drill(d);
+  else ctx->c.res_skip = 0;
+  return MPS_OK;
+}
+// mps_cg_solve_csr_noalloc on the default stream with a drill.
+extern "C" int mps_drill_csr(const int64_t* d, int device, size_t n, const uint64_t* rowptr, const uint32_t* col,
+                             const double* val, const double* b, double* x, double allowable_residual,
+                             int64_t* iterations, char* err, size_t err_len) {
+  const mps::ResidentDrill drill = resident_drill(d);
+  return csr_entry(device, n, rowptr, col, val, b, x, allowable_residual, 0, nullptr, &drill, iterations, err, err_len);
+}
+// Resident solves of this process on a device: ended, and given up or refused by the device.
+extern "C" void mps_resident_counts(int device, int64_t* solved, int64_t* given_up) {
+  *solved = mps::g_resident_solved[device];
+  *given_up = mps::g_resident_given_up[device];
 }

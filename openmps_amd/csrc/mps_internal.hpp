@@ -65,6 +65,14 @@ struct Counters {
 struct ResidentCtl;  // mps_resident.hpp
 constexpr size_t kResHead = 384;  // its head and results, read by the host after a solve
 
+// Rehearsal of the ways in which resident workgroups give a solve up (tests only; a
+// solve with a drill runs instantiations of its own): the limits of their waits in
+// ticks of 10 ns, and one workgroup that holds back before one exchange.
+struct ResidentDrill {
+  long long start_ticks, wait_ticks, hold_ticks;
+  unsigned hold_group, hold_generation;
+};
+
 constexpr int kAmgMaxLevels = 20;  // grid levels of the cell-grid multigrid
 
 constexpr int kFeat = 132;     // warm-start feature width
@@ -316,6 +324,8 @@ struct Context {
   // up), and how many solves not to try after one was refused
   ResidentCtl* res_ctl = nullptr;
   unsigned* res_host = nullptr;  // pinned, kResHead bytes
+  bool drilling = false;
+  ResidentDrill drill{};
   int res_skip = 0;
   bool solve_ended = false;  // solve_b was recorded by the solver (a residual follows it)
 
@@ -549,7 +559,8 @@ void ppe_solve(Context& c);              // mps_cg.hip
 void settle_solve(Context& c);           // mps_cg.hip: the last solve's time into stats (first use)
 void residual64(Context& c, double& rr, double& bb, bool track);
 void reduce2(Context& c, const double* a, const double* b, int nparts);  // -> c.red_host[0..1]
-void residual64_launch(Context& c);  // r = b - A x; |r|^2, |b|^2 -> c.red_out[0..1] (no sync)
+// r = b - A x; |r|^2, |b|^2 -> c.red_out[0..1] (no sync); ctl: of the resident solve before it
+void residual64_launch(Context& c, const ResidentCtl* ctl = nullptr);
 struct FeatRec;
 bool learned_residual32(Context& c, FeatRec* rec);  // mps_cg.hip: see there
 void ml_setup_ahead(Context& c);  // mps_cg.hip: the multilevel set-up on the auxiliary stream

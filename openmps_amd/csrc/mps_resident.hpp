@@ -49,7 +49,8 @@ constexpr int kResWords64 = 4;  // values of one slot at most (a line holds 8)
 struct ResidentCtl {
   unsigned started;
   unsigned abort;
-  unsigned pad[30];
+  ResidentDrill drill;
+  unsigned pad[22];
   long long out[32];  // results of a solve (read by the host together with the head)
   unsigned long long slot[kResRing][kResSlots * kResPitch];
 };
@@ -61,6 +62,9 @@ static_assert(offsetof(ResidentCtl, slot) == kResHead, "what the host reads");
 // generation (2 s: only a lost workgroup gets there).
 constexpr long long kResStartTicks = 500000;
 constexpr long long kResWaitTicks = 200000000;
+struct Patience {
+  long long start, wait;
+};
 
 template <class T>
 __device__ __forceinline__ T agent_load(const T* p) {
@@ -73,9 +77,25 @@ __device__ __forceinline__ void agent_store(T* p, T v) {
 // The wavefront's stores have completed at their destination.
 __device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+template <bool DRILL>
+__device__ __forceinline__ Patience resident_patience(const ResidentCtl* c) {
+  if constexpr (DRILL) return Patience{c->drill.start_ticks, c->drill.wait_ticks};
+  return Patience{kResStartTicks, kResWaitTicks};
+}
+// Before the stores of generation g: the workgroup that a drill holds back.
+template <bool DRILL>
+__device__ __forceinline__ void resident_hold(const ResidentCtl* c, unsigned g, unsigned idx) {
+  if constexpr (DRILL) {
+    if (g != c->drill.hold_generation || idx != c->drill.hold_group) return;
+    const long long t0 = wall_clock64(), t = c->drill.hold_ticks;
+    while (wall_clock64() - t0 < t) {
+    }
+  }
+}
+
 // Block-uniform; every thread calls it.  True once all workgroups of the grid
 // have started and none has refused (ok == false).
-__device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok) {
+__device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok, const Patience& w) {
   __shared__ int s_go;
   if (threadIdx.x == 0) {
     if (!ok) {
@@ -86,7 +106,7 @@ __device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok) {
     const long long t0 = wall_clock64();
     int go = 1;
     while (agent_load(&c->started) < gridDim.x) {
-      if (agent_load(&c->abort) || wall_clock64() - t0 > kResStartTicks) {
+      if (agent_load(&c->abort) || wall_clock64() - t0 > w.start) {
         agent_store(&c->abort, 1u);
         go = 0;
         break;
@@ -123,14 +143,15 @@ __device__ __forceinline__ const double* resident_slot(const ResidentCtl* c, uns
   return reinterpret_cast<const double*>(&c->slot[g % kResRing][k * kResPitch + word]);
 }
 // It once it is published; ok: false if the wait was given up.
-__device__ __forceinline__ double resident_word(ResidentCtl* c, unsigned g, unsigned k, int word, bool& ok) {
+__device__ __forceinline__ double resident_word(ResidentCtl* c, unsigned g, unsigned k, int word, bool& ok,
+                                                const Patience& w) {
   const unsigned long long* s = &c->slot[g % kResRing][k * kResPitch + word];
   unsigned long long b = agent_load(s);
   if (b == kResEmpty) {
     const long long t0 = wall_clock64();
     do {
       b = agent_load(s);
-      if (b == kResEmpty && (agent_load(&c->abort) || wall_clock64() - t0 > kResWaitTicks)) {
+      if (b == kResEmpty && (agent_load(&c->abort) || wall_clock64() - t0 > w.wait)) {
         agent_store(&c->abort, 1u);
         ok = false;
         break;
@@ -142,7 +163,7 @@ __device__ __forceinline__ double resident_word(ResidentCtl* c, unsigned g, unsi
 
 // Values word and word + 1 of workgroup k's slot, polled together.
 __device__ __forceinline__ void resident_words(ResidentCtl* c, unsigned g, unsigned k, int word, bool& ok, double& v0,
-                                               double& v1) {
+                                               double& v1, const Patience& w) {
   const unsigned long long* s = &c->slot[g % kResRing][k * kResPitch + word];
   unsigned long long a = agent_load(s), b = agent_load(s + 1);
   if (a == kResEmpty || b == kResEmpty) {
@@ -151,7 +172,7 @@ __device__ __forceinline__ void resident_words(ResidentCtl* c, unsigned g, unsig
       a = agent_load(s);
       b = agent_load(s + 1);
       if ((a == kResEmpty || b == kResEmpty) &&
-          (agent_load(&c->abort) || wall_clock64() - t0 > kResWaitTicks)) {
+          (agent_load(&c->abort) || wall_clock64() - t0 > w.wait)) {
         agent_store(&c->abort, 1u);
         ok = false;
         break;
@@ -181,7 +202,7 @@ __device__ __forceinline__ void flag_clear(double* p) {
 __device__ __forceinline__ void flag_store(double* p, double v) { agent_store(p, v != v ? __builtin_nan("") : v); }
 // Entries p[0 .. N) once they are there; ok: false if the wait was given up.
 template <int N, class T>
-__device__ __forceinline__ void flag_wait(ResidentCtl* c, const T* const (&p)[N], T (&v)[N], bool& ok) {
+__device__ __forceinline__ void flag_wait(ResidentCtl* c, const T* const (&p)[N], T (&v)[N], bool& ok, const Patience& w) {
   auto look = [&] {
     bool there = true;
 #pragma unroll
@@ -193,7 +214,7 @@ __device__ __forceinline__ void flag_wait(ResidentCtl* c, const T* const (&p)[N]
   if (look()) return;
   const long long t0 = wall_clock64();
   while (!look())
-    if (agent_load(&c->abort) || wall_clock64() - t0 > kResWaitTicks) {
+    if (agent_load(&c->abort) || wall_clock64() - t0 > w.wait) {
       agent_store(&c->abort, 1u);
       ok = false;
       return;
@@ -209,10 +230,11 @@ __device__ __forceinline__ void resident_empty(ResidentCtl* c, unsigned g, unsig
 
 // Clears the control block (and whatever `extra` words of a status) before a
 // resident launch: one launch of kResSlots threads.
-__device__ __forceinline__ void resident_clear(ResidentCtl* c) {
+__device__ __forceinline__ void resident_clear(ResidentCtl* c, const ResidentDrill& drill) {
   if (threadIdx.x == 0) {
     c->started = 0;
     c->abort = 0;
+    c->drill = drill;
   }
   for (int g = 0; g < kResRing; g++)
     for (int k = threadIdx.x; k < kResSlots; k += blockDim.x)
