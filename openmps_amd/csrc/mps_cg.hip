@@ -814,7 +814,7 @@ __device__ __forceinline__ double resident_sum(ResidentCtl* ctl, unsigned gen, u
 // REG on that fit.
 template <class M, int REG, int WAVES, bool DRILL = false>
 __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restrict__ x, double* r, double* p,
-                                                           double* __restrict__ q,
+                                                           double* __restrict__ x0,
                                                            const double* __restrict__ part_rr,
                                                            const double* __restrict__ part_bb, CgStatus* st,
                                                            StopRule sr, long long max_iter, ResidentCtl* ctl,
@@ -862,6 +862,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   }
   const double dg = in ? row.diag() : 0.0;
   double ri = in ? r[i] : 0.0, xi = in ? x[i] : 0.0, pi = 0.0, qi = 0.0;
+  if (in) x0[i] = xi;  // x as it was, for the caller if the solve is given up
   double rr = scalar_of(block_sum<NT>(threadIdx.x < G ? part_rr[threadIdx.x] : 0.0, lds));
   double rr_prev = 0.0, bb = 0.0, tol = 0.0;
   if (sr.rule == MPS_STOP_RHS_NORM) bb = scalar_of(block_sum<NT>(threadIdx.x < G ? part_bb[threadIdx.x] : 0.0, lds));
@@ -973,11 +974,10 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
     gen++;
     if (!ok) return;
   }
-  if (in) r[i] = ri;
   if (in) {
     x[i] = xi;
+    r[i] = ri;
     p[i] = pi;
-    q[i] = qi;
   }
   if (lead()) {
     st->rr[it & 1] = rr;
@@ -2687,7 +2687,7 @@ struct MixedArgs {
   unsigned rows;  // workgroups that have rows
   Sell<double> A;
   const double* b;
-  double *x, *r64;
+  double *x, *x0, *r64;
   const uint32_t* len;
   const uint2* pos;
   const float* ghost;
@@ -2907,6 +2907,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
   }
   const float ghost = in ? A.ghost[i] : 0.0f;
   double x = in ? A.x[i] : 0.0;
+  if (in) A.x0[i] = x;  // as in k_cg_resident
   if (in) agent_store(A.z + i, 0.0f);  // rows outside every cell keep z = 0
 
   // ---- cells ----
@@ -3730,9 +3731,10 @@ size_t resident_lds(K kernel, int grid, int per_cu) {
 
 // Launches the resident CG on stream s (r, the partial sums of r.r and b.b
 // from k_cg_init already enqueued; ctl and st cleared by it); false if it
-// cannot run.  The result is in st (ctl->abort: nothing was solved).
+// cannot run.  The result is in st; ctl->abort: it was given up, x may be that of some
+// rows, and x0 holds it as it was (restore_x).
 template <class M>
-bool resident_cg_launch(const M& A, const Launch& L, double* x, double* r, double* p, double* q, const double* part_rr,
+bool resident_cg_launch(const M& A, const Launch& L, double* x, double* r, double* p, double* x0, const double* part_rr,
                         const double* part_bb, CgStatus* st, const StopRule& sr, long long max_iter, ResidentCtl* ctl,
                         const ResidentDrill* drill, hipStream_t s) {
   if (L.rpb != static_cast<size_t>(NT)) return false;  // one row per thread
@@ -3744,10 +3746,16 @@ bool resident_cg_launch(const M& A, const Launch& L, double* x, double* r, doubl
   }
   if (lds == 0) return false;
   hipLaunchKernelGGL(k_resident_clear, dim3(1), dim3(NT), 0, s, ctl, st, drill ? *drill : ResidentDrill{});
-  hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(NT), lds, s, A, x, r, p, q, part_rr, part_bb, st, sr, max_iter, ctl,
+  hipLaunchKernelGGL(kernel, dim3(L.grid), dim3(NT), lds, s, A, x, r, p, x0, part_rr, part_bb, st, sr, max_iter, ctl,
                      static_cast<uint32_t>(lds));
   check_launch();
   return true;
+}
+
+// After a solve that was given up: the launched kernels start from the caller's x, so
+// that their target is the one that was asked for.
+void restore_x(double* x, const double* x0, size_t n, hipStream_t s) {
+  MPS_HIP(hipMemcpyAsync(x, x0, n * sizeof(double), hipMemcpyDeviceToDevice, s));
 }
 
 // The start of the FP64 CG: r = b - A x and the partial sums of r.r and b.b.
@@ -3797,6 +3805,7 @@ bool resident_cg64(Context& c, const Sell<double>& A, const Launch& L, const Sto
   collect_events(c, c.st_host->converged ? c.st_host->iterations : 0x7fffffffffffffffLL);
   turn.ended(c.st_host->ran != 0);
   if (!c.st_host->ran) {
+    restore_x(c.sol, c.q, c.ppe_n, c.stream);
     c.res_skip = kResSkip;
     return false;
   }
@@ -4491,6 +4500,7 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   A.A = sell<double>(c, c.sval, c.diag, L.rpb);
   A.b = c.b;
   A.x = c.sol;
+  A.x0 = c.q;
   A.r64 = c.r;
   A.len = c.row_len;
   A.pos = c.qpos;
@@ -4561,6 +4571,7 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   c.rec_ready = false;
   turn.ended(c.res_host[1] == 0);
   if (c.res_host[1]) {
+    restore_x(c.sol, c.q, n, c.stream);
     c.res_skip = kResSkip;
     return false;
   }
@@ -5797,6 +5808,7 @@ void csr_solve(size_t n, const uint64_t* rowptr, const uint32_t* col, const doub
           return;
         }
         hs = CgStatus{};
+        restore_x(x, q, n, s);
       }
     }
   }

@@ -10,6 +10,8 @@ import pytest
 import cases
 from openmps_amd import _lib as L
 from test_gpu_resident import EPS, banded
+from test_gpu_resident_mixed import TOL, make, scene
+from test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +72,64 @@ def test_last_exchange_left_by_all_but_the_first(n, reach):
     assert how == (0, 1)
     # (the bound of test_gpu_resident.py)
     assert res <= 1.01 * EPS + 1e-12 * np.linalg.norm(b) / np.linalg.norm(b - A @ x0)
+
+
+@pytest.mark.parametrize("group", [0, 3])
+@pytest.mark.parametrize("n,reach", [(4000, 200), (100_000, 300)])
+def test_x_of_a_solve_given_up(n, reach, group):
+    """The workgroup that holds back before the last exchange stores its rows
+    of x, the others do not: the launched kernels start from x as it was, and
+    return what they (and the resident solve) return from there, bit for bit."""
+    solve, A, b, x0 = matrix(n, reach)
+    x, its, how = solve()
+    assert how == (1, 0)
+    y, its2, how = solve(group=group, exchange=2 * its - 1)
+    assert how == (0, 1)
+    assert its2 == its and np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("group", [0, 3])
+@pytest.mark.parametrize("n,reach", [(4000, 200), (100_000, 300)])
+def test_x_of_a_csr_solve_given_up(n, reach, group):
+    A, b, x0, _ = banded(n, reach, 9, 0, n)
+    hip = Hip()
+    mat = [hip.put(A.indptr.astype(np.uint64)), hip.put(A.indices.astype(np.uint32)), hip.put(A.data), hip.put(b)]
+    lib = hooks()
+    p = ctypes.c_void_p
+    lib.mps_drill_csr.argtypes = [ctypes.POINTER(ctypes.c_int64), ctypes.c_int, ctypes.c_size_t, p, p, p, p, p,
+                                  ctypes.c_double, ctypes.POINTER(ctypes.c_int64), ctypes.c_char_p, ctypes.c_size_t]
+
+    def solve(**kw):
+        x, it, err, was = hip.put(x0), ctypes.c_int64(-1), ctypes.create_string_buffer(256), counts()
+        rc = lib.mps_drill_csr(numbers(**kw), 0, n, *mat, x, EPS, ctypes.byref(it), err, 256)
+        assert rc == L.MPS_OK, err.value.decode()
+        return hip.get(x, x0), it.value, solved(was)
+
+    x, its, how = solve(wait=200 * MS, hold=0)
+    assert how == (1, 0)
+    y, its2, how = solve(group=group, exchange=2 * its - 1)
+    hip.free()
+    assert how == (0, 1)
+    assert its2 == its and np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("prec", ["ml", "amg"])
+@pytest.mark.parametrize("cols,rows", [(20, 40), (127, 253)])
+def test_x_of_a_refinement_given_up(prec, cols, rows):
+    """Given up after at least one sweep has been added to x: the launched
+    solve runs the sweeps that the resident one runs from the start."""
+    def step(**kw):
+        c = make(scene(cols, rows, 2.1, 3.1, False), prec)
+        drill(c, **kw)
+        was = counts()
+        c.forward_time(1e-4)
+        st = c.solve_stats()
+        return c.aux("ppe_x"), [st[k] for k in ("iterations", "outer_iterations", "rr0", "rr")], solved(was)
+
+    x, st, how = step()
+    assert how == (1, 0) and st[1] >= 2
+    # two exchanges an iteration (the multigrid: three at least), some more a sweep: past the first sweep, before the end
+    y, st2, how = step(exchange=(2 if prec == "ml" else 3) * st[0] - 4)
+    print(f"  {prec}: {st}, launched {st2}", flush=True)
+    assert how == (0, 1)
+    assert st2 == st and np.array_equal(x, y)
