@@ -3693,8 +3693,10 @@ struct ResidentTurn {
     int idle = 0;
     if (d >= 0 && d < kMaxDevices && g_resident_busy[d].compare_exchange_strong(idle, 1)) dev = d;
   }
-  ~ResidentTurn() {
+  ~ResidentTurn() { leave(); }
+  void leave() {
     if (dev >= 0) g_resident_busy[dev].store(0);
+    dev = -1;
   }
   // what became of the launched solve
   void ended(bool solved) const { (solved ? g_resident_solved : g_resident_given_up)[dev]++; }
@@ -4570,20 +4572,22 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   collect_events(c);
   c.rec_ready = false;
   turn.ended(c.res_host[1] == 0);
+  turn.leave();  // (to the fallback's CG, or another's)
   if (c.res_host[1]) {
     restore_x(c.sol, c.q, n, c.stream);
     c.res_skip = kResSkip;
     return false;
   }
-  c.solve_ended = true;
   c.replay_ready = MPS_K_CG_SPMV32;
   MixedResult r;
   std::memcpy(&r, reinterpret_cast<const char*>(c.res_host) + offsetof(ResidentCtl, out), sizeof r);
   for (int k = 0; k < Context::kSweepPred; k++) c.pred(k) = r.pred[k];
-  if (r.stalled && !r.done && r.rr == r.rr && r.total < A.total_cap)
-    refine_fallback(c, sr, r.rr0, r.rr, r.total, r.outer);
-  else
+  if (r.stalled && !r.done && r.rr == r.rr && r.total < A.total_cap) {
+    refine_fallback(c, sr, r.rr0, r.rr, r.total, r.outer);  // (the solve ends with it)
+  } else {
+    c.solve_ended = true;
     refine_finished(c, r.done != 0, r.total, r.outer, r.rr0, r.rr, r.bb);
+  }
   return true;
 }
 

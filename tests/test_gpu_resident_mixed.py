@@ -92,3 +92,22 @@ def test_target_below_rounding(prec):
     c.forward_time(1e-4)
     st = c.solve_stats()
     assert st["fallback"] == 1 and st["outer_iterations"] >= 3
+
+
+@pytest.mark.parametrize("prec", ["ml", "amg"])
+@pytest.mark.parametrize("cols,rows", [(20, 40), (127, 253)])
+def test_fallback_is_part_of_the_solve(prec, cols, rows):
+    """The plain CG that finishes a stalled refinement: its time is in solve_ms,
+    and the refinement holds nothing that keeps it from running resident."""
+    c = make(scene(cols, rows, 2.1, 3.1, False), prec)
+    c.set_solver(kind=L.SOLVER_MIXED_IR, stop_rule=L.STOP_RHS_NORM, precond=PREC[prec], tol=1e-25)
+    c.set_profiling(True)
+    c.forward_time(1e-4)
+    st, k = c.solve_stats(), c.kernel_stats()
+    # both are launches between the solve's two events
+    inside = k["cg_spmv32"]["ms"] + k["cg_spmv"]["ms"]
+    print(f"  {prec}: solve {st['solve_ms']:.3f} ms, its kernels {inside:.3f} ms, launches {k['cg_spmv']['launches']}",
+          flush=True)
+    assert st["fallback"] == 1
+    assert st["solve_ms"] >= inside
+    assert k["cg_spmv"]["launches"] == 1 and k["cg_update"]["launches"] == 0
