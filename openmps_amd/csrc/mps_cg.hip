@@ -4212,11 +4212,20 @@ void enqueue_block_list(Context& c, bool copy) {
 namespace {
 bool block_list_ready(const Context& c) { return c.ml_list_serial == c.search_serial; }
 
+// Returns with the list's length on the host.  The search has waited for a list of
+// its own; one that a set-up enqueued (the solver was changed after the search) may
+// still be on its way, also from the auxiliary stream, which c.stream waits for by now.
+void block_list_length(Context& c) {
+  if (c.ml_count_serial == c.search_serial) return;
+  MPS_HIP(hipStreamSynchronize(c.stream));
+  c.ml_count_serial = c.search_serial;
+}
+
 // The multilevel solver's set-up on c.stream, which does not depend on the
 // initial guess: Jacobi factors, the aggregate sums of A from the FP64 system
 // (row sums in z, r, d as scratch, unless the fill of this system summed the
 // rows already), and the list of the 4x4 cell blocks that hold particles (its
-// length reaches the host with the solver's first synchronisation).
+// length: block_list_length).
 void ml_setup(Context& c) {
   const size_t n = c.ppe_n;
   const Launch L = cg_grid(n);
@@ -4597,12 +4606,10 @@ void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max
   ensure_zrec(c, n);
   const MatFreeRec A = matfree_rec(c, L.rpb);
   float* const zval = reinterpret_cast<float*>(c.zrec) + 2;  // z_i at zval[4 i]
-  const bool listed = block_list_ready(c);  // the search listed the blocks
   if (!join_ml_setup(c)) ml_setup(c);  // enqueued ahead on the auxiliary stream, or now
-  if (listed) {
-    pack_slots(c, false);
-    if (resident_mixed<false>(c, sr, max_iter)) return;
-  }
+  block_list_length(c);
+  pack_slots(c, false);
+  if (resident_mixed<false>(c, sr, max_iter)) return;
   const MlGeom g = ml_geom(c);
   const size_t stride = c.part_ml_cap;
   const CellGrid G = ml_grid(c, g);
@@ -4613,31 +4620,20 @@ void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max
   check_launch();
   double* p_pq = c.part3b;
   const long long limit = inner_limit(c, max_iter);
+  const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
+  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
   // per particle: r (read, written), q, z; per slot of the packed layout: id
-  // and Jacobi factor; per lane: the aggregate scales (set once nact is known)
-  double b_prec = n * 16.0;
-  uint32_t nact = 0;
-  size_t pgrid = 1;
-  bool packed = listed;
+  // and Jacobi factor; per lane: the aggregate scales
+  const double b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
   auto prec = [&](double norm, long long it) {
     const PrecArgs a{G,      c.ml_list, nact,   c.ml_pid, c.ml_dv, c.ml_sc,   c.r,       1.0 / norm,
                      c.r32,  c.d32,     c.q32,  c.dinv32, zval,    4u,        p_pq,      L.grid,
                      c.part_ml, stride, c.st32};
     hipLaunchKernelGGL(k_ml_prec<0>, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, a, it);
   };
-  double b_spmv = b_base;
+  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
   c.replay_ready = MPS_K_CG_SPMV32;
   refine(c, sr, [&](double norm, double sweep_tol) {
-    // refine() has synchronised the stream (residual) before every sweep: the
-    // block count and the wide nnz are on the host
-    nact = static_cast<uint32_t>(c.counters_host->ml_active);
-    b_spmv = b_base + 2.0 * mf_nnz_wide(c);
-    pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
-    b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
-    if (!packed) {
-      pack_slots(c, false);
-      packed = true;
-    }
     MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
     tracked(c, MPS_K_CG_INIT32, n * 25.0, [&] { prec(norm, 0); });
     long long launched = 0;
@@ -4673,7 +4669,6 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   ensure_zrec(c, n);
   const MatFreeRec A = matfree_rec(c, L.rpb);
   float* const zval = reinterpret_cast<float*>(c.zrec) + 2;  // z_i at zval[4 i]
-  const bool listed = block_list_ready(c);  // the search listed the blocks
   amg_setup(c);
   clear_direction_sums(c);
   const MlGeom g = ml_geom(c);
@@ -4682,10 +4677,9 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
   }
-  if (listed) {
-    pack_slots(c, true);
-    if (resident_mixed<true>(c, sr, max_iter)) return;
-  }
+  block_list_length(c);
+  pack_slots(c, true);
+  if (resident_mixed<true>(c, sr, max_iter)) return;
   const size_t stride = c.part_ml_cap;
   const CellGrid G = ml_grid(c, g);
   hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
@@ -4694,15 +4688,14 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   check_launch();
   double* p_pq = c.part3b;
   const long long limit = inner_limit(c, max_iter);
-  uint32_t nact = 0;
-  size_t pgrid = 1;
-  bool packed = listed;
+  const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
+  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
   // per pass over the particles (k_ml_prec<1>, then k_ml_prec<2>): r, q or z
   // per particle, the packed ids and Jacobi factors per slot, P_s's rows (18
   // bytes per particle); the cycle: level 0's direction sums written and
   // gathered (9 + 9 + 1 floats per point), then r, x, e and the stencils of
   // every level, twice
-  double b_pass = n * 30.0;
+  const double b_pass = n * 30.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 8);
   const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
   const double b_cycle = static_cast<double>(c.amg_pts) * 2 * (36 + 16) + npts0 * 19.0 * 4;
   const size_t tq_stride = c.amg_tq_stride;
@@ -4737,19 +4730,9 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
         hipLaunchKernelGGL(k_ml_prec<2>, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, a, it);
     });
   };
-  double b_spmv = b_base;
+  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
   c.replay_ready = MPS_K_CG_SPMV32;
   refine(c, sr, [&](double norm, double sweep_tol) {
-    // refine() has synchronised the stream before every sweep: the block
-    // count and the wide nnz are on the host
-    nact = static_cast<uint32_t>(c.counters_host->ml_active);
-    b_spmv = b_base + 2.0 * mf_nnz_wide(c);
-    pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
-    b_pass = n * 30.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 8);
-    if (!packed) {
-      pack_slots(c, true);
-      packed = true;
-    }
     MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
     tracked(c, MPS_K_CG_INIT32, n * 25.0, [&] { prec(norm, 0); });
     long long launched = 0;
@@ -5614,7 +5597,6 @@ bool batch_amg(const Context& c) { return c.solver.precond == MPS_PRECOND_AMG; }
 void amg_prepare(Context& c) {
   const size_t n = c.ppe_n;
   ensure_zrec(c, n);
-  const bool listed = block_list_ready(c);
   amg_setup(c);
   const MlGeom g = ml_geom(c);
   if (c.part_ml_cap < g.sgrid) {
@@ -5622,7 +5604,7 @@ void amg_prepare(Context& c) {
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
   }
-  if (!listed) MPS_HIP(hipStreamSynchronize(c.stream));  // the count of occupied cell blocks
+  block_list_length(c);
   pack_slots(c, true);
   clear_direction_sums(c);
   hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
@@ -5634,9 +5616,8 @@ void amg_prepare(Context& c) {
 void ml_prepare(Context& c) {
   const size_t n = c.ppe_n;
   ensure_zrec(c, n);
-  const bool listed = block_list_ready(c);
   if (!join_ml_setup(c)) ml_setup(c);
-  if (!listed) MPS_HIP(hipStreamSynchronize(c.stream));  // the count of occupied cell blocks
+  block_list_length(c);
   pack_slots(c, false);
   hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
                      c.zrec, c.r32, c.d32);

@@ -294,6 +294,7 @@ struct Context {
   float4* ml_sc = nullptr;
   size_t ml_pack_cap = 0;      // lanes (64 per listed block)
   long long ml_list_serial = -1;       // search whose cells the list is of
+  long long ml_count_serial = -1;      // search whose list's length is in counters_host
   bool rec_ready = false;              // zrec holds the installed system's positions
   size_t agg_cap = 0;
   size_t agg_off[4] = {0, 0, 0, 0};  // level l at agg_inv + agg_off[l]

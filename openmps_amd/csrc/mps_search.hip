@@ -638,6 +638,7 @@ void search(Context& c) {
   // flags, the lists' length and the block count in one copy (Counters)
   MPS_HIP(hipMemcpyAsync(c.counters_host, c.counters, offsetof(Counters, nnz), hipMemcpyDeviceToHost, c.stream));
   MPS_HIP(hipStreamSynchronize(c.stream));
+  c.ml_count_serial = c.ml_list_serial;
   c.nbr_total = c.counters_host->nbr_total;
   add_bytes(c, MPS_K_NEIGHBORS, 4.0 * c.nbr_total);
   c.have_neighbors = true;

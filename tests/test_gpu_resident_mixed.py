@@ -111,3 +111,50 @@ def test_fallback_is_part_of_the_solve(prec, cols, rows):
     assert st["fallback"] == 1
     assert st["solve_ms"] >= inside
     assert k["cg_spmv"]["launches"] == 1 and k["cg_update"]["launches"] == 0
+
+
+@pytest.mark.parametrize("warm", ["previous", "learned"])
+@pytest.mark.parametrize("prec", ["ml", "amg", "auto"])
+@pytest.mark.parametrize("cols,rows", [(5, 9), (60, 117), (300, 600)])
+def test_solver_chosen_after_the_search(cols, rows, prec, warm):
+    """A search under the FP64 solver lists no blocks of cells for the
+    preconditioners: the set-up of the first mixed solve does, on the auxiliary
+    stream if the learned start runs before it, and the solve has to wait for
+    their number.  Same system, same solver: the same bits as with the solver
+    chosen first, in the first solve and in a second one."""
+    from openmps_amd import learned
+    model = learned.Model(3)
+
+    def run(late):
+        sc = scene(cols, rows, 2.1, 3.1, False)
+        c = Computer(1e-10, sc[0])
+        c.add_particles(sc[1])
+        learned.attach_model(c, model)
+
+        def choose():
+            c.set_solver(kind=L.SOLVER_MIXED_IR, stop_rule=L.STOP_RHS_NORM, tol=TOL,
+                         precond=dict(PREC, auto=L.PRECOND_AUTO)[prec],
+                         warm_start=L.WARM_LEARNED if warm == "learned" else L.WARM_PREVIOUS)
+
+        if not late:
+            choose()
+        c.set_time(1e-4, 1e-4)
+        for stage in ("search", "density", "error_correction", "explicit", "density"):
+            c.stage(stage)
+        if late:
+            choose()
+        out = []
+        for _ in range(2):
+            c.stage("ppe_assemble")
+            c.stage("ppe_solve")
+            st = c.solve_stats()
+            assert st["rel_residual"] <= TOL
+            out.append((c.aux("ppe_x"), st["iterations"], st["precond_used"]))
+        return out
+
+    early, late = run(False), run(True)
+    print(f"  {prec} {warm}: {[v[1:] for v in early]}, chosen late {[v[1:] for v in late]}", flush=True)
+    if prec == "auto":  # (its second choice follows the times of the first)
+        early, late = early[:1], late[:1]
+    for (x, it, used), (x2, it2, used2) in zip(early, late):
+        assert it == it2 and used == used2 and np.array_equal(x, x2)
