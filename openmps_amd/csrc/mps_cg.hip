@@ -582,7 +582,7 @@ __global__ void __launch_bounds__(NT) k_cg_check(const double* __restrict__ part
 // rows fit one per thread of the workgroups that the chip holds at once: each
 // thread keeps x, r, p, q and its row's first REG matrix entries in registers,
 // the next entries (10 bytes each) in LDS as far as it goes, and streams the
-// rest.  A workgroup gathers r into an LDS copy of exactly the rows its columns
+// few that may be left (kResStream).  A workgroup gathers r into an LDS copy of exactly the rows its columns
 // name, every iteration (cell-ordered rows couple to three short ranges of rows,
 // far apart: copying the whole span took 2 us more per iteration at 131k rows).
 // Two exchanges per iteration: p.q, and r.r while the gather waits for the
@@ -629,19 +629,22 @@ struct CsrRow {
 __device__ __forceinline__ SellRow<double> row_of(const Sell<double>& A, size_t i, bool in) { return {A, i, in}; }
 __device__ __forceinline__ CsrRow row_of(const Csr& A, size_t i, bool in) { return {A, i, in}; }
 
-// Smallest and largest value over the block (every thread contributes).
-__device__ __forceinline__ void block_range(uint32_t& lo, uint32_t& hi) {
-  __shared__ uint32_t s[2 * (NT / 64)];
+// The smallest lo, the largest hi and the largest m over the block (every thread contributes).
+__device__ __forceinline__ void block_range(uint32_t& lo, uint32_t& hi, uint32_t& m) {
+  __shared__ uint32_t s[3 * (NT / 64)];
   lo = wave_min_u32(lo);
   hi = wave_max_u32(hi);
+  m = wave_max_u32(m);
   if ((threadIdx.x & 63) == 0) {
     s[threadIdx.x >> 6] = lo;
     s[NT / 64 + (threadIdx.x >> 6)] = hi;
+    s[2 * (NT / 64) + (threadIdx.x >> 6)] = m;
   }
   __syncthreads();
   for (int k = 0; k < NT / 64; k++) {
     lo = min(lo, s[k]);
     hi = max(hi, s[NT / 64 + k]);
+    m = max(m, s[2 * (NT / 64) + k]);
   }
   __syncthreads();
 }
@@ -700,11 +703,11 @@ __device__ __forceinline__ uint32_t number_marked(const Gathered& g) {
 
 // Marks and numbers the rows that a workgroup gathers: the columns col(k), k < m,
 // of every thread's row i and the row itself (in: the thread has a row).  lo:
-// the lowest of them, wn: their number.  Block-uniform; false: they span too
-// many rows.
+// the lowest of them, wn: their number, longest: the largest m.  Block-uniform; false:
+// they span too many rows, or a row is longer than `most`.
 template <class Col>
-__device__ __forceinline__ bool gather_rows(const Gathered& ga, bool in, uint32_t i, uint32_t m, Col col, uint32_t& lo,
-                                            uint32_t& wn) {
+__device__ __forceinline__ bool gather_rows(const Gathered& ga, bool in, uint32_t i, uint32_t m, uint32_t most, Col col,
+                                            uint32_t& lo, uint32_t& wn, uint32_t& longest) {
   lo = in ? i : 0xffffffffu;
   uint32_t hi = in ? i : 0u;
   for (uint32_t k = 0; k < m; k++) {
@@ -713,13 +716,14 @@ __device__ __forceinline__ bool gather_rows(const Gathered& ga, bool in, uint32_
     hi = max(hi, j);
   }
   for (uint32_t k = threadIdx.x; k < kResWords; k += NT) ga.mark[k] = 0u;
-  block_range(lo, hi);
+  longest = m;
+  block_range(lo, hi, longest);
   wn = 0;
   if (hi < lo) {  // no rows at all
     lo = 0;
     return true;
   }
-  if (hi - lo >= kResRange) return false;
+  if (hi - lo >= kResRange || longest > most) return false;
   if (in) ga.set(i - lo);
   for (uint32_t k = 0; k < m; k++) ga.set(col(k) - lo);
   __syncthreads();
@@ -733,6 +737,17 @@ __device__ __forceinline__ void gather_list(const Gathered& ga, uint16_t* list) 
     for (; bits; bits &= bits - 1) list[at++] = static_cast<uint16_t>(32 * w + __ffs(bits) - 1);
   }
 }
+// A row's entries in LDS at most, and those that k_cg_resident may stream every
+// iteration beyond them and the registers'.  Such an entry is a chain of loads and a
+// wait for its r: 0.5 us with one workgroup a compute unit, 1.0 with two, where the
+// launched product takes 0.15 and 0.47.  The lines lie where the two take as long
+// (longest rows, streamed entries, launched and resident us an iteration): one, 2k rows
+// 80 (23) 18.5 / 15.3, 96 (39) 20.9 / 24.2, 132 (75) 27 / 43; 50k 27 / 17, 31 / 26, 41 /
+// 78; two, 166k rows 48 (17) 30 / 28, 68 (37) 38 / 52, 132 67 / 131.  Longer rows
+// are refused on the device.
+constexpr uint32_t kResLdsRows = 64;
+template <int WAVES>
+constexpr uint32_t kResStream = WAVES == 2 ? 24 : 18;
 constexpr uint32_t kMarkBytes = 6 * kResWords;  // marks and numbers, at the start of the dynamic LDS
 
 // The gathered entries of a vector into LDS, as they were published.
@@ -827,42 +842,47 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   const bool in = i < rw.hi;
   const auto row = row_of(A, i, in);
   const uint32_t m = row.m, self = static_cast<uint32_t>(i);
+  double xi = in ? x[i] : 0.0;
+  if (in) x0[i] = xi;  // x as it was, for the caller if the solve is given up
+  const Patience patience = resident_patience<DRILL>(ctl);
   const Gathered ga{reinterpret_cast<uint32_t*>(win), reinterpret_cast<uint16_t*>(win) + 2 * kResWords};
-  uint32_t lo, wn;
-  const bool narrow = gather_rows(ga, in, self, m, [&](uint32_t k) { return row.col(k); }, lo, wn);
+  constexpr uint32_t kOnChip = REG + kResStream<WAVES>;
+  uint32_t lo, wn, longest;
+  const bool narrow =
+      gather_rows(ga, in, self, m, kOnChip + kResLdsRows, [&](uint32_t k) { return row.col(k); }, lo, wn, longest);
   // LDS behind the gathered r: the list of its rows, entries of the matrix
   const uint32_t list_at = max(wn * 8u, kMarkBytes), mat_at = (list_at + 2 * wn + 15u) & ~15u;
-  const bool ok_lds = narrow && mat_at <= bytes;
+  const uint32_t lrows = mat_at <= bytes ? min((bytes - mat_at) / (10u * NT), kResLdsRows) : 0u;
+  if (!narrow || mat_at > bytes || longest > kOnChip + lrows) {
+    (void)resident_start(ctl, false, patience);
+    return;
+  }
   uint16_t* const list = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(win) + list_at);
-  const uint32_t lrows = ok_lds ? min((bytes - mat_at) / (10u * NT), 64u) : 0u;
   double* const lval = reinterpret_cast<double*>(reinterpret_cast<char*>(win) + mat_at);
   uint16_t* const lcol = reinterpret_cast<uint16_t*>(lval + static_cast<size_t>(lrows) * NT);
   const uint32_t kl = min(m, static_cast<uint32_t>(REG) + lrows);  // entries in registers and LDS
   // the row's first entries: values, and columns as their numbers, two a register
   double a[REG];
   uint32_t off[REG / 2];
-  const uint32_t own = (ok_lds && in) ? ga.at(self - lo) : 0u;  // past the row's end: its own r, value 0
+  const uint32_t own = in ? ga.at(self - lo) : 0u;  // past the row's end: its own r, value 0
 #pragma unroll
   for (int k = 0; k < REG; k++) {
     a[k] = 0.0;
     uint32_t d = own;
     if (static_cast<uint32_t>(k) < m) {
       a[k] = row.val(k);
-      if (ok_lds) d = ga.at(row.col(k) - lo);
+      d = ga.at(row.col(k) - lo);
     }
     if (k & 1) off[k >> 1] |= d << 16;
     else off[k >> 1] = d;
   }
-  if (ok_lds) {
-    for (uint32_t k = REG; k < kl; k++) {
-      lval[(k - REG) * NT + threadIdx.x] = row.val(k);
-      lcol[(k - REG) * NT + threadIdx.x] = static_cast<uint16_t>(ga.at(row.col(k) - lo));
-    }
-    gather_list(ga, list);
+  for (uint32_t k = REG; k < kl; k++) {
+    lval[(k - REG) * NT + threadIdx.x] = row.val(k);
+    lcol[(k - REG) * NT + threadIdx.x] = static_cast<uint16_t>(ga.at(row.col(k) - lo));
   }
+  gather_list(ga, list);
   const double dg = in ? row.diag() : 0.0;
-  double ri = in ? r[i] : 0.0, xi = in ? x[i] : 0.0, pi = 0.0, qi = 0.0;
-  if (in) x0[i] = xi;  // x as it was, for the caller if the solve is given up
+  double ri = in ? r[i] : 0.0, pi = 0.0, qi = 0.0;
   double rr = scalar_of(block_sum<NT>(threadIdx.x < G ? part_rr[threadIdx.x] : 0.0, lds));
   double rr_prev = 0.0, bb = 0.0, tol = 0.0;
   if (sr.rule == MPS_STOP_RHS_NORM) bb = scalar_of(block_sum<NT>(threadIdx.x < G ? part_bb[threadIdx.x] : 0.0, lds));
@@ -871,8 +891,7 @@ __global__ void __launch_bounds__(NT, WAVES) k_cg_resident(M A, double* __restri
   if (in) flag_clear(p + i);
   stores_done();
   __syncthreads();
-  const Patience patience = resident_patience<DRILL>(ctl);
-  if (!resident_start(ctl, ok_lds, patience)) return;
+  if (!resident_start(ctl, true, patience)) return;
   unsigned gen = 0;
   long long it = 1;
   bool conv = false, ok = true;
@@ -2863,8 +2882,9 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
   const uint32_t self = static_cast<uint32_t>(i), m = in ? A.len[i] : 0u;
   const SellRow<double> row(A.A, i, in);
   const Gathered ga{reinterpret_cast<uint32_t*>(win), reinterpret_cast<uint16_t*>(win) + 2 * kResWords};
-  uint32_t lo, wn;
-  const bool narrow = gather_rows(ga, in, self, m, [&](uint32_t k) { return row.col(k); }, lo, wn);
+  uint32_t lo, wn, longest;
+  const bool narrow =
+      gather_rows(ga, in, self, m, 0xffffffffu, [&](uint32_t k) { return row.col(k); }, lo, wn, longest);
   // dynamic LDS: the gathered vector (first the marks), the list of its rows, the cycle's levels, matrix entries
   const uint32_t list_at = max(wn * 8u, kMarkBytes), lev_at = (list_at + 2 * wn + 15u) & ~15u;
   const uint32_t mat_at = lev_at + (AMG ? lds_level_bytes(A.lvp, A.lvq, amg_npts(A.g.L[A.g.levels - 1])) : 0u);
