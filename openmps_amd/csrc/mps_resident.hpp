@@ -46,9 +46,12 @@ constexpr int kResPitch = 8;    // a slot per 64-byte line: polls of one slot do
 constexpr unsigned long long kResEmpty = ~0ull;  // no partial sum: NaNs are published as one quiet pattern
 
 constexpr int kResWords64 = 4;  // values of one slot at most (a line holds 8)
+// Why a solve was abandoned: a wait ended at its limit (some workgroups may have gone
+// on), or a workgroup refused the system before any of them started.
+constexpr unsigned kResGivenUp = 1, kResRefused = 2;
 struct ResidentCtl {
   unsigned started;
-  unsigned abort;
+  unsigned abort;  // kResGivenUp, kResRefused
   ResidentDrill drill;
   unsigned pad[22];
   long long out[32];  // results of a solve (read by the host together with the head)
@@ -99,15 +102,19 @@ __device__ __forceinline__ bool resident_start(ResidentCtl* c, bool ok, const Pa
   __shared__ int s_go;
   if (threadIdx.x == 0) {
     if (!ok) {
-      agent_store(&c->abort, 1u);
+      agent_store(&c->abort, kResRefused);
       stores_done();
     }
     __hip_atomic_fetch_add(&c->started, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const long long t0 = wall_clock64();
     int go = 1;
     while (agent_load(&c->started) < gridDim.x) {
-      if (agent_load(&c->abort) || wall_clock64() - t0 > w.start) {
-        agent_store(&c->abort, 1u);
+      if (agent_load(&c->abort)) {
+        go = 0;
+        break;
+      }
+      if (wall_clock64() - t0 > w.start) {
+        agent_store(&c->abort, kResGivenUp);
         go = 0;
         break;
       }
@@ -152,7 +159,7 @@ __device__ __forceinline__ double resident_word(ResidentCtl* c, unsigned g, unsi
     do {
       b = agent_load(s);
       if (b == kResEmpty && (agent_load(&c->abort) || wall_clock64() - t0 > w.wait)) {
-        agent_store(&c->abort, 1u);
+        agent_store(&c->abort, kResGivenUp);
         ok = false;
         break;
       }
@@ -173,7 +180,7 @@ __device__ __forceinline__ void resident_words(ResidentCtl* c, unsigned g, unsig
       b = agent_load(s + 1);
       if ((a == kResEmpty || b == kResEmpty) &&
           (agent_load(&c->abort) || wall_clock64() - t0 > w.wait)) {
-        agent_store(&c->abort, 1u);
+        agent_store(&c->abort, kResGivenUp);
         ok = false;
         break;
       }
@@ -215,7 +222,7 @@ __device__ __forceinline__ void flag_wait(ResidentCtl* c, const T* const (&p)[N]
   const long long t0 = wall_clock64();
   while (!look())
     if (agent_load(&c->abort) || wall_clock64() - t0 > w.wait) {
-      agent_store(&c->abort, 1u);
+      agent_store(&c->abort, kResGivenUp);
       ok = false;
       return;
     }

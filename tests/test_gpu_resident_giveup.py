@@ -88,29 +88,87 @@ def test_x_of_a_solve_given_up(n, reach, group):
     assert its2 == its and np.array_equal(x, y)
 
 
+class CsrSolve:
+    """mps_cg_solve_csr_noalloc on one system, or with a drill (keywords)."""
+
+    def __init__(self, A, b, x0):
+        self.hip, self.n, self.x0 = Hip(), len(b), x0
+        self.args = [self.hip.put(v) for v in (A.indptr.astype(np.uint64), A.indices.astype(np.uint32), A.data, b, x0)]
+        p = ctypes.c_void_p
+        hooks().mps_drill_csr.argtypes = [
+            ctypes.POINTER(ctypes.c_int64), ctypes.c_int, ctypes.c_size_t, p, p, p, p, p, ctypes.c_double,
+            ctypes.POINTER(ctypes.c_int64), ctypes.c_char_p, ctypes.c_size_t]
+
+    def __call__(self, **kw):
+        it, err, was, x = ctypes.c_int64(-1), ctypes.create_string_buffer(256), counts(), self.args[4]
+        assert self.hip.h.hipMemcpy(x, self.x0.ctypes.data, self.x0.nbytes, 1) == 0  # host to device
+        if kw:
+            rc = L.lib().mps_drill_csr(numbers(**kw), 0, self.n, *self.args, EPS, ctypes.byref(it), err, 256)
+        else:
+            rc = L.lib().mps_cg_solve_csr_noalloc(0, self.n, *self.args, EPS, 0, None, ctypes.byref(it), err, 256)
+        assert rc == L.MPS_OK, err.value.decode()
+        return self.hip.get(x, self.x0), it.value, solved(was)
+
+
+@pytest.fixture
+def csr_solves():
+    """Makes CsrSolves; afterwards no refusal is remembered by the process."""
+    made = []
+
+    def make(A, b, x0):
+        made.append(CsrSolve(A, b, x0))
+        return made[-1]
+
+    yield make
+    for s in made:
+        for _ in range(65):
+            how = s()[2]
+            if how != (0, 0):
+                break
+        s.hip.free()
+
+
 @pytest.mark.parametrize("group", [0, 3])
 @pytest.mark.parametrize("n,reach", [(4000, 200), (100_000, 300)])
-def test_x_of_a_csr_solve_given_up(n, reach, group):
+def test_x_of_a_csr_solve_given_up(csr_solves, n, reach, group):
     A, b, x0, _ = banded(n, reach, 9, 0, n)
-    hip = Hip()
-    mat = [hip.put(A.indptr.astype(np.uint64)), hip.put(A.indices.astype(np.uint32)), hip.put(A.data), hip.put(b)]
-    lib = hooks()
-    p = ctypes.c_void_p
-    lib.mps_drill_csr.argtypes = [ctypes.POINTER(ctypes.c_int64), ctypes.c_int, ctypes.c_size_t, p, p, p, p, p,
-                                  ctypes.c_double, ctypes.POINTER(ctypes.c_int64), ctypes.c_char_p, ctypes.c_size_t]
-
-    def solve(**kw):
-        x, it, err, was = hip.put(x0), ctypes.c_int64(-1), ctypes.create_string_buffer(256), counts()
-        rc = lib.mps_drill_csr(numbers(**kw), 0, n, *mat, x, EPS, ctypes.byref(it), err, 256)
-        assert rc == L.MPS_OK, err.value.decode()
-        return hip.get(x, x0), it.value, solved(was)
-
+    solve = csr_solves(A, b, x0)
     x, its, how = solve(wait=200 * MS, hold=0)
     assert how == (1, 0)
     y, its2, how = solve(group=group, exchange=2 * its - 1)
-    hip.free()
     assert how == (0, 1)
     assert its2 == its and np.array_equal(x, y)
+
+
+def test_csr_refusals_are_remembered(csr_solves):
+    """After a refused system the next 1, 2, 4, ... 64 calls of its size are not
+    tried, but other sizes are; after a wait that ended at its limit none of
+    any size.  A resident solve ends either."""
+    from test_gpu_resident_routes import one_long_row
+    long, small, big = (csr_solves(*a) for a in (one_long_row(300, 140), one_long_row(301, 5), banded(4000, 200, 9, 0, 1)[:3]))
+    short = csr_solves(*one_long_row(300, 5))
+    ref = [s(wait=200 * MS, hold=0)[0] for s in (small, big)]
+    x, _, how = long()
+    assert how == (0, 1)
+    for left in (1, 2, 4, 8, 16, 32, 64, 64):
+        for _ in range(left):
+            y, _, how = long()
+            assert how == (0, 0) and np.array_equal(x, y)
+        y, _, how = small()
+        assert how == (1, 0) and np.array_equal(y, ref[0])
+        y, _, how = long()
+        assert how == (0, 1) and np.array_equal(x, y)
+    for _ in range(64):
+        assert short()[2] == (0, 0)
+    assert short()[2] == (1, 0) and short()[2] == (1, 0)
+    assert long()[2] == (0, 1) and long()[2] == (0, 0) and long()[2] == (0, 1)
+    for left in (1, 2):
+        y, _, how = big(group=0, exchange=0)
+        assert how == (0, 1) and np.array_equal(y, ref[1])
+        for k in range(left):
+            y, _, how = (small, big)[k]()
+            assert how == (0, 0) and np.array_equal(y, ref[k])
+    assert small()[2] == (1, 0) and big()[2] == (1, 0)
 
 
 @pytest.mark.parametrize("prec", ["ml", "amg"])
