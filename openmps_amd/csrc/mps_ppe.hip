@@ -295,7 +295,11 @@ struct DirA {
 };
 __device__ __forceinline__ DirA make_pair_da(int dir, double a) { return DirA{dir, a}; }
 
-// One row of k_ppe_fill; kk returns its stored non-zeros.
+// One row of k_ppe_fill; kk returns its stored non-zeros.  Bound by the gathers of the
+// neighbours and the partly written lines; so the walk keeps the columns only, and a
+// row is stored once, ascending (values stored by the walk as well, for rows that
+// turn out ascending, cost the others a second store: 1.00M particles in a kept lattice
+// order 279 -> 345 us, shuffled 1251 -> 1717, 133k shuffled 114 -> 143).
 template <bool ROWS9>
 __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __restrict__ x,
                                          const double* __restrict__ z, const uint8_t* __restrict__ type, NV nb,
@@ -355,12 +359,6 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
                    for (int v = 0; v < 4; v++) {
                      s = l[v] ? s + -a[v] : s;
                      if (l[v]) {
-                       // stored at once, in list order; the merge below writes rows whose
-                       // list is not ascending again
-                       const size_t o = base + static_cast<size_t>(ne) * 64;
-                       val[o] = a[v];
-                       if (wide) col[o] = j[v];
-                       col16[o] = static_cast<int16_t>(static_cast<long long>(j[v]) - static_cast<long long>(self));
                        if (ne == 0 || j[v] < prev) {
                          if (nr < kRuns) {
 #pragma unroll
@@ -387,8 +385,17 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
     // ROWS9: the row's cell when it takes part (its row length is known from the count pass)
     const uint32_t k9 = ROWS9 ? ag.aggkey[i] : kNoCell;
     const int c9x = static_cast<int>(k9 / ag.gnz), c9z = static_cast<int>(k9 % ag.gnz);
-    // the share of a stored entry in the aggregate row sums
-    auto share = [&](uint32_t j, double a) {
+    // value of an emitted column j in slot kk, and its share of the aggregate row sums
+    auto emit = [&](uint32_t j) {
+      const double2 pj = xz[j];
+      const double dx = pj.x - xi, dz = pj.y - zi;
+      const double r = sqrt(dx * dx + dz * dz);
+      const size_t o = base + static_cast<size_t>(kk) * 64;
+      const double a = 3 * k.rl / k.n0l / (r * r * r);
+      val[o] = a;
+      if (wide) col[o] = j;
+      col16[o] = static_cast<int16_t>(static_cast<long long>(j) - static_cast<long long>(self));
+      kk++;
       if (ki != kNoCell) {
         const uint32_t kj = ag.key[j];
         if (kj != kNoCell) {
@@ -408,19 +415,6 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
         if (kj != kNoCell) dir = 3 * (static_cast<int>(kj / ag.gnz) - c9x + 1) + static_cast<int>(kj % ag.gnz) - c9z + 1;
       }
       return make_pair_da(dir, a);
-    };
-    // value of an emitted column j in slot kk (and its share)
-    auto emit = [&](uint32_t j) {
-      const double2 pj = xz[j];
-      const double dx = pj.x - xi, dz = pj.y - zi;
-      const double r = sqrt(dx * dx + dz * dz);
-      const size_t o = base + static_cast<size_t>(kk) * 64;
-      const double a = 3 * k.rl / k.n0l / (r * r * r);
-      val[o] = a;
-      if (wide) col[o] = j;
-      col16[o] = static_cast<int16_t>(static_cast<long long>(j) - static_cast<long long>(self));
-      kk++;
-      return share(j, a);
     };
     // consecutive columns of one direction are summed in a run and the run
     // added to its direction's sum when the direction changes (in cell order
@@ -445,14 +439,10 @@ __device__ __forceinline__ void fill_row(size_t n, size_t i, const double* __res
       }
     };
     if (staged && nr <= 1) {
-      // one ascending run (the particles in cell order: the list visits the
-      // cells, and each cell's members, in ascending index order): stored by
-      // the walk; the sums need the diagonal first, so they read the values back
-      kk = ne;
-      if (ki != kNoCell || k9 != kNoCell) {
+      // one ascending run (a kept order may be one, here or there): the staged
+      // columns in their order
 #pragma unroll 4
-        for (uint32_t v = 0; v < ne; v++) add9(share(stage[v][t], val[base + static_cast<size_t>(v) * 64]));
-      }
+      for (uint32_t v = 0; v < ne; v++) add9(emit(stage[v][t]));
     } else if (staged) {
       // 9-way merge of the staged runs (LDS only on its dependency chain),
       // the ascending columns written first, the values computed after
