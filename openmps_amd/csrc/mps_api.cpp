@@ -663,14 +663,14 @@ int mps_stage_search(mps_ctx* ctx) {
 int mps_stage_density(mps_ctx* ctx) {
   return mps::guard(ctx, [&](Context& c) {
     mps::require_neighbors(c);
-    mps::density(c, false, false, true);
+    mps::density(c, false);
     mps::sync(c);
   });
 }
 int mps_stage_error_correction(mps_ctx* ctx) {
   return mps::guard(ctx, [&](Context& c) {
     mps::require_neighbors(c);
-    mps::density(c, true, false, false);
+    mps::density(c, true);
     mps::sync(c);
   });
 }
@@ -684,7 +684,7 @@ int mps_stage_explicit(mps_ctx* ctx) {
 int mps_stage_save_x(mps_ctx* ctx) {
   return mps::guard(ctx, [&](Context& c) {
     mps::require_neighbors(c);
-    mps::density(c, false, true, false);
+    mps::save_x(c);
     mps::sync(c);
   });
 }

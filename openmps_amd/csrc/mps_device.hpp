@@ -55,13 +55,17 @@ __device__ __forceinline__ bool ghost_pos(double xi, double zi, double sx, doubl
 // ids and fields are loaded before the current group's arithmetic.  (Density
 // and acceleration pass, bound by FP64 issue: 2k particles 23 -> 16 us, 131k 46
 // -> 37, 1.05M 215 -> 180.)
-template <class T, class Load, class Use>
+//
+// What is loaded ahead at a list's end is thrown away: the first group's again, or
+// TIGHT, the particle's own, which costs nothing where gathers miss the caches (a
+// shuffled order) and a few registers.
+template <class T, bool TIGHT = false, class Load, class Use>
 __device__ __forceinline__ void walk_list(uint32_t i, uint32_t m, const uint32_t* __restrict__ ids, uint32_t kmax,
                                           Load load, Use use) {
   if (m == 0) return;
   auto group = [&](uint32_t q, uint32_t j[4]) {
-    const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, q, kmax));
-    j[0] = g.x;
+    const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, !TIGHT || q < m ? q : 0u, kmax));
+    j[0] = (!TIGHT || q < m) ? g.x : i;
     j[1] = (q + 1 < m) ? g.y : i;
     j[2] = (q + 2 < m) ? g.z : i;
     j[3] = (q + 3 < m) ? g.w : i;
@@ -69,7 +73,7 @@ __device__ __forceinline__ void walk_list(uint32_t i, uint32_t m, const uint32_t
   uint32_t j[4], jn[4];
   T f[4];
   group(0, j);
-  group(m > 4 ? 4u : 0u, jn);
+  group(TIGHT || m > 4 ? 4u : 0u, jn);
 #pragma unroll
   for (int v = 0; v < 4; v++) f[v] = load(j[v]);
   for (uint32_t q = 0; q < m; q += 4) {
@@ -77,7 +81,7 @@ __device__ __forceinline__ void walk_list(uint32_t i, uint32_t m, const uint32_t
     uint32_t j2[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) fn[v] = load(jn[v]);
-    group(q + 8 < m ? q + 8 : 0u, j2);
+    group(TIGHT || q + 8 < m ? q + 8 : 0u, j2);
     bool in[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) in[v] = q + v < m;
@@ -88,6 +92,25 @@ __device__ __forceinline__ void walk_list(uint32_t i, uint32_t m, const uint32_t
       jn[v] = j2[v];
       f[v] = fn[v];
     }
+  }
+}
+
+// walk_list without loads ahead: a third fewer registers, and none thrown away at the
+// list's end; the wavefronts that a compute unit then holds hide the loads once there
+// are enough of them (from about 100k particles on; k_density).
+template <class T, class Load, class Use>
+__device__ __forceinline__ void walk_plain(uint32_t i, uint32_t m, const uint32_t* __restrict__ ids, uint32_t kmax,
+                                           Load load, Use use) {
+  for (uint32_t q = 0; q < m; q += 4) {
+    const uint4 g = *reinterpret_cast<const uint4*>(ids + nbr_slot(i, q, kmax));
+    const uint32_t j[4] = {g.x, (q + 1 < m) ? g.y : i, (q + 2 < m) ? g.z : i, (q + 3 < m) ? g.w : i};
+    T f[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) f[v] = load(j[v]);
+    bool in[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) in[v] = q + v < m;
+    use(j, f, in);
   }
 }
 
@@ -130,7 +153,7 @@ __device__ __forceinline__ void walk_uniform(uint32_t i, uint32_t m, uint32_t mw
 
 // The walk of a pass whose expensive terms only count for the nearer neighbours
 // (r < r_e, while the list reaches r_lap): far(j, p, f1, in, e) gets four
-// neighbours' positions p and fields f1 (load1), adds the terms of all of them
+// neighbours' positions p (pos) and fields f1 (load1), adds the terms of all of them
 // and sets e[v] for the nearer ones; near(p, f2, e) gets those with the fields
 // f2 (load2) and adds their terms, in list order.
 //
@@ -146,9 +169,9 @@ __device__ __forceinline__ void walk_uniform(uint32_t i, uint32_t m, uint32_t mw
 // quarters of the list.
 constexpr uint32_t kNearQueue = 24;
 inline bool near_pays(double re, double rl) { return re * re < 0.75 * rl * rl; }
-template <bool NEAR, int THREADS, class F1, class F2, class Load1, class Load2, class Far, class Near>
+template <bool NEAR, int THREADS, class F1, class F2, class Pos, class Load1, class Load2, class Far, class Near>
 __device__ __forceinline__ void walk_near(uint32_t i, uint32_t m, const uint32_t* __restrict__ ids, uint32_t kmax,
-                                          const double2* __restrict__ xz, uint32_t (*queue)[THREADS], Load1 load1,
+                                          Pos pos, uint32_t (*queue)[THREADS], Load1 load1,
                                           Load2 load2, Far far, Near near) {
   if (m == 0) return;
   auto group = [&](uint32_t q, uint32_t j[4]) {
@@ -166,7 +189,7 @@ __device__ __forceinline__ void walk_near(uint32_t i, uint32_t m, const uint32_t
   group(m > 4 ? 4u : 0u, jn);
 #pragma unroll
   for (int v = 0; v < 4; v++) {
-    p[v] = xz[j[v]];
+    p[v] = pos(j[v]);
     f[v] = load1(j[v]);
     if (!NEAR) g[v] = load2(j[v]);
   }
@@ -177,7 +200,7 @@ __device__ __forceinline__ void walk_near(uint32_t i, uint32_t m, const uint32_t
       uint32_t j2[4];
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        pn[v] = xz[jn[v]];
+        pn[v] = pos(jn[v]);
         fn[v] = load1(jn[v]);
         if (!NEAR) gn[v] = load2(jn[v]);
       }
@@ -213,7 +236,7 @@ __device__ __forceinline__ void walk_near(uint32_t i, uint32_t m, const uint32_t
         for (int v = 0; v < 4; v++) {
           e[v] = k + v < found;
           const uint32_t jk = e[v] ? queue[k + v < kNearQueue ? k + v : 0u][threadIdx.x] : i;
-          pk[v] = xz[jk];
+          pk[v] = pos(jk);
           gk[v] = load2(jk);
         }
         near(pk, gk, e);

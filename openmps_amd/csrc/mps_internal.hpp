@@ -515,10 +515,12 @@ void caller_order(Context& c, bool out, double* const* dev, void* const* host, v
 
 // ---- stage entry points (defined in the .hip units) ------------------------------
 void search(Context& c);                 // mps_search.hip
-void density(Context& c, bool ecs, bool savex, bool dens);  // mps_particles.hip
+// mps_particles.hip: number densities, or (ecs) the error correction; SaveX
+void density(Context& c, bool ecs);
+void save_x(Context& c);
 void density_variation(Context& c, double* out_dev);
 void explicit_forces(Context& c);
-// density(c, true, false, true) followed by explicit_forces(c), the two list
+// the density and error-correction passes followed by explicit_forces(c), the list
 // walks fused into one kernel (same results)
 void density_and_explicit(Context& c);
 void explicit_update(Context& c);  // wall targets and the integration of the explicit stage
@@ -529,7 +531,7 @@ void pressure_gradient(Context& c, bool packed);
 void dynamic_stabilize(Context& c, bool packed);
 void ppe_assemble(Context& c);           // mps_ppe.hip
 void pack_state(Context& c);             // mps_particles.hip: xz, uw from x, z, u, w
-// density(c, false, true, true) followed by ppe_assemble(c), the density walk
+// the density pass and save_x(c) followed by ppe_assemble(c), the density walk
 // and the PPE count walk fused into one kernel (same results)
 void density_save_and_assemble(Context& c);
 void ppe_make_fp32(Context& c);

@@ -51,80 +51,120 @@ __device__ __forceinline__ size_t thread_particle() {
   return blk * static_cast<size_t>(blockDim.x) + threadIdx.x;
 }
 
-// ComputeNeighborDensities (Computer.hpp:780-833), fused with
-// NeighborDensityVariationSpeed + ComputeErrorCorrection (:838-910) and with
-// SaveX (:1025-1039) as the template flags ask.
-template <bool DENS, bool ECS, bool SAVEX>
+// SaveX (Computer.hpp:1025-1039).
+__global__ void __launch_bounds__(kBlock) k_save_x(size_t n, const double* __restrict__ x,
+                                                   const double* __restrict__ z, const uint8_t* __restrict__ type,
+                                                   double* __restrict__ ox, double* __restrict__ oz) {
+  const size_t i = thread_particle();
+  if (i >= n || type[i] == kDummy || type[i] == kDisabled) return;
+  ox[i] = x[i];
+  oz[i] = z[i];
+}
+
+// ComputeNeighborDensities (Computer.hpp:780-833), or ECS:
+// NeighborDensityVariationSpeed + ComputeErrorCorrection (:838-910).
+//
+// Bound by the gathers, in small scenes by a wavefront's own chain; WALK is the
+// fastest of three (density and error correction pass, us at 2.1k / 36k / 133k / 1.00M
+// particles in cell order, radii 2.1 / 3.1):
+//   kNear (walk_near)  10.0 10.8 17.9 83   10.5 11.1 19.4  99
+//   kAhead (walk_list) 11.5 12.1 19.0 90   12.0 13.0 22.5 121
+//   kPlain             12.6 12.9 18.7 80   14.0 14.3 22.7 109
+// and 36k / 1.00M at 2.4 / 2.4, where nearly every neighbour is near: kAhead 9.2 57 and
+// 10.1 72, kPlain 9.9 54 and 10.8 71.  In a shuffled order, 133k / 1.00M, the positions
+// kNear gathers again cost the density pass more than it saves (81 1518, kPlain
+// 64 1123), not the error correction (113 1950, 114 1992).
+enum Walk { kPlain, kAhead, kNear };
+template <bool ECS, int WALK>
 __global__ void __launch_bounds__(kBlock) k_density(size_t n, const double* __restrict__ x,
                                                     const double* __restrict__ z,
                                                     const double* __restrict__ u,
                                                     const double* __restrict__ w,
                                                     const uint8_t* __restrict__ type, NV nb, Consts k,
                                                     double* __restrict__ nd, double* __restrict__ nws,
-                                                    double* __restrict__ ecs, double* __restrict__ ox,
-                                                    double* __restrict__ oz) {
+                                                    double* __restrict__ ecs) {
   const size_t i = thread_particle();
   if (i >= n) return;
   const uint8_t ti = type[i];
-  const bool alive = (ti != kDummy) && (ti != kDisabled);
-  const double xi = x[i], zi = z[i];
-  if (SAVEX && alive) {
-    ox[i] = xi;
-    oz[i] = zi;
-  }
-  if (!alive) {
-    if (DENS) nws[i] = k.n0;
+  if (ti == kDummy || ti == kDisabled) {
+    if (!ECS) nws[i] = k.n0;
     return;
   }
+  const double xi = x[i], zi = z[i];
   double ui = 0, wi = 0;
   if (ECS) {
     ui = u[i];
     wi = w[i];
   }
-  double s = 0.0, h = 0.0;
-  struct F {
-    double x, z, u, w;
-  };
-  walk_list<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
-               [&](uint32_t j) {
-                 F f{x[j], z[j], 0.0, 0.0};
-                 if (ECS) {
-                   f.u = u[j];
-                   f.w = w[j];
-                 }
-                 return f;
-               },
-               [&](const uint32_t*, const F* f, const bool* in) {
-                 double wg[4], hs[4];
-                 bool e[4];
+  double s = 0.0;
+  const uint32_t self = static_cast<uint32_t>(i), m = nb.count[i];
+  if constexpr (WALK == kNear) {
+    struct None {};
+    __shared__ uint32_t queue[kNearQueue][kBlock];
+    walk_near<true, kBlock, None, double2>(
+        self, m, nb.ids, nb.kmax, [&](uint32_t j) { return make_double2(x[j], z[j]); }, queue,
+        [&](uint32_t) { return None{}; },
+        [&](uint32_t j) { return ECS ? make_double2(u[j], w[j]) : make_double2(0.0, 0.0); },
+        [&](const uint32_t*, const double2* q, const None*, const bool* in, bool* e) {
 #pragma unroll
-                 for (int v = 0; v < 4; v++) {
-                   const double dx = f[v].x - xi, dz = f[v].z - zi;
-                   const double r2 = dx * dx + dz * dz;
-                   e[v] = in[v] && r2 < k.re2;
-                   const double r = sqrt(r2);
-                   wg[v] = weight(r, k.re);
-                   hs[v] = (dx * (f[v].u - ui) + dz * (f[v].w - wi)) / (r * r * r);
-                 }
+          for (int v = 0; v < 4; v++) {
+            const double dx = q[v].x - xi, dz = q[v].y - zi;
+            e[v] = in[v] && dx * dx + dz * dz < k.re2;
+          }
+        },
+        [&](const double2* q, const double2* f, const bool* e) {
+          double t[4];
 #pragma unroll
-                 for (int v = 0; v < 4; v++) {
-                   if (DENS) s = e[v] ? s + wg[v] : s;
-                   if (ECS) h = e[v] ? h + hs[v] : h;
-                 }
-               });
-  double thisNws, thisN;
-  if (DENS) {
-    thisNws = s;
-    thisN = (s < k.n0) ? k.n0 : s;  // std::max(thisN, n0)
-    nws[i] = thisNws;
-    nd[i] = thisN;
+          for (int v = 0; v < 4; v++) {
+            const double dx = q[v].x - xi, dz = q[v].y - zi, r = sqrt(dx * dx + dz * dz);
+            t[v] = ECS ? (dx * (f[v].x - ui) + dz * (f[v].y - wi)) / (r * r * r) : weight(r, k.re);
+          }
+#pragma unroll
+          for (int v = 0; v < 4; v++) s = e[v] ? s + t[v] : s;
+        });
   } else {
-    thisNws = nws[i];
-    thisN = nd[i];
+    struct F {
+      double x, z, u, w;
+    };
+    auto load = [&](uint32_t j) {
+      F f{x[j], z[j], 0.0, 0.0};
+      if (ECS) {
+        f.u = u[j];
+        f.w = w[j];
+      }
+      return f;
+    };
+    auto use = [&](const uint32_t*, const F* f, const bool* in) {
+      double r2[4], t[4];
+      bool e[4];
+      auto radius = [&](int v) {
+        const double dx = f[v].x - xi, dz = f[v].z - zi;
+        r2[v] = dx * dx + dz * dz;
+        e[v] = in[v] && r2[v] < k.re2;
+      };
+      if constexpr (WALK == kPlain) {  // (all or none of a wavefront's lanes have one near, often enough)
+#pragma unroll
+        for (int v = 0; v < 4; v++) radius(v);
+        if (!(e[0] || e[1] || e[2] || e[3])) return;
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        if constexpr (WALK != kPlain) radius(v);
+        const double dx = f[v].x - xi, dz = f[v].z - zi, r = sqrt(r2[v]);
+        t[v] = ECS ? (dx * (f[v].u - ui) + dz * (f[v].w - wi)) / (r * r * r) : weight(r, k.re);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; v++) s = e[v] ? s + t[v] : s;
+    };
+    if constexpr (WALK == kAhead) walk_list<F>(self, m, nb.ids, nb.kmax, load, use);
+    else walk_plain<F>(self, m, nb.ids, nb.kmax, load, use);
   }
-  if (ECS) {
-    const double speed = (thisNws < k.n0) ? 0.0 : -k.re * h;
-    const double e = (thisN - k.n0) / k.n0;
+  if (!ECS) {
+    nws[i] = s;
+    nd[i] = (s < k.n0) ? k.n0 : s;  // std::max(thisN, n0)
+  } else {
+    const double speed = (nws[i] < k.n0) ? 0.0 : -k.re * s;
+    const double e = (nd[i] - k.n0) / k.n0;
     ecs[i] = fabs(e) * speed + fabs(speed) * e;
   }
 }
@@ -155,7 +195,8 @@ __global__ void __launch_bounds__(kBlock) k_hs(size_t n, const double* __restric
 }
 
 // ComputeExplicitForces first pass (Computer.hpp:928-987): HL viscosity over
-// non-dummy neighbours, the SPP ghost term, plus gravity.
+// non-dummy neighbours, the SPP ghost term, plus gravity.  (walk_list holds 140
+// registers: 1.00M particles 165 us, 155 this way; 2.1k 16.6, 16.8.)
 __global__ void __launch_bounds__(kBlock) k_explicit(size_t n, const double* __restrict__ x,
                                                      const double* __restrict__ z,
                                                      const double* __restrict__ u,
@@ -172,7 +213,7 @@ __global__ void __launch_bounds__(kBlock) k_explicit(size_t n, const double* __r
     double x, z, u, w;
     uint8_t t;
   };
-  walk_list<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
+  walk_plain<F>(static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax,
                [&](uint32_t j) { return F{x[j], z[j], u[j], w[j], type[j]}; },
                [&](const uint32_t*, const F* f, const bool* in) {
                  double tx[4], tz[4], cx[4], cz[4];
@@ -383,7 +424,8 @@ __global__ void __launch_bounds__(kBlock) k_gradient(size_t n, const double2* __
   };
   __shared__ uint32_t queue[NEAR ? kNearQueue : 1][kBlock];
   walk_near<NEAR, kBlock, None, F>(
-      static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax, xz, queue, [&](uint32_t) { return None{}; },
+      static_cast<uint32_t>(i), nb.count[i], nb.ids, nb.kmax, [&](uint32_t j) { return xz[j]; }, queue,
+      [&](uint32_t) { return None{}; },
       [&](uint32_t j) { return F{p[j], type[j]}; },
       [&](const uint32_t*, const double2* q, const None*, const bool* in, bool* e) {
 #pragma unroll
@@ -578,26 +620,27 @@ NV nview(const Context& c) { return NV{c.nbr, c.ncount, c.kstride}; }
 
 }  // namespace
 
-void density(Context& c, bool ecs, bool savex, bool dens) {
+void density(Context& c, bool ecs) {
   const size_t n = c.n;
   if (n == 0) return;
   const Consts k = consts(c);
-  const NV nb = nview(c);
-  const double bytes = n * (16.0 + 1 + 4) + 4.0 * c.nbr_total + (ecs ? 16.0 * n + 8.0 * n : 0) +
-                       (dens ? 16.0 * n : 16.0 * n) + (savex ? 16.0 * n : 0);
-  const int kid = savex ? MPS_K_DENSITY_SAVE : MPS_K_DENSITY_ECS;
-  tracked(c, kid, bytes, [&] {
-    const dim3 g(grid_for(n)), b(kBlock);
-#define MPS_DENS(D, E, S)                                                                         \
-  hipLaunchKernelGGL((k_density<D, E, S>), g, b, 0, c.stream, n, c.x, c.z, c.u, c.w,              \
-                     static_cast<const uint8_t*>(c.type), nb, k, c.nd, c.nws, c.ecs, c.ox, c.oz)
-    if (dens && ecs && !savex) MPS_DENS(true, true, false);
-    else if (dens && !ecs && savex) MPS_DENS(true, false, true);
-    else if (dens && !ecs && !savex) MPS_DENS(true, false, false);
-    else if (!dens && ecs && !savex) MPS_DENS(false, true, false);
-    else if (!dens && !ecs && savex) MPS_DENS(false, false, true);
-    else MPS_DENS(true, true, true);
-#undef MPS_DENS
+  const bool pays = near_pays(k.re, k.rl);
+  const Walk walk = pays && (ecs || (c.lists_ascending && n <= 400000)) ? kNear : n <= 100000 ? kAhead : kPlain;
+  auto kernel = ecs ? (walk == kNear ? k_density<true, kNear> : walk == kAhead ? k_density<true, kAhead> : k_density<true, kPlain>)
+                    : (walk == kNear ? k_density<false, kNear> : walk == kAhead ? k_density<false, kAhead> : k_density<false, kPlain>);
+  tracked(c, MPS_K_DENSITY_ECS, n * (16.0 + 1 + 4 + 16) + 4.0 * c.nbr_total + (ecs ? 16.0 * n + 8.0 * n : 0), [&] {
+    hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, c.x, c.z, c.u, c.w,
+                       static_cast<const uint8_t*>(c.type), nview(c), k, c.nd, c.nws, c.ecs);
+  });
+  check_launch();
+}
+
+void save_x(Context& c) {
+  const size_t n = c.n;
+  if (n == 0) return;
+  tracked(c, MPS_K_DENSITY_SAVE, n * 33.0, [&] {
+    hipLaunchKernelGGL(k_save_x, dim3(grid_for(n)), dim3(kBlock), 0, c.stream, n, static_cast<const double*>(c.x),
+                       static_cast<const double*>(c.z), static_cast<const uint8_t*>(c.type), c.ox, c.oz);
   });
   check_launch();
 }
