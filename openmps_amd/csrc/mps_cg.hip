@@ -2927,7 +2927,6 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
   }
   const float ghost = in ? A.ghost[i] : 0.0f;
   double x = in ? A.x[i] : 0.0;
-  if (in) A.x0[i] = x;  // as in k_cg_resident
   if (in) agent_store(A.z + i, 0.0f);  // rows outside every cell keep z = 0
 
   // ---- cells ----
@@ -2980,6 +2979,8 @@ __global__ void __launch_bounds__(NT, WAVES) k_mixed_resident(MixedArgs A) {
           __builtin_bit_cast(_Float16, static_cast<uint16_t>((h[e >> 1] >> (16 * (e & 1))) & 0xffffu)));
     out[8] = static_cast<float>(__builtin_bit_cast(_Float16, q9c[u]));
   };
+
+  if (in) A.x0[i] = x;  // as in k_cg_resident (here neither its load nor its store is waited for)
 
   // ---- the cycle's levels from l0 on, in every workgroup's LDS ----
   const AmgGrid& g = A.g;
