@@ -4504,9 +4504,9 @@ constexpr uint32_t kResLevelBytes = 96 * 1024;
 // false: the launched solve has to run (nothing was solved).  Which scenes:
 // no cell with more particles than its wavefront's registers, columns within
 // 16-bit offsets, one row a thread, at most 512 workgroups (kResSlots), two a
-// compute unit.
+// compute unit.  b_iter: the bytes accounted for an iteration.
 template <bool AMG>
-bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
+bool resident_mixed(Context& c, const StopRule& sr, long long max_iter, double b_iter) {
   const size_t n = c.ppe_n;
   const Launch L = cg_grid(n);
   const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
@@ -4612,6 +4612,9 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter) {
   MixedResult r;
   std::memcpy(&r, reinterpret_cast<const char*>(c.res_host) + offsetof(ResidentCtl, out), sizeof r);
   for (int k = 0; k < Context::kSweepPred; k++) c.pred(k) = r.pred[k];
+  // as the launched kernels account for it: residuals, sweep starts, iterations
+  add_bytes(c, MPS_K_CG_SPMV32,
+            (r.outer + 1 - A.have_r) * spmv_bytes(c, 8, 8.0 + 8 + 8) + r.outer * (n * 25.0) + r.total * b_iter);
   if (r.stalled && !r.done && r.rr == r.rr && r.total < A.total_cap) {
     refine_fallback(c, sr, r.rr0, r.rr, r.total, r.outer);  // (the solve ends with it)
   } else {
@@ -4630,7 +4633,13 @@ void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max
   if (!join_ml_setup(c)) ml_setup(c);  // enqueued ahead on the auxiliary stream, or now
   block_list_length(c);
   pack_slots(c, false);
-  if (resident_mixed<false>(c, sr, max_iter)) return;
+  const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
+  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
+  // per particle: r (read, written), q, z; per slot of the packed layout: id
+  // and Jacobi factor; per lane: the aggregate scales
+  const double b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
+  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
+  if (resident_mixed<false>(c, sr, max_iter, b_spmv + b_prec)) return;
   const MlGeom g = ml_geom(c);
   const size_t stride = c.part_ml_cap;
   const CellGrid G = ml_grid(c, g);
@@ -4641,18 +4650,12 @@ void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max
   check_launch();
   double* p_pq = c.part3b;
   const long long limit = inner_limit(c, max_iter);
-  const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
-  const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
-  // per particle: r (read, written), q, z; per slot of the packed layout: id
-  // and Jacobi factor; per lane: the aggregate scales
-  const double b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
   auto prec = [&](double norm, long long it) {
     const PrecArgs a{G,      c.ml_list, nact,   c.ml_pid, c.ml_dv, c.ml_sc,   c.r,       1.0 / norm,
                      c.r32,  c.d32,     c.q32,  c.dinv32, zval,    4u,        p_pq,      L.grid,
                      c.part_ml, stride, c.st32};
     hipLaunchKernelGGL(k_ml_prec<0>, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, a, it);
   };
-  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
   c.replay_ready = MPS_K_CG_SPMV32;
   refine(c, sr, [&](double norm, double sweep_tol) {
     MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
@@ -4700,15 +4703,6 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   }
   block_list_length(c);
   pack_slots(c, true);
-  if (resident_mixed<true>(c, sr, max_iter)) return;
-  const size_t stride = c.part_ml_cap;
-  const CellGrid G = ml_grid(c, g);
-  hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
-                     c.zrec, c.r32, c.d32);
-  c.rec_ready = true;
-  check_launch();
-  double* p_pq = c.part3b;
-  const long long limit = inner_limit(c, max_iter);
   const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
   const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
   // per pass over the particles (k_ml_prec<1>, then k_ml_prec<2>): r, q or z
@@ -4719,6 +4713,16 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   const double b_pass = n * 30.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 8);
   const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
   const double b_cycle = static_cast<double>(c.amg_pts) * 2 * (36 + 16) + npts0 * 19.0 * 4;
+  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
+  if (resident_mixed<true>(c, sr, max_iter, b_spmv + 2 * b_pass + b_cycle)) return;
+  const size_t stride = c.part_ml_cap;
+  const CellGrid G = ml_grid(c, g);
+  hipLaunchKernelGGL(k_rec_init, dim3(grid_for(n)), dim3(256), 0, c.stream, n, static_cast<const uint2*>(c.qpos),
+                     c.zrec, c.r32, c.d32);
+  c.rec_ready = true;
+  check_launch();
+  double* p_pq = c.part3b;
+  const long long limit = inner_limit(c, max_iter);
   const size_t tq_stride = c.amg_tq_stride;
   // it == 0 (the sweep's start) is accounted as a whole by the caller
   auto prec = [&](double norm, long long it) {
@@ -4751,7 +4755,6 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
         hipLaunchKernelGGL(k_ml_prec<2>, dim3(static_cast<unsigned>(pgrid)), dim3(NTP), 0, c.stream, a, it);
     });
   };
-  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
   c.replay_ready = MPS_K_CG_SPMV32;
   refine(c, sr, [&](double norm, double sweep_tol) {
     MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));

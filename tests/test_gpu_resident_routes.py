@@ -1,7 +1,5 @@
 """Which systems the resident solvers take: both sides of each line, counted,
 and the solution checked on either."""
-import ctypes
-
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -9,7 +7,8 @@ import scipy.sparse as sp
 import cases
 from openmps_amd import _lib as L
 from test_gpu_resident import EPS
-from test_gpu_resident_giveup import counts, solved
+from test_gpu_resident_giveup import counts, drill, solved
+from test_gpu_resident_mixed import make, scene
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +41,30 @@ def test_long_rows(n, m, resident):
     print(f"  {n} rows, the longest of {m}: (ended, given up) {how}", flush=True)
     assert how == ((1, 0) if resident else (0, 1))
     assert np.linalg.norm(b - A @ x) <= 1.01 * EPS * r0 + 1e-12 * np.linalg.norm(b)  # (as test_gpu_resident.py)
+
+
+@pytest.mark.parametrize("profiling", [False, True])
+@pytest.mark.parametrize("prec", ["ml", "amg"])
+@pytest.mark.parametrize("cols,rows", [(20, 40), (127, 253)])
+def test_bytes_of_a_resident_refinement(prec, cols, rows, profiling):
+    """The kernel statistics account for a resident refinement, one launch, the
+    bytes that they account for the launched kernels of the same solve (given up
+    at its first exchange, then launched)."""
+    kernels = ("cg_spmv32", "ml_prec", "amg_cycle", "cg_init32", "ir_residual")
+
+    def step(**kw):
+        c = make(scene(cols, rows, 2.1, 3.1, False), prec)
+        drill(c, **kw)
+        c.set_profiling(profiling)
+        c.reset_kernel_stats()
+        was = counts()
+        c.forward_time(1e-4)
+        k = c.kernel_stats()
+        return sum(k[name]["bytes"] for name in kernels), k["cg_spmv32"]["launches"], solved(was)
+
+    own, launches, how = step()
+    assert how == (1, 0) and launches == 1
+    launched, launches, how = step(exchange=0)
+    print(f"  {prec}: {own:.6e} bytes, launched {launched:.6e}", flush=True)
+    assert how == (0, 1) and launches > 1
+    assert own == pytest.approx(launched, rel=1e-12)
