@@ -559,7 +559,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 
 // need the diagonal first, read values and offsets back (344 MB more fetched at
 // 1.05M particles, from the last-level cache); a
 // column's direction follows from the difference of the two cells' indices (they
-// are neighbours; the grid has a border, so dz + gnz dx is unique); the direction
+// are neighbours, and with three rows of cells dz + gnz dx is unique); the direction
 // sums are collected in LDS and stored together (72 bytes a row, one after the
 // other, touched 72 lines a store).
 // Every store is within the slice's `width` slots: a row's entries were counted
@@ -924,7 +924,9 @@ void ppe_finish(Context& c, const PpeConsts& k) {
     // only lists of particles in cell order ascend; those of a kept storage order
     // need k_ppe_fill's merge (in cell order it is never the faster: 253 vs 187 us
     // at 1.05M particles, 47.6 vs 47.5 us at 131k, 18 vs 15 us at 2k)
-    if (c.lists_ascending) {
+    // (and it tells neighbouring cells apart by the difference of their numbers, which
+    // takes three rows of cells: a domain of no height has two)
+    if (c.lists_ascending && c.gnz >= 3) {
       hipLaunchKernelGGL(want9 ? k_ppe_fill_cells<true> : k_ppe_fill_cells<false>, dim3(grid_for(n)), dim3(kBlock), 0,
                          c.stream, n, c.x, c.z, static_cast<const uint8_t*>(c.type), nb, k,
                          static_cast<const uint64_t*>(c.slice_off), static_cast<const uint32_t*>(c.slice_width), c.sval,

@@ -105,6 +105,38 @@ def test_fill_in_cell_and_kept_order(n, precond):
         assert np.array_equal(a, b, equal_nan=a.dtype.kind == "f")
 
 
+@pytest.mark.parametrize("height", [0.0, 0.5])
+@pytest.mark.parametrize("precond", [L.PRECOND_MULTILEVEL, L.PRECOND_AMG])
+def test_fill_in_a_flat_domain(precond, height):
+    """A domain of no height has two rows of cells and no border above them: the
+    difference of two cells' numbers does not tell which neighbours they are.
+    Cell order against the kept order, as above."""
+    rng = np.random.Generator(np.random.PCG64(5))
+    nl = cases.make("gpu", cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, 2.1, L0, 0, 0, 1, 1, 3.1), 1e-9).env()["neighbor_length"]
+    n, w = 420, 6
+    env = cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, 2.1, L0, 0.0, 0.0, n // w * L0, height * nl, 3.1)
+    at = np.arange(n)
+    parts = dict(x=(at // w + 0.5 + rng.uniform(-0.2, 0.2, n)) * L0, z=(at % w + 0.5 + rng.uniform(-0.2, 0.2, n)) * L0,
+                 u=rng.standard_normal(n) * 1e-2, w=rng.standard_normal(n) * 1e-2, p=rng.uniform(0, 100, n), n=np.zeros(n),
+                 type=np.zeros(n, np.uint8))
+    order = np.lexsort((at, np.floor(parts["z"] / nl), np.floor(parts["x"] / nl)))
+    parts = {k: v[order] for k, v in parts.items()}
+    out = []
+    for keep in (False, True):
+        c = cases.make("gpu", env, 1e-9)
+        c.set_storage_order(keep=keep)
+        assert c.grid()["nz"] == 2 + (height > 0)
+        c.set_solver(kind=L.SOLVER_MIXED_IR, stop_rule=L.STOP_RHS_NORM, precond=precond, tol=1e-9)
+        c.add_particles(parts)
+        c.set_time(1e-4, 1e-4)
+        for st in ("search", "density", "error_correction", "explicit", "density", "save_x", "ppe_assemble", "ppe_solve"):
+            c.stage(st)
+        out.append((c.neighbors()[0], *c.ppe(), c.aux("ppe_x"), np.array(c.solve_stats()["iterations"])))
+    print(f"  {out[0][0].max()} neighbours at most, iterations {out[0][-1]} and {out[1][-1]}", flush=True)
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("nx,nz", [(1, 1), (40, 50), (61, 125), (62, 126), (128, 129), (181, 182)])
 def test_cell_counts(nx, nz):
     """Grids around the size at which the scan of the cell counts goes from one
