@@ -278,6 +278,8 @@ void upload_caller_order(Context& c, const void* host, void* dev, size_t elem) {
 
 void ensure_ppe_vectors(Context& c, size_t n) {
   if (n <= c.ppe_alloc && c.r) return;
+  c.ppe_alloc = 0;
+  c.have_ppe = false;
   const size_t m = (n + 63) / 64 * 64 + 64;
   const size_t ns = m / 64 + 1;
   dfree(c.row_len); dfree(c.slice_width); dfree(c.slice_off); dfree(c.diag); dfree(c.diag32);

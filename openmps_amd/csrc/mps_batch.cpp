@@ -158,6 +158,7 @@ void batch_forward(mps_batch& b, double dt_fixed, double* dt_out) {
     rows += c.n;
   }
   if (rows > b.feats_cap) {
+    b.feats_cap = 0;
     give_back_features(b);
     dfree(b.feats);
     dfree(b.ypred);

@@ -4156,6 +4156,7 @@ void solve_mixed_cg(Context& c, const Op& A, double b_base, bool wide, const Sto
 // Multilevel preconditioner: two kernels per iteration (see k_ml_prec).
 void ensure_zrec(Context& c, size_t n) {
   if (c.zrec_cap < n) {
+    c.zrec_cap = 0;
     dfree(c.zrec);
     c.zrec = dalloc<uint4>(n);
     c.zrec_cap = n;
@@ -4212,6 +4213,7 @@ CellGrid ml_grid(const Context& c, const MlGeom& g) {
 void enqueue_block_list(Context& c, bool copy) {
   const MlGeom g = ml_geom(c);
   if (c.ml_blk_cap < g.nblk) {
+    c.ml_blk_cap = 0;
     dfree(c.ml_flag);
     dfree(c.ml_off);
     dfree(c.ml_list);
@@ -4254,11 +4256,13 @@ void ml_setup(Context& c) {
                      static_cast<const double*>(c.diag), c.dinv32);
   const MlGeom g = ml_geom(c);
   if (c.agg_cap < g.total_aggs) {
+    c.agg_cap = 0;
     dfree(c.agg_inv);
     c.agg_inv = dalloc<float>(g.total_aggs);
     c.agg_cap = g.total_aggs;
   }
   if (c.part_ml_cap < g.sgrid) {
+    c.part_ml_cap = 0;
     dfree(c.part_ml);
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
@@ -4287,6 +4291,7 @@ void ensure_q9(Context& c, size_t nslots) {
   const size_t m = std::max<size_t>(nslots, 64);
   const size_t words = m + (m + 7) / 8;  // uint4 words: the rows, then the ninth coefficients
   if (c.amg_q9_cap < words) {
+    c.amg_q9_cap = 0;
     dfree(c.amg_q9);
     c.amg_q9 = dalloc<uint4>(words);
     c.amg_q9_cap = words;
@@ -4349,6 +4354,7 @@ void amg_setup(Context& c) {
   c.amg_levels = lv;
   c.amg_pts = off;
   if (c.amg_cap < off) {
+    c.amg_cap = 0;
     dfree(c.amg_S64);
     dfree(c.amg_S);
     dfree(c.amg_dinv);
@@ -4404,6 +4410,7 @@ void pack_slots(Context& c, bool amg) {
   const size_t pgrid = std::max<size_t>(1, (nact + NTP / 64 - 1) / (NTP / 64));
   const size_t slots = static_cast<size_t>(std::max<uint32_t>(nact, 1)) * 64;
   if (c.ml_pack_cap < slots) {
+    c.ml_pack_cap = 0;
     dfree(c.ml_pid);
     dfree(c.ml_dv);
     dfree(c.ml_sc);
@@ -4438,6 +4445,7 @@ void clear_direction_sums(Context& c) {
   const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
   c.amg_tq_stride = (npts0 + 63) & ~static_cast<size_t>(63);
   if (c.amg_tq_cap < 9 * c.amg_tq_stride) {
+    c.amg_tq_cap = 0;
     dfree(c.amg_tq);
     c.amg_tq = dalloc<float>(9 * c.amg_tq_stride);
     c.amg_tq_cap = 9 * c.amg_tq_stride;
@@ -4697,6 +4705,7 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   clear_direction_sums(c);
   const MlGeom g = ml_geom(c);
   if (c.part_ml_cap < g.sgrid) {
+    c.part_ml_cap = 0;
     dfree(c.part_ml);
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;
@@ -5334,6 +5343,7 @@ int effective_precond(const Context& c) {
 
 void ensure_amg_rows(Context& c, size_t n) {
   if (c.amg_rows_cap < n) {
+    c.amg_rows_cap = 0;
     dfree(c.amg_rows);
     c.amg_rows = dalloc<double>(9 * n);
     c.amg_rows_cap = n;
@@ -5511,6 +5521,7 @@ bool learned_residual32(Context& c, FeatRec* rec) {
   // five partial sums per block
   const int G = static_cast<int>((c.ppe_n + 255) / 256);
   if (c.learn_part_cap < static_cast<size_t>(G)) {
+    c.learn_part_cap = 0;
     dfree(c.learn_part);
     c.learn_part = dalloc<double>(5 * static_cast<size_t>(G));
     c.learn_part_cap = G;
@@ -5575,21 +5586,22 @@ void BatchWork::ensure(size_t scenes) {
   stream = s;
   ev_a = a;
   ev_b = b;
-  cap = std::max<size_t>(scenes, 8);
-  tab = dalloc<unsigned char>(kKinds * cap * kArgBytes);
-  first = dalloc<uint32_t>(kKinds * (cap + 1));
-  st = dalloc<CgStatus>(cap);
+  const size_t most = std::max<size_t>(scenes, 8);
+  tab = dalloc<unsigned char>(kKinds * most * kArgBytes);
+  first = dalloc<uint32_t>(kKinds * (most + 1));
+  st = dalloc<CgStatus>(most);
   void* h = nullptr;
-  MPS_HIP(hipHostMalloc(&h, kKinds * cap * kArgBytes, hipHostMallocDefault));
+  MPS_HIP(hipHostMalloc(&h, kKinds * most * kArgBytes, hipHostMallocDefault));
   tab_host = static_cast<unsigned char*>(h);
-  MPS_HIP(hipHostMalloc(&h, kKinds * (cap + 1) * sizeof(uint32_t), hipHostMallocDefault));
+  MPS_HIP(hipHostMalloc(&h, kKinds * (most + 1) * sizeof(uint32_t), hipHostMallocDefault));
   first_host = static_cast<uint32_t*>(h);
-  MPS_HIP(hipHostMalloc(&h, cap * sizeof(CgStatus), hipHostMallocDefault));
+  MPS_HIP(hipHostMalloc(&h, most * sizeof(CgStatus), hipHostMallocDefault));
   st_host = static_cast<CgStatus*>(h);
-  std::memset(tab_host, 0, kKinds * cap * kArgBytes);
+  std::memset(tab_host, 0, kKinds * most * kArgBytes);
   if (!stream) MPS_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   if (!ev_a) MPS_HIP(hipEventCreate(&ev_a));
   if (!ev_b) MPS_HIP(hipEventCreate(&ev_b));
+  cap = most;
 }
 
 void BatchWork::release() {
@@ -5624,6 +5636,7 @@ void amg_prepare(Context& c) {
   amg_setup(c);
   const MlGeom g = ml_geom(c);
   if (c.part_ml_cap < g.sgrid) {
+    c.part_ml_cap = 0;
     dfree(c.part_ml);
     c.part_ml = dalloc<double>(2 * g.sgrid);
     c.part_ml_cap = g.sgrid;

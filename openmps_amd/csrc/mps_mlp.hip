@@ -822,6 +822,7 @@ size_t Model::param_count(int k) {
 
 void Model::ensure_batch(size_t m) {
   if (m <= cap) return;
+  cap = 0;  // (a size is forgotten before its buffers are: an allocation may fail)
   dfree(xb); dfree(tb); dfree(z1); dfree(z2); dfree(a2); dfree(h1b); dfree(y); dfree(dy);
   dfree(da2b); dfree(dh1); dfree(da1b); dfree(idx);
   xb = dalloc<__bf16>(m * kFeatPad);
@@ -961,6 +962,7 @@ void Model::adam(hipStream_t s, float lr) {
 void Model::pack_host_rows(size_t m, const float* x_host) {
   ensure_batch(m);
   if (m > xf_cap) {
+    xf_cap = 0;
     dfree(xf);
     xf = dalloc<float>(m * kFeat);
     xf_cap = m;
@@ -1035,11 +1037,13 @@ void learned_features(Context& c) {
   if (n == 0) return;
   if (c.feats_borrowed) {  // rows and predictions in a batch's buffers: the records only
     if (!c.feat_rec || c.feats_cap < n) {
+      c.feats_cap = 0;
       dfree(c.feat_rec);
       c.feat_rec = dalloc<FeatRec>(n);
       c.feats_cap = n;
     }
   } else if (!c.feats || c.feats_cap < n) {
+    c.feats_cap = 0;
     dfree(c.feats);
     dfree(c.ypred);
     dfree(c.feat_rec);

@@ -749,6 +749,8 @@ __global__ void __launch_bounds__(kBlock) k_to_f32(size_t n, const double* __res
 
 void ensure_sell_capacity(Context& c, size_t nslices, size_t slots) {
   if (slots > c.sell_cap) {
+    c.sell_cap = 0;
+    c.have_ppe = false;
     dfree(c.sval);
     dfree(c.scol);
     dfree(c.sval32);
@@ -770,10 +772,10 @@ PpeConsts ppe_prepare(Context& c) {
   const size_t n = c.n;
   c.ppe_n = n;
   c.nslices = (n + 63) / 64;
-  c.have_ppe = true;
-  c.have_ppe32 = false;
   // worst case: every row as long as the longest neighbour list
   if (n > 0) ensure_sell_capacity(c, c.nslices, c.nslices * 64 * static_cast<size_t>(c.kmax));
+  c.have_ppe = true;
+  c.have_ppe32 = false;
   const double extent = std::max(c.env.max_x - c.env.min_x, c.env.max_z - c.env.min_z);
   c.qpos_inv_h = (extent > 0) ? 1073741824.0 / extent : 1.0 / c.env.l0;
   PpeConsts k{c.env.r_e, c.env.r_e * c.env.r_e, c.env.r_lap, c.env.r_lap * c.env.r_lap, c.env.n0,

@@ -41,3 +41,24 @@ def test_gradients_row_counts(rows):
             err = np.linalg.norm(g[k] - want[k]) / np.linalg.norm(dy) / max(1.0, np.linalg.norm(want[k]) / np.linalg.norm(dy))
             print(f"  {rows} rows, {k}: {err:.1e}", flush=True)
             assert err <= 1e-3, (k, err)
+
+
+def test_rows_that_no_memory_holds():
+    """A call whose buffers cannot be allocated (2^40 rows; nothing is read)
+    fails, and the next calls work: fewer rows than before it, and more."""
+    from openmps_amd import _lib as L
+    from openmps_amd.learned import Model
+    m = Model(0)
+    m.set_params(random_params(5))
+    rng = np.random.Generator(np.random.PCG64(1))
+    x = rng.normal(size=(600, FEAT)).astype(np.float32)
+    t = rng.normal(size=600).astype(np.float32)
+    y, (loss, g) = m.forward(x[:300]), m.gradients(x[:300], t[:300])
+    few = np.zeros(4, np.float32)
+    assert L.lib().mps_model_forward(m._h, 1 << 40, few.ctypes.data, few.ctypes.data) == L.MPS_ERR_HIP
+    assert np.array_equal(m.forward(x[:300]), y) and np.array_equal(m.forward(x[:200]), y[:200])
+    loss2, g2 = m.gradients(x[:300], t[:300])
+    assert abs(loss2 - loss) <= 1e-5 * loss  # (its atomics add in any order)
+    for k in g:
+        assert np.linalg.norm(g2[k] - g[k]) <= 1e-5 * np.linalg.norm(g[k])
+    assert np.array_equal(m.forward(x)[:300], y)
