@@ -1,14 +1,14 @@
 """Which systems the resident solvers take: both sides of each line, counted,
-and the solution checked on either."""
+the solution checked on either, and the same bits from the launched kernels."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
 
 import cases
 from openmps_amd import _lib as L
-from test_gpu_resident import EPS
+from test_gpu_resident import EPS, SIZES, banded
 from test_gpu_resident_giveup import counts, drill, solved
-from test_gpu_resident_mixed import make, scene
+from test_gpu_resident_mixed import SHAPES, make, scene
 
 pytestmark = pytest.mark.gpu
 
@@ -68,3 +68,54 @@ def test_bytes_of_a_resident_refinement(prec, cols, rows, profiling):
     print(f"  {prec}: {own:.6e} bytes, launched {launched:.6e}", flush=True)
     assert how == (0, 1) and launches > 1
     assert own == pytest.approx(launched, rel=1e-12)
+
+
+def both_ways(make_context, run):
+    """A solve as it comes, and by the launched kernels (given up at its first
+    exchange; a drill has no shape for two workgroups a compute unit)."""
+    out = []
+    for kw in ({}, dict(exchange=0)):
+        c = make_context()
+        drill(c, **kw)
+        was = counts()
+        run(c)
+        st = c.solve_stats()
+        out.append((solved(was), c.aux("ppe_x"), [st[k] for k in ("iterations", "outer_iterations", "rr0", "rr")]))
+    return out
+
+
+# workgroups of 512 rows on the 256 compute units, one or two on each
+ONE, TWO = 131_072, 262_144
+
+
+@pytest.mark.parametrize("n,reach,long_rows,far", SIZES)
+def test_systems_resident_and_launched(n, reach, long_rows, far):
+    """Bit for bit the same, and resident where rows and spans fit (above)."""
+    A, b, x0, _ = banded(n, reach, long_rows, far, n + reach)
+    longest = np.diff(A.indptr).max() - 1
+    first, last = A.indices[A.indptr[:-1]], A.indices[A.indptr[1:] - 1]  # (sorted rows)
+    span = max(last[k:k + 512].max() - first[k:k + 512].min() for k in range(0, n, 512))
+    resident = n <= TWO and span < 65536 and longest <= (82 if n <= ONE else 49)
+
+    def context():
+        c = cases.make("gpu", cases.CG["env"], EPS)
+        c.set_ppe(A.indptr, A.indices, A.data, b, x0)
+        return c
+
+    (how, x, st), (how2, x2, st2) = both_ways(context, lambda c: c.stage("ppe_solve"))
+    print(f"  {n} rows, longest {longest}, span {span}: (ended, given up) {how} and {how2}, {st}", flush=True)
+    assert how == ((1, 0) if resident else (0, 1) if n <= TWO else (0, 0))
+    assert how2 != (1, 0) or n <= 512  # (a single workgroup waits for no other)
+    assert st == st2 and np.array_equal(x, x2)
+
+
+@pytest.mark.parametrize("prec", ["ml", "amg"])
+@pytest.mark.parametrize("cols,rows,r_e,r_lap,still", SHAPES)
+def test_scenes_resident_and_launched(prec, cols, rows, r_e, r_lap, still):
+    """Bit for bit the same; resident up to one workgroup a compute unit (multigrid) or two."""
+    sc = scene(cols, rows, r_e, r_lap, still)
+    (how, x, st), (how2, x2, st2) = both_ways(lambda: make(sc, prec), lambda c: c.forward_time(1e-4))
+    print(f"  {prec} {len(x)} particles: (ended, given up) {how} and {how2}, {st}", flush=True)
+    assert how == ((1, 0) if len(x) <= (ONE if prec == "amg" else TWO) else (0, 0))
+    assert how2 != (1, 0) or len(x) <= 512
+    assert st == st2 and np.array_equal(x, x2)
