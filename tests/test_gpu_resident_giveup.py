@@ -191,3 +191,62 @@ def test_x_of_a_refinement_given_up(prec, cols, rows):
     print(f"  {prec}: {st}, launched {st2}", flush=True)
     assert how == (0, 1)
     assert st2 == st and np.array_equal(x, y)
+
+
+def test_start_limit():
+    """Workgroups that do not all start within the limit (none here) leave: the
+    launched kernels solve, from then on for 64 solves, and after those the
+    resident ones try again."""
+    n = 100_000
+    A, b, x0, _ = banded(n, 300, 9, 0, n)
+    c = cases.make("gpu", cases.CG["env"], EPS)
+    c.set_ppe(A.indptr, A.indices, A.data, b, x0)
+
+    def solve():
+        was = counts()
+        c.set_aux("ppe_x", x0)
+        c.stage("ppe_solve")
+        return c.aux("ppe_x"), solved(was)
+
+    x, how = solve()
+    assert how == (1, 0)
+    drill(c, start=0, group=1 << 20)
+    y, how = solve()
+    assert how == (0, 1) and np.array_equal(x, y)
+    for _ in range(64):
+        y, how = solve()
+        assert how == (0, 0) and np.array_equal(x, y)
+    y, how = solve()
+    assert how == (0, 1) and np.array_equal(x, y)
+    drill(c)
+    y, how = solve()
+    assert how == (1, 0) and np.array_equal(x, y)
+
+
+def test_two_threads():
+    """One resident solve at a time: a second thread's solve, while the first one
+    holds back, takes the launched kernels and waits for nothing."""
+    import threading
+    import time
+    n = 100_000
+    A, b, x0, _ = banded(n, 300, 9, 0, n)
+    one, two = (cases.make("gpu", cases.CG["env"], EPS) for _ in range(2))
+    for c in (one, two):
+        c.set_ppe(A.indptr, A.indices, A.data, b, x0)
+        c.stage("ppe_solve")
+        x = c.aux("ppe_x")
+        c.set_aux("ppe_x", x0)
+    drill(one, wait=2000 * MS, hold=300 * MS)
+    was = counts()
+    t = threading.Thread(target=one.stage, args=("ppe_solve",))
+    t.start()
+    time.sleep(0.1)  # (one's kernel runs for 0.3 s at least)
+    t0 = time.perf_counter()
+    two.stage("ppe_solve")
+    took = time.perf_counter() - t0
+    busy = t.is_alive()
+    t.join()
+    print(f"  the second thread's solve took {took * 1e3:.1f} ms, the first one was still running: {busy}", flush=True)
+    assert solved(was) == (1, 0)
+    for c in (one, two):
+        assert np.array_equal(c.aux("ppe_x"), x)
