@@ -4125,7 +4125,7 @@ void solve_mixed_cg(Context& c, const Op& A, double b_base, bool wide, const Sto
   double b_iter = b_base;
   refine(c, sr, [&](double norm, double sweep_tol) {
     // refine() has synchronised the stream (residual) before every sweep
-    if (wide) b_iter = b_base + 2.0 * mf_nnz_wide(c);
+    if (wide) b_iter = b_base + 2.0 * c.mf_nnz_wide;
     MPS_HIP(hipMemsetAsync(c.st32, 0, sizeof(CgStatus), c.stream));
     tracked(c, MPS_K_CG_INIT32, b_iter + n * 8.0, [&] {
       hipLaunchKernelGGL(k_cgf_init<Op>, dim3(L.grid), dim3(NT), 0, c.stream, A,
@@ -4519,7 +4519,7 @@ bool resident_mixed(Context& c, const StopRule& sr, long long max_iter, double b
   const Launch L = cg_grid(n);
   const uint32_t nact = static_cast<uint32_t>(c.counters_host->ml_active);
   const int grid = std::max(L.grid, static_cast<int>((nact + NT / 64 - 1) / (NT / 64)));
-  if (L.rpb != static_cast<size_t>(NT) || c.cap > 4u * kPerLane || mf_nnz_wide(c) > 0 || grid > kResSlots) return false;
+  if (L.rpb != static_cast<size_t>(NT) || c.cap > 4u * kPerLane || c.mf_nnz_wide > 0 || grid > kResSlots) return false;
   if (c.res_skip > 0) {
     c.res_skip--;
     return false;
@@ -4646,7 +4646,7 @@ void solve_mixed_ml(Context& c, double b_base, const StopRule& sr, long long max
   // per particle: r (read, written), q, z; per slot of the packed layout: id
   // and Jacobi factor; per lane: the aggregate scales
   const double b_prec = n * 16.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 16);
-  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
+  const double b_spmv = b_base + 2.0 * c.mf_nnz_wide;
   if (resident_mixed<false>(c, sr, max_iter, b_spmv + b_prec)) return;
   const MlGeom g = ml_geom(c);
   const size_t stride = c.part_ml_cap;
@@ -4722,7 +4722,7 @@ void solve_mixed_amg(Context& c, double b_base, const StopRule& sr, long long ma
   const double b_pass = n * 30.0 + static_cast<double>(nact) * 64 * (8.0 * kPerLane + 8);
   const size_t npts0 = static_cast<size_t>(c.amg_box[2]) * c.amg_box[3];
   const double b_cycle = static_cast<double>(c.amg_pts) * 2 * (36 + 16) + npts0 * 19.0 * 4;
-  const double b_spmv = b_base + 2.0 * mf_nnz_wide(c);
+  const double b_spmv = b_base + 2.0 * c.mf_nnz_wide;
   if (resident_mixed<true>(c, sr, max_iter, b_spmv + 2 * b_pass + b_cycle)) return;
   const size_t stride = c.part_ml_cap;
   const CellGrid G = ml_grid(c, g);

@@ -226,10 +226,8 @@ struct Context {
   uint8_t* slice_wide = nullptr;
   int16_t* col16 = nullptr;  // sell_cap entries, beside scol
   double mf_nnz_wide = 0;
-  bool mf_wide_pending = false;  // mf_nnz_wide still in counters_host
-  // [0] off-diagonal nnz, [1] wide nnz, [2..5] the cell box of the rows with
-  // off-diagonals (gnx - 1 - min x, max x, gnz - 1 - min z, max z: atomic maxima)
-  uint32_t amg_box[4] = {0, 0, 0, 0};  // cells x0, z0, nx, nz of that box (the multigrid's level 0)
+  // cells x0, z0, nx, nz of the box of the rows with off-diagonals (the multigrid's level 0)
+  uint32_t amg_box[4] = {0, 0, 0, 0};
   bool amg_box_ready = false;          // the box belongs to the installed system
   uint4* box_part = nullptr;           // per-block partial boxes
   double nnz_offdiag = 0, sell_slots = 0;
@@ -535,7 +533,6 @@ void pack_state(Context& c);             // mps_particles.hip: xz, uw from x, z,
 // and the PPE count walk fused into one kernel (same results)
 void density_save_and_assemble(Context& c);
 void ppe_make_fp32(Context& c);
-double mf_nnz_wide(Context& c);  // mps_ppe.hip: nnz of the wide slices; valid once the stream was synchronised
 // mps_ppe.hip: the box of cells of the rows with off-diagonals (c.amg_box),
 // computed now (one synchronisation) unless the assembly left it
 void amg_box(Context& c);

@@ -901,7 +901,6 @@ void ppe_finish(Context& c, const PpeConsts& k) {
   c.sell_slots = c.counters_host->slots;
   // the wide slices' stored count (byte accounting only), from the count pass
   c.mf_nnz_wide = static_cast<double>(c.counters_host->nnz_wide);
-  c.mf_wide_pending = false;
   c.amg_box_ready = false;
   if (want_box) amg_box_from_counters(c);
   // row sums of the multilevel preconditioner's aggregates, when that solver will run
@@ -1007,13 +1006,6 @@ void amg_box(Context& c) {
   amg_box_from_counters(c);
 }
 
-double mf_nnz_wide(Context& c) {
-  if (c.mf_wide_pending) {
-    c.mf_nnz_wide = static_cast<double>(c.counters_host->nnz_wide);
-    c.mf_wide_pending = false;
-  }
-  return c.mf_nnz_wide;
-}
 
 // FP32 copies of an already assembled system (the mixed solver on a system
 // installed through mps_set_ppe, or after switching solvers).

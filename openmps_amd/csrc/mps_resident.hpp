@@ -27,8 +27,11 @@
 //
 // Every wait is bounded.  Before the first iteration the workgroups wait until
 // all of them have started (they might not fit beside other work on the GPU)
-// or the time limit has passed; then they all leave without having written
-// anything, and the caller runs the launched kernels instead.
+// or the time limit has passed; then they leave, having written scratch only
+// (the empty marks over p, zeros over z, x's copy).  One that gives up later
+// leaves the others to give up at the exchanges it is missing from, or, at the
+// last one, to finish and store their rows of x.  Either way `abort` is set, and
+// the caller puts x back (restore_x) and runs the launched kernels instead.
 #pragma once
 
 #include <hip/hip_runtime.h>
