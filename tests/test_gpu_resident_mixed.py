@@ -158,3 +158,34 @@ def test_solver_chosen_after_the_search(cols, rows, prec, warm):
         early, late = early[:1], late[:1]
     for (x, it, used), (x2, it2, used2) in zip(early, late):
         assert it == it2 and used == used2 and np.array_equal(x, x2)
+
+
+@pytest.mark.parametrize("prec", ["ml", "amg", "auto"])
+@pytest.mark.parametrize("cols,rows", [(5, 9), (60, 117), (300, 600)])
+def test_solver_chosen_after_the_assembly(cols, rows, prec):
+    """The system assembled under the FP64 solver, which sums no rows for the
+    preconditioners: set-up and block list come with the solve.  The sums are
+    taken in another order, which can move a stop test by one iteration of a
+    sweep (as above)."""
+    def run(late):
+        sc = scene(cols, rows, 2.1, 3.1, False)
+        c = Computer(1e-10, sc[0])
+        c.add_particles(sc[1])
+        opts = dict(kind=L.SOLVER_MIXED_IR, stop_rule=L.STOP_RHS_NORM, tol=TOL, precond=dict(PREC, auto=L.PRECOND_AUTO)[prec])
+        if not late:
+            c.set_solver(**opts)
+        c.set_time(1e-4, 1e-4)
+        for stage in ("search", "density", "error_correction", "explicit", "density", "ppe_assemble"):
+            c.stage(stage)
+        if late:
+            c.set_solver(**opts)
+        c.stage("ppe_solve")
+        A, rhs, x = solved(c)
+        assert np.linalg.norm(rhs - A @ x) <= 1.01 * TOL * np.linalg.norm(rhs)
+        return c.solve_stats()
+
+    a, b = run(False), run(True)
+    print(f"  {prec}: {a['iterations']} iterations in {a['outer_iterations']} sweeps, {b['iterations']} in "
+          f"{b['outer_iterations']}", flush=True)
+    assert a["precond_used"] == b["precond_used"] and a["outer_iterations"] == b["outer_iterations"]
+    assert abs(a["iterations"] - b["iterations"]) <= a["outer_iterations"]
