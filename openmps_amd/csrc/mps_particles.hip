@@ -625,6 +625,7 @@ void density(Context& c, bool ecs) {
   if (n == 0) return;
   const Consts k = consts(c);
   const bool pays = near_pays(k.re, k.rl);
+  // (the lines lie between the sizes of k_density's table at which the faster one changes)
   const Walk walk = pays && (ecs || (c.lists_ascending && n <= 400000)) ? kNear : n <= 100000 ? kAhead : kPlain;
   auto kernel = ecs ? (walk == kNear ? k_density<true, kNear> : walk == kAhead ? k_density<true, kAhead> : k_density<true, kPlain>)
                     : (walk == kNear ? k_density<false, kNear> : walk == kAhead ? k_density<false, kAhead> : k_density<false, kPlain>);

@@ -65,6 +65,32 @@ def test_uneven_neighbourhoods(n, r_e, r_lap):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("n,r_e,r_lap,keep", [(100_000, 2.4, 2.4, False), (100_001, 2.4, 2.4, False), (100_000, 2.1, 3.1, True),
+                                              (100_001, 2.1, 3.1, True), (400_000, 2.1, 3.1, False),
+                                              (400_001, 2.1, 3.1, False)])
+def test_walks_chosen_by_size_and_order(n, r_e, r_lap, keep):
+    """Both sides of the sizes at which the density and error-correction passes
+    change their walk, in cell order and in a kept, random one."""
+    probe = cases.make("gpu", cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, r_e, L0, 0, 0, 1, 1, r_lap), 1e-9)
+    nl = probe.env()["neighbor_length"]
+    side = int(np.ceil(np.sqrt(n) * L0 / nl)) + 1
+    env = cases.env(1e-3, 0.1, 9.8, 998.2, 1e-6, r_e, L0, 0.0, 0.0, side * nl, side * nl, r_lap)
+    rng = np.random.Generator(np.random.PCG64(n))
+    at, w = rng.permutation(n), int(np.ceil(np.sqrt(n)))
+    parts = dict(x=(at // w + 0.5 + rng.uniform(-0.3, 0.3, n)) * L0, z=(at % w + 0.5 + rng.uniform(-0.3, 0.3, n)) * L0,
+                 u=rng.standard_normal(n) * 1e-2, w=rng.standard_normal(n) * 1e-2, p=rng.uniform(0, 100, n), n=np.zeros(n),
+                 type=rng.choice(np.array([0, 0, 0, 0, 1, 2], np.uint8), n))
+    g, o = cases.make("gpu", env, 1e-9), cases.make("oracle", env, 1e-9)
+    g.set_storage_order(keep=keep)
+    for c in (g, o):
+        c.add_particles(parts)
+        c.set_time(1e-4, 1e-4)
+    for st in ("search", "density", "error_correction", "explicit", "save_x"):
+        g.stage(st)
+        o.stage(st)
+        compare_stage(g, o, st)
+
+
 @pytest.mark.parametrize("precond", [None, L.PRECOND_MULTILEVEL, L.PRECOND_AMG])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 257, 3000])
 def test_fill_in_cell_and_kept_order(n, precond):
