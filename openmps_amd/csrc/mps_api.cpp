@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <exception>
 #include <new>
 
@@ -254,7 +255,49 @@ const std::vector<uint32_t>& storage_order(Context& c) {
   return c.orig_host;
 }
 
+// Whether one array of this size is permuted on the host: up to kHostOrder
+// particles, and from the second time that an array moves under a permutation,
+// so that a single read after every search does not pay for the copy of the
+// order.  One array of 225 particles takes 23.4 us out and 17.2 us in on the
+// host, 25.6 and 18.4 us through the kernel; of 2062 11.5 and 11.3 against 24.4
+// and 22.2; of 9104 25.5 and 24.0 against 26.7 and 24.0; of 36119 71 and 65
+// against 35 and 31.
+constexpr size_t kHostOrder = 8192;
+bool permute_on_host(Context& c) {
+  if (c.n == 0 || c.n > kHostOrder || c.order_serial == 0) return false;
+  if (c.order_host_serial == c.order_serial) return true;
+  const bool again = c.order_moved_serial == c.order_serial;
+  c.order_moved_serial = c.order_serial;
+  return again;
+}
+
+template <class T>
+void download_permuted(Context& c, const void* dev, void* host) {
+  const std::vector<uint32_t>& o = storage_order(c);
+  std::vector<T> tmp(c.n);
+  MPS_HIP(hipMemcpyAsync(tmp.data(), dev, c.n * sizeof(T), hipMemcpyDeviceToHost, c.stream));
+  MPS_HIP(hipStreamSynchronize(c.stream));
+  for (size_t k = 0; k < c.n; k++)
+    std::memcpy(static_cast<unsigned char*>(host) + o[k] * sizeof(T), &tmp[k], sizeof(T));
+}
+
+template <class T>
+void upload_permuted(Context& c, const void* host, void* dev) {
+  const std::vector<uint32_t>& o = storage_order(c);
+  std::vector<T> tmp(c.n);
+  for (size_t k = 0; k < c.n; k++)
+    std::memcpy(&tmp[k], static_cast<const unsigned char*>(host) + o[k] * sizeof(T), sizeof(T));
+  MPS_HIP(hipMemcpyAsync(dev, tmp.data(), c.n * sizeof(T), hipMemcpyHostToDevice, c.stream));
+  MPS_HIP(hipStreamSynchronize(c.stream));
+}
+
 void download_caller_order(Context& c, const void* dev, void* host, size_t elem) {
+  if (permute_on_host(c)) {
+    if (elem == 8) download_permuted<uint64_t>(c, dev, host);
+    else if (elem == 4) download_permuted<uint32_t>(c, dev, host);
+    else download_permuted<uint8_t>(c, dev, host);
+    return;
+  }
   double* d[kCallerFields] = {};
   void* h[kCallerFields] = {};
   void* src = const_cast<void*>(dev);
@@ -266,6 +309,12 @@ void download_caller_order(Context& c, const void* dev, void* host, size_t elem)
 }
 
 void upload_caller_order(Context& c, const void* host, void* dev, size_t elem) {
+  if (permute_on_host(c)) {
+    if (elem == 8) upload_permuted<uint64_t>(c, host, dev);
+    else if (elem == 4) upload_permuted<uint32_t>(c, host, dev);
+    else upload_permuted<uint8_t>(c, host, dev);
+    return;
+  }
   double* d[kCallerFields] = {};
   void* h[kCallerFields] = {};
   void* src = const_cast<void*>(host);

@@ -178,6 +178,7 @@ struct Context {
   bool keep_order = false;          // MPS_ORDER_KEEP: the search does not permute
   std::vector<uint32_t> orig_host;  // host copy of orig for order_host_serial
   long long order_host_serial = -1;
+  long long order_moved_serial = -1;  // of the last single array moved through the kernel
   // arrays the permutation writes into, then swapped with the live ones
   static constexpr int kMoved = 14;  // FP64 per-particle arrays the permutation moves
   double* spare_d[kMoved] = {};

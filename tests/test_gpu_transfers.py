@@ -64,3 +64,36 @@ def test_results_in_the_callers_order():
         out.append((cnt, ids, c.particles()["n"], c.density_variation()))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("count", [1, 225, 8192, 8193])
+def test_one_array_again_under_one_permutation(count):
+    """The first and every later transfer of one array under a permutation, on
+    both sides of the size where later ones are permuted on the host, after
+    particles were added and after a new permutation."""
+    print(f"  transfers again: {count} particles", flush=True)
+    env, s, rng = scattered(count, 11 * count)
+    first = (count + 1) // 2
+    c = cases.make("gpu", env, 1e-8)
+    kept = cases.make("gpu", env, 1e-8)
+    kept.set_storage_order(True)
+    for part in (slice(0, first), slice(first, count)):
+        if part.start == part.stop:
+            continue
+        for m in (c, kept):
+            m.add_particles({k: v[part] for k, v in s.items()})
+        for _ in range(2):
+            for m in (c, kept):
+                m.stage("search")
+                m.stage("density")
+            for _ in range(3):
+                assert np.array_equal(c.density_variation(), kept.density_variation())
+                for a, b in zip(c.neighbors(), kept.neighbors()):
+                    assert np.array_equal(a, b)
+                v = rng.standard_normal(part.stop)
+                c.set_aux("ecs", v)
+                assert np.array_equal(c.aux("ecs"), v)
+                assert np.array_equal(c.aux("ecs"), v)
+            got = c.particles()
+            for k in FIELDS[:4] + ("type",):
+                assert np.array_equal(got[k], s[k][:part.stop]), k
